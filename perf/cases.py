@@ -14,6 +14,7 @@ import importlib
 import math
 
 import numpy as np
+import torch
 
 fr = importlib.import_module("faster-rwkv_amd")
 
@@ -145,3 +146,138 @@ def tolerance(case):
     Measured between prompts as one pass and as one-token steps: RWKV-4 up to 3.6e-3 of the logits' norm, the largest
     difference 1.6e-2 of their rms; RWKV-5.2 5.4e-3 and 2.2e-2.  Four times that."""
     return {"rel": 0.015, "max": 0.065} if case["version"] == "4" else {"rel": 0.022, "max": 0.09}
+
+
+class _Weights:
+    """The random weights of a "synthetic:" model (counter-based: splitmix64, Box-Muller), in the order in which the
+    model draws them."""
+
+    def __init__(self, case):
+        self.seed, self.drawn, self.quant = 1236 + len(case["weights"]), 0, case["weights"] == "int8"
+
+    @staticmethod
+    def _signed(x):
+        x &= (1 << 64) - 1
+        return x - (1 << 64) if x >> 63 else x
+
+    @classmethod
+    def _splitmix(cls, x):
+        x = x + cls._signed(0x9E3779B97F4A7C15)
+        x = (x ^ ((x >> 30) & ((1 << 34) - 1))) * cls._signed(0xBF58476D1CE4E5B9)
+        x = (x ^ ((x >> 27) & ((1 << 37) - 1))) * cls._signed(0x94D049BB133111EB)
+        return x ^ ((x >> 31) & ((1 << 33) - 1))
+
+    @classmethod
+    def _unit(cls, key, i):
+        return (((cls._splitmix(i + key) >> 40) & 0xFFFFFF) + 1).float() * (1.0 / 16777216.0)
+
+    @classmethod
+    def _normal(cls, key, i):
+        u1, u2 = cls._unit(key, 2 * i), cls._unit(key, 2 * i + 1)
+        log = torch.log(u1.double()).float()
+        return torch.sqrt(-2.0 * log) * torch.cos((6.2831855 * u2).double()).float()
+
+    def _key(self):
+        self.drawn += 1
+        x = torch.tensor(self._signed(self.seed * 0x100000001B3 + self.drawn))
+        return int(self._splitmix(x))
+
+    def uniform(self, n, lo, hi, half=True):
+        v = lo + (hi - lo) * self._unit(self._key(), torch.arange(n, device="cuda"))
+        return (v.half() if half else v).double()
+
+    def matrix(self, k, n):
+        key, w = self._key(), torch.empty(k, n, device="cuda", dtype=torch.float64)
+        rows = max(1, (1 << 25) // n)
+        for lo in range(0, k, rows):
+            at = torch.arange(lo * n, min(k, lo + rows) * n, device="cuda")
+            w[lo:lo + rows] = (0.02 * self._normal(key, at)).half().double().view(-1, n)
+        return self._coded(w.float()) if self.quant else w
+
+    @staticmethod
+    def _coded(w):
+        """What a matrix is in uint8 codes with row and column offsets and ranges in binary16."""
+        mx = w.min(0).values.half().float()
+        w = w - mx
+        my = w.min(1).values.half().float()
+        w = w - my[:, None]
+        rx = w.max(0).values.clamp(min=1e-4).half().float()
+        w = w / rx
+        ry = w.max(1).values.clamp(min=1e-4).half().float()
+        q = torch.round(w / ry[:, None] * 255.0).clamp(0, 255).double()
+        return q * (rx.double() / 255.0) * ry.double()[:, None] + mx.double() + my.double()[:, None]
+
+    def rows(self, ids, c):
+        key, at = self._key(), torch.as_tensor(ids, device="cuda", dtype=torch.int64)[:, None] * c
+        v = (0.02 * self._normal(key, at + torch.arange(c, device="cuda"))).double()
+        return _norm(v).half().double()
+
+
+def _norm(x):
+    return (x - x.mean(-1, keepdim=True)) / torch.sqrt(x.var(-1, unbiased=False, keepdim=True) + 1e-5)
+
+
+def _running(x, decay):
+    """y[t] = decay y[t-1] + x[t], along the first axis."""
+    d, n = decay, 1
+    while n < len(x):
+        x = torch.cat([x[:n], x[n:] + d * x[:-n]])
+        d, n = d * d, 2 * n
+    return x
+
+
+def _attention4(w, c, mixed):
+    mk, mv, mr = (w.uniform(c, 0, 1) for _ in range(3))
+    decay, first = torch.exp(-torch.exp(w.uniform(c, -5, 1, False))), w.uniform(c, -1, 1, False)
+    k, v, r = mixed(mk) @ w.matrix(c, c), mixed(mv) @ w.matrix(c, c), torch.sigmoid(mixed(mr) @ w.matrix(c, c))
+    e = torch.exp(k)
+    num, den = _running(e * v, decay), _running(e, decay)
+    now = torch.exp(first + k)
+    before = [torch.cat([torch.zeros_like(s[:1]), s[:-1]]) for s in (num, den)]
+    return (r * (before[0] + now * v) / (before[1] + now)) @ w.matrix(c, c)
+
+
+def _attention5(w, c, heads, mixed):
+    s = c // heads
+    mk, mv, mr, mg = (w.uniform(c, 0, 1) for _ in range(4))
+    decay, first = torch.exp(-torch.exp(w.uniform(c, -6, 0, False))), w.uniform(c, -1, 1, False)
+    k, v, r, g = (mixed(m) @ w.matrix(c, c) for m in (mk, mv, mr, mg))
+    decay, first = decay.view(heads, s, 1), first.view(heads, s, 1)
+    state, out = torch.zeros(heads, s, s, device="cuda", dtype=torch.float64), []
+    for kt, vt, rt in zip(k.view(-1, heads, s, 1), v.view(-1, heads, 1, s), r.view(-1, heads, 1, s)):
+        kv = kt * vt
+        out.append(rt @ (state + first * kv))
+        state = state * decay + kv
+    out = _norm(torch.stack(out).view(-1, heads, s)).view(-1, c)
+    return (out * torch.nn.functional.silu(g)) @ w.matrix(c, c)
+
+
+@torch.no_grad()
+def exact(case, seed):
+    """The logits in 64 bits, from the weights as the model holds them (binary16, or uint8 codes with their scales)."""
+    rng = np.random.default_rng(seed)
+    prompt = rng.integers(0, case["vocab"], case["prompt"])
+    steps = rng.integers(0, case["vocab"], case["steps"])
+    past = rng.integers(0, case["vocab"], 0 if case["fresh"] else 16)
+    ids = np.concatenate([past, prompt, steps])
+    c, f, w = case["c"], case["f"], _Weights(case)
+    table = _Weights(case)
+    table.drawn = case["layers"] * (16 if case["heads"] else 14) + 1  # the embedding comes after the layers and the head
+    x = table.rows(ids, c)
+
+    for layer in range(case["layers"]):
+        def mixed(m):
+            return xx * m + torch.cat([torch.zeros_like(xx[:1]), xx[:-1]]) * (1 - m)
+        xx = _norm(x)
+        x = x + (_attention5(w, c, case["heads"], mixed) if case["heads"] else _attention4(w, c, mixed))
+        xx = _norm(x)
+        mk, mr = w.uniform(c, 0, 1), w.uniform(c, 0, 1)
+        k = torch.relu(mixed(mk) @ w.matrix(c, f)) ** 2
+        v = k @ w.matrix(f, c)
+        x = x + v * torch.sigmoid(mixed(mr) @ w.matrix(c, c))
+        if (layer + 1) % 6 == 0:
+            x = x / 2
+    if not case["score"]:
+        x = x[(len(past) if len(prompt) == 0 else len(past) + len(prompt) - 1):]
+    logits = (_norm(x) @ w.matrix(c, case["vocab"])).cpu().numpy()
+    return logits if case["score"] else list(logits)
