@@ -80,6 +80,8 @@ _SIGS = {
     "frhip_gemv": (_i, [_vp, _WP, _vp, _i, _vp]),
     "frhip_cast": (_i, [_vp, _i, _vp, _i, _sz, _vp]),
     "frhip_fill": (_i, [_vp, _i, C.c_float, _sz, _vp]),
+    "frhip_fill_many": (_i, [_i, _vp, _vp, _vp, _vp, _vp]),
+    "frhip_copy_many": (_i, [_i, _vp, _vp, _vp, _vp]),
     "frhip_scalar_div_f16": (_i, [_vp, C.c_float, _sz, _vp]),
     "frhip_gather_rows": (_i, [_vp, _vp, _vp, _i, _i, _vp]),
     "frhip_slice": (_i, [_vp, _vp, _i, _vp, _vp, _vp, _vp, _i, _vp]),

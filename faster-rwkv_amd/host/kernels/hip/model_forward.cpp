@@ -135,6 +135,25 @@ static std::shared_ptr<DecodePlan> make_plan(Model *model, ModelExtra &ex) {
   return p;
 }
 
+// Device-to-device copies of the state tensors of one call, issued together (frhip_copy_many: a launch per 64 of them).
+// The sources are held until then.
+struct CopyList {
+  std::vector<Tensor> held;
+  std::vector<void *> dst;
+  std::vector<const void *> src;
+  std::vector<size_t> bytes;
+  void add(Tensor &to, const Tensor &from) {
+    held.push_back(from);
+    dst.push_back(to.data_ptr());
+    src.push_back(from.data_ptr());
+    bytes.push_back(from.nbytes());
+  }
+  void issue() {
+    if (!dst.empty())
+      FRHIP_CHECK(frhip_copy_many(static_cast<int>(dst.size()), dst.data(), src.data(), bytes.data(), stream()));
+  }
+};
+
 // The fused path updates the recurrent state in place, in buffers the plan owns, and Model::states()
 // hands out those buffers.  The reference's operators return fresh tensors every step
 // (kernels/cuda/att.cu:344-353), so a caller may keep a copy of states() as a snapshot and give it back
@@ -161,12 +180,14 @@ static void detach_if_snapshotted(Model *model, DecodePlan &p) {
   old.aa = p.aa, old.bb = p.bb, old.pp = p.pp, old.wkv = p.wkv;
   for (int s = 0; s < 2; s++) old.sx_att[s] = p.sx_att[s], old.sx_ffn[s] = p.sx_ffn[s];
   alloc_state_buffers(p);
+  CopyList copies;
   for (int l = 0; l < p.L; l++)
     for (size_t j = 0; j < p.n_state(); j++) {
       Tensor &src = old.view(p.parity, l, j), &dst = p.view(p.parity, l, j);
-      FRHIP_CHECK(frhip_memcpy_async(dst.data_ptr(), src.data_ptr(), src.nbytes(), FRHIP_D2D, stream()));
+      copies.add(dst, src);
       if (st[l][j].shares_storage_with(src)) st[l][j] = dst;
     }
+  copies.issue();
   FRHIP_CHECK(frhip_stream_sync(stream()));
   for (auto *set : {p.graph, p.chain})
     for (int i = 0; i < 2; i++) {
@@ -182,6 +203,8 @@ static void detach_if_snapshotted(Model *model, DecodePlan &p) {
 static void adopt_states(Model *model, DecodePlan &p) {
   auto &st = model->states();
   RV_CHECK(static_cast<int>(st.size()) == p.L);
+  CopyList copies;
+  bool from_host = false;
   for (int l = 0; l < p.L; l++) {
     RV_CHECK(st[l].size() == p.n_state());
     for (size_t j = 0; j < p.n_state(); j++) {
@@ -190,11 +213,15 @@ static void adopt_states(Model *model, DecodePlan &p) {
       RV_CHECK(st[l][j].nbytes() == mine.nbytes() && st[l][j].dtype() == mine.dtype())
           << "state " << l << "/" << j << " has the wrong shape or dtype";
       Tensor src = st[l][j].device() == Device::kHIP ? st[l][j] : Copy(st[l][j], Device::kHIP);
-      FRHIP_CHECK(frhip_memcpy_async(mine.data_ptr(), src.data_ptr(), src.nbytes(), FRHIP_D2D, stream()));
-      if (src.data_ptr() != st[l][j].data_ptr()) FRHIP_CHECK(frhip_stream_sync(stream()));  // src dies here
-      st[l][j] = mine;
+      copies.add(mine, src);
+      from_host = from_host || src.data_ptr() != st[l][j].data_ptr();
     }
   }
+  copies.issue();
+  for (int l = 0; l < p.L; l++)
+    for (size_t j = 0; j < p.n_state(); j++)
+      if (st[l][j].data_ptr() != p.view(p.parity, l, j).data_ptr()) st[l][j] = p.view(p.parity, l, j);
+  if (from_host) FRHIP_CHECK(frhip_stream_sync(stream()));  // the copies on the device die with this call
 }
 
 // `chained`: the token comes from the arg-max pairs the previous step left in device memory (pairs_dev)

@@ -49,6 +49,19 @@ Tensor &fill_(Tensor &x, float value) {
   return x;
 }
 
+void fill_many_(std::vector<Tensor> &xs, const std::vector<float> &vals) {
+  RV_CHECK(xs.size() == vals.size());
+  std::vector<void *> dst;
+  std::vector<int> dtype;
+  std::vector<size_t> count;
+  for (auto &x : xs) {
+    dst.push_back(x.data_ptr());
+    dtype.push_back(to_frhip_dtype(x.dtype()));
+    count.push_back(static_cast<size_t>(x.numel()));
+  }
+  FRHIP_CHECK(frhip_fill_many(static_cast<int>(xs.size()), dst.data(), dtype.data(), vals.data(), count.data(), stream()));
+}
+
 Tensor cast_dtype(const Tensor &x, DType dtype) {
   if (x.dtype() == dtype) return x;
   Tensor y = Tensor::Empty(x.shape(), dtype, Device::kHIP);
@@ -415,6 +428,7 @@ att_seq_v5(const Tensor &x, const Tensor &sx, const Tensor &s, const Tensor &ln_
 }
 
 KernelRegister fill_reg("fill_", Device::kHIP, fill_);
+KernelRegister fill_many_reg("fill_many_", Device::kHIP, fill_many_);
 KernelRegister cast_reg("cast_dtype", Device::kHIP, cast_dtype);
 KernelRegister scalar_div_reg("scalar_div_", Device::kHIP, scalar_div_);
 KernelRegister layernorm_reg("layernorm", Device::kHIP, layernorm);

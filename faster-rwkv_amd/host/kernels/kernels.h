@@ -72,6 +72,8 @@ FR_OP(T2, ffn_seq, "ffn_seq", x.device(), FR_FFN_PARAMS, FR_FFN_ARGS)
 // ---- primitives ----------------------------------------------------------------
 FR_OP(T1, cast_dtype, "cast_dtype", x.device(), (CT x, DType dtype), (x, dtype))
 FR_OP(Tensor &, fill_, "fill_", x.device(), (Tensor & x, float val), (x, val))
+// fill_ of several tensors of one device, all of one call's launches together (hip only; Model::ResetStates)
+FR_OP(void, fill_many_, "fill_many_", xs.at(0).device(), (std::vector<Tensor> &xs, const std::vector<float> &vals), (xs, vals))
 FR_OP(T1, scalar_div_, "scalar_div_", x.device(), (Tensor & x, float val), (x, val))
 FR_OP(T1, layernorm, "layernorm", x.device(), (CT x, CT weight, CT bias), (x, weight, bias))
 FR_OP(T1, groupnorm, "groupnorm", x.device(), (CT x, int num_groups, CT weight, CT bias),

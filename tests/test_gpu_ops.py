@@ -268,3 +268,39 @@ def test_gather_rows():
     out = DevBuf.empty((5, 256), np.float16)
     fr.check(L().frhip_gather_rows(keep(tab).ptr, keep(ids).ptr, out.ptr, 5, 512, None))
     assert np.array_equal(out.numpy(), tab[ids])
+
+
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 130])
+def test_fill_and_copy_of_many_buffers(n):
+    """Every buffer of a call is filled / copied whole and nothing beside it is touched: sizes around 16 bytes and
+    around a workgroup's 4096, empty ones, odd addresses (single bytes of a copy, 2-byte steps of a fill), and counts
+    around the 64 buffers of a launch."""
+    sizes = [0, 2, 14, 16, 18, 4094, 4096, 4098, 80000, 3 << 19]
+    total = sum(sizes[i % len(sizes)] + 64 for i in range(n))
+    host = rng.integers(0, 255, total).astype(np.uint8)
+    src, dst = keep(host), keep(np.full(total, 0xAB, np.uint8))
+    copied, filled = np.full(total, 0xAB, np.uint8), host.copy()
+    at, to, frm, nbytes, fill, dtypes, values, counts = 0, [], [], [], [], [], [], []
+    for i in range(n):
+        nb = sizes[i % len(sizes)]
+        o = at + (0, 2, 5)[i % 3]
+        to.append(dst.ptr + o), frm.append(src.ptr + o), nbytes.append(nb)
+        copied[o:o + nb] = host[o:o + nb]
+        f32 = i // 2 % 2 == 0
+        o = at + (0, 4 if f32 else 2)[i % 2]
+        fill.append(src.ptr + o), dtypes.append(fr.F32 if f32 else fr.F16)
+        values.append(-1e30 if f32 else 0.25 * i), counts.append(nb // (4 if f32 else 2))
+        v = np.full(counts[-1], values[-1], np.float32 if f32 else np.float16).view(np.uint8)
+        filled[o:o + v.size] = v
+        at += (nb + 64) // 16 * 16
+    arr = lambda t, v: (t * len(v))(*v)
+    copy = lambda k, d: L().frhip_copy_many(k, arr(C.c_void_p, d), arr(C.c_void_p, frm), arr(C.c_size_t, nbytes), None)
+    fil = lambda k, t, c: L().frhip_fill_many(k, arr(C.c_void_p, fill), arr(C.c_int, t), arr(C.c_float, values),
+                                              arr(C.c_size_t, c), None)
+    fr.check(copy(n, to))
+    fr.check(fil(n, dtypes, counts))
+    fr.check(L().frhip_device_sync())
+    assert np.array_equal(dst.numpy(), copied)
+    assert np.array_equal(src.numpy(), filled)
+    assert copy(n, [None] * n) == (-1 if any(nbytes) else 0)
+    assert fil(n, [fr.U8] * n, counts) == -1
