@@ -686,20 +686,16 @@ static void gemm_ldw_launch(dim3 grid, hipStream_t st, const GemmArgs& a) {
 // 32-column blocks; the loops are instantiated per block count, so the products are the same
 // MFMAs in the same k order as in the other kernels and the results are bit-identical.  Loader
 // wave, LDS ring (three or four K-steps of 64, whatever fits 160 KB at the launch's widest tile)
-// and swizzle are those of gemm_ldw_kernel.  gemm_vw_kernel<256> has eight MFMA waves (4 x 2 of
-// 64 rows each) over tiles of 256 rows and at most 160 columns; the host takes it where it saves
-// a round (1024 x 2048 x 10240 as one segment: 58 us against 71 us in two rounds of 128-row tiles).
-// Its predicated epilogue (edge tiles) spills a few registers; the main loop does not.
+// and swizzle are those of gemm_ldw_kernel.  Tiles of 256 rows: gemm_vw256_kernel below.
 // ---------------------------------------------------------------------------
-constexpr int kVwMaxW = 8;
+constexpr int kVwMaxW = 8, kVwMaxRounds = 32;
 
-template <int BM, int W>
+template <int W>
 __device__ __forceinline__ void vw_loader(const GemmSeg& sg, unsigned char* smem, int stage_bytes, int ns, int m0, int n0,
                                           int M, int N, int K, int lane) {
-  constexpr int kVwABytes = BM * kLdwBK * 2;
-  constexpr int kAInstr = kVwABytes / 1024, kBInstr = 4 * W, kPer = (kAInstr + kBInstr) <= 63 ? (kAInstr + kBInstr) : 0;
-  if constexpr (kPer == 0) return;  // wider than the wait counter allows: the host never plans such a tile
-
+  constexpr int BM = 128, kVwABytes = BM * kLdwBK * 2;
+  constexpr int kAInstr = kVwABytes / 1024, kBInstr = 4 * W, kPer = kAInstr + kBInstr;
+  static_assert(kPer <= 63, "the wait counter's range");
   const int lr = lane >> 3, ls = (lane & 7) ^ lr;
   const h1* pa[kAInstr];
   const h1* pb[kBInstr];
@@ -762,10 +758,10 @@ __device__ __forceinline__ void vw_loader(const GemmSeg& sg, unsigned char* smem
   }
 }
 
-template <int BM, int NJ>
+template <int NJ>
 __device__ __forceinline__ void vw_mma(const GemmArgs& a, const GemmSeg& sg, const unsigned char* smem, int stage_bytes, int ns,
                                        int brow0, int m0, int n0, int M, int N, bool full, int lane, int wm) {
-  constexpr int kVwABytes = BM * kLdwBK * 2;
+  constexpr int kVwABytes = 128 * kLdwBK * 2;
   f16v acc[2][NJ];
 #pragma unroll
   for (int i = 0; i < 2; i++)
@@ -779,29 +775,23 @@ __device__ __forceinline__ void vw_mma(const GemmArgs& a, const GemmSeg& sg, con
     __builtin_amdgcn_s_barrier();
     const unsigned char* st = smem + slot * stage_bytes;
     slot = slot + 1 == ns ? 0 : slot + 1;
-    // fragments of KG x 16 k are requested together; with eight MFMA waves a lane has 168
-    // registers and holds two of the four k-blocks of a step at a time
-    constexpr int KG = BM == 128 ? 4 : 2;
+    h8 fa[4][2], fb[4][NJ];
 #pragma unroll
-    for (int kh = 0; kh < 4; kh += KG) {
-      h8 fa[KG][2], fb[KG][NJ];
+    for (int kb = 0; kb < 4; kb++) {
+      const int q = kb * 2 + (lane >> 5);
 #pragma unroll
-      for (int kb = 0; kb < KG; kb++) {
-        const int q = (kh + kb) * 2 + (lane >> 5);
+      for (int i = 0; i < 2; i++) fa[kb][i] = *reinterpret_cast<const h8*>(st + ldw_at(wm * 64 + i * 32 + (lane & 31), q));
 #pragma unroll
-        for (int i = 0; i < 2; i++) fa[kb][i] = *reinterpret_cast<const h8*>(st + ldw_at(wm * 64 + i * 32 + (lane & 31), q));
+      for (int j = 0; j < NJ; j++)
+        fb[kb][j] = *reinterpret_cast<const h8*>(st + kVwABytes + ldw_at(brow0 + j * 32 + (lane & 31), q));
+    }
+#pragma unroll
+    for (int kb = 0; kb < 4; kb++)
+#pragma unroll
+      for (int i = 0; i < 2; i++)
 #pragma unroll
         for (int j = 0; j < NJ; j++)
-          fb[kb][j] = *reinterpret_cast<const h8*>(st + kVwABytes + ldw_at(brow0 + j * 32 + (lane & 31), q));
-      }
-#pragma unroll
-      for (int kb = 0; kb < KG; kb++)
-#pragma unroll
-        for (int i = 0; i < 2; i++)
-#pragma unroll
-          for (int j = 0; j < NJ; j++)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[kb][i], fb[kb][j], acc[i][j], 0, 0, 0);
-    }
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[kb][i], fb[kb][j], acc[i][j], 0, 0, 0);
   }
   if (full)
     gemm_epilogue_t<2, NJ, true>(a, sg, acc, m0 + wm * 64, n0 + brow0, M, N, lane);
@@ -809,21 +799,23 @@ __device__ __forceinline__ void vw_mma(const GemmArgs& a, const GemmSeg& sg, con
     gemm_epilogue_t<2, NJ, false>(a, sg, acc, m0 + wm * 64, n0 + brow0, M, N, lane);
 }
 
-template <int BM>
-__global__ __launch_bounds__(BM * 2 + 64) void gemm_vw_kernel(GemmArgs a) {
-  constexpr int kVwABytes = BM * kLdwBK * 2, kLoader = BM / 32;  // BM / 32 MFMA waves of 64 rows x half the width, then the loader
+// Workgroups are dealt to the eight XCDs in turn (linear index mod 8), each with an L2 of its own.  XCD x takes the
+// x-th eighth of the tiles, counted in blocks of four N tiles by all strips of rows, so that the 32 it runs at a time
+// share about four N tiles and eight strips.  (A matter of traffic only: the map is one to one, and any assignment of
+// tiles to workgroups gives the same results.)
+__device__ __forceinline__ void xcd_tile(int& bx, int& by) {
+  const int gx = gridDim.x, gy = gridDim.y, lin = blockIdx.y * gx + blockIdx.x, n = gx * gy;
+  const int x = lin & 7, id = x * (n >> 3) + min(x, n & 7) + (lin >> 3);
+  const int blk = id / (4 * gy), rem = id - blk * 4 * gy, bw = min(4, gx - 4 * blk);
+  by = rem / bw;
+  bx = 4 * blk + rem % bw;
+}
+
+__global__ __launch_bounds__(320) void gemm_vw_kernel(GemmArgs a) {
+  constexpr int BM = 128, kVwABytes = BM * kLdwBK * 2, kLoader = 4;  // four MFMA waves of 64 rows x half the width, then the loader
   extern __shared__ __attribute__((aligned(16))) unsigned char gemm_smem[];
-  // Workgroups are dealt to the eight XCDs in turn (linear index mod 8), each with an L2 of its own.
-  // XCD x therefore takes the x-th eighth of the N tiles, for every strip of rows: it fetches
-  // those weights once and one segment's rows of A, instead of every segment's.  (A matter of
-  // traffic only: any assignment of tiles to workgroups gives the same results.)
-  int bx = blockIdx.x, by = blockIdx.y;
-  if (gridDim.x % 8 == 0) {
-    const int lin = by * gridDim.x + bx, per = gridDim.x / 8;
-    const int r = lin >> 3;
-    bx = (lin & 7) * per + r % per;
-    by = r / per;
-  }
+  int bx, by;
+  xcd_tile(bx, by);
   int sidx = 0;
 #pragma unroll
   for (int i = 1; i < kGemmMaxSeg; i++) sidx += (i < a.nseg && bx >= a.tile_start[i]) ? 1 : 0;
@@ -839,13 +831,13 @@ __global__ __launch_bounds__(BM * 2 + 64) void gemm_vw_kernel(GemmArgs a) {
   const int stage_bytes = kVwABytes + a.vw_maxw * 4096, ns = a.vw_ns;
   if (wave == kLoader) {
     switch (width) {
-      case 2: vw_loader<BM, 2>(sg, gemm_smem, stage_bytes, ns, m0, n0, M, N, K, lane); break;
-      case 3: vw_loader<BM, 3>(sg, gemm_smem, stage_bytes, ns, m0, n0, M, N, K, lane); break;
-      case 4: vw_loader<BM, 4>(sg, gemm_smem, stage_bytes, ns, m0, n0, M, N, K, lane); break;
-      case 5: vw_loader<BM, 5>(sg, gemm_smem, stage_bytes, ns, m0, n0, M, N, K, lane); break;
-      case 6: vw_loader<BM, 6>(sg, gemm_smem, stage_bytes, ns, m0, n0, M, N, K, lane); break;
-      case 7: vw_loader<BM, BM == 128 ? 7 : 6>(sg, gemm_smem, stage_bytes, ns, m0, n0, M, N, K, lane); break;  // 256 rows: never wider than 5
-      default: vw_loader<BM, BM == 128 ? 8 : 6>(sg, gemm_smem, stage_bytes, ns, m0, n0, M, N, K, lane); break;
+      case 2: vw_loader<2>(sg, gemm_smem, stage_bytes, ns, m0, n0, M, N, K, lane); break;
+      case 3: vw_loader<3>(sg, gemm_smem, stage_bytes, ns, m0, n0, M, N, K, lane); break;
+      case 4: vw_loader<4>(sg, gemm_smem, stage_bytes, ns, m0, n0, M, N, K, lane); break;
+      case 5: vw_loader<5>(sg, gemm_smem, stage_bytes, ns, m0, n0, M, N, K, lane); break;
+      case 6: vw_loader<6>(sg, gemm_smem, stage_bytes, ns, m0, n0, M, N, K, lane); break;
+      case 7: vw_loader<7>(sg, gemm_smem, stage_bytes, ns, m0, n0, M, N, K, lane); break;
+      default: vw_loader<8>(sg, gemm_smem, stage_bytes, ns, m0, n0, M, N, K, lane); break;
     }
     return;
   }
@@ -855,27 +847,135 @@ __global__ __launch_bounds__(BM * 2 + 64) void gemm_vw_kernel(GemmArgs a) {
   const int brow0 = wn ? nj0 * 32 : 0;
   const bool full = m0 + BM <= M && n0 + width * 32 <= N;
   switch (nj) {
-    case 1: vw_mma<BM, 1>(a, sg, gemm_smem, stage_bytes, ns, brow0, m0, n0, M, N, full, lane, wm); break;
-    case 2: vw_mma<BM, 2>(a, sg, gemm_smem, stage_bytes, ns, brow0, m0, n0, M, N, full, lane, wm); break;
-    case 3: vw_mma<BM, 3>(a, sg, gemm_smem, stage_bytes, ns, brow0, m0, n0, M, N, full, lane, wm); break;
-    default: vw_mma<BM, BM == 128 ? 4 : 3>(a, sg, gemm_smem, stage_bytes, ns, brow0, m0, n0, M, N, full, lane, wm); break;
+    case 1: vw_mma<1>(a, sg, gemm_smem, stage_bytes, ns, brow0, m0, n0, M, N, full, lane, wm); break;
+    case 2: vw_mma<2>(a, sg, gemm_smem, stage_bytes, ns, brow0, m0, n0, M, N, full, lane, wm); break;
+    case 3: vw_mma<3>(a, sg, gemm_smem, stage_bytes, ns, brow0, m0, n0, M, N, full, lane, wm); break;
+    default: vw_mma<4>(a, sg, gemm_smem, stage_bytes, ns, brow0, m0, n0, M, N, full, lane, wm); break;
   }
 }
 
-// Cuts the launch into tiles of bm rows for gemm_vw_kernel<bm>: the fewest rounds over `cus` compute
-// units whose widest tile fits.  Returns the number of rounds, or 0: the launch is too small for
-// tiles of at least bm x 128 (the other kernels' 64-row tiles serve it better) or too ragged.
+// ---------------------------------------------------------------------------
+// The same tiles, 256 rows high: eight waves, 4 x 2, each 64 rows x half the width.
+//
+// With one MFMA wave per SIMD (gemm_vw_kernel) nothing runs while the first fragments of a step come
+// out of LDS after the barrier.  Here every SIMD has two, and a step is twice the
+// products for 1.33 times the bytes (256 x 256 against 128 x 256).  There is no loader wave: a ninth
+// wave would leave each wave 168 registers (three on one SIMD), too few for 128 accumulators; the waves
+// issue their share of a step's loads (at most 8 instructions of 1 KB) right behind a barrier, one step
+// ahead into the second stage.  (A third stage, which tiles of up to 160 columns leave room for, and loads
+// two steps ahead were measured: no faster, 4099 x 8192 x 2048 166 us against 161.)
+// Rows past the matrix are clamped in the lane offsets, so edge tiles load like the others.
+// ---------------------------------------------------------------------------
+constexpr int kVw256Threads = 512, kVw256ABytes = 256 * kLdwBK * 2;
+
+template <int NJ>
+__device__ __forceinline__ void vw256_body(const GemmArgs& a, const GemmSeg& sg, unsigned char* smem, int width, int brow0,
+                                           int m0, int n0, int lane, int wave) {
+  const int M = a.M, K = a.K, N = sg.N, nk = K / kLdwBK, wm = wave >> 1;
+  const unsigned stage_bytes = kVw256ABytes + a.vw_maxw * 4096;
+  // this wave's loads: row groups 4 wave .. + 3 of A, row groups wave, wave + 8, ... of B (there are 4 width)
+  unsigned va[4], vb[4];
+  const int lr = lane >> 3, ls = (lane & 7) ^ lr;
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const int ga = wave * 4 + i, gb = wave + 8 * i;
+    const int ra = m0 + ga * 8 + lr, rb = n0 + gb * 8 + lr;
+    va[i] = (unsigned)((ra < M ? ra : M - 1) - m0) * (unsigned)(K * 2) + (ls ^ (ga & 1)) * 16;
+    vb[i] = (unsigned)((rb < N ? rb : N - 1) - n0) * (unsigned)(K * 2) + (ls ^ (gb & 1)) * 16;
+  }
+  const unsigned char* abase = uniform_ptr(reinterpret_cast<const unsigned char*>(sg.A) + (size_t)m0 * K * 2);
+  const unsigned char* bbase = uniform_ptr(sg.B + (size_t)n0 * K * 2);
+  const unsigned lds0 = (unsigned)(size_t)((__attribute__((address_space(3))) unsigned char*)smem);
+  const int nb = 4 * width;
+  auto issue = [&](int step) {
+    const unsigned st = lds0 + (step & 1) * stage_bytes;
+    const unsigned char* ak = abase + (size_t)step * (kLdwBK * 2);
+    const unsigned char* bk = bbase + (size_t)step * (kLdwBK * 2);
+#pragma unroll
+    for (int i = 0; i < 4; i++) load_lds_saddr(va[i], ak, st + (wave * 4 + i) * 1024);
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+      if (wave + 8 * i < nb) load_lds_saddr(vb[i], bk, st + kVw256ABytes + (wave + 8 * i) * 1024);
+  };
+  f16v acc[2][NJ];
+#pragma unroll
+  for (int i = 0; i < 2; i++)
+#pragma unroll
+    for (int j = 0; j < NJ; j++)
+#pragma unroll
+      for (int v = 0; v < 16; v++) acc[i][j][v] = 0.f;
+  issue(0);
+  for (int k = 0; k < nk; k++) {
+    // this wave's loads of step k have landed and its fragments of step k-1 are in registers; behind the
+    // barrier that holds for all eight, so step k may be read and the slot of step k-1 refilled
+    __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    if (k + 1 < nk) issue(k + 1);
+    const unsigned char* st = smem + (k & 1) * stage_bytes;
+#pragma unroll
+    for (int kb = 0; kb < 4; kb++) {
+      h8 fa[2], fb[NJ];
+      const int q = kb * 2 + (lane >> 5);
+#pragma unroll
+      for (int i = 0; i < 2; i++) fa[i] = *reinterpret_cast<const h8*>(st + ldw_at(wm * 64 + i * 32 + (lane & 31), q));
+#pragma unroll
+      for (int j = 0; j < NJ; j++)
+        fb[j] = *reinterpret_cast<const h8*>(st + kVw256ABytes + ldw_at(brow0 + j * 32 + (lane & 31), q));
+#pragma unroll
+      for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < NJ; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[i], fb[j], acc[i][j], 0, 0, 0);
+    }
+  }
+  if (m0 + 256 <= M && n0 + width * 32 <= N)
+    gemm_epilogue_t<2, NJ, true>(a, sg, acc, m0 + wm * 64, n0 + brow0, M, N, lane);
+  else
+    gemm_epilogue_t<2, NJ, false>(a, sg, acc, m0 + wm * 64, n0 + brow0, M, N, lane);
+}
+
+__global__ __launch_bounds__(kVw256Threads) void gemm_vw256_kernel(GemmArgs a) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char gemm_smem[];
+  int bx, by;
+  xcd_tile(bx, by);
+  int sidx = 0;
+#pragma unroll
+  for (int i = 1; i < kGemmMaxSeg; i++) sidx += (i < a.nseg && bx >= a.tile_start[i]) ? 1 : 0;
+  const GemmSeg& sg = a.seg[sidx];
+  const int ti = bx - a.tile_start[sidx];
+  const int base = a.vw_base[sidx], wide = a.vw_wide[sidx];
+  const int width = base + (ti < wide ? 1 : 0);  // 32-column blocks of this tile
+  const int n0 = (ti * base + (ti < wide ? ti : wide)) * 32;
+  const int m0 = by * 256;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int nj0 = (width + 1) >> 1;
+  const int nj = (wave & 1) ? width - nj0 : nj0;
+  const int brow0 = (wave & 1) ? nj0 * 32 : 0;
+  switch (nj) {  // every wave passes the same barriers, whatever its width
+    case 1: vw256_body<1>(a, sg, gemm_smem, width, brow0, m0, n0, lane, wave); break;
+    case 2: vw256_body<2>(a, sg, gemm_smem, width, brow0, m0, n0, lane, wave); break;
+    case 3: vw256_body<3>(a, sg, gemm_smem, width, brow0, m0, n0, lane, wave); break;
+    default: vw256_body<4>(a, sg, gemm_smem, width, brow0, m0, n0, lane, wave); break;
+  }
+}
+
+// Cuts the launch into tiles of bm rows (128: gemm_vw_kernel, 256: gemm_vw256_kernel): the fewest rounds over
+// `cus` compute units whose widest tile fits.  Returns what the launch is expected to take, or 0: it is too small
+// for tiles of at least bm x 96 (the other kernels' 64-row tiles serve it better) or too ragged.
+// The expectation is rounds x (fixed + slope x widest tile), in 0.1 us at K = 2048; both parts grow with K alike.
+// Measured rounds, us: 128 rows, widths 5 / 6 / 8: 26.4 / 30.5 / 38.2; 256 rows, 3 / 4 / 5 / 6 / 8: 30.3 / 38.7 /
+// 46.0 / 51.9 / 66.8.  256-row tiles are the cheaper ones per product from about six blocks on, and where they
+// save a round.
 static int plan_vw(GemmArgs& a, int bm, int cus, dim3* grid, size_t* lds) {
   const int mt = (a.M + bm - 1) / bm;
   const int abytes = bm * kLdwBK * 2;
-  const int wcap = bm == 128 ? kVwMaxW : 5;  // 256 rows: three stages of (256 + 160) x 64 halves are 156 KB of the 160 KB
   int cb[kGemmMaxSeg], total = 0;
   for (int s = 0; s < a.nseg; s++) {
     cb[s] = (a.seg[s].N + 31) / 32;
     total += cb[s];
   }
-  for (int rounds = 1; rounds <= 4; rounds++) {
-    const int P = rounds * cus / mt;  // tiles per strip of 128 rows
+  for (int rounds = 1; rounds <= kVwMaxRounds; rounds++) {
+    const int P = rounds * cus / mt;  // tiles per strip of rows
     if (P < a.nseg) continue;
     int t[kGemmMaxSeg], used = 0;
     for (int s = 0; s < a.nseg; s++) {
@@ -902,8 +1002,8 @@ static int plan_vw(GemmArgs& a, int bm, int cus, dim3* grid, size_t* lds) {
       maxw = w > maxw ? w : maxw;
       minw = cb[s] / t[s] < minw ? cb[s] / t[s] : minw;
     }
-    if (maxw > wcap) continue;
-    if (minw < 2 || maxw < 4) return 0;
+    if (maxw > kVwMaxW) continue;
+    if (minw < 2 || maxw < 3) return 0;
     int tiles = 0;
     for (int s = 0; s < a.nseg; s++) {
       a.tile_start[s] = tiles;
@@ -915,24 +1015,26 @@ static int plan_vw(GemmArgs& a, int bm, int cus, dim3* grid, size_t* lds) {
     a.tile_start[a.nseg] = tiles;
     a.vw_maxw = maxw;
     const size_t stage = abytes + (size_t)maxw * 4096;
-    a.vw_ns = stage * 4 <= 160 * 1024 ? 4 : 3;
+    a.vw_ns = bm == 256 ? 2 : stage * 4 <= 160 * 1024 ? 4 : 3;
     if (stage * a.vw_ns > 160 * 1024) return 0;
     *lds = stage * a.vw_ns;
     *grid = dim3(tiles, mt);
-    return rounds;
+    return rounds * (bm == 128 ? 75 + 39 * maxw : 100 + 72 * maxw);
   }
   return 0;
 }
 
-template <int BM>
-static void gemm_vw_launch(dim3 grid, size_t lds, hipStream_t st, const GemmArgs& a) {
-  static bool raised = false;
-  if (!raised) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_vw_kernel<BM>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                              160 * 1024);
-    raised = true;
-  }
-  hipLaunchKernelGGL((gemm_vw_kernel<BM>), grid, dim3(BM * 2 + 64), lds, st, a);
+static void gemm_vw_launch(int bm, dim3 grid, size_t lds, hipStream_t st, const GemmArgs& a) {
+  static const bool raised = [] {
+    for (const void* f : {reinterpret_cast<const void*>(&gemm_vw_kernel), reinterpret_cast<const void*>(&gemm_vw256_kernel)})
+      (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    return true;
+  }();
+  (void)raised;
+  if (bm == 256)
+    hipLaunchKernelGGL(gemm_vw256_kernel, grid, dim3(kVw256Threads), lds, st, a);
+  else
+    hipLaunchKernelGGL(gemm_vw_kernel, grid, dim3(320), lds, st, a);
 }
 
 static constexpr size_t gemm_lds_bytes(int bm, int bk) { return (size_t)(bm + BN) * (bk + 8) * 2; }
@@ -1080,28 +1182,39 @@ int launch_gemm(GemmArgs& a, bool u8, hipStream_t st, const char* what, void* dq
   static const bool vw = !(getenv("FRHIP_GEMM_VW") && atoi(getenv("FRHIP_GEMM_VW")) == 0);
   static const int force_vw_bm = getenv("FRHIP_GEMM_VW_BM") ? atoi(getenv("FRHIP_GEMM_VW_BM")) : 0;  // measurement aid
   if (!u8 && ldw && vw && !force_bm) {
-    // 128-row tiles unless 256-row tiles (eight MFMA waves) need fewer rounds
-    GemmArgs b1 = a, b2 = a;
-    dim3 g1, g2;
-    size_t l1 = 0, l2 = 0;
-    const int r1 = plan_vw(b1, 128, compute_units(), &g1, &l1);
-    const int r2 = force_vw_bm == 128 ? 0 : plan_vw(b2, 256, compute_units(), &g2, &l2);
-    // A grouped launch that needs two rounds although each of its products alone fits one (ffn r,k at T = 1024:
-    // 2048 columns in one round of 64 x 128 tiles, 8192 in one round of 128 x 256) goes out as separate launches.
+    struct Plan {
+      GemmArgs a;
+      dim3 grid;
+      size_t lds = 0;
+      int bm = 0, cost = 0;
+    };
+    auto plan = [&](const GemmArgs& g) {
+      Plan p1, p2;
+      p1.a = p2.a = g;
+      p1.bm = 128, p2.bm = 256;
+      p1.cost = plan_vw(p1.a, 128, compute_units(), &p1.grid, &p1.lds);
+      p2.cost = force_vw_bm == 128 ? 0 : plan_vw(p2.a, 256, compute_units(), &p2.grid, &p2.lds);
+      return p2.cost && (!p1.cost || p2.cost < p1.cost || force_vw_bm == 256) ? p2 : p1;
+    };
+    const Plan p = plan(a);
+    // A grouped launch whose products are cheaper one by one (2048 columns in one round of 64 x 128 tiles, 8192 in
+    // one round of 128 x 256, together two rounds) goes out as separate launches.  One round of 64-row tiles takes
+    // 16.5 us at K = 2048, another launch about 3 us.
     static const bool separate = !(getenv("FRHIP_GEMM_SEPARATE") && atoi(getenv("FRHIP_GEMM_SEPARATE")) == 0);
-    if (separate && a.nseg > 1 && (r1 == 0 || r1 >= 2) && (r2 == 0 || r2 >= 2)) {
-      bool each_one_round = true;
-      for (int sgi = 0; sgi < a.nseg && each_one_round; sgi++) {
+    if (separate && a.nseg > 1) {
+      bool known = true;
+      int sum = 30 * (a.nseg - 1);
+      for (int sgi = 0; sgi < a.nseg && known; sgi++) {
         GemmArgs one = a;
         one.nseg = 1;
         one.seg[0] = a.seg[sgi];
-        dim3 g;
-        size_t l = 0;
-        const int rr1 = plan_vw(one, 128, compute_units(), &g, &l), rr2 = plan_vw(one, 256, compute_units(), &g, &l);
         const long t64 = (long)((a.seg[sgi].N + BN - 1) / BN) * ((a.M + 63) / 64);
-        each_one_round = rr1 == 1 || rr2 == 1 || (rr1 == 0 && rr2 == 0 && t64 <= compute_units());
+        const int c = plan(one).cost;
+        known = c != 0 || t64 <= compute_units();
+        sum += c ? c : 165;
       }
-      if (each_one_round) {
+      const long t64g = (long)tiles * ((a.M + 63) / 64);
+      if (known && (p.cost ? sum < p.cost : t64g > compute_units())) {
         for (int sgi = 0; sgi < a.nseg; sgi++) {
           GemmArgs one = a;
           one.nseg = 1;
@@ -1111,12 +1224,8 @@ int launch_gemm(GemmArgs& a, bool u8, hipStream_t st, const char* what, void* dq
         return 0;
       }
     }
-    if (r2 && (!r1 || r2 < r1 || force_vw_bm == 256)) {
-      gemm_vw_launch<256>(g2, l2, st, b2);
-      return check_launch(what);
-    }
-    if (r1) {
-      gemm_vw_launch<128>(g1, l1, st, b1);
+    if (p.cost) {
+      gemm_vw_launch(p.bm, p.grid, p.lds, st, p.a);
       return check_launch(what);
     }
   }

@@ -67,6 +67,24 @@ def test_gemm_against_oracle(T, K, N, quant):
         assert not out[len(ks):].any()
 
 
+@pytest.mark.parametrize("T,K,N", [(2048, 64, 8192),    # 256 x 256 tiles, two stages, a single K-step
+                                   (2048, 128, 6100),   # 256 x 192, two K-steps, ragged columns
+                                   (4099, 192, 2048),   # 256 x 160 / 128, three stages; the last strip has three rows
+                                   (1025, 320, 10000),  # one row in the last strip, ragged columns
+                                   (512, 192, 6144),    # 128 x 96: the narrowest planned tile
+                                   (3000, 128, 10240)]) # more than four rounds' worth of 128 x 128 tiles
+def test_gemm_planned_tiles_against_oracle(T, K, N):
+    """Tile heights, widths, stage counts and edges of the planned binary16 launches.  Both sides add K exact products
+    in fp32, in another order: K 2^-24 of the sum of the magnitudes at most, which 3e-6 sqrt(K) max|y| covers here."""
+    x = h(rng.standard_normal((T, K)))
+    w = h(rng.standard_normal((K, N)) * 0.02)
+    pw, wref = make_weight(w, False)
+    ref = po.gemm_f16(x, wref, "f32")
+    y = DevBuf.empty((T, N), np.float32)
+    fr.check(L().frhip_gemm(keep(x).ptr, pw.ref, y.ptr, T, fr.F32, None))
+    assert np.abs(y.numpy() - ref).max() <= 3e-6 * np.sqrt(K) * np.abs(ref).max() + 1e-5
+
+
 def test_gemm_sigmoid_and_silu_epilogues_every_binary16_bit_exact():
     """Every finite binary16 value goes through the product's sigmoid epilogue (identity weight, so the
     accumulator is the input exactly) and must come out as the oracle's double-evaluated sigmoid (and its silu), bit for bit;
