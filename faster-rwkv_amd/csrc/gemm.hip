@@ -338,17 +338,31 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_kernel(GemmArgs a) {
     }
   };
 
+  // slice z of ksplit takes K-steps [z base + min(z, rem), ...): the first rem slices one step more
+  int kbeg = 0, kend = K;
+  if (U8 && a.ksplit > 1) {
+    const int z = blockIdx.z, steps = K / BK, per = steps / a.ksplit, rem = steps % a.ksplit;
+    kbeg = (z * per + min(z, rem)) * BK;
+    kend = kbeg + (per + (z < rem ? 1 : 0)) * BK;
+  }
   Stage s0;
-  load_tiles(s0, 0);
-  for (int k0 = 0; k0 < K; k0 += BK) {
+  load_tiles(s0, kbeg);
+  for (int k0 = kbeg; k0 < kend; k0 += BK) {
     __syncthreads();  // everyone is done reading the previous tile
     store_tiles(s0, k0);
     __syncthreads();
-    if (k0 + BK < K) load_tiles(s0, k0 + BK);
+    if (k0 + BK < kend) load_tiles(s0, k0 + BK);
     compute_tile();
   }
 
-  gemm_epilogue<BM>(a, sg, acc, m0, n0, M, N, lane, wm, wn);
+  if (U8 && a.ksplit > 1) {
+    GemmSeg sp = sg;  // this slice's sums go out as fp32; the epilogue proper follows in gemm_splitk_reduce_kernel
+    sp.out = a.partial + (size_t)blockIdx.z * a.partial_stride + a.part_off[sidx];
+    sp.epi = G_STORE_F32;
+    gemm_epilogue<BM>(a, sp, acc, m0, n0, M, N, lane, wm, wn);
+  } else {
+    gemm_epilogue<BM>(a, sg, acc, m0, n0, M, N, lane, wm, wn);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1066,10 +1080,89 @@ static int env_bk() {
   return e ? atoi(e) : 0;
 }
 
+static bool env_on(const char* name) {
+  const char* e = getenv(name);
+  return !(e && atoi(e) == 0);
+}
+
+// Few rows (a short prompt): 64 x 128 tiles leave most compute units without a workgroup, and a workgroup pulls its
+// weights through a ring of two K-steps (48 KB in flight), so a launch takes K / 64 round trips to memory however few
+// rows there are (T = 64, 2048 x 2048: 16 workgroups, 17-25 us for 8 MB).  With scratch for the partial sums such a
+// launch is split over K into as many slices as there are idle compute units (at least four K-steps each), and the
+// reduction pass adds the slices in order and applies each product's epilogue.  A group that is too wide for that as a
+// whole goes out product by product, so that its narrow members still can.  FRHIP_GEMM_FEW_ROWS=0: off.
+// uint8 weights of at most kU8DirectRows rows (one strip of tiles) are dequantised on their way into LDS, once each:
+// 1 byte of traffic per weight, where the expansion and a binary16 product move 5 (1 in, 2 out, 2 in again).  The
+// slices are those of the binary16 launch, so the sums are the same bits whichever form of the weight is multiplied.
+// *taken stays false, and nothing is launched, if the launch is not of this form.
+constexpr int kU8DirectRows = 64;
+static int launch_few_rows(GemmArgs& a, bool u8, hipStream_t st, const char* what, void* dq, float* few_rows,
+                           size_t few_rows_floats, bool* taken) {
+  int tiles = 0;
+  bool narrow = true;
+  for (int s = 0; s < a.nseg; s++) {
+    a.tile_start[s] = tiles;
+    tiles += (a.seg[s].N + BN - 1) / BN;
+    narrow = narrow && a.seg[s].N % 16 == 0;
+  }
+  for (int s = a.nseg; s <= kGemmMaxSeg; s++) a.tile_start[s] = INT_MAX;
+  a.tile_start[a.nseg] = tiles;
+  const int m64 = (a.M + 63) / 64, ksteps = a.K / kLdwBK, cus = compute_units();
+  if (ksteps < 4) return 0;
+  if (narrow && (long)tiles * m64 * 2 <= cus) {
+    size_t cols = 0;
+    for (int s = 0; s < a.nseg; s++) {
+      a.part_off[s] = (size_t)a.M * cols;
+      cols += (size_t)a.seg[s].N;
+    }
+    a.part_off[a.nseg] = (size_t)a.M * cols;
+    const size_t stride = (a.part_off[a.nseg] + 63) / 64 * 64;
+    long S = cus / ((long)tiles * m64);
+    if (S > ksteps / 4) S = ksteps / 4;  // at least four K-steps per slice: twice the ring's depth in flight
+    if ((size_t)S * stride > few_rows_floats) S = (long)(few_rows_floats / stride);
+    if (S < 2) return 0;
+    *taken = true;
+    a.ksplit = (int)S;
+    a.partial = few_rows;
+    a.partial_stride = stride;
+    const dim3 grid(tiles, m64, (unsigned)S);
+    if (u8)
+      gemm_launch_one<64, 64, true>(grid, st, a);
+    else
+      gemm_ldw_launch<64>(grid, st, a);
+    if (int rc = check_launch(what)) return rc;
+    launch_splitk_reduce(st, a);
+    return check_launch(what);
+  }
+  if (a.nseg == 1 || (long)tiles * m64 >= cus) return 0;  // a group that fills the part as it is stays one launch
+  for (int s = 0; s < a.nseg; s++)
+    *taken = *taken || ((long)((a.seg[s].N + BN - 1) / BN) * m64 * 2 <= cus && a.seg[s].N % 16 == 0);
+  if (!*taken) return 0;
+  for (int s = 0; s < a.nseg; s++) {
+    GemmArgs one = a;
+    one.nseg = 1;
+    one.seg[0] = a.seg[s];
+    if (int rc = launch_gemm(one, u8, st, what, dq, nullptr, 0, 0, few_rows, few_rows_floats)) return rc;
+  }
+  return 0;
+}
+
 int launch_gemm(GemmArgs& a, bool u8, hipStream_t st, const char* what, void* dq, float* partial, size_t partial_stride,
                 int max_split, float* few_rows, size_t few_rows_floats) {
   if (a.M <= 0) return 0;
   if (a.K <= 0 || a.K % 64 != 0) return set_error(FRHIP_ESHAPE, "gemm: K must be a positive multiple of 64");
+  static const bool splitk = env_on("FRHIP_GEMM_SPLITK");
+  static const int force_bm = getenv("FRHIP_GEMM_BM") ? atoi(getenv("FRHIP_GEMM_BM")) : 0;  // measurement aid
+  // binary16 weights go to the kernel with the loader wave (FRHIP_GEMM_LDW=0 selects the other one:
+  // measurement aid); uint8 weights need the registers in between for the dequantisation
+  static const bool ldw = env_on("FRHIP_GEMM_LDW"), few = env_on("FRHIP_GEMM_FEW_ROWS");
+  const bool few_ok = ldw && splitk && few && !force_bm && few_rows;
+  const bool direct = u8 && dq && a.M >= kDequantRows && a.M <= kU8DirectRows;
+  if (few_ok && direct) {
+    bool taken = false;
+    const int rc = launch_few_rows(a, true, st, what, dq, few_rows, few_rows_floats, &taken);
+    if (taken) return rc;
+  }
   if (u8 && dq && a.M >= kDequantRows) {
     // Expanding N x K codes costs 3 bytes of traffic per weight.  The uint8 kernel's in-flight dequantisation costs a launch
     // of many rows about 0.4 x 2 T FLOP per weight at the binary16 kernel's rate, and a launch of few rows cannot be spread
@@ -1090,6 +1183,11 @@ int launch_gemm(GemmArgs& a, bool u8, hipStream_t st, const char* what, void* dq
     if (int rc = dequant_u8_group_async(a.nseg, qs, mxs, rxs, mys, rys, dsts, a.K, ns, st)) return rc;
     u8 = false;
   }
+  if (!u8 && few_ok) {
+    bool taken = false;
+    const int rc = launch_few_rows(a, false, st, what, dq, few_rows, few_rows_floats, &taken);
+    if (taken) return rc;
+  }
   int tiles = 0;
   for (int s = 0; s < a.nseg; s++) {
     a.tile_start[s] = tiles;
@@ -1099,66 +1197,15 @@ int launch_gemm(GemmArgs& a, bool u8, hipStream_t st, const char* what, void* dq
   a.tile_start[a.nseg] = tiles;
   // 128-row tiles unless that leaves fewer than ~1.5 workgroups per CU; then 64-row tiles
   const int m128 = (a.M + 127) / 128;
-  static const int force_bm = getenv("FRHIP_GEMM_BM") ? atoi(getenv("FRHIP_GEMM_BM")) : 0;  // measurement aid
   const bool small = force_bm ? force_bm == 64 : (long)tiles * m128 < (long)compute_units() * 3 / 2;
   static const int force_bk = env_bk();
   const bool deep = force_bk ? force_bk == 128 : true;
   const bool deep_ok = deep && a.K % 128 == 0;
-  // binary16 weights go to the kernel with the loader wave (FRHIP_GEMM_LDW=0 selects the other one:
-  // measurement aid); uint8 weights need the registers in between for the dequantisation
-  static const bool ldw = !(getenv("FRHIP_GEMM_LDW") && atoi(getenv("FRHIP_GEMM_LDW")) == 0);
   // Split K: a single product with few outputs and a long K (ffn value: 1024 x 8192 x 2048) fills the compute units only
   // with 64 x 128 tiles, which ask L2 for 1.5 times the bytes of 128 x 128 tiles per product and are bound by just that
   // (786 MB in 57 us).  With scratch for the partial sums the launch runs ksplit slices of K over 128 x 128 tiles, and a
   // second kernel adds the slices in order and applies the epilogue.  The sums are grouped by slice, so the result can
   // differ from the unsplit launch in the last fp32 bit before the rounding to binary16.  FRHIP_GEMM_SPLITK=0: off.
-  static const bool splitk = !(getenv("FRHIP_GEMM_SPLITK") && atoi(getenv("FRHIP_GEMM_SPLITK")) == 0);
-  // Few rows (a short prompt): 64 x 128 tiles leave most compute units without a workgroup, and a workgroup pulls its
-  // weights through a ring of two K-steps (48 KB in flight), so a launch takes K / 64 round trips to memory however few
-  // rows there are (T = 64, 2048 x 2048: 16 workgroups, 17-25 us for 8 MB).  With scratch for the partial sums such a
-  // launch is split over K into as many slices as there are idle compute units (at least four K-steps each), and the
-  // reduction pass adds the slices in order and applies each product's epilogue.  A group that is too wide for that as a
-  // whole goes out product by product, so that its narrow members still can.  FRHIP_GEMM_FEW_ROWS=0: off.
-  static const bool few = !(getenv("FRHIP_GEMM_FEW_ROWS") && atoi(getenv("FRHIP_GEMM_FEW_ROWS")) == 0);
-  if (!u8 && ldw && splitk && few && !force_bm && few_rows) {
-    const int m64 = (a.M + 63) / 64, ksteps = a.K / kLdwBK, cus = compute_units();
-    bool eligible = (long)tiles * m64 * 2 <= cus && ksteps >= 4;
-    for (int sgi = 0; sgi < a.nseg; sgi++) eligible = eligible && a.seg[sgi].N % 16 == 0;
-    if (eligible) {
-      size_t cols = 0;
-      for (int sgi = 0; sgi < a.nseg; sgi++) {
-        a.part_off[sgi] = (size_t)a.M * cols;
-        cols += (size_t)a.seg[sgi].N;
-      }
-      a.part_off[a.nseg] = (size_t)a.M * cols;
-      const size_t stride = (a.part_off[a.nseg] + 63) / 64 * 64;
-      long S = cus / ((long)tiles * m64);
-      if (S > ksteps / 4) S = ksteps / 4;  // at least four K-steps per slice: twice the ring's depth in flight
-      if ((size_t)S * stride > few_rows_floats) S = (long)(few_rows_floats / stride);
-      if (S >= 2) {
-        a.ksplit = (int)S;
-        a.partial = few_rows;
-        a.partial_stride = stride;
-        gemm_ldw_launch<64>(dim3(tiles, m64, (unsigned)S), st, a);
-        if (int rc = check_launch(what)) return rc;
-        launch_splitk_reduce(st, a);
-        return check_launch(what);
-      }
-    } else if (a.nseg > 1 && ksteps >= 4 && (long)tiles * m64 < cus) {  // a group that fills the part as it is stays one launch
-      bool some = false;
-      for (int sgi = 0; sgi < a.nseg; sgi++)
-        some = some || ((long)((a.seg[sgi].N + BN - 1) / BN) * m64 * 2 <= cus && a.seg[sgi].N % 16 == 0);
-      if (some) {
-        for (int sgi = 0; sgi < a.nseg; sgi++) {
-          GemmArgs one = a;
-          one.nseg = 1;
-          one.seg[0] = a.seg[sgi];
-          if (int rc = launch_gemm(one, false, st, what, nullptr, nullptr, 0, 0, few_rows, few_rows_floats)) return rc;
-        }
-        return 0;
-      }
-    }
-  }
   if (!u8 && ldw && splitk && !force_bm && partial && max_split >= 2 && a.nseg == 1 && a.K >= 4096 && a.seg[0].N % 16 == 0 &&
       (a.seg[0].epi == G_STORE_F16 || a.seg[0].epi == G_STORE_F32 || a.seg[0].epi == G_RESIDUAL || a.seg[0].epi == G_FFN_OUT) &&
       (size_t)a.M * a.seg[0].N <= partial_stride) {

@@ -156,6 +156,12 @@ def test_ffn_seq(T, C_, F_, quant):
     assert_close_f16(x_out.numpy(), ref_x, max_ulp=3, max_frac=0.2, what="x_out", floor_rms=1.0)
 
 
+@pytest.mark.parametrize("T,C_,F_", [(4, 512, 1792), (64, 512, 2048), (65, 768, 3072), (128, 2048, 8192), (129, 512, 1792)])
+def test_ffn_seq_uint8_dequantised_in_the_product(T, C_, F_):
+    """One strip of 64 or 128 rows, split over K; 129 rows are expanded first.  Bounds as in test_ffn_seq."""
+    test_ffn_seq(T, C_, F_, True)
+
+
 @pytest.mark.parametrize("T,C_,F_", [(64, 512, 1792), (1024, 2048, 8192), (1, 512, 1024), (200, 768, 3072)])
 @pytest.mark.parametrize("quant", [False, True])
 def test_ffn_seq_with_the_halving_folded_in(T, C_, F_, quant):
