@@ -91,11 +91,13 @@ int fr_model_run(void *m, const int *ids, int n, float *logits, int capacity) {
 long long fr_model_run_full(void *m, const int *ids, int n, float *logits, long long capacity) {
   return guarded([&]() -> long long {
     auto *model = static_cast<rwkv::Model *>(m);
-    rwkv::Tensor out = rwkv::Copy(
-        rwkv::ModelForwardSeq(model, model->_act_device, std::vector<int>(ids, ids + n), true), rwkv::Device::kCPU);
+    rwkv::Tensor out = rwkv::ModelForwardSeq(model, model->_act_device, std::vector<int>(ids, ids + n), true);
     const long long v = static_cast<long long>(out.numel());
     if (v > capacity) throw FRException("logits buffer too small");
-    std::memcpy(logits, out.data_ptr<float>(), sizeof(float) * static_cast<size_t>(v));
+    if (out.device() == rwkv::Device::kHIP)
+      rwkv::hip::read_to_host(*rwkv::hip::extra_of(model), out, logits);
+    else
+      std::memcpy(logits, out.data_ptr<float>(), sizeof(float) * static_cast<size_t>(v));
     return v;
   });
 }

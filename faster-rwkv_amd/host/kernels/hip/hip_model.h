@@ -11,18 +11,22 @@ namespace rwkv {
 class Model;
 namespace hip {
 
+struct ReadBack;    // pinned ring for large results (read_back.cpp)
 struct DecodePlan;  // fused one-token forward: buffers + captured graphs (model_forward.cpp)
 
 struct ModelExtra {
   Tensor emb_table;                 // [V, C]: one slab; Model::_embd_weights are row views into it
   std::vector<const void *> packed; // keys registered in the weight table, released with the model
   std::shared_ptr<DecodePlan> plan;
+  std::shared_ptr<ReadBack> read_back;
   int32_t last_argmax = -1;               // index of the largest logit of the last fused one-token pass ...
   const void *last_argmax_of = nullptr;   // ... and the logits buffer it belongs to
   ~ModelExtra();
 };
 
 std::shared_ptr<ModelExtra> extra_of(Model *model);
+// A device tensor into `dst` (src.nbytes() bytes of host memory), after the work queued so far; returns when it is there.
+void read_to_host(ModelExtra &ex, const Tensor &src, void *dst);
 bool device_argmax(Model *model, const Tensor &logits, int *id);
 // `steps` greedy tokens from `first_id` with the token choice left on the device (model_forward.cpp).
 bool GreedyDecode(Model *model, int first_id, int steps, int *out_ids, Tensor *last_logits = nullptr);

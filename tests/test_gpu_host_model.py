@@ -365,6 +365,21 @@ def test_full_output_gives_the_logits_of_every_position(model_files):
     m.close()
 
 
+@pytest.mark.parametrize("rows,vocab", [(4, 50000), (13, 65536), (61, 50277)])  # below the ring, 4 chunks, 12 chunks and a remainder
+def test_the_logits_of_a_long_text_arrive_whole(rows, vocab):
+    """Every row of the read-back equals the one-token pass over the same prefix, up to the rounding of the two
+    products (the bound of the test above); a lost, late or misplaced piece is another row's logits."""
+    m = fr.Model("synthetic:v=4,L=2,C=256,F=1024,V=%d,seed=9" % vocab, "hip fp16")
+    ids = np.random.default_rng(rows).integers(0, vocab, rows).astype(np.int32)
+    m.reset()
+    full = m.run_full(ids)
+    assert full.shape == (rows, vocab)
+    m.reset()
+    for t in range(rows):
+        assert np.abs(full[t] - m.run(int(ids[t]))).max() <= 2e-2, t
+    m.close()
+
+
 def test_sampled_generation_follows_the_oracle_sampler(model_files):
     """chat.cpp's loop with a seeded Sampler: the C++ loop on the hip model picks the tokens that the
     sampler oracle picks from the same logits."""
