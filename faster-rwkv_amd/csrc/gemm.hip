@@ -5,10 +5,11 @@
 // Both operands are K-contiguous, which is the layout v_mfma_f32_32x32x16_f16 wants:
 // a lane's A (or B) fragment is 8 consecutive k of one row, i.e. one 16-byte load.
 // Workgroup tile 128x128 (64x128 for launches that would otherwise leave CUs idle), 2x2 compute
-// waves of 64x64 (2x2 MFMA tiles, 64 fp32 accumulators per lane).  Three kernels:
-//   gemm_vw_kernel   binary16 weights, launches large enough for tiles of 128 x 128 and more:
+// waves of 64x64 (2x2 MFMA tiles, 64 fp32 accumulators per lane).  Four kernels:
+//   gemm_vw_kernel   binary16 weights, launches large enough for tiles of 128 x 96 and more:
 //                    tile widths are chosen per launch so that the workgroups fill the compute
 //                    units in whole rounds; loader wave and LDS ring as in gemm_ldw_kernel;
+//   gemm_vw256_kernel  the same with tiles of 256 rows and eight waves that load and multiply;
 //   gemm_ldw_kernel  binary16 weights: a fifth wave streams the tiles global -> LDS directly
 //                    through a ring of four 64-deep K steps; the compute waves never load;
 //   gemm_kernel      uint8 weights: tiles go global -> registers -> LDS (rows padded by 16 bytes
@@ -879,6 +880,9 @@ __global__ __launch_bounds__(320) void gemm_vw_kernel(GemmArgs a) {
 // ahead into the second stage.  (A third stage, which tiles of up to 160 columns leave room for, and loads
 // two steps ahead were measured: no faster, 4099 x 8192 x 2048 166 us against 161.)
 // Rows past the matrix are clamped in the lane offsets, so edge tiles load like the others.
+// What bounds it: a step of 256 x 256 reads 192 KB of fragments from LDS and writes 64 KB to it, 2048 cycles at
+// 128 bytes per cycle, as many as its MFMAs take on each SIMD.  3000 x 5120 x 20480: 825 -> 571 us (1.1 PFLOP/s),
+// 4099 x 2048 x 10240: 230 -> 171 us, against the fixed 128 x 128 tiles both launches had before.
 // ---------------------------------------------------------------------------
 constexpr int kVw256Threads = 512, kVw256ABytes = 256 * kLdwBK * 2;
 
@@ -1094,6 +1098,8 @@ static bool env_on(const char* name) {
 // uint8 weights of at most kU8DirectRows rows (one strip of tiles) are dequantised on their way into LDS, once each:
 // 1 byte of traffic per weight, where the expansion and a binary16 product move 5 (1 in, 2 out, 2 in again).  The
 // slices are those of the binary16 launch, so the sums are the same bits whichever form of the weight is multiplied.
+// 13 rows of 2048 x 10240 (ffn r,k): 18.6 us against 17.7 + 9.5; 8192 x 2048: 13.7 against 15.0 + 8.6; 2048 x 2048:
+// 9.0 against 7.3 + 5.2.  Above 64 rows a second strip would dequantise every code again.
 // *taken stays false, and nothing is launched, if the launch is not of this form.
 constexpr int kU8DirectRows = 64;
 static int launch_few_rows(GemmArgs& a, bool u8, hipStream_t st, const char* what, void* dq, float* few_rows,
