@@ -80,6 +80,7 @@ __global__ __launch_bounds__(256) void ln_mix_seq_kernel(LnMixSeq a) {
 // of one load, two reductions and one store per workgroup, so what counts is how many workgroups
 // a compute unit has to overlap: at T = 1024, C = 2048 four rows per workgroup (one workgroup per
 // CU, every row read 1.25 times) take 8.7 us, two 7.4 us, one (every row read twice) 7.0 us.
+// NG = 3 (C up to 6144): 1000 x 5120 takes 14.2 us, ln_mix_seq_kernel 45.8.
 constexpr int kLnRows = 1;
 
 template <int NG>
@@ -567,6 +568,8 @@ static int launch_ln_mix(int T, int C, const void* x, const void* state, const v
     hipLaunchKernelGGL(ln_mix_rows_kernel<1>, dim3(nwg), dim3(256), 0, st, a);
   else if (C % 8 == 0 && C <= 4096)
     hipLaunchKernelGGL(ln_mix_rows_kernel<2>, dim3(nwg), dim3(256), 0, st, a);
+  else if (C % 8 == 0 && C <= 6144)
+    hipLaunchKernelGGL(ln_mix_rows_kernel<3>, dim3(nwg), dim3(256), 0, st, a);
   else
     hipLaunchKernelGGL(ln_mix_seq_kernel, dim3(T), dim3(256), 4 * (size_t)C, st, a);
   return check_launch("ln_mix_seq");

@@ -162,6 +162,12 @@ def test_ffn_seq_uint8_dequantised_in_the_product(T, C_, F_):
     test_ffn_seq(T, C_, F_, True)
 
 
+@pytest.mark.parametrize("T,C_", [(9, 4096), (5, 4160), (9, 5120), (1, 6144), (3, 6208)])  # two, three groups per thread; beyond them
+def test_ffn_seq_wide_rows(T, C_):
+    """The layernorm and mix of wide rows, at the edges of the register form.  Bounds as in test_ffn_seq."""
+    test_ffn_seq(T, C_, 128, False)
+
+
 @pytest.mark.parametrize("T,C_,F_", [(64, 512, 1792), (1024, 2048, 8192), (1, 512, 1024), (200, 768, 3072)])
 @pytest.mark.parametrize("quant", [False, True])
 def test_ffn_seq_with_the_halving_folded_in(T, C_, F_, quant):
