@@ -80,7 +80,6 @@ __global__ __launch_bounds__(256) void ln_mix_seq_kernel(LnMixSeq a) {
 // of one load, two reductions and one store per workgroup, so what counts is how many workgroups
 // a compute unit has to overlap: at T = 1024, C = 2048 four rows per workgroup (one workgroup per
 // CU, every row read 1.25 times) take 8.7 us, two 7.4 us, one (every row read twice) 7.0 us.
-// NG = 3 (C up to 6144): 1000 x 5120 takes 14.2 us, ln_mix_seq_kernel 45.8.
 constexpr int kLnRows = 1;
 
 template <int NG>
@@ -181,6 +180,79 @@ __global__ __launch_bounds__(256) void ln_mix_rows_kernel(LnMixSeq a) {
       }
       prev = xx;
     }
+  }
+}
+
+// Rows beyond 4096 elements, up to 256 * NE, C % 512 == 0: the row and the one before it stay in registers too, but
+// thread t owns elements t, t + 256, ... as in ln_mix_seq_kernel, and every sum is taken in that kernel's order: the same
+// bits as the general form, at any address.  (Groups of 8 consecutive elements, as above, would be another order of the
+// same sums.)  Bound by its 2-byte loads and stores.  1000 x 5120: 25.4 us, ln_mix_seq_kernel 38.2.
+// C % 512: the compiler unrolls the general form's last loop by two and four, and only in the remainder of an odd count
+// does it round (x - mean) * inv once to binary16 (v_fma_mixlo_f16) instead of to fp32 and then to binary16.
+template <int NE>
+__global__ __launch_bounds__(256) void ln_mix_wide_kernel(LnMixSeq a) {
+  __shared__ float red[2][2][4];
+  const int C = a.C, t = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  h1 xr[2][NE];  // [0]: the row before, [1]: this row
+  const h1* row[2] = {a.x + (size_t)(t ? t - 1 : 0) * C, a.x + (size_t)t * C};
+#pragma unroll
+  for (int n = 0; n < NE; n++) {
+    const int i = tid + n * 256, ic = i < C ? i : 0;
+    xr[0][n] = row[0][ic];
+    xr[1][n] = row[1][ic];
+  }
+  float mean[2], inv[2];
+#pragma unroll
+  for (int r = 0; r < 2; r++) {
+    float s = 0.f;
+#pragma unroll
+    for (int n = 0; n < NE; n++)
+      if (tid + n * 256 < C) s += (float)xr[r][n];
+    s = wave_sum(s);
+    if (lane == 0) red[0][r][wv] = s;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < 2; r++) {
+    float s = 0.f;
+#pragma unroll
+    for (int w = 0; w < 4; w++) s += red[0][r][w];
+    mean[r] = s / (float)C;
+    float q = 0.f;
+#pragma unroll
+    for (int n = 0; n < NE; n++)
+      if (tid + n * 256 < C) {
+        const float d = (float)xr[r][n] - mean[r];
+        q += d * d;
+      }
+    q = wave_sum(q);
+    if (lane == 0) red[1][r][wv] = q;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < 2; r++) {
+    float q = 0.f;
+#pragma unroll
+    for (int w = 0; w < 4; w++) q += red[1][r][w];
+    float var = q / (float)C;
+    var = var > 0.f ? var : 0.f;
+    inv[r] = 1.0f / sqrtf(var + 1e-5f);
+  }
+#pragma unroll
+  for (int n = 0; n < NE; n++) {
+    const int i = tid + n * 256;
+    if (i >= C) break;
+    const h1 g = a.ln_w[i], b = a.ln_b[i];
+    h1 xx[2];
+#pragma unroll
+    for (int r = 0; r < 2; r++) {
+      float p = ((float)xr[r][n] - mean[r]) * inv[r];
+      asm("" : "+v"(p));  // rounded to fp32 before the conversion: no v_fma_mixlo_f16
+      xx[r] = ((h1)p * g) + b;
+    }
+    const h1 sx = t == 0 ? a.state[i] : xx[0];
+    for (int m = 0; m < a.nmix; m++) a.out[m][(size_t)t * C + i] = mix1(xx[1], sx, a.mix[m][i]);
+    if (t == a.T - 1) a.xx_last[i] = xx[1];
   }
 }
 
@@ -568,8 +640,8 @@ static int launch_ln_mix(int T, int C, const void* x, const void* state, const v
     hipLaunchKernelGGL(ln_mix_rows_kernel<1>, dim3(nwg), dim3(256), 0, st, a);
   else if (C % 8 == 0 && C <= 4096)
     hipLaunchKernelGGL(ln_mix_rows_kernel<2>, dim3(nwg), dim3(256), 0, st, a);
-  else if (C % 8 == 0 && C <= 6144)
-    hipLaunchKernelGGL(ln_mix_rows_kernel<3>, dim3(nwg), dim3(256), 0, st, a);
+  else if (C % 512 == 0 && C > 4096 && C <= 6144)
+    hipLaunchKernelGGL(ln_mix_wide_kernel<24>, dim3(T), dim3(256), 0, st, a);
   else
     hipLaunchKernelGGL(ln_mix_seq_kernel, dim3(T), dim3(256), 4 * (size_t)C, st, a);
   return check_launch("ln_mix_seq");

@@ -162,10 +162,65 @@ def test_ffn_seq_uint8_dequantised_in_the_product(T, C_, F_):
     test_ffn_seq(T, C_, F_, True)
 
 
-@pytest.mark.parametrize("T,C_", [(9, 4096), (5, 4160), (9, 5120), (1, 6144), (3, 6208)])  # two, three groups per thread; beyond them
+@pytest.mark.parametrize("T,C_", [(9, 4096), (5, 4160), (9, 5120), (1, 6144), (3, 6208)])  # 16-byte groups; general form; one element at a time (twice); general form
 def test_ffn_seq_wide_rows(T, C_):
-    """The layernorm and mix of wide rows, at the edges of the register form.  Bounds as in test_ffn_seq."""
+    """The layernorm and mix of wide rows, at the edges of the register forms.  Bounds as in test_ffn_seq."""
     test_ffn_seq(T, C_, 128, False)
+
+
+def _ln_rows(x, g, b, strided):
+    """LN of the rows of x in fp32 with the sums taken thread by thread (256 threads: elements t, t + 256, ..., or groups
+    of 8 consecutive ones), then over the lanes of a wave (pairs, fours, eights, rows of 16, the four rows in turn), then
+    over the four waves."""
+    f = np.float32
+    rows, C_ = x.shape
+    if strided:
+        own = np.zeros((rows, -(-C_ // 256) * 256), f)
+        own[:, :C_] = x
+        valid = (np.arange(own.shape[1]) < C_).reshape(-1, 256)
+        own = own.reshape(rows, -1, 256).transpose(1, 0, 2)
+    else:
+        n = -(-C_ // 2048) * 2048
+        own, valid = np.zeros((rows, n), f), np.arange(n) < C_
+        own[:, :C_] = x
+        own = own.reshape(rows, -1, 256, 8).transpose(1, 3, 0, 2).reshape(-1, rows, 256)
+        valid = valid.reshape(-1, 256, 8).transpose(0, 2, 1).reshape(-1, 256)
+
+    def total(v):
+        s = np.zeros((rows, 256), f)
+        for e, ok in zip(v, valid):
+            s = np.where(ok, s + e, s)
+        for _ in range(4):
+            s = s[:, 0::2] + s[:, 1::2]
+        s = s.reshape(rows, 4, 4)
+        w = ((s[:, :, 0] + s[:, :, 1]) + s[:, :, 2]) + s[:, :, 3]
+        return ((w[:, 0] + w[:, 1]) + w[:, 2]) + w[:, 3]
+
+    mean = total(own) / f(C_)
+    d = own - mean[None, :, None]
+    var = np.maximum(total(d * d) / f(C_), f(0))
+    inv = f(1) / np.sqrt(var + f(1e-5))
+    return ((x.astype(f) - mean[:, None]) * inv[:, None]).astype(np.float16) * g + b
+
+
+@pytest.mark.parametrize("C_", [4608, 5120, 6144, 6656])
+def test_layernorm_of_wide_rows_sums_in_one_order(C_):
+    """The new shift state is LN of the last row, bit for bit, with thread t summing elements t, t + 256, ... whichever
+    form of the kernel a width takes (6656: the general one); vectors that start at an odd binary16 address are taken as they are.  (The inputs
+    tell that order from groups of 8 consecutive elements.)"""
+    rows = 96
+    x, g, b = h(rng.standard_normal((rows, C_)) * 2 + 1), h(1 + 0.1 * rng.standard_normal(C_)), h(0.1 * rng.standard_normal(C_))
+    want = _ln_rows(x, g, b, True)
+    assert (want.view(np.uint16) != _ln_rows(x, g, b, False).view(np.uint16)).any(axis=1).sum() >= 3
+    odd = [keep(np.concatenate([h([7]), v])) for v in (h(rng.standard_normal(C_)), g, b, h(rng.uniform(0, 1, C_)), h(rng.uniform(0, 1, C_)))]
+    kw, vw, rw = (make_weight(h(rng.standard_normal(s) * 0.02), False)[0] for s in ((C_, 64), (64, C_), (C_, C_)))
+    x_dev, x_out, xx_out = keep(x), DevBuf.empty((8, C_), np.float16), DevBuf.empty(C_ + 1, np.float16)
+    ws = DevBuf(L().frhip_seq_workspace_bytes(8, C_, 64))
+    for last in range(rows):
+        T = min(last + 1, 1 + last % 8)
+        fr.check(L().frhip_ffn_seq(T, C_, 64, x_dev.ptr + 2 * C_ * (last + 1 - T), *[v.ptr + 2 for v in odd], kw.ref, vw.ref,
+                                   rw.ref, x_out.ptr, xx_out.ptr + 2, 0, ws.ptr, None))
+        assert np.array_equal(xx_out.numpy()[1:].view(np.uint16), want[last].view(np.uint16)), last
 
 
 @pytest.mark.parametrize("T,C_,F_", [(64, 512, 1792), (1024, 2048, 8192), (1, 512, 1024), (200, 768, 3072)])
