@@ -1165,7 +1165,10 @@ int launch_gemm(GemmArgs& a, bool u8, hipStream_t st, const char* what, void* dq
   // measurement aid); uint8 weights need the registers in between for the dequantisation
   static const bool ldw = env_on("FRHIP_GEMM_LDW"), few = env_on("FRHIP_GEMM_FEW_ROWS");
   const bool few_ok = ldw && splitk && few && !force_bm && few_rows;
-  const bool direct = u8 && dq && a.M >= kDequantRows && a.M <= kU8DirectRows;
+  bool direct = u8 && dq && a.M >= kDequantRows && a.M <= kU8DirectRows;
+  for (int s = 0; s < a.nseg; s++)  // the uint8 kernel reads codes and row scales 16 bytes at a time; the expansion takes any address
+    direct = direct && ((reinterpret_cast<uintptr_t>(a.seg[s].B) | reinterpret_cast<uintptr_t>(a.seg[s].ry) |
+                         reinterpret_cast<uintptr_t>(a.seg[s].my)) & 15) == 0;
   if (few_ok && direct) {
     bool taken = false;
     const int rc = launch_few_rows(a, true, st, what, dq, few_rows, few_rows_floats, &taken);

@@ -1,4 +1,6 @@
 """GPU parity tests of the seq-mode (prompt) operators against the oracle."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -160,6 +162,27 @@ def test_ffn_seq(T, C_, F_, quant):
 def test_ffn_seq_uint8_dequantised_in_the_product(T, C_, F_):
     """One strip of 64 or 128 rows, split over K; 129 rows are expanded first.  Bounds as in test_ffn_seq."""
     test_ffn_seq(T, C_, F_, True)
+
+
+@pytest.mark.parametrize("T", [4, 13, 64, 65])
+def test_ffn_seq_uint8_scales_at_any_address(T):
+    """Row scales and codes that do not start at a multiple of 16 bytes are taken, with the same bits."""
+    C_, F_ = 512, 1792
+    x, sx = h(rng.standard_normal((T, C_)) * 2), h(rng.standard_normal(C_))
+    vecs = [keep(v) for v in (x, sx, h(1 + 0.1 * rng.standard_normal(C_)), h(0.1 * rng.standard_normal(C_)), h(rng.uniform(0, 1, C_)), h(rng.uniform(0, 1, C_)))]
+    weights = [make_weight(h(rng.standard_normal(s) * 0.02), True)[0] for s in ((C_, F_), (F_, C_), (C_, C_))]
+    moved = []
+    for w in weights:
+        q, mx, rx, my, ry = w.parts
+        ptrs = [keep(np.concatenate([np.zeros(b, np.uint8), np.ascontiguousarray(v).reshape(-1).view(np.uint8)])).ptr + b
+                for v, b in ((q.T, 4), (mx, 2), (rx, 2), (my, 2), (ry, 2))]
+        moved.append(fr.Weight(*ptrs, w.K, w.N, fr.U8))
+    outs = []
+    for kw, vw, rw in ([w.ref for w in weights], [C.byref(m) for m in moved]):
+        x_out, xx_out, ws = DevBuf.empty((T, C_), np.float16), DevBuf.empty(C_, np.float16), DevBuf(L().frhip_seq_workspace_bytes(T, C_, F_))
+        fr.check(L().frhip_ffn_seq(T, C_, F_, *[v.ptr for v in vecs], kw, vw, rw, x_out.ptr, xx_out.ptr, 0, ws.ptr, None))
+        outs.append(x_out.numpy())
+    assert np.array_equal(outs[0].view(np.uint16), outs[1].view(np.uint16))
 
 
 @pytest.mark.parametrize("T,C_", [(9, 4096), (5, 4160), (9, 5120), (1, 6144), (3, 6208)])  # 16-byte groups; general form; one element at a time (twice); general form
