@@ -406,6 +406,15 @@ __device__ __forceinline__ const unsigned char* uniform_ptr(const void* p) {
   return reinterpret_cast<const unsigned char*>(((unsigned long long)hi << 32) | lo);
 }
 
+// The barrier between K-steps whose waits the kernel places itself.  The builtin is no memory fence for the compiler:
+// without the empty statements it could move a fragment read across (nothing else stands between the barrier and the
+// reads in a step that issues no loads).  No instruction of its own.
+__device__ __forceinline__ void step_barrier() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
 constexpr int kLdwThreads = 320;
 constexpr int kLdwStages = 4;
 constexpr int kLdwBK = 64;
@@ -496,7 +505,7 @@ __global__ __launch_bounds__(kLdwThreads) void gemm_ldw_kernel(GemmArgs a) {
       } else {
         __builtin_amdgcn_s_waitcnt(0x0F70);    // vmcnt(0)
       }
-      __builtin_amdgcn_s_barrier();            // barrier k: step k may be read, step k-1 has been read by all
+      step_barrier();            // barrier k: step k may be read, step k-1 has been read by all
       if (k + 2 < nk) issue(k + 2);            // into the slot of step k-2
     }
     return;
@@ -512,7 +521,7 @@ __global__ __launch_bounds__(kLdwThreads) void gemm_ldw_kernel(GemmArgs a) {
 #pragma unroll
       for (int v = 0; v < 16; v++) acc[i][j][v] = 0.f;
   for (int k = 0; k < nk; k++) {
-    __builtin_amdgcn_s_barrier();
+    step_barrier();
     const unsigned char* st = gemm_smem + (k % kLdwStages) * kStageBytes;
     h8 fa[4][MI], fb[4][2];
 #pragma unroll
@@ -765,7 +774,7 @@ __device__ __forceinline__ void vw_loader(const GemmSeg& sg, unsigned char* smem
       __builtin_amdgcn_s_waitcnt(((kPer >> 4) << 14) | 0x0F70 | (kPer & 15));  // vmcnt(kPer): step k has landed
     else
       __builtin_amdgcn_s_waitcnt(0x0F70);
-    __builtin_amdgcn_s_barrier();  // step k may be read; step k-1 has been read by all
+    step_barrier();  // step k may be read; step k-1 has been read by all
     if (k + 2 < nk) {
       issue(k + 2, slot);          // ns >= 3: not the slot of step k or k+1
       slot = slot + 1 == ns ? 0 : slot + 1;
@@ -787,7 +796,7 @@ __device__ __forceinline__ void vw_mma(const GemmArgs& a, const GemmSeg& sg, con
   const int nk = a.K / kLdwBK;
   int slot = 0;
   for (int k = 0; k < nk; k++) {
-    __builtin_amdgcn_s_barrier();
+    step_barrier();
     const unsigned char* st = smem + slot * stage_bytes;
     slot = slot + 1 == ns ? 0 : slot + 1;
     h8 fa[4][2], fb[4][NJ];
@@ -929,7 +938,7 @@ __device__ __forceinline__ void vw256_body(const GemmArgs& a, const GemmSeg& sg,
     // this wave's loads of step k have landed and its fragments of step k-1 are in registers; behind the
     // barrier that holds for all eight, so step k may be read and the slot of step k-1 refilled
     __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0)
-    __builtin_amdgcn_s_barrier();
+    step_barrier();
     if (k + 1 < nk) issue(k + 1);
     const unsigned char* st = smem + (k & 1) * stage_bytes;
 #pragma unroll

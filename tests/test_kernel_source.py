@@ -1,0 +1,20 @@
+"""Properties of the kernels' source that no run shows reliably."""
+import glob
+import os
+import re
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "faster-rwkv_amd", "csrc")
+
+
+def test_bare_barriers_stand_between_compiler_fences():
+    """The barrier builtin does not keep the compiler from moving LDS accesses across it (__syncthreads does): it has an
+    empty statement that clobbers memory on either side."""
+    fence = 'asm volatile("" ::: "memory");'
+    found = 0
+    for path in sorted(glob.glob(os.path.join(CSRC, "*.hip")) + glob.glob(os.path.join(CSRC, "*.h"))):
+        lines = [re.sub(r"\s*//.*", "", line).strip() for line in open(path)]
+        for i, line in enumerate(lines):
+            if "__builtin_amdgcn_s_barrier" in line:
+                found += 1
+                assert (lines[i - 1], lines[i + 1]) == (fence, fence), "%s:%d" % (os.path.basename(path), i + 1)
+    assert found
