@@ -103,6 +103,7 @@ _SIGS = {
     "frhip_argmax_blocks_f32_mirror": (_i, [_vp, _i, _vp, _vp, _i, _vp]),
     "frhip_gemm": (_i, [_vp, _WP, _vp, _i, _i, _vp]),
     "frhip_gemm_act": (_i, [_vp, _WP, _vp, _i, _i, _vp]),
+    "frhip_gemm_route": (_i, [_i, _i, _i, _vp, _i, _vp]),
     "frhip_copy_probe": (_i, [_vp, _vp, _sz, _vp]),
     "frhip_read_probe": (_i, [_vp, _sz, _vp, _vp]),
     "frhip_mfma_probe": (_i, [_i, _i, _vp, _vp, _vp, _vp]),

@@ -988,14 +988,41 @@ __global__ __launch_bounds__(kVw256Threads) void gemm_vw256_kernel(GemmArgs a) {
   }
 }
 
-// Cuts the launch into tiles of bm rows (128: gemm_vw_kernel, 256: gemm_vw256_kernel): the fewest rounds over
-// `cus` compute units whose widest tile fits.  Returns what the launch is expected to take, or 0: it is too small
-// for tiles of at least bm x 96 (the other kernels' 64-row tiles serve it better) or too ragged.
-// The expectation is rounds x (fixed + slope x widest tile), in 0.1 us at K = 2048; both parts grow with K alike.
-// Measured rounds, us: 128 rows, widths 5 / 6 / 8: 26.4 / 30.5 / 38.2; 256 rows, 3 / 4 / 5 / 6 / 8: 30.3 / 38.7 /
-// 46.0 / 51.9 / 66.8.  256-row tiles are the cheaper ones per product from about six blocks on, and where they
-// save a round.
-static int plan_vw(GemmArgs& a, int bm, int cus, dim3* grid, size_t* lds) {
+// How one launch of binary16 weights, not split over K, is cut into tiles.
+struct GemmRoute {
+  int rows = 0;        // of a tile: 64 (gemm_ldw_kernel<64>), 128 (gemm_vw_kernel), 256 (gemm_vw256_kernel); 0: none of these
+  int blocks = 0;      // widest tile, in blocks of 32 columns
+  int rounds = 0;      // over the compute units
+  double us = 0;       // what the launch is expected to take
+  dim3 grid;
+  size_t lds = 0;
+  GemmArgs a;          // with the tile tables of this cut
+};
+
+static long tiles64(const GemmArgs& a) {
+  long n = 0;
+  for (int s = 0; s < a.nseg; s++) n += (long)((a.seg[s].N + BN - 1) / BN) * ((a.M + 63) / 64);
+  return n;
+}
+
+// Expected times, us, with k = K / 2048: 2 + rounds x (a part that does not depend on K + k x (fixed + slope x widest
+// tile)).  Fitted to 825 products of 65 to 4099 rows, K 768 to 20480, N 768 to 65536, weights from memory: the kernels
+// chosen by them take 0.3 % longer than the best of each product's, none but a few at equal prices more than 4 %.
+// Rounds at K = 2048 as measured: 64 rows 14-18; 128 rows, widths 3 / 5 / 8: 22 / 26 / 38; 256 rows, widths 3 / 5 / 7 /
+// 8: 36 / 44 / 54 / 65 (the widest tiles of full strips run at the lowest clock).  300 x 2048 x 6144: 19.2 us as one
+// round of 64-row tiles, 22.7 as 128 x 96; 3000 x 2048 x 8192: 105.5 as 256 rows, 119 as 128; 640 x 2048 x 65536, three
+// strips of 256 rows, half of the last one empty: 200 as 128 rows, 217 as 256.
+static double us_64(int rounds, double k) { return 2 + rounds * (2.4 + 14.2 * k); }
+static double us_128(int rounds, double k, int w) { return 2 + rounds * (5 + k * (5 + 3.55 * w)); }
+static double us_256(int rounds, double k, int w) { return 2 + rounds * (6.6 + k * (11.8 + 5.45 * w + (w == 8 ? 3 : 0))); }
+constexpr double kLaunchUs = 3;  // one more launch
+
+// Cuts the launch into tiles of bm rows (128 or 256): the fewest rounds over `cus` compute units whose widest tile
+// fits.  r.rows stays 0 if it is too small for tiles of at least bm x 96, or too ragged.
+static GemmRoute plan_vw(const GemmArgs& args, int bm, int cus) {
+  GemmRoute r;
+  r.a = args;
+  GemmArgs& a = r.a;
   const int mt = (a.M + bm - 1) / bm;
   const int abytes = bm * kLdwBK * 2;
   int cb[kGemmMaxSeg], total = 0;
@@ -1019,8 +1046,8 @@ static int plan_vw(GemmArgs& a, int bm, int cus, dim3* grid, size_t* lds) {
     while (used < P) {
       int best = 0;
       for (int s = 1; s < a.nseg; s++) {
-        const long l = (long)cb[s] * t[best], r = (long)cb[best] * t[s];
-        if (l > r || (l == r && heavy(s) > heavy(best))) best = s;
+        const long l = (long)cb[s] * t[best], q = (long)cb[best] * t[s];
+        if (l > q || (l == q && heavy(s) > heavy(best))) best = s;
       }
       t[best]++;
       used++;
@@ -1032,7 +1059,7 @@ static int plan_vw(GemmArgs& a, int bm, int cus, dim3* grid, size_t* lds) {
       minw = cb[s] / t[s] < minw ? cb[s] / t[s] : minw;
     }
     if (maxw > kVwMaxW) continue;
-    if (minw < 2 || maxw < 3) return 0;
+    if (minw < 2 || maxw < 3) return r;
     int tiles = 0;
     for (int s = 0; s < a.nseg; s++) {
       a.tile_start[s] = tiles;
@@ -1045,12 +1072,61 @@ static int plan_vw(GemmArgs& a, int bm, int cus, dim3* grid, size_t* lds) {
     a.vw_maxw = maxw;
     const size_t stage = abytes + (size_t)maxw * 4096;
     a.vw_ns = bm == 256 ? 2 : stage * 4 <= 160 * 1024 ? 4 : 3;
-    if (stage * a.vw_ns > 160 * 1024) return 0;
-    *lds = stage * a.vw_ns;
-    *grid = dim3(tiles, mt);
-    return rounds * (bm == 128 ? 75 + 39 * maxw : 100 + 72 * maxw);
+    if (stage * a.vw_ns > 160 * 1024) return r;
+    r.lds = stage * a.vw_ns;
+    r.grid = dim3(tiles, mt);
+    r.blocks = maxw;
+    r.rounds = rounds;
+    r.us = bm == 128 ? us_128(rounds, a.K / 2048.0, maxw) : us_256(rounds, a.K / 2048.0, maxw);
+    r.rows = bm;
+    return r;
   }
-  return 0;
+  return r;
+}
+
+// The cheapest cut.  rows stays 0 where the planned tiles do not fit and fixed 64-row tiles take more than a round.
+static GemmRoute gemm_route(const GemmArgs& a, int cus) {
+  static const int force_bm = getenv("FRHIP_GEMM_VW_BM") ? atoi(getenv("FRHIP_GEMM_VW_BM")) : 0;  // measurement aid
+  GemmRoute r = plan_vw(a, 128, cus);
+  if (force_bm != 128) {
+    GemmRoute r2 = plan_vw(a, 256, cus);
+    if (r2.rows && (!r.rows || r2.us < r.us || force_bm == 256)) r = r2;
+  }
+  const int rounds = (int)((tiles64(a) + cus - 1) / cus);
+  const double us = us_64(rounds, a.K / 2048.0);
+  if (r.rows ? us < r.us && !force_bm : rounds == 1) {
+    r.rows = 64;
+    r.blocks = BN / 32;
+    r.rounds = rounds;
+    r.us = us;
+    r.a = a;
+    int tiles = 0;
+    for (int s = 0; s < a.nseg; s++) {
+      r.a.tile_start[s] = tiles;
+      tiles += (a.seg[s].N + BN - 1) / BN;
+    }
+    for (int s = a.nseg; s <= kGemmMaxSeg; s++) r.a.tile_start[s] = INT_MAX;
+    r.a.tile_start[a.nseg] = tiles;
+    r.grid = dim3(tiles, (a.M + 63) / 64);
+  }
+  return r;
+}
+
+// A grouped launch whose products are cheaper one by one (2048 columns in one round of 64 x 128 tiles, 8192 in two of
+// 128 x 192, together three) goes out as separate launches.  FRHIP_GEMM_SEPARATE=0: never.
+static bool one_by_one(const GemmArgs& a, const GemmRoute& whole, int cus) {
+  static const bool separate = !(getenv("FRHIP_GEMM_SEPARATE") && atoi(getenv("FRHIP_GEMM_SEPARATE")) == 0);
+  if (!separate || a.nseg < 2) return false;
+  double us = kLaunchUs * (a.nseg - 1);
+  for (int s = 0; s < a.nseg; s++) {
+    GemmArgs one = a;
+    one.nseg = 1;
+    one.seg[0] = a.seg[s];
+    const GemmRoute r = gemm_route(one, cus);
+    if (!r.rows) return false;
+    us += r.us;
+  }
+  return whole.rows ? us < whole.us : true;
 }
 
 static void gemm_vw_launch(int bm, dim3 grid, size_t lds, hipStream_t st, const GemmArgs& a) {
@@ -1247,52 +1323,22 @@ int launch_gemm(GemmArgs& a, bool u8, hipStream_t st, const char* what, void* dq
   }
   // FRHIP_GEMM_VW=0 keeps binary16 launches on the fixed 128 / 64 x 128 tiles (measurement aid)
   static const bool vw = !(getenv("FRHIP_GEMM_VW") && atoi(getenv("FRHIP_GEMM_VW")) == 0);
-  static const int force_vw_bm = getenv("FRHIP_GEMM_VW_BM") ? atoi(getenv("FRHIP_GEMM_VW_BM")) : 0;  // measurement aid
   if (!u8 && ldw && vw && !force_bm) {
-    struct Plan {
-      GemmArgs a;
-      dim3 grid;
-      size_t lds = 0;
-      int bm = 0, cost = 0;
-    };
-    auto plan = [&](const GemmArgs& g) {
-      Plan p1, p2;
-      p1.a = p2.a = g;
-      p1.bm = 128, p2.bm = 256;
-      p1.cost = plan_vw(p1.a, 128, compute_units(), &p1.grid, &p1.lds);
-      p2.cost = force_vw_bm == 128 ? 0 : plan_vw(p2.a, 256, compute_units(), &p2.grid, &p2.lds);
-      return p2.cost && (!p1.cost || p2.cost < p1.cost || force_vw_bm == 256) ? p2 : p1;
-    };
-    const Plan p = plan(a);
-    // A grouped launch whose products are cheaper one by one (2048 columns in one round of 64 x 128 tiles, 8192 in
-    // one round of 128 x 256, together two rounds) goes out as separate launches.  One round of 64-row tiles takes
-    // 16.5 us at K = 2048, another launch about 3 us.
-    static const bool separate = !(getenv("FRHIP_GEMM_SEPARATE") && atoi(getenv("FRHIP_GEMM_SEPARATE")) == 0);
-    if (separate && a.nseg > 1) {
-      bool known = true;
-      int sum = 30 * (a.nseg - 1);
-      for (int sgi = 0; sgi < a.nseg && known; sgi++) {
+    const GemmRoute r = gemm_route(a, compute_units());
+    if (one_by_one(a, r, compute_units())) {
+      for (int sgi = 0; sgi < a.nseg; sgi++) {
         GemmArgs one = a;
         one.nseg = 1;
         one.seg[0] = a.seg[sgi];
-        const long t64 = (long)((a.seg[sgi].N + BN - 1) / BN) * ((a.M + 63) / 64);
-        const int c = plan(one).cost;
-        known = c != 0 || t64 <= compute_units();
-        sum += c ? c : 165;
+        if (int rc = launch_gemm(one, false, st, what, nullptr, nullptr, 0, 0, nullptr, 0)) return rc;
       }
-      const long t64g = (long)tiles * ((a.M + 63) / 64);
-      if (known && (p.cost ? sum < p.cost : t64g > compute_units())) {
-        for (int sgi = 0; sgi < a.nseg; sgi++) {
-          GemmArgs one = a;
-          one.nseg = 1;
-          one.seg[0] = a.seg[sgi];
-          if (int rc = launch_gemm(one, false, st, what, nullptr, nullptr, 0, 0, nullptr, 0)) return rc;
-        }
-        return 0;
-      }
+      return 0;
     }
-    if (p.cost) {
-      gemm_vw_launch(p.bm, p.grid, p.lds, st, p.a);
+    if (r.rows) {
+      if (r.rows == 64)
+        gemm_ldw_launch<64>(r.grid, st, r.a);
+      else
+        gemm_vw_launch(r.rows, r.grid, r.lds, st, r.a);
       return check_launch(what);
     }
   }
@@ -1345,6 +1391,36 @@ extern "C" int frhip_gemm(const void* x, const frhip_weight* w, void* y, int T, 
   a.K = w->K;
   gemm_add_seg(a, x, w, y, out_dtype == FRHIP_F32 ? G_STORE_F32 : G_STORE_F16);
   return launch_gemm(a, w->dtype == FRHIP_U8, static_cast<hipStream_t>(s), "gemm");
+}
+
+extern "C" int frhip_gemm_route(int T, int K, int nproducts, const int* N, int compute_units, int* out) {
+  if (!N || !out) return set_error(FRHIP_EINVAL, "gemm_route: null pointer");
+  if (T <= 0 || K <= 0 || K % 64 != 0 || nproducts < 1 || nproducts > kGemmMaxSeg || compute_units < 1)
+    return set_error(FRHIP_ESHAPE, "gemm_route: no such launch");
+  GemmArgs a;
+  memset(&a, 0, sizeof(a));
+  a.M = T;
+  a.K = K;
+  for (int s = 0; s < nproducts; s++) {
+    if (N[s] <= 0) return set_error(FRHIP_ESHAPE, "gemm_route: no such launch");
+    a.seg[s].N = N[s];
+  }
+  a.nseg = nproducts;
+  const GemmRoute whole = gemm_route(a, compute_units);
+  const bool split = one_by_one(a, whole, compute_units);
+  for (int s = 0; s < nproducts; s++) {
+    GemmRoute r = whole;
+    if (split) {
+      GemmArgs one = a;
+      one.nseg = 1;
+      one.seg[0] = a.seg[s];
+      r = gemm_route(one, compute_units);
+    }
+    out[3 * s] = r.rows;
+    out[3 * s + 1] = r.blocks;
+    out[3 * s + 2] = r.rounds;
+  }
+  return split ? nproducts : 1;
 }
 
 static_assert(FRHIP_ACT_SIGMOID == G_SIGMOID && FRHIP_ACT_RELU2 == G_RELU2 && FRHIP_ACT_SILU == G_SILU, "activation codes");
