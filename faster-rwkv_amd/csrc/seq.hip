@@ -186,20 +186,24 @@ __global__ __launch_bounds__(256) void ln_mix_rows_kernel(LnMixSeq a) {
 // Rows beyond 4096 elements, up to 256 * NE, C % 512 == 0: the row and the one before it stay in registers too, but
 // thread t owns elements t, t + 256, ... as in ln_mix_seq_kernel, and every sum is taken in that kernel's order: the same
 // bits as the general form, at any address.  (Groups of 8 consecutive elements, as above, would be another order of the
-// same sums.)  Bound by its 2-byte loads and stores.  1000 x 5120: 25.4 us, ln_mix_seq_kernel 38.2.
+// same sums.)  Few rows are bound by the chain of loads, so
+// each batch of them goes out together; many by the 2-byte loads and stores.  1000 x 5120: 14.5 us (13 rows: 5.7),
+// ln_mix_seq_kernel 37.7 (29.9).
 // C % 512: the compiler unrolls the general form's last loop by two and four, and only in the remainder of an odd count
 // does it round (x - mean) * inv once to binary16 (v_fma_mixlo_f16) instead of to fp32 and then to binary16.
 template <int NE>
 __global__ __launch_bounds__(256) void ln_mix_wide_kernel(LnMixSeq a) {
   __shared__ float red[2][2][4];
   const int C = a.C, t = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  h1 xr[2][NE];  // [0]: the row before, [1]: this row
+  h1 xr[2][NE], gam[NE], bet[NE];  // [0]: the row before, [1]: this row
   const h1* row[2] = {a.x + (size_t)(t ? t - 1 : 0) * C, a.x + (size_t)t * C};
 #pragma unroll
   for (int n = 0; n < NE; n++) {
     const int i = tid + n * 256, ic = i < C ? i : 0;
     xr[0][n] = row[0][ic];
     xr[1][n] = row[1][ic];
+    gam[n] = a.ln_w[ic];
+    bet[n] = a.ln_b[ic];
   }
   float mean[2], inv[2];
 #pragma unroll
@@ -240,19 +244,30 @@ __global__ __launch_bounds__(256) void ln_mix_wide_kernel(LnMixSeq a) {
   }
 #pragma unroll
   for (int n = 0; n < NE; n++) {
-    const int i = tid + n * 256;
-    if (i >= C) break;
-    const h1 g = a.ln_w[i], b = a.ln_b[i];
-    h1 xx[2];
 #pragma unroll
     for (int r = 0; r < 2; r++) {
       float p = ((float)xr[r][n] - mean[r]) * inv[r];
       asm("" : "+v"(p));  // rounded to fp32 before the conversion: no v_fma_mixlo_f16
-      xx[r] = ((h1)p * g) + b;
+      xr[r][n] = ((h1)p * gam[n]) + bet[n];
     }
-    const h1 sx = t == 0 ? a.state[i] : xx[0];
-    for (int m = 0; m < a.nmix; m++) a.out[m][(size_t)t * C + i] = mix1(xx[1], sx, a.mix[m][i]);
-    if (t == a.T - 1) a.xx_last[i] = xx[1];
+  }
+  if (t == 0) {
+#pragma unroll
+    for (int n = 0; n < NE; n++) xr[0][n] = a.state[tid + n * 256 < C ? tid + n * 256 : 0];
+  }
+  for (int m = 0; m < a.nmix; m++) {  // the loads of one vector together, then its stores
+    h1 mx[NE];
+#pragma unroll
+    for (int n = 0; n < NE; n++) mx[n] = a.mix[m][tid + n * 256 < C ? tid + n * 256 : 0];
+    h1* out = a.out[m] + (size_t)t * C;
+#pragma unroll
+    for (int n = 0; n < NE; n++)
+      if (tid + n * 256 < C) out[tid + n * 256] = mix1(xr[1][n], xr[0][n], mx[n]);
+  }
+  if (t == a.T - 1) {
+#pragma unroll
+    for (int n = 0; n < NE; n++)
+      if (tid + n * 256 < C) a.xx_last[tid + n * 256] = xr[1][n];
   }
 }
 
