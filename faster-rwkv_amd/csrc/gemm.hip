@@ -9,7 +9,8 @@
 //   gemm_vw_kernel   binary16 weights, launches large enough for tiles of 128 x 96 and more:
 //                    tile widths are chosen per launch so that the workgroups fill the compute
 //                    units in whole rounds; loader wave and LDS ring as in gemm_ldw_kernel;
-//   gemm_vw256_kernel  the same with tiles of 256 rows and eight waves that load and multiply;
+//                    (128 rows; 256 rows where all tiles are whole and narrow)
+//   gemm_vw256_kernel  tiles of 256 rows and eight waves that load and multiply;
 //   gemm_ldw_kernel  binary16 weights: a fifth wave streams the tiles global -> LDS directly
 //                    through a ring of four 64-deep K steps; the compute waves never load;
 //   gemm_kernel      uint8 weights: tiles go global -> registers -> LDS (rows padded by 16 bytes
@@ -710,14 +711,16 @@ static void gemm_ldw_launch(dim3 grid, hipStream_t st, const GemmArgs& a) {
 // 32-column blocks; the loops are instantiated per block count, so the products are the same
 // MFMAs in the same k order as in the other kernels and the results are bit-identical.  Loader
 // wave, LDS ring (three or four K-steps of 64, whatever fits 160 KB at the launch's widest tile)
-// and swizzle are those of gemm_ldw_kernel.  Tiles of 256 rows: gemm_vw256_kernel below.
+// and swizzle are those of gemm_ldw_kernel.  gemm_vw_kernel<256> has eight MFMA waves (4 x 2 of
+// 64 rows each) and takes whole tiles of at most 160 columns; gemm_vw256_kernel below takes the others.
 // ---------------------------------------------------------------------------
 constexpr int kVwMaxW = 8, kVwMaxRounds = 32;
+constexpr int kVw256LoaderMaxW = 5;  // three stages of (256 + 160) x 64 halves are 156 KB of the 160 KB
 
-template <int W>
+template <int BM, int W>
 __device__ __forceinline__ void vw_loader(const GemmSeg& sg, unsigned char* smem, int stage_bytes, int ns, int m0, int n0,
                                           int M, int N, int K, int lane) {
-  constexpr int BM = 128, kVwABytes = BM * kLdwBK * 2;
+  constexpr int kVwABytes = BM * kLdwBK * 2;
   constexpr int kAInstr = kVwABytes / 1024, kBInstr = 4 * W, kPer = kAInstr + kBInstr;
   static_assert(kPer <= 63, "the wait counter's range");
   const int lr = lane >> 3, ls = (lane & 7) ^ lr;
@@ -782,10 +785,10 @@ __device__ __forceinline__ void vw_loader(const GemmSeg& sg, unsigned char* smem
   }
 }
 
-template <int NJ>
+template <int BM, int NJ>
 __device__ __forceinline__ void vw_mma(const GemmArgs& a, const GemmSeg& sg, const unsigned char* smem, int stage_bytes, int ns,
                                        int brow0, int m0, int n0, int M, int N, bool full, int lane, int wm) {
-  constexpr int kVwABytes = 128 * kLdwBK * 2;
+  constexpr int kVwABytes = BM * kLdwBK * 2;
   f16v acc[2][NJ];
 #pragma unroll
   for (int i = 0; i < 2; i++)
@@ -799,25 +802,31 @@ __device__ __forceinline__ void vw_mma(const GemmArgs& a, const GemmSeg& sg, con
     step_barrier();
     const unsigned char* st = smem + slot * stage_bytes;
     slot = slot + 1 == ns ? 0 : slot + 1;
-    h8 fa[4][2], fb[4][NJ];
+    // fragments of KG x 16 k are requested together; with eight MFMA waves and the loader a lane has 168
+    // registers and holds two of the four k-blocks of a step at a time
+    constexpr int KG = BM == 128 ? 4 : 2;
 #pragma unroll
-    for (int kb = 0; kb < 4; kb++) {
-      const int q = kb * 2 + (lane >> 5);
+    for (int kh = 0; kh < 4; kh += KG) {
+      h8 fa[KG][2], fb[KG][NJ];
 #pragma unroll
-      for (int i = 0; i < 2; i++) fa[kb][i] = *reinterpret_cast<const h8*>(st + ldw_at(wm * 64 + i * 32 + (lane & 31), q));
+      for (int kb = 0; kb < KG; kb++) {
+        const int q = (kh + kb) * 2 + (lane >> 5);
 #pragma unroll
-      for (int j = 0; j < NJ; j++)
-        fb[kb][j] = *reinterpret_cast<const h8*>(st + kVwABytes + ldw_at(brow0 + j * 32 + (lane & 31), q));
-    }
-#pragma unroll
-    for (int kb = 0; kb < 4; kb++)
-#pragma unroll
-      for (int i = 0; i < 2; i++)
+        for (int i = 0; i < 2; i++) fa[kb][i] = *reinterpret_cast<const h8*>(st + ldw_at(wm * 64 + i * 32 + (lane & 31), q));
 #pragma unroll
         for (int j = 0; j < NJ; j++)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[kb][i], fb[kb][j], acc[i][j], 0, 0, 0);
+          fb[kb][j] = *reinterpret_cast<const h8*>(st + kVwABytes + ldw_at(brow0 + j * 32 + (lane & 31), q));
+      }
+#pragma unroll
+      for (int kb = 0; kb < KG; kb++)
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+          for (int j = 0; j < NJ; j++)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[kb][i], fb[kb][j], acc[i][j], 0, 0, 0);
+    }
   }
-  if (full)
+  if (BM == 256 || full)  // 256 rows: whole tiles only
     gemm_epilogue_t<2, NJ, true>(a, sg, acc, m0 + wm * 64, n0 + brow0, M, N, lane);
   else
     gemm_epilogue_t<2, NJ, false>(a, sg, acc, m0 + wm * 64, n0 + brow0, M, N, lane);
@@ -837,8 +846,11 @@ __device__ __forceinline__ void xcd_tile(int& bx, int& by) {
   by = 4 * blk + rem % bw;
 }
 
-__global__ __launch_bounds__(320) void gemm_vw_kernel(GemmArgs a) {
-  constexpr int BM = 128, kVwABytes = BM * kLdwBK * 2, kLoader = 4;  // four MFMA waves of 64 rows x half the width, then the loader
+// BM / 32 MFMA waves of 64 rows x half the width, then the loader.  BM = 256: launches of whole tiles of at most
+// kVw256LoaderMaxW blocks.
+template <int BM>
+__global__ __launch_bounds__(BM * 2 + 64) void gemm_vw_kernel(GemmArgs a) {
+  constexpr int kVwABytes = BM * kLdwBK * 2, kLoader = BM / 32, kCap = BM == 128 ? kVwMaxW : kVw256LoaderMaxW;
   extern __shared__ __attribute__((aligned(16))) unsigned char gemm_smem[];
   int bx, by;
   xcd_tile(bx, by);
@@ -857,13 +869,13 @@ __global__ __launch_bounds__(320) void gemm_vw_kernel(GemmArgs a) {
   const int stage_bytes = kVwABytes + a.vw_maxw * 4096, ns = a.vw_ns;
   if (wave == kLoader) {
     switch (width) {
-      case 2: vw_loader<2>(sg, gemm_smem, stage_bytes, ns, m0, n0, M, N, K, lane); break;
-      case 3: vw_loader<3>(sg, gemm_smem, stage_bytes, ns, m0, n0, M, N, K, lane); break;
-      case 4: vw_loader<4>(sg, gemm_smem, stage_bytes, ns, m0, n0, M, N, K, lane); break;
-      case 5: vw_loader<5>(sg, gemm_smem, stage_bytes, ns, m0, n0, M, N, K, lane); break;
-      case 6: vw_loader<6>(sg, gemm_smem, stage_bytes, ns, m0, n0, M, N, K, lane); break;
-      case 7: vw_loader<7>(sg, gemm_smem, stage_bytes, ns, m0, n0, M, N, K, lane); break;
-      default: vw_loader<8>(sg, gemm_smem, stage_bytes, ns, m0, n0, M, N, K, lane); break;
+      case 2: vw_loader<BM, 2>(sg, gemm_smem, stage_bytes, ns, m0, n0, M, N, K, lane); break;
+      case 3: vw_loader<BM, 3>(sg, gemm_smem, stage_bytes, ns, m0, n0, M, N, K, lane); break;
+      case 4: vw_loader<BM, 4>(sg, gemm_smem, stage_bytes, ns, m0, n0, M, N, K, lane); break;
+      case 5: vw_loader<BM, 5>(sg, gemm_smem, stage_bytes, ns, m0, n0, M, N, K, lane); break;
+      case 6: vw_loader<BM, kCap < 6 ? kCap : 6>(sg, gemm_smem, stage_bytes, ns, m0, n0, M, N, K, lane); break;
+      case 7: vw_loader<BM, kCap < 7 ? kCap : 7>(sg, gemm_smem, stage_bytes, ns, m0, n0, M, N, K, lane); break;
+      default: vw_loader<BM, kCap>(sg, gemm_smem, stage_bytes, ns, m0, n0, M, N, K, lane); break;
     }
     return;
   }
@@ -873,10 +885,10 @@ __global__ __launch_bounds__(320) void gemm_vw_kernel(GemmArgs a) {
   const int brow0 = wn ? nj0 * 32 : 0;
   const bool full = m0 + BM <= M && n0 + width * 32 <= N;
   switch (nj) {
-    case 1: vw_mma<1>(a, sg, gemm_smem, stage_bytes, ns, brow0, m0, n0, M, N, full, lane, wm); break;
-    case 2: vw_mma<2>(a, sg, gemm_smem, stage_bytes, ns, brow0, m0, n0, M, N, full, lane, wm); break;
-    case 3: vw_mma<3>(a, sg, gemm_smem, stage_bytes, ns, brow0, m0, n0, M, N, full, lane, wm); break;
-    default: vw_mma<4>(a, sg, gemm_smem, stage_bytes, ns, brow0, m0, n0, M, N, full, lane, wm); break;
+    case 1: vw_mma<BM, 1>(a, sg, gemm_smem, stage_bytes, ns, brow0, m0, n0, M, N, full, lane, wm); break;
+    case 2: vw_mma<BM, 2>(a, sg, gemm_smem, stage_bytes, ns, brow0, m0, n0, M, N, full, lane, wm); break;
+    case 3: vw_mma<BM, 3>(a, sg, gemm_smem, stage_bytes, ns, brow0, m0, n0, M, N, full, lane, wm); break;
+    default: vw_mma<BM, (kCap + 1) / 2>(a, sg, gemm_smem, stage_bytes, ns, brow0, m0, n0, M, N, full, lane, wm); break;
   }
 }
 
@@ -990,7 +1002,8 @@ __global__ __launch_bounds__(kVw256Threads) void gemm_vw256_kernel(GemmArgs a) {
 
 // How one launch of binary16 weights, not split over K, is cut into tiles.
 struct GemmRoute {
-  int rows = 0;        // of a tile: 64 (gemm_ldw_kernel<64>), 128 (gemm_vw_kernel), 256 (gemm_vw256_kernel); 0: none of these
+  int rows = 0;        // of a tile: 64 (gemm_ldw_kernel<64>), 128 (gemm_vw_kernel<128>), 256 (the other two); 0: none of these
+  bool loader = true;  // 256 rows: gemm_vw_kernel<256>, not gemm_vw256_kernel
   int blocks = 0;      // widest tile, in blocks of 32 columns
   int rounds = 0;      // over the compute units
   double us = 0;       // what the launch is expected to take
@@ -1015,6 +1028,7 @@ static long tiles64(const GemmArgs& a) {
 static double us_64(int rounds, double k) { return 2 + rounds * (2.4 + 14.2 * k); }
 static double us_128(int rounds, double k, int w) { return 2 + rounds * (5 + k * (5 + 3.55 * w)); }
 static double us_256(int rounds, double k, int w) { return 2 + rounds * (6.6 + k * (11.8 + 5.45 * w + (w == 8 ? 3 : 0))); }
+static double us_256_loader(int rounds, double k, int w) { return 2 + rounds * (5.7 + k * (5.8 + 6.8 * w)); }
 constexpr double kLaunchUs = 3;  // one more launch
 
 // Cuts the launch into tiles of bm rows (128 or 256): the fewest rounds over `cus` compute units whose widest tile
@@ -1071,13 +1085,23 @@ static GemmRoute plan_vw(const GemmArgs& args, int bm, int cus) {
     a.tile_start[a.nseg] = tiles;
     a.vw_maxw = maxw;
     const size_t stage = abytes + (size_t)maxw * 4096;
-    a.vw_ns = bm == 256 ? 2 : stage * 4 <= 160 * 1024 ? 4 : 3;
+    if (bm == 256) {
+      // Whole tiles of up to 160 columns: the loader wave's form, whose loads are two steps ahead.  All 256 compute
+      // units multiply real data then and the clock is the lowest, which costs it less: 512 x 5120 x 20480 101 us
+      // against 115, 2048 x 20480 x 5120 375 against 423, 1024 x 2048 x 10240 44 against 46.  With a part of a tile
+      // empty the other form is the faster one (1793 x 5120 x 5120: 101 against 119): its edge tiles load like whole ones.
+      r.loader = a.M % 256 == 0 && maxw <= kVw256LoaderMaxW;
+      for (int s = 0; s < a.nseg; s++) r.loader = r.loader && a.seg[s].N % 32 == 0;
+    }
+    a.vw_ns = !r.loader ? 2 : stage * 4 <= 160 * 1024 ? 4 : 3;
     if (stage * a.vw_ns > 160 * 1024) return r;
     r.lds = stage * a.vw_ns;
     r.grid = dim3(tiles, mt);
     r.blocks = maxw;
     r.rounds = rounds;
-    r.us = bm == 128 ? us_128(rounds, a.K / 2048.0, maxw) : us_256(rounds, a.K / 2048.0, maxw);
+    r.us = bm == 128 ? us_128(rounds, a.K / 2048.0, maxw)
+           : r.loader ? us_256_loader(rounds, a.K / 2048.0, maxw)
+                      : us_256(rounds, a.K / 2048.0, maxw);
     r.rows = bm;
     return r;
   }
@@ -1129,17 +1153,20 @@ static bool one_by_one(const GemmArgs& a, const GemmRoute& whole, int cus) {
   return whole.rows ? us < whole.us : true;
 }
 
-static void gemm_vw_launch(int bm, dim3 grid, size_t lds, hipStream_t st, const GemmArgs& a) {
+static void gemm_vw_launch(const GemmRoute& r, hipStream_t st) {
   static const bool raised = [] {
-    for (const void* f : {reinterpret_cast<const void*>(&gemm_vw_kernel), reinterpret_cast<const void*>(&gemm_vw256_kernel)})
+    for (const void* f : {reinterpret_cast<const void*>(&gemm_vw_kernel<128>), reinterpret_cast<const void*>(&gemm_vw_kernel<256>),
+                          reinterpret_cast<const void*>(&gemm_vw256_kernel)})
       (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     return true;
   }();
   (void)raised;
-  if (bm == 256)
-    hipLaunchKernelGGL(gemm_vw256_kernel, grid, dim3(kVw256Threads), lds, st, a);
+  if (r.rows == 128)
+    hipLaunchKernelGGL(gemm_vw_kernel<128>, r.grid, dim3(320), r.lds, st, r.a);
+  else if (r.loader)
+    hipLaunchKernelGGL(gemm_vw_kernel<256>, r.grid, dim3(576), r.lds, st, r.a);
   else
-    hipLaunchKernelGGL(gemm_vw_kernel, grid, dim3(320), lds, st, a);
+    hipLaunchKernelGGL(gemm_vw256_kernel, r.grid, dim3(kVw256Threads), r.lds, st, r.a);
 }
 
 static constexpr size_t gemm_lds_bytes(int bm, int bk) { return (size_t)(bm + BN) * (bk + 8) * 2; }
@@ -1338,7 +1365,7 @@ int launch_gemm(GemmArgs& a, bool u8, hipStream_t st, const char* what, void* dq
       if (r.rows == 64)
         gemm_ldw_launch<64>(r.grid, st, r.a);
       else
-        gemm_vw_launch(r.rows, r.grid, r.lds, st, r.a);
+        gemm_vw_launch(r, st);
       return check_launch(what);
     }
   }
@@ -1416,9 +1443,10 @@ extern "C" int frhip_gemm_route(int T, int K, int nproducts, const int* N, int c
       one.seg[0] = a.seg[s];
       r = gemm_route(one, compute_units);
     }
-    out[3 * s] = r.rows;
-    out[3 * s + 1] = r.blocks;
-    out[3 * s + 2] = r.rounds;
+    out[4 * s] = r.rows;
+    out[4 * s + 1] = r.blocks;
+    out[4 * s + 2] = r.rounds;
+    out[4 * s + 3] = r.rows != 0 && r.loader;
   }
   return split ? nproducts : 1;
 }

@@ -295,8 +295,9 @@ int frhip_att_seq_v5(int T, int C, int H, const void *x, const void *sx, const f
 /* How a launch of `nproducts` (1..4) binary16 products [T][K] x [K][N[i]] would be cut into tiles on a part with that
  * many compute units, without scratch to split it over K: a pure function of the sizes, for tests and measurements.
  * Returns the number of launches (1: all products together; nproducts: one by one) or a negative FRHIP_E*.
- * out[3 i]: rows of a tile of product i's launch (64, 128, 256; 0: fixed 128 x 128 or 64 x 128 tiles, several rounds),
- * out[3 i + 1]: its widest tile in blocks of 32 columns, out[3 i + 2]: its rounds over the compute units. */
+ * out[4 i]: rows of a tile of product i's launch (64, 128, 256; 0: fixed 128 x 128 or 64 x 128 tiles, several rounds),
+ * out[4 i + 1]: its widest tile in blocks of 32 columns, out[4 i + 2]: its rounds over the compute units,
+ * out[4 i + 3]: 1 if a wave of its own loads the tiles. */
 int frhip_gemm_route(int T, int K, int nproducts, const int *N, int compute_units, int *out);
 
 /* ---- bandwidth probes: DIAGNOSTICS, not operators (measurement aids of bench.py and of the

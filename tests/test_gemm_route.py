@@ -9,18 +9,18 @@ fr = importlib.import_module("faster-rwkv_amd")
 
 
 def route(T, K, *N):
-    """-> launches, [(rows of a tile, widest tile in blocks of 32 columns, rounds)] per product"""
-    out = (C.c_int * (3 * len(N)))()
+    """-> launches, [(rows of a tile, widest tile in blocks of 32 columns, rounds, loader wave)] per product"""
+    out = (C.c_int * (4 * len(N)))()
     launches = fr.lib().frhip_gemm_route(T, K, len(N), (C.c_int * len(N))(*N), 256, out)
     assert launches > 0, launches
-    return launches, [tuple(out[3 * i:3 * i + 3]) for i in range(len(N))]
+    return launches, [tuple(out[4 * i:4 * i + 4]) for i in range(len(N))]
 
 
 @pytest.mark.parametrize("T,K,N", [(300, 2048, 6144),   # 19.2 against 22.7 as 128 x 96
                                    (129, 2048, 10240),  # 19.0 against 21.6
                                    (129, 2560, 8960)])  # 24.8 against 26.3
 def test_one_round_of_64_row_tiles_is_kept_where_it_is_cheaper(T, K, N):
-    assert route(T, K, N) == (1, [(64, 4, 1)])
+    assert route(T, K, N) == (1, [(64, 4, 1, 1)])
 
 
 @pytest.mark.parametrize("T,K,N,rows", [(3000, 2048, 8192, 256),   # 105.5 against 119 as three rounds of 128 rows
@@ -32,13 +32,26 @@ def test_tile_height(T, K, N, rows):
     assert route(T, K, N)[1][0][0] == rows
 
 
+@pytest.mark.parametrize("T,K,N,loader", [(512, 5120, 20480, 1),    # 101 against 115 without the loader wave
+                                          (1024, 5120, 20480, 1),   # 200 against 219
+                                          (2048, 20480, 5120, 1),   # 375 against 423
+                                          (768, 2560, 11520, 1),    # 51 against 59
+                                          (1793, 5120, 5120, 0),    # 119 with it against 101: rows past the end
+                                          (1025, 320, 10000, 0),
+                                          (2048, 2048, 5110, 0),    # columns past the end
+                                          (2048, 2048, 8192, 0)])   # wider than its stages allow
+def test_loader_wave_of_256_row_tiles(T, K, N, loader):
+    rows, blocks, _, got = route(T, K, N)[1][0]
+    assert (rows, got) == (256, loader) and (blocks <= 5 or not loader)
+
+
 def test_an_extra_launch_costs_the_same_whatever_k():
     """2048 and 8192 columns one by one save part of a round, which grows with K; the launch they cost does not."""
     assert [route(3074, k, 2048, 8192)[0] for k in (512, 1024, 2048, 4096)] == [1, 1, 2, 2]
 
 
 def test_refused_sizes():
-    lib, n, out = fr.lib(), (C.c_int * 1)(64), (C.c_int * 3)()
+    lib, n, out = fr.lib(), (C.c_int * 1)(64), (C.c_int * 4)()
     for args in ((0, 64, 1), (4, 96, 1), (4, 64, 0), (4, 64, 5)):
         assert lib.frhip_gemm_route(*args, n, 256, out) == -2
     assert lib.frhip_gemm_route(4, 64, 1, None, 256, out) == -1
