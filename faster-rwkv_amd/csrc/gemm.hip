@@ -714,7 +714,7 @@ static void gemm_ldw_launch(dim3 grid, hipStream_t st, const GemmArgs& a) {
 // and swizzle are those of gemm_ldw_kernel.  gemm_vw_kernel<256> has eight MFMA waves (4 x 2 of
 // 64 rows each) and takes whole tiles of at most 160 columns; gemm_vw256_kernel below takes the others.
 // ---------------------------------------------------------------------------
-constexpr int kVwMaxW = 8, kVwMaxRounds = 32;
+constexpr int kVwMaxW = 8;
 constexpr int kVw256LoaderMaxW = 5;  // three stages of (256 + 160) x 64 halves are 156 KB of the 160 KB
 
 template <int BM, int W>
@@ -1044,8 +1044,10 @@ static GemmRoute plan_vw(const GemmArgs& args, int bm, int cus) {
     cb[s] = (a.seg[s].N + 31) / 32;
     total += cb[s];
   }
-  for (int rounds = 1; rounds <= kVwMaxRounds; rounds++) {
-    const int P = rounds * cus / mt;  // tiles per strip of rows
+  // From the fewest rounds that tiles of the largest width allow; it ends at tiles of one block at the latest.  (With a
+  // limit of 32 rounds 8193 x 2048 x 65536 took 3.14 ms on fixed 128 x 128 tiles, 2.06 so, one row less 1.97.)
+  for (long rounds = ((long)total * mt + (long)kVwMaxW * cus - 1) / ((long)kVwMaxW * cus);; rounds++) {
+    const int P = (int)(rounds * cus / mt);  // tiles per strip of rows
     if (P < a.nseg) continue;
     int t[kGemmMaxSeg], used = 0;
     for (int s = 0; s < a.nseg; s++) {
@@ -1098,10 +1100,10 @@ static GemmRoute plan_vw(const GemmArgs& args, int bm, int cus) {
     r.lds = stage * a.vw_ns;
     r.grid = dim3(tiles, mt);
     r.blocks = maxw;
-    r.rounds = rounds;
-    r.us = bm == 128 ? us_128(rounds, a.K / 2048.0, maxw)
-           : r.loader ? us_256_loader(rounds, a.K / 2048.0, maxw)
-                      : us_256(rounds, a.K / 2048.0, maxw);
+    r.rounds = (int)rounds;
+    r.us = bm == 128 ? us_128(r.rounds, a.K / 2048.0, maxw)
+           : r.loader ? us_256_loader(r.rounds, a.K / 2048.0, maxw)
+                      : us_256(r.rounds, a.K / 2048.0, maxw);
     r.rows = bm;
     return r;
   }

@@ -45,6 +45,19 @@ def test_loader_wave_of_256_row_tiles(T, K, N, loader):
     assert (rows, got) == (256, loader) and (blocks <= 5 or not loader)
 
 
+@pytest.mark.parametrize("T", [8192, 8193, 16000, 100000])
+def test_no_limit_on_rounds(T):
+    """The logits of every position of a long text: planned tiles, however many rounds they take."""
+    rows, blocks, rounds, _ = route(T, 2048, 65536)[1][0]
+    assert (rows, blocks) == (256, 8) and -(-T // 256) * 256 <= rounds * 256 < -(-T // 256) * 256 + 512
+
+
+def test_many_products_of_few_columns():
+    """More strips than compute units: a round holds a part of a strip."""
+    assert route(300000, 64, 96, 96, 96, 96)[1][0][0] in (0, 128, 256)
+    assert route(300000, 64, 32)[1][0][0] == 0
+
+
 def test_an_extra_launch_costs_the_same_whatever_k():
     """2048 and 8192 columns one by one save part of a round, which grows with K; the launch they cost does not."""
     assert [route(3074, k, 2048, 8192)[0] for k in (512, 1024, 2048, 4096)] == [1, 1, 2, 2]
