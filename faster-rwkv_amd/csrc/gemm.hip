@@ -1037,6 +1037,8 @@ static GemmRoute plan_vw(const GemmArgs& args, int bm, int cus) {
   GemmRoute r;
   r.a = args;
   GemmArgs& a = r.a;
+  // gemm_vw256_kernel addresses the 256 rows of a tile with 32-bit byte offsets
+  if (bm == 256 && (size_t)a.K * 2 * 256 > 0xffffffffull) return r;
   const int mt = (a.M + bm - 1) / bm;
   const int abytes = bm * kLdwBK * 2;
   int cb[kGemmMaxSeg], total = 0;

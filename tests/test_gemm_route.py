@@ -58,6 +58,14 @@ def test_many_products_of_few_columns():
     assert route(300000, 64, 32)[1][0][0] == 0
 
 
+def test_rows_too_long_for_32_bit_offsets_are_not_cut_into_256_row_tiles():
+    """gemm_vw256_kernel's lane offsets reach 255 rows and 128 bytes beyond a tile's first: 2 K 256 must stay below 2^32."""
+    k = (1 << 32) // 512 - 64
+    assert k % 64 == 0 and route(3000, k, 8192)[1][0] == (256, 7, 2, 0)
+    for more in (64, 128, 1 << 20):
+        assert route(3000, k + more, 8192)[1][0][0] in (64, 128)
+
+
 def test_an_extra_launch_costs_the_same_whatever_k():
     """2048 and 8192 columns one by one save part of a round, which grows with K; the launch they cost does not."""
     assert [route(3074, k, 2048, 8192)[0] for k in (512, 1024, 2048, 4096)] == [1, 1, 2, 2]
