@@ -80,9 +80,10 @@ __global__ void fill_kernel(T* x, T v, size_t n) {
 }
 
 // Many small buffers per launch: blockIdx.y picks the buffer, the workgroups of a row walk it in steps of 16 bytes per
-// thread (2 bytes where an address or a size is not a multiple of 16).  Bound by launches, not by bytes: the 120 state
-// tensors of a 24-layer RWKV-4 model (1.6 MB) are two launches of about 3 us; as blocking copies from the host they took
-// 1.48 ms, and the 120 device-to-device copies into the decode buffers 0.22 ms.
+// thread (where an address or a size is not a multiple of 16: 2 bytes of a fill, single bytes of a copy).  Bound by
+// launches, not by bytes: the 120 state tensors of a 24-layer RWKV-4 model (C = 2048: 0.79 MB) are two
+// launches of about 3 us; as blocking copies from the host they took 1.48 ms, and the 120 device-to-device copies into
+// the decode buffers 0.22 ms.
 constexpr int kManyBuffers = 64;  // 24 bytes of kernel arguments each
 struct ManyBuffers {
   void* dst[kManyBuffers];
@@ -634,7 +635,7 @@ int frhip_fill_many(int n, void* const* dst, const int* dtype, const float* valu
   for (int i = 0; i < n; i++) {
     if (!dst[i] && count[i]) return set_error(FRHIP_EINVAL, "fill_many: null buffer");
     if (dtype[i] != FRHIP_F16 && dtype[i] != FRHIP_F32) return set_error(FRHIP_EINVAL, "fill_many: unknown dtype");
-    if (reinterpret_cast<uintptr_t>(dst[i]) % (dtype[i] == FRHIP_F16 ? 2 : 4)) return set_error(FRHIP_EINVAL, "fill_many: misaligned buffer");
+    if (count[i] && reinterpret_cast<uintptr_t>(dst[i]) % (dtype[i] == FRHIP_F16 ? 2 : 4)) return set_error(FRHIP_EINVAL, "fill_many: misaligned buffer");
   }
   for (int i = 0; i < n;) {
     ManyFill a;

@@ -121,9 +121,10 @@ int frhip_cast(const void *src, int src_dtype, void *dst, int dst_dtype, size_t 
 int frhip_fill(void *x, int dtype, float value, size_t n, frhip_stream s);
 /* fill_ and device-to-device copies of `n` separate buffers with one launch per 64 of them: the tensors of a recurrent
  * state (120 of them in a 24-layer RWKV-4 model) are small, and a launch or copy of its own costs each more than its bytes.
- * Buffers may have any alignment and size (fill_many: sizes are multiples of the element, dtype FRHIP_F16 or FRHIP_F32;
- * `value` per buffer).  Null entries are refused before anything is launched; a buffer of no bytes is skipped.  The
- * destinations do not overlap each other or a source. */
+ * copy_many: any address and number of bytes.  fill_many: `count` elements of dtype FRHIP_F16 or FRHIP_F32, at an address
+ * that is a multiple of the element's size; `value` per buffer.  A buffer of no bytes is skipped, whatever its
+ * address.  What does not fit is refused before anything is launched.  The destinations do not overlap each other or a
+ * source. */
 int frhip_fill_many(int n, void *const *dst, const int *dtype, const float *value, const size_t *count, frhip_stream s);
 int frhip_copy_many(int n, void *const *dst, const void *const *src, const size_t *bytes, frhip_stream s);
 /* scalar_div_: kernels/cuda/element_wise.cu:8-19 (binary16, divisor rounded to half first). */

@@ -30,6 +30,19 @@ def test_workspace_query_and_argument_checks_do_not_need_a_gpu():
     assert b"null" in lib.frhip_error_string()
 
 
+def test_fill_many_and_copy_many_look_at_buffers_of_some_bytes_only():
+    """An empty buffer is skipped whatever its address (nothing is launched); an element that would straddle its
+    alignment is refused."""
+    L = fr.lib()
+    fill = lambda ptr, dtype, count: L.frhip_fill_many(1, (C.c_void_p * 1)(ptr), (C.c_int * 1)(dtype), (C.c_float * 1)(0),
+                                                       (C.c_size_t * 1)(count), None)
+    for ptr in (None, 4096, 4097, 4098):
+        for dtype in (fr.F16, fr.F32):
+            assert fill(ptr, dtype, 0) == 0
+        assert L.frhip_copy_many(1, (C.c_void_p * 1)(ptr), (C.c_void_p * 1)(None), (C.c_size_t * 1)(0), None) == 0
+    assert fill(4097, fr.F16, 1) == fill(4098, fr.F32, 1) == fill(None, fr.F16, 1) == fill(4096, fr.U8, 0) == -1
+
+
 def test_host_library_loads_and_reports_errors_as_status():
     h = fr.host()
     m = h.fr_model_create(b"/nonexistent/model.fr", b"tpu fp16")
