@@ -40,7 +40,7 @@ def h(x):
 @pytest.mark.parametrize("T,K,N", [(1024, 2048, 2048), (512, 2560, 8960), (100, 8192, 2048), (1, 64, 128), (130, 128, 200), (7, 1792, 512),
                                    # wide enough for the variable-width tiles: ragged N (last block partial), ragged T
                                    (1024, 256, 7000), (900, 128, 6144),
-                                   # one round of 256-row tiles beats two of 128-row tiles: the eight-wave form, full and ragged
+                                   # one round of 256-row tiles beats two of 128-row tiles: with a loader wave (whole tiles) and without
                                    (1024, 128, 10240), (1000, 128, 10000)])
 @pytest.mark.parametrize("quant", [False, True])
 def test_gemm_against_oracle(T, K, N, quant):
@@ -71,7 +71,8 @@ def test_gemm_against_oracle(T, K, N, quant):
 
 @pytest.mark.parametrize("T,K,N", [(2048, 64, 8192),    # 256 x 256 tiles, two stages, a single K-step
                                    (2048, 128, 6100),   # 256 x 192, two K-steps, ragged columns
-                                   (4099, 192, 2048),   # 256 x 160 / 128, three stages; the last strip has three rows
+                                   (4099, 192, 2048),   # 256 x 160 / 128; the last strip has three rows
+                                   (1024, 192, 10240),  # 256 x 160, whole tiles: the loader wave's form, three stages
                                    (1025, 320, 10000),  # one row in the last strip, ragged columns
                                    (512, 192, 6144),    # 128 x 96: the narrowest planned tile
                                    (3000, 128, 10240)]) # more than four rounds' worth of 128 x 128 tiles
@@ -133,7 +134,7 @@ def _common(C_):
     return (h(1 + 0.1 * rng.standard_normal(C_)), h(0.1 * rng.standard_normal(C_)))
 
 
-# (1024, 2048, 8192): r and k as separate one-round launches, the value product split over K in two slices;
+# (1024, 2048, 8192): r and k as one round of 256-row tiles, the value product split over K in two slices;
 # (300, 2048, 8192): the value product in four slices over ragged row tiles; (512, 2560, 8960): three slices of 47, 47 and 46 K-steps
 # (16, 2048, 8192), (130, 2048, 8192), (200, 2560, 8960): short prompts at full width -- products split over K across the idle compute
 # units: r,k grouped in one split launch (16 rows), product by product because the group is too wide (130, 200 rows), the value
@@ -158,10 +159,55 @@ def test_ffn_seq(T, C_, F_, quant):
     assert_close_f16(x_out.numpy(), ref_x, max_ulp=3, max_frac=0.2, what="x_out", floor_rms=1.0)
 
 
+def _routes(T, K, *N):
+    """frhip_gemm_route on 256 compute units -> launches, [(rows of a tile, widest tile in blocks of 32 columns, rounds, loader wave)]"""
+    out = (C.c_int * (4 * len(N)))()
+    launches = L().frhip_gemm_route(T, K, len(N), (C.c_int * len(N))(*N), 256, out)
+    return launches, [tuple(out[4 * i:4 * i + 4]) for i in range(len(N))]
+
+
+@pytest.mark.parametrize("T,C_,F_,rk,v", [
+    # every product on 256-row tiles whose last strip has 16 rows: sigmoid, relu^2 and the output's epilogue, predicated
+    (16400, 320, 256, (1, [(256, 8, 1, 0)] * 2), (256, 4, 1, 0)),
+    (2049, 1024, 4096, (1, [(256, 6, 1, 0)] * 2), None),  # ... one row in the last strip, 16 K-steps
+    (3074, 320, 4736, (2, [(64, 4, 1, 1), (256, 8, 1, 0)]), None),  # r and k one by one, on tiles of different heights
+    (12288, 448, 896, (1, [(256, 5, 2, 1)] * 2), (256, 3, 1, 1))])  # whole tiles: the loader wave's form, grouped and alone
+def test_ffn_seq_on_planned_tiles(T, C_, F_, rk, v):
+    """The fused epilogues on 256-row tiles, with rows past the end and without, in groups and one by one.  Bounds as in
+    test_ffn_seq."""
+    assert _routes(T, C_, C_, F_) == rk
+    assert v is None or _routes(T, F_, C_)[1] == [v]
+    test_ffn_seq(T, C_, F_, False)
+
+
 @pytest.mark.parametrize("T,C_,F_", [(4, 512, 1792), (64, 512, 2048), (65, 768, 3072), (128, 2048, 8192), (129, 512, 1792)])
 def test_ffn_seq_uint8_dequantised_in_the_product(T, C_, F_):
-    """One strip of 64 or 128 rows, split over K; 129 rows are expanded first.  Bounds as in test_ffn_seq."""
+    """Up to 64 rows the split product dequantises by itself; from 65 rows on the codes are expanded first.  Bounds as in
+    test_ffn_seq."""
     test_ffn_seq(T, C_, F_, True)
+
+
+# (576, 1856): ragged tiles; (2560, 8960): r,k of 13 rows in two slices of 20 K-steps, the value product in twelve of 11 or 12
+@pytest.mark.parametrize("T", [4, 13, 63, 64, 65, 129])
+@pytest.mark.parametrize("C_,F_", [(576, 1856), (2560, 8960)])
+def test_ffn_seq_uint8_gives_the_bits_of_its_binary16_image(T, C_, F_):
+    """A uint8 weight and its dequantised image as a binary16 weight: the same slices of K, so the same bits, whether the
+    product dequantises (up to 64 rows) or the codes are expanded first."""
+    x, sx = h(rng.standard_normal((T, C_)) * 2), h(rng.standard_normal(C_))
+    vecs = [keep(a) for a in (x, sx, *_common(C_), h(rng.uniform(0, 1, C_)), h(rng.uniform(0, 1, C_)))]
+    coded = [make_weight(h(rng.standard_normal(s) * 0.02), True)[0] for s in ((C_, F_), (F_, C_), (C_, C_))]
+    images = []
+    for w in coded:
+        img = DevBuf.empty((w.N, w.K), np.float16)
+        _alive.append(img)
+        fr.check(L().frhip_dequant_u8(w.ref, img.ptr, None))
+        images.append(fr.Weight(img.ptr, None, None, None, None, w.K, w.N, fr.F16))
+    outs = []
+    for kw, vw, rw in ([w.ref for w in coded], [C.byref(w) for w in images]):
+        x_out, xx_out, ws = DevBuf.empty((T, C_), np.float16), DevBuf.empty(C_, np.float16), DevBuf(L().frhip_seq_workspace_bytes(T, C_, F_))
+        fr.check(L().frhip_ffn_seq(T, C_, F_, *[a.ptr for a in vecs], kw, vw, rw, x_out.ptr, xx_out.ptr, 0, ws.ptr, None))
+        outs.append(x_out.numpy())
+    assert np.array_equal(outs[0].view(np.uint16), outs[1].view(np.uint16))
 
 
 @pytest.mark.parametrize("T", [4, 13, 64, 65])
@@ -307,6 +353,14 @@ def test_att_seq_v4(T, C_, quant, fresh):
         g = got.numpy().astype(np.float64) * np.exp(po_.numpy().astype(np.float64) - ref[4].astype(np.float64))
         assert np.allclose(g, want, rtol=2e-3, atol=2e-3 * np.abs(want).max())
     assert np.abs(po_.numpy() - ref[4]).max() < 30  # offsets stay in a sane range
+
+
+@pytest.mark.parametrize("T,C_,kvr,o", [(16400, 320, (256, 5, 2, 0), (256, 4, 1, 0)),  # predicated epilogues: 16 rows in the last strip
+                                        (4096, 448, (256, 3, 1, 1), (64, 4, 1, 1))])   # whole tiles: the loader wave's form
+def test_att_seq_v4_on_planned_tiles(T, C_, kvr, o):
+    """k, v, r grouped and the residual's epilogue on 256-row tiles.  Bounds as in test_att_seq_v4."""
+    assert _routes(T, C_, C_, C_, C_) == (1, [kvr] * 3) and _routes(T, C_, C_) == (1, [o])
+    test_att_seq_v4(T, C_, False, False)
 
 
 @pytest.mark.parametrize("T,C_", [(1024, 2048), (700, 512), (5000, 256)])  # 5000: beyond 128 chunks of 32 steps, the scan's serial pass
