@@ -33,8 +33,9 @@ struct GemmArgs {
   // gemm_vw_kernel: a segment's tiles are vw_base (the first vw_wide of them vw_base + 1) blocks of 32 columns wide
   int vw_base[kGemmMaxSeg], vw_wide[kGemmMaxSeg], vw_maxw, vw_ns;
   GemmSeg seg[kGemmMaxSeg];
-  // split K (single-segment launches of gemm_ldw_kernel<128> only): slice z of ksplit accumulates K / ksplit of the
-  // product into partial + z * partial_stride as fp32 [M][N]; gemm_splitk_reduce_kernel adds the slices and applies the epilogue
+  // split K (ksplit >= 2; gemm_ldw_kernel<128> with one segment, gemm_ldw_kernel<64> and the uint8 gemm_kernel<64, 64> with
+  // up to four): slice z of ksplit accumulates its K-steps of segment s into partial + z * partial_stride + part_off[s] as
+  // fp32 [M][N]; gemm_splitk_reduce_kernel adds the slices and applies the epilogues
   int ksplit;
   float* partial;
   size_t partial_stride;
@@ -43,12 +44,13 @@ struct GemmArgs {
   int div2;
 };
 
-// dq: optional scratch of gemm_dequant_bytes(a) bytes.  With it, uint8 weights of a launch with at least
+// dq: optional scratch, 2 bytes per weight of the launch.  With it, uint8 weights of a launch with at least
 // kDequantRows rows are expanded once to binary16 (the standalone dequantisation: the same bits as the
-// in-kernel one) and the launch takes the binary16 kernel.
+// in-kernel one) and the launch takes the binary16 kernel, unless it has at most 64 rows and goes out split over K
+// (few_rows): the uint8 kernel dequantises those on the way into LDS.
 // partial: optional fp32 scratch of max_split slices of partial_stride floats (>= M * N each) for splitting K.
 // few_rows: optional fp32 scratch of few_rows_floats floats; with it a launch of so few rows that 64 x 128 tiles leave
-// at least half of the compute units idle goes out product by product, each split over K across the idle units.
+// at least half of the compute units idle is split over K across the idle units, whole or product by product.
 constexpr size_t kFewRowsFloats = (size_t)512 * 64 * 128;  // two 64 x 128 tiles per compute unit of a 256-unit part
 constexpr int kFewRowsMax = 360;                          // rows up to which the seq operators carry that scratch
 int launch_gemm(GemmArgs& a, bool u8, hipStream_t st, const char* what, void* dq = nullptr, float* partial = nullptr,

@@ -17,7 +17,8 @@
 //                    against bank conflicts), the loads of step k+1 issued before the MFMAs of
 //                    step k, and are dequantised to binary16 on the way into LDS with the same
 //                    formula as the standalone dequantisation, so the product sees exactly the
-//                    dequantised matrix.
+//                    dequantised matrix (launches of up to 64 rows, and calls without scratch
+//                    for the expanded weights).
 // Products are exact in fp32, accumulation is fp32 in ascending k, and the result is rounded once
 // to the output type (kernels/cuda/matmul.cpp:38-42,64-68); all kernels give the same bits, except
 // that a launch split over K (launch_gemm) adds its slices' fp32 sums at the end.
@@ -705,9 +706,8 @@ static void gemm_ldw_launch(dim3 grid, hipStream_t st, const GemmArgs& a) {
 // A launch of 128 x 128 tiles over T = 1024 rows rarely comes out as a whole number of rounds over
 // the compute units (k,v,r of a 2048-wide model: 384 tiles on 256 CUs take as long as 512), and a
 // wider tile moves fewer bytes per product.  Here the host cuts every segment of a launch into
-// tiles of 128 rows x (32 w) columns, w = base or base + 1 per segment, so that the launch has as
-// many workgroups as the part has compute units (or twice, three times as many), and no tile
-// straddles two segments.  The two wave columns of a workgroup take ceil(w/2) and floor(w/2)
+// tiles of 128 rows x (32 w) columns, w = base or base + 1 per segment, so that the launch fills
+// a whole number of rounds over the compute units, and no tile straddles two segments.  The two wave columns of a workgroup take ceil(w/2) and floor(w/2)
 // 32-column blocks; the loops are instantiated per block count, so the products are the same
 // MFMAs in the same k order as in the other kernels and the results are bit-identical.  Loader
 // wave, LDS ring (three or four K-steps of 64, whatever fits 160 KB at the launch's widest tile)
@@ -904,8 +904,8 @@ __global__ __launch_bounds__(BM * 2 + 64) void gemm_vw_kernel(GemmArgs a) {
 // two steps ahead were measured: no faster, 4099 x 8192 x 2048 166 us against 161.)
 // Rows past the matrix are clamped in the lane offsets, so edge tiles load like the others.
 // What bounds it: a step of 256 x 256 reads 192 KB of fragments from LDS and writes 64 KB to it, 2048 cycles at
-// 128 bytes per cycle, as many as its MFMAs take on each SIMD.  3000 x 5120 x 20480: 825 -> 571 us (1.1 PFLOP/s),
-// 4099 x 2048 x 10240: 230 -> 171 us, against the fixed 128 x 128 tiles both launches had before.
+// 128 bytes per cycle, as many as its MFMAs take on each SIMD.  3000 x 5120 x 20480: 811 -> 580 us (1.08 PFLOP/s),
+// 4099 x 2048 x 10240: 229 -> 172 us, against the fixed 128 x 128 tiles both launches had before (in turn on one part).
 // ---------------------------------------------------------------------------
 constexpr int kVw256Threads = 512, kVw256ABytes = 256 * kLdwBK * 2;
 
