@@ -56,8 +56,10 @@ constexpr int kGemmThreads = 256;
 // is below 1e-6, plus one ulp each for v_exp_f32, the sum and v_rcp_f32: under 20 fp32 ulps.  An
 // estimate further than 64 ulps from the midpoint of two binary16 values therefore rounds as the
 // exact value does; the others (about 1 in 60) are queued per lane and evaluated in double
-// afterwards, one per lane and pass.
-__device__ __forceinline__ void sigmoid_h16(const f16v& c, h1 (&y)[16]) {
+// afterwards, one per lane and pass.  `live`: the elements that are stored.  Rows past the matrix hold copies of its
+// last row, so one pending element would be sixteen: 777 x 2048 x (2048 sigmoid + 8192), whose last strip of 256 rows has
+// nine, took 89 us with all of them queued and takes 57.5 (1024 rows: 59).
+__device__ __forceinline__ void sigmoid_h16(const f16v& c, h1 (&y)[16], uint32_t live) {
   h1 x[16];
   uint32_t pend = 0;
 #pragma unroll
@@ -70,6 +72,7 @@ __device__ __forceinline__ void sigmoid_h16(const f16v& c, h1 (&y)[16]) {
     y[v] = (h1)s32;
     pend |= safe ? 0u : (1u << v);
   }
+  pend &= live;
   while (pend) {
     const int v = __builtin_ctz(pend);
     pend &= pend - 1;
@@ -87,7 +90,7 @@ __device__ __forceinline__ void sigmoid_h16(const f16v& c, h1 (&y)[16]) {
 // for the exponential, v_rcp_f32 for the quotient: under 20 and 3 fp32 ulps off) are taken when
 // they are further than 64 ulps from a binary16 rounding boundary and in the normal binary16
 // range; the other elements are queued and go through silu_h itself.
-__device__ __forceinline__ void silu_h16(const f16v& c, h1 (&y)[16]) {
+__device__ __forceinline__ void silu_h16(const f16v& c, h1 (&y)[16], uint32_t live) {
   h1 x[16];
   uint32_t pend = 0;
   auto far_from_boundary = [](float v) {
@@ -106,6 +109,7 @@ __device__ __forceinline__ void silu_h16(const f16v& c, h1 (&y)[16]) {
     y[v] = (h1)qf;
     pend |= safe ? 0u : (1u << v);
   }
+  pend &= live;
   while (pend) {
     const int v = __builtin_ctz(pend);
     pend &= pend - 1;
@@ -138,6 +142,14 @@ __device__ __forceinline__ void gemm_epilogue_t(const GemmArgs& a, const GemmSeg
 #pragma unroll
       for (int j = 0; j < NJ; j++) g(i, j, acc[i][j]);
   };
+  // blocks without a stored element; only for the costly epilogues: with the test in all of them the short launches of
+  // gemm_ldw_kernel<64> took 0.4-0.8 us longer (33 x 1024 x 5120: 6.5 -> 6.9)
+  auto outside = [&](int i, int j) { return !FULL && (row0 + i * 32 >= M || col0 + j * 32 >= N); };
+  auto live_of = [&](int i, int j) {  // bit v: element v of the block lies inside the matrix
+    uint32_t m = 0;
+    for_tile(i, j, [&](int v, bool ok, size_t) { m |= ok ? 1u << v : 0u; });
+    return m;
+  };
   switch (sg.epi) {
     case G_STORE_F16:
       for_blocks([&](int i, int j, const f16v& c) {
@@ -151,8 +163,9 @@ __device__ __forceinline__ void gemm_epilogue_t(const GemmArgs& a, const GemmSeg
       break;
     case G_SIGMOID:
       for_blocks([&](int i, int j, const f16v& c) {
+        if (outside(i, j)) return;
         h1 y[16];
-        sigmoid_h16(c, y);
+        sigmoid_h16(c, y, live_of(i, j));
         for_tile(i, j, [&](int v, bool ok, size_t o) { if (ok) static_cast<h1*>(sg.out)[o] = y[v]; });
       });
       break;
@@ -166,8 +179,9 @@ __device__ __forceinline__ void gemm_epilogue_t(const GemmArgs& a, const GemmSeg
       break;
     case G_SILU:
       for_blocks([&](int i, int j, const f16v& c) {
+        if (outside(i, j)) return;
         h1 y[16];
-        silu_h16(c, y);
+        silu_h16(c, y, live_of(i, j));
         for_tile(i, j, [&](int v, bool ok, size_t o) { if (ok) static_cast<h1*>(sg.out)[o] = y[v]; });
       });
       break;
@@ -621,7 +635,7 @@ __device__ __forceinline__ void splitk_reduce_body(const GemmArgs& a, const Gemm
         f16v c;
 #pragma unroll
         for (int i = 0; i < 16; i++) c[i] = acc[i];
-        if (sg.epi == G_SIGMOID) sigmoid_h16(c, y); else silu_h16(c, y);
+        if (sg.epi == G_SIGMOID) sigmoid_h16(c, y, 0xffffu); else silu_h16(c, y, 0xffffu);
       }
       break;
     case G_RELU2:

@@ -33,6 +33,13 @@ def _rng_per_test(request):
     rng = np.random.default_rng([777, zlib.crc32(request.node.name.encode())])
 
 
+def _routes(T, K, *N):
+    """frhip_gemm_route on 256 compute units -> launches, [(rows of a tile, widest tile in blocks of 32 columns, rounds, loader wave)]"""
+    out = (C.c_int * (4 * len(N)))()
+    launches = L().frhip_gemm_route(T, K, len(N), (C.c_int * len(N))(*N), 256, out)
+    return launches, [tuple(out[4 * i:4 * i + 4]) for i in range(len(N))]
+
+
 def h(x):
     return np.asarray(x, np.float32).astype(np.float16)
 
@@ -123,6 +130,32 @@ def test_gemm_act_relu2_and_silu_match_the_oracle():
     assert L().frhip_gemm_act(keep(x).ptr, pw.ref, y.ptr, 256, 7, None) == -1
 
 
+@pytest.mark.parametrize("act", [2, 4])  # FRHIP_ACT_SIGMOID, FRHIP_ACT_SILU
+def test_rows_past_the_end_do_not_slow_an_epilogue(act):
+    """777 and 1024 rows are the same four strips of 256-row tiles, the last one with 9 or 256 rows.  The elements that
+    are not stored, copies of the last row, may not be worked off one by one (that took half as long again and more)."""
+    assert _routes(777, 2048, 10240)[1][0][:3] == _routes(1024, 2048, 10240)[1][0][:3] == (256, 5, 1)
+    x, pw = keep(h(rng.standard_normal((1024, 2048)))), fr.PackedWeight(w_kn=h(rng.standard_normal((2048, 10240)) * 0.02))
+    y = DevBuf.empty((1024, 10240), np.float16)
+    events = [C.c_void_p() for _ in range(2)]
+    for e in events:
+        fr.check(L().frhip_event_create(C.byref(e)))
+    best = {777: 1e9, 1024: 1e9}
+    for _ in range(12):
+        for T in best:
+            ms = C.c_float()
+            fr.check(L().frhip_event_record(events[0], None))
+            for _ in range(4):
+                fr.check(L().frhip_gemm_act(x.ptr, pw.ref, y.ptr, T, act, None))
+            fr.check(L().frhip_event_record(events[1], None))
+            fr.check(L().frhip_event_sync(events[1]))
+            fr.check(L().frhip_event_elapsed_ms(*events, C.byref(ms)))
+            best[T] = min(best[T], ms.value)
+    for e in events:
+        fr.check(L().frhip_event_destroy(e))
+    assert best[777] <= 1.2 * best[1024], best
+
+
 def test_gemm_rejects_bad_shapes():
     w = fr.PackedWeight(w_kn=h(rng.standard_normal((96, 64))))
     y = DevBuf.empty((4, 64), np.float32)
@@ -157,13 +190,6 @@ def test_ffn_seq(T, C_, F_, quant):
                                keep(mr).ptr, kw.ref, vw.ref, rw.ref, x_out.ptr, xx_out.ptr, 0, ws.ptr, None))
     assert_close_f16(xx_out.numpy(), ref_xx, max_ulp=1, what="xx_last")
     assert_close_f16(x_out.numpy(), ref_x, max_ulp=3, max_frac=0.2, what="x_out", floor_rms=1.0)
-
-
-def _routes(T, K, *N):
-    """frhip_gemm_route on 256 compute units -> launches, [(rows of a tile, widest tile in blocks of 32 columns, rounds, loader wave)]"""
-    out = (C.c_int * (4 * len(N)))()
-    launches = L().frhip_gemm_route(T, K, len(N), (C.c_int * len(N))(*N), 256, out)
-    return launches, [tuple(out[4 * i:4 * i + 4]) for i in range(len(N))]
 
 
 @pytest.mark.parametrize("T,C_,F_,rk,v", [
