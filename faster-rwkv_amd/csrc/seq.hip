@@ -183,14 +183,15 @@ __global__ __launch_bounds__(256) void ln_mix_rows_kernel(LnMixSeq a) {
   }
 }
 
-// Rows beyond 4096 elements, up to 256 * NE, C % 512 == 0: the row and the one before it stay in registers too, but
+// Rows beyond 4096 elements, up to 256 * NE: the row and the one before it stay in registers too, but
 // thread t owns elements t, t + 256, ... as in ln_mix_seq_kernel, and every sum is taken in that kernel's order: the same
 // bits as the general form, at any address.  (Groups of 8 consecutive elements, as above, would be another order of the
 // same sums.)  Few rows are bound by the chain of loads, so
 // each batch of them goes out together; many by the 2-byte loads and stores.  1000 x 5120: 14.5 us (13 rows: 5.7),
 // ln_mix_seq_kernel 37.7 (29.9).
-// C % 512: the compiler unrolls the general form's last loop by two and four, and only in the remainder of an odd count
-// does it round (x - mean) * inv once to binary16 (v_fma_mixlo_f16) instead of to fp32 and then to binary16.
+// The compiler unrolls the general form's last loop by two; a thread with an odd count of elements takes its last one in
+// the remainder, where (x - mean) * inv is rounded once to binary16 (v_fma_mixlo_f16) instead of to fp32 and then to
+// binary16.  Both roundings are written out here.
 template <int NE>
 __global__ __launch_bounds__(256) void ln_mix_wide_kernel(LnMixSeq a) {
   __shared__ float red[2][2][4];
@@ -246,9 +247,16 @@ __global__ __launch_bounds__(256) void ln_mix_wide_kernel(LnMixSeq a) {
   for (int n = 0; n < NE; n++) {
 #pragma unroll
     for (int r = 0; r < 2; r++) {
-      float p = ((float)xr[r][n] - mean[r]) * inv[r];
-      asm("" : "+v"(p));  // rounded to fp32 before the conversion: no v_fma_mixlo_f16
-      xr[r][n] = ((h1)p * gam[n]) + bet[n];
+      const float d = (float)xr[r][n] - mean[r];
+      float p = d * inv[r];
+      asm("" : "+v"(p));  // rounded to fp32 before the conversion
+      h1 nrm = (h1)p;
+      if (n >= 16 && n % 2 == 0) {  // C > 4096: every thread has 16 elements before its last
+        uint32_t once;
+        asm("v_fma_mixlo_f16 %0, %1, %2, 0" : "=v"(once) : "v"(d), "v"(inv[r]));
+        if (tid + (n + 1) * 256 >= C) nrm = __builtin_bit_cast(h1, (uint16_t)once);
+      }
+      xr[r][n] = (nrm * gam[n]) + bet[n];
     }
   }
   if (t == 0) {
@@ -655,7 +663,7 @@ static int launch_ln_mix(int T, int C, const void* x, const void* state, const v
     hipLaunchKernelGGL(ln_mix_rows_kernel<1>, dim3(nwg), dim3(256), 0, st, a);
   else if (C % 8 == 0 && C <= 4096)
     hipLaunchKernelGGL(ln_mix_rows_kernel<2>, dim3(nwg), dim3(256), 0, st, a);
-  else if (C % 512 == 0 && C > 4096 && C <= 6144)
+  else if (C > 4096 && C <= 6144)
     hipLaunchKernelGGL(ln_mix_wide_kernel<24>, dim3(T), dim3(256), 0, st, a);
   else
     hipLaunchKernelGGL(ln_mix_seq_kernel, dim3(T), dim3(256), 4 * (size_t)C, st, a);
