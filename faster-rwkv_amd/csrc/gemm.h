@@ -32,6 +32,7 @@ struct GemmArgs {
   size_t part_off[kGemmMaxSeg + 1]; // split launches: where each segment's [M][N] block starts within a slice of `partial` (floats); [nseg] = all
   // gemm_vw_kernel: a segment's tiles are vw_base (the first vw_wide of them vw_base + 1) blocks of 32 columns wide
   int vw_base[kGemmMaxSeg], vw_wide[kGemmMaxSeg], vw_maxw, vw_ns;
+  int few_strips;  // gemm_few_kernel: strips of rows
   GemmSeg seg[kGemmMaxSeg];
   // split K (ksplit >= 2; gemm_ldw_kernel<128> with one segment, gemm_ldw_kernel<64> and the uint8 gemm_kernel<64, 64> with
   // up to four): slice z of ksplit accumulates its K-steps of segment s into partial + z * partial_stride + part_off[s] as
@@ -55,6 +56,17 @@ constexpr size_t kFewRowsFloats = (size_t)512 * 64 * 128;  // two 64 x 128 tiles
 constexpr int kFewRowsMax = 360;                          // rows up to which the seq operators carry that scratch
 int launch_gemm(GemmArgs& a, bool u8, hipStream_t st, const char* what, void* dq = nullptr, float* partial = nullptr,
                 size_t partial_stride = 0, int max_split = 0, float* few_rows = nullptr, size_t few_rows_floats = 0);
+// Products of a few rows in one launch, K split over the waves of a workgroup (gemm_few.hip).  plan_few: the tile that is
+// expected to be the quickest and its us; mt = 0: not a launch of this form.  It depends on the sizes alone, not on the
+// weight type, so that a uint8 weight and its binary16 image take the same sums.  few_takes: the addresses allow it.
+constexpr int kFewKernelRows = 512;
+struct FewPlan {
+  int mt = 0, nt = 0;  // blocks of 16 rows and 16 columns of a workgroup
+  double us = 0;
+};
+FewPlan plan_few(const GemmArgs& a, int cus);
+bool few_takes(const GemmArgs& a, bool u8);
+int launch_gemm_few(const GemmArgs& a, const FewPlan& p, bool u8, hipStream_t st, const char* what);
 constexpr int kDequantRows = FRHIP_SEQ_EXPAND_ROWS;
 // uint8 [N][K] -> binary16 [N][K] with the frozen formula (ops.hip)
 int dequant_u8_async(const unsigned char* q, const h1* mx, const h1* rx, const h1* my, const h1* ry, h1* dst, int K, int N,

@@ -27,14 +27,11 @@
 #include <climits>
 #include <cstring>
 
-#include "gemm.h"
+#include "gemm_device.h"
 
 #pragma clang fp contract(off)
 
 namespace frhip {
-
-typedef float f16v __attribute__((ext_vector_type(16)));
-typedef float f4v __attribute__((ext_vector_type(4)));
 
 constexpr int BN = 128;
 constexpr int kGemmThreads = 256;
@@ -45,83 +42,6 @@ constexpr int kGemmThreads = 256;
 // element every store becomes a branch to an out-of-line block; on the 1024 x 6144 product that
 // was 11 of 59 us.)  The epilogue kind is uniform over the launch segment: one switch, and for the
 // kinds that read operands all 16 of a block are requested before the first is used.
-// sigmoid_h of the 16 accumulators a lane holds of one 32 x 32 block, the same bits at a fraction
-// of the cost.  Called element by element, sigmoid_h makes a wave take its double branch whenever
-// any of its 64 lanes needs it (every other element), and its fp32 estimate alone (expf and a
-// correctly rounded division, ~35 VALU instructions) is 128 x 35 instructions per lane and tile:
-// the sigmoid epilogue of a 128 x 224 tile took 26 us where a plain store takes 2.5 us.
-// Here the estimate is v_exp_f32 and v_rcp_f32.  Its error: t = -x log2(e) is one rounded product,
-// |dt| <= 9e-8 |t|, so exp2(t) is off by at most 6.2e-8 |t| relative, which reaches the result
-// scaled by e/(1+e); over the range that is not handed to the exact path anyway (x > -9.3) that
-// is below 1e-6, plus one ulp each for v_exp_f32, the sum and v_rcp_f32: under 20 fp32 ulps.  An
-// estimate further than 64 ulps from the midpoint of two binary16 values therefore rounds as the
-// exact value does; the others (about 1 in 60) are queued per lane and evaluated in double
-// afterwards, one per lane and pass.  `live`: the elements that are stored.  Rows past the matrix hold copies of its
-// last row, so one pending element would be sixteen: 777 x 2048 x (2048 sigmoid + 8192), whose last strip of 256 rows has
-// nine, took 89 us with all of them queued and takes 57.5 (1024 rows: 59).
-__device__ __forceinline__ void sigmoid_h16(const f16v& c, h1 (&y)[16], uint32_t live) {
-  h1 x[16];
-  uint32_t pend = 0;
-#pragma unroll
-  for (int v = 0; v < 16; v++) {
-    x[v] = (h1)c[v];
-    const float e = __builtin_amdgcn_exp2f((float)x[v] * -1.44269504088896340736f);
-    const float s32 = __builtin_amdgcn_rcpf(1.0f + e);
-    const uint32_t frac = __float_as_uint(s32) & 0x1FFFu;  // the 13 fp32 mantissa bits binary16 drops
-    const bool safe = s32 > 1e-4f && (frac - (0x1000u - 64u)) > 128u;
-    y[v] = (h1)s32;
-    pend |= safe ? 0u : (1u << v);
-  }
-  pend &= live;
-  while (pend) {
-    const int v = __builtin_ctz(pend);
-    pend &= pend - 1;
-    h1 xv = x[0];
-#pragma unroll
-    for (int u = 1; u < 16; u++) xv = (v == u) ? x[u] : xv;
-    const h1 r = sigmoid_h_exact(xv);
-#pragma unroll
-    for (int u = 0; u < 16; u++) y[u] = (v == u) ? r : y[u];
-  }
-}
-
-// silu_h of a block's 16 accumulators, the same bits, built like sigmoid_h16.  silu_h rounds
-// e^-x to binary16, adds 1 in binary16 and divides x by the sum in fp32.  The estimates (v_exp_f32
-// for the exponential, v_rcp_f32 for the quotient: under 20 and 3 fp32 ulps off) are taken when
-// they are further than 64 ulps from a binary16 rounding boundary and in the normal binary16
-// range; the other elements are queued and go through silu_h itself.
-__device__ __forceinline__ void silu_h16(const f16v& c, h1 (&y)[16], uint32_t live) {
-  h1 x[16];
-  uint32_t pend = 0;
-  auto far_from_boundary = [](float v) {
-    const uint32_t frac = __float_as_uint(v) & 0x1FFFu;
-    const float m = __builtin_fabsf(v);
-    return m > 1e-4f && m < 60000.f && (frac - (0x1000u - 64u)) > 128u;
-  };
-#pragma unroll
-  for (int v = 0; v < 16; v++) {
-    x[v] = (h1)c[v];
-    const float xf = (float)x[v];
-    const float ef = __builtin_amdgcn_exp2f(xf * -1.44269504088896340736f);
-    const h1 d = (h1)1.0f + (h1)ef;
-    const float qf = xf * __builtin_amdgcn_rcpf((float)d);
-    const bool safe = far_from_boundary(ef) && far_from_boundary(qf);
-    y[v] = (h1)qf;
-    pend |= safe ? 0u : (1u << v);
-  }
-  pend &= live;
-  while (pend) {
-    const int v = __builtin_ctz(pend);
-    pend &= pend - 1;
-    h1 xv = x[0];
-#pragma unroll
-    for (int u = 1; u < 16; u++) xv = (v == u) ? x[u] : xv;
-    const h1 r = silu_h(xv);
-#pragma unroll
-    for (int u = 0; u < 16; u++) y[u] = (v == u) ? r : y[u];
-  }
-}
-
 template <int MI, int NJ, bool FULL>
 __device__ __forceinline__ void gemm_epilogue_t(const GemmArgs& a, const GemmSeg& sg, const f16v (&acc)[MI][NJ],
                                                 int row0, int col0, int M, int N, int lane) {
@@ -165,7 +85,7 @@ __device__ __forceinline__ void gemm_epilogue_t(const GemmArgs& a, const GemmSeg
       for_blocks([&](int i, int j, const f16v& c) {
         if (outside(i, j)) return;
         h1 y[16];
-        sigmoid_h16(c, y, live_of(i, j));
+        sigmoid_batch(c, y, live_of(i, j));
         for_tile(i, j, [&](int v, bool ok, size_t o) { if (ok) static_cast<h1*>(sg.out)[o] = y[v]; });
       });
       break;
@@ -181,7 +101,7 @@ __device__ __forceinline__ void gemm_epilogue_t(const GemmArgs& a, const GemmSeg
       for_blocks([&](int i, int j, const f16v& c) {
         if (outside(i, j)) return;
         h1 y[16];
-        silu_h16(c, y, live_of(i, j));
+        silu_batch(c, y, live_of(i, j));
         for_tile(i, j, [&](int v, bool ok, size_t o) { if (ok) static_cast<h1*>(sg.out)[o] = y[v]; });
       });
       break;
@@ -401,36 +321,6 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_kernel(GemmArgs a) {
 // term moves them one slot apart: SQ_LDS_BANK_CONFLICT is 0 and a read takes 4 cycles (without
 // that term every read was a two-way conflict: 8 cycles).
 // ---------------------------------------------------------------------------
-// global_load_lds_dwordx4 with the address as a scalar base plus a 32-bit lane offset.  The builtin
-// takes a 64-bit address per lane, which costs the loader one vector add per load; on the SIMD it
-// shares with an MFMA wave each of those waits for a gap between that wave's MFMAs, and the whole
-// workgroup waits for the loader at the step's barrier (per K-step of a 128 x 256 tile: loader 2150
-// cycles from barrier to barrier, MFMA waves 1550-1700 plus 540-700 waiting).  In this form a load
-// needs scalar instructions only.  `lds` is the destination's LDS byte address (lane l writes 16 bytes
-// at lds + 16 l); the wait counts are the caller's business, as with the builtin.
-// M0 is written here without the compiler knowing (it refuses m0 in a clobber list: a reserved register).  That is safe
-// as used: a workgroup issues either these loads or the builtin's (a tile lies wholly inside the matrices or it does not),
-// never both, so no value the compiler keeps in M0 for the builtin is ever live across this statement.
-__device__ __forceinline__ void load_lds_saddr(unsigned voff, const void* sbase, unsigned lds) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "s"(lds) : "memory");
-}
-
-// The same address for every lane, in scalar registers (the compiler cannot always prove it).
-__device__ __forceinline__ const unsigned char* uniform_ptr(const void* p) {
-  const unsigned long long v = reinterpret_cast<unsigned long long>(p);
-  const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)v), hi = __builtin_amdgcn_readfirstlane((unsigned)(v >> 32));
-  return reinterpret_cast<const unsigned char*>(((unsigned long long)hi << 32) | lo);
-}
-
-// The barrier between K-steps whose waits the kernel places itself.  The builtin is no memory fence for the compiler:
-// without the empty statements it could move a fragment read across (nothing else stands between the barrier and the
-// reads in a step that issues no loads).  No instruction of its own.
-__device__ __forceinline__ void step_barrier() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
-
 constexpr int kLdwThreads = 320;
 constexpr int kLdwStages = 4;
 constexpr int kLdwBK = 64;
@@ -635,7 +525,7 @@ __device__ __forceinline__ void splitk_reduce_body(const GemmArgs& a, const Gemm
         f16v c;
 #pragma unroll
         for (int i = 0; i < 16; i++) c[i] = acc[i];
-        if (sg.epi == G_SIGMOID) sigmoid_h16(c, y, 0xffffu); else silu_h16(c, y, 0xffffu);
+        if (sg.epi == G_SIGMOID) sigmoid_batch(c, y, 0xffffu); else silu_batch(c, y, 0xffffu);
       }
       break;
     case G_RELU2:
@@ -1234,36 +1124,59 @@ static bool env_on(const char* name) {
 // 9.0 against 7.3 + 5.2.  Above 64 rows a second strip would dequantise every code again.
 // *taken stays false, and nothing is launched, if the launch is not of this form.
 constexpr int kU8DirectRows = 64;
+
+// Slices of K for a launch of few rows on 64 x 128 tiles, 0 if it is not split as a whole.
+static int few_rows_slices(const GemmArgs& a, size_t few_rows_floats, int cus) {
+  long tiles = 0;
+  size_t cols = 0;
+  for (int s = 0; s < a.nseg; s++) {
+    if (a.seg[s].N % 16 != 0) return 0;
+    tiles += (a.seg[s].N + BN - 1) / BN;
+    cols += (size_t)a.seg[s].N;
+  }
+  const int m64 = (a.M + 63) / 64, ksteps = a.K / kLdwBK;
+  if (tiles * m64 * 2 > cus) return 0;
+  const size_t stride = ((size_t)a.M * cols + 63) / 64 * 64;
+  long S = cus / (tiles * m64);
+  if (S > ksteps / 4) S = ksteps / 4;  // at least four K-steps per slice: twice the ring's depth in flight
+  if ((size_t)S * stride > few_rows_floats) S = (long)(few_rows_floats / stride);
+  return S < 2 ? 0 : (int)S;
+}
+
+// ... or, a group that does not fill the part, product by product, so that its narrow members are
+static bool few_rows_one_by_one(const GemmArgs& a, int cus) {
+  const int m64 = (a.M + 63) / 64;
+  long tiles = 0;
+  bool any = false;
+  for (int s = 0; s < a.nseg; s++) {
+    const long t = (a.seg[s].N + BN - 1) / BN;
+    tiles += t;
+    any = any || (t * m64 * 2 <= cus && a.seg[s].N % 16 == 0);
+  }
+  return a.nseg > 1 && tiles * m64 < cus && any;
+}
+
 static int launch_few_rows(GemmArgs& a, bool u8, hipStream_t st, const char* what, void* dq, float* few_rows,
                            size_t few_rows_floats, bool* taken) {
-  int tiles = 0;
-  bool narrow = true;
-  for (int s = 0; s < a.nseg; s++) {
-    a.tile_start[s] = tiles;
-    tiles += (a.seg[s].N + BN - 1) / BN;
-    narrow = narrow && a.seg[s].N % 16 == 0;
-  }
-  for (int s = a.nseg; s <= kGemmMaxSeg; s++) a.tile_start[s] = INT_MAX;
-  a.tile_start[a.nseg] = tiles;
-  const int m64 = (a.M + 63) / 64, ksteps = a.K / kLdwBK, cus = compute_units();
-  if (ksteps < 4) return 0;
-  if (narrow && (long)tiles * m64 * 2 <= cus) {
+  const int cus = compute_units();
+  if (a.K / kLdwBK < 4) return 0;
+  if (const int S = few_rows_slices(a, few_rows_floats, cus)) {
+    int tiles = 0;
     size_t cols = 0;
     for (int s = 0; s < a.nseg; s++) {
+      a.tile_start[s] = tiles;
+      tiles += (a.seg[s].N + BN - 1) / BN;
       a.part_off[s] = (size_t)a.M * cols;
       cols += (size_t)a.seg[s].N;
     }
+    for (int s = a.nseg; s <= kGemmMaxSeg; s++) a.tile_start[s] = INT_MAX;
+    a.tile_start[a.nseg] = tiles;
     a.part_off[a.nseg] = (size_t)a.M * cols;
-    const size_t stride = (a.part_off[a.nseg] + 63) / 64 * 64;
-    long S = cus / ((long)tiles * m64);
-    if (S > ksteps / 4) S = ksteps / 4;  // at least four K-steps per slice: twice the ring's depth in flight
-    if ((size_t)S * stride > few_rows_floats) S = (long)(few_rows_floats / stride);
-    if (S < 2) return 0;
     *taken = true;
-    a.ksplit = (int)S;
+    a.ksplit = S;
     a.partial = few_rows;
-    a.partial_stride = stride;
-    const dim3 grid(tiles, m64, (unsigned)S);
+    a.partial_stride = (a.part_off[a.nseg] + 63) / 64 * 64;
+    const dim3 grid(tiles, (a.M + 63) / 64, (unsigned)S);
     if (u8)
       gemm_launch_one<64, 64, true>(grid, st, a);
     else
@@ -1272,10 +1185,8 @@ static int launch_few_rows(GemmArgs& a, bool u8, hipStream_t st, const char* wha
     launch_splitk_reduce(st, a);
     return check_launch(what);
   }
-  if (a.nseg == 1 || (long)tiles * m64 >= cus) return 0;  // a group that fills the part as it is stays one launch
-  for (int s = 0; s < a.nseg; s++)
-    *taken = *taken || ((long)((a.seg[s].N + BN - 1) / BN) * m64 * 2 <= cus && a.seg[s].N % 16 == 0);
-  if (!*taken) return 0;
+  if (!few_rows_one_by_one(a, cus)) return 0;
+  *taken = true;
   for (int s = 0; s < a.nseg; s++) {
     GemmArgs one = a;
     one.nseg = 1;
@@ -1283,6 +1194,52 @@ static int launch_few_rows(GemmArgs& a, bool u8, hipStream_t st, const char* wha
     if (int rc = launch_gemm(one, u8, st, what, dq, nullptr, 0, 0, few_rows, few_rows_floats)) return rc;
   }
   return 0;
+}
+
+// Slices of K of a single product with few outputs and a long K on 128 x 128 tiles (below), 0 if it is not split.
+static int long_k_slices(const GemmArgs& a, size_t partial_stride, int max_split, int cus) {
+  const int epi = a.seg[0].epi;
+  if (max_split < 2 || a.nseg != 1 || a.K < 4096 || a.seg[0].N % 16 != 0 || (size_t)a.M * a.seg[0].N > partial_stride ||
+      (epi != G_STORE_F16 && epi != G_STORE_F32 && epi != G_RESIDUAL && epi != G_FFN_OUT))
+    return 0;
+  const long t128 = (long)((a.seg[0].N + BN - 1) / BN) * ((a.M + 127) / 128);
+  int S = (int)(cus / t128);
+  if (S > max_split) S = max_split;
+  while (S >= 2 && a.K / (kLdwBK * S) < 16) S--;
+  return S >= 2 && t128 * S * 5 >= (long)cus * 3 ? S : 0;  // the slices fill at least 60 % of the CUs
+}
+
+// What launch_gemm's other binary16 forms are expected to take, us, in its order: split over K on 64-row tiles, product by
+// product, split over K on 128-row tiles, planned tiles.  The split forms are fitted to 600 measured products (5 to 7 % rms),
+// their reduction launch included.
+static double tiled_us(const GemmArgs& a, size_t partial_stride, int max_split, size_t few_rows_floats, int cus) {
+  const double outs = [&] { double n = 0; for (int s = 0; s < a.nseg; s++) n += (double)a.M * a.seg[s].N; return n; }();
+  auto each = [&](size_t floats) {
+    double us = 0;
+    for (int s = 0; s < a.nseg; s++) {
+      GemmArgs one = a;
+      one.nseg = 1;
+      one.seg[0] = a.seg[s];
+      us += tiled_us(one, 0, 0, floats, cus);
+    }
+    return us;
+  };
+  const int ksteps = a.K / kLdwBK;
+  if (few_rows_floats && ksteps >= 4) {
+    if (const int S = few_rows_slices(a, few_rows_floats, cus))
+      return 6.8 + 0.37 * ((ksteps + S - 1) / S) + outs / a.M * a.K * 2 / 11.3e6 + 0.067 * S + outs * S * 8 / 4.27e6;
+    if (few_rows_one_by_one(a, cus)) return each(few_rows_floats);
+  }
+  if (const int S = long_k_slices(a, partial_stride, max_split, cus)) return 10 + 0.66 * ((ksteps + S - 1) / S) + outs * S * 8 / 7.1e6;
+  const GemmRoute r = gemm_route(a, cus);
+  if (one_by_one(a, r, cus)) return each(0);
+  return r.rows ? r.us : us_64((int)((tiles64(a) + cus - 1) / cus), a.K / 2048.0);
+}
+
+// plan_few's tile where it is worth it, with the scratch that the other forms would have
+static FewPlan few_plan(const GemmArgs& a, size_t partial_stride, int max_split, size_t few_rows_floats, int cus) {
+  const FewPlan p = plan_few(a, cus);
+  return p.mt && p.us * 1.1 <= tiled_us(a, partial_stride, max_split, few_rows_floats, cus) ? p : FewPlan();
 }
 
 int launch_gemm(GemmArgs& a, bool u8, hipStream_t st, const char* what, void* dq, float* partial, size_t partial_stride,
@@ -1295,6 +1252,14 @@ int launch_gemm(GemmArgs& a, bool u8, hipStream_t st, const char* what, void* dq
   // measurement aid); uint8 weights need the registers in between for the dequantisation
   static const bool ldw = env_on("FRHIP_GEMM_LDW"), few = env_on("FRHIP_GEMM_FEW_ROWS");
   const bool few_ok = ldw && splitk && few && !force_bm && few_rows;
+  // Few rows: one launch with K split over the waves of a workgroup where that is expected to be the quicker form by a
+  // tenth (both estimates are good to that).  Every workgroup of it reads all rows of X: a long K over few columns is quicker
+  // split over K in memory (64 x 20480 x 5120: 45 us against 64; 77 x 8192 x 2048: 17.3 both), many rows of wide products on
+  // planned tiles (256 x 5120 x (5120 + 20480): 91 against 143).  Decided by the sizes alone: uint8 codes and their binary16
+  // image, expanded here or kept by the caller, give the same bits.
+  const FewPlan fp = ldw && splitk && few && !force_bm ? few_plan(a, partial ? partial_stride : 0, partial ? max_split : 0, few_ok ? few_rows_floats : 0, compute_units())
+                                                       : FewPlan();
+  if (fp.mt && few_takes(a, u8)) return launch_gemm_few(a, fp, u8, st, what);
   bool direct = u8 && dq && a.M >= kDequantRows && a.M <= kU8DirectRows;
   for (int s = 0; s < a.nseg; s++)  // the uint8 kernel reads codes and row scales 16 bytes at a time; the expansion takes any address
     direct = direct && ((reinterpret_cast<uintptr_t>(a.seg[s].B) | reinterpret_cast<uintptr_t>(a.seg[s].ry) |
@@ -1323,6 +1288,7 @@ int launch_gemm(GemmArgs& a, bool u8, hipStream_t st, const char* what, void* dq
     }
     if (int rc = dequant_u8_group_async(a.nseg, qs, mxs, rxs, mys, rys, dsts, a.K, ns, st)) return rc;
     u8 = false;
+    if (fp.mt && few_takes(a, false)) return launch_gemm_few(a, fp, false, st, what);
   }
   if (!u8 && few_ok) {
     bool taken = false;
@@ -1347,14 +1313,8 @@ int launch_gemm(GemmArgs& a, bool u8, hipStream_t st, const char* what, void* dq
   // (786 MB in 57 us).  With scratch for the partial sums the launch runs ksplit slices of K over 128 x 128 tiles, and a
   // second kernel adds the slices in order and applies the epilogue.  The sums are grouped by slice, so the result can
   // differ from the unsplit launch in the last fp32 bit before the rounding to binary16.  FRHIP_GEMM_SPLITK=0: off.
-  if (!u8 && ldw && splitk && !force_bm && partial && max_split >= 2 && a.nseg == 1 && a.K >= 4096 && a.seg[0].N % 16 == 0 &&
-      (a.seg[0].epi == G_STORE_F16 || a.seg[0].epi == G_STORE_F32 || a.seg[0].epi == G_RESIDUAL || a.seg[0].epi == G_FFN_OUT) &&
-      (size_t)a.M * a.seg[0].N <= partial_stride) {
-    const long t128 = (long)tiles * m128;
-    int S = (int)(compute_units() / t128);
-    if (S > max_split) S = max_split;
-    while (S >= 2 && a.K / (kLdwBK * S) < 16) S--;
-    if (S >= 2 && t128 * S * 5 >= (long)compute_units() * 3) {  // the slices fill at least 60 % of the CUs
+  if (!u8 && ldw && splitk && !force_bm && partial) {
+    if (const int S = long_k_slices(a, partial_stride, max_split, compute_units())) {
       a.ksplit = S;
       a.partial = partial;
       a.partial_stride = partial_stride;
@@ -1467,6 +1427,25 @@ extern "C" int frhip_gemm_route(int T, int K, int nproducts, const int* N, int c
     out[4 * s + 3] = r.rows != 0 && r.loader;
   }
   return split ? nproducts : 1;
+}
+
+extern "C" int frhip_gemm_few_tile(int T, int K, int nproducts, const int* N, int compute_units, int* out) {
+  if (!N || !out) return set_error(FRHIP_EINVAL, "gemm_few_tile: null pointer");
+  if (T <= 0 || K <= 0 || K % 64 != 0 || nproducts < 1 || nproducts > kGemmMaxSeg || compute_units < 1)
+    return set_error(FRHIP_ESHAPE, "gemm_few_tile: no such launch");
+  GemmArgs a;
+  memset(&a, 0, sizeof(a));
+  a.M = T;
+  a.K = K;
+  a.nseg = nproducts;
+  for (int s = 0; s < nproducts; s++) {
+    if (N[s] <= 0) return set_error(FRHIP_ESHAPE, "gemm_few_tile: no such launch");
+    a.seg[s].N = N[s];
+  }
+  const FewPlan p = few_plan(a, 0, 0, 0, compute_units);
+  out[0] = p.mt;
+  out[1] = p.nt;
+  return 0;
 }
 
 static_assert(FRHIP_ACT_SIGMOID == G_SIGMOID && FRHIP_ACT_RELU2 == G_RELU2 && FRHIP_ACT_SILU == G_SILU, "activation codes");

@@ -300,6 +300,10 @@ int frhip_att_seq_v5(int T, int C, int H, const void *x, const void *sx, const f
  * out[4 i + 1]: its widest tile in blocks of 32 columns, out[4 i + 2]: its rounds over the compute units,
  * out[4 i + 3]: 1 if a wave of its own loads the tiles. */
 int frhip_gemm_route(int T, int K, int nproducts, const int *N, int compute_units, int *out);
+/* Whether such a launch goes, instead, to the kernel for a few rows (K split over the waves of a workgroup), and with which
+ * tile: out[0], out[1] = blocks of 16 rows and of 16 columns of a workgroup, 0, 0 if it is cut as above.  A pure function
+ * of the sizes too. */
+int frhip_gemm_few_tile(int T, int K, int nproducts, const int *N, int compute_units, int *out);
 
 /* ---- bandwidth probes: DIAGNOSTICS, not operators (measurement aids of bench.py and of the
  *      hardware-counter calibration; no counterpart in the reference, nothing on the model path calls them) */
