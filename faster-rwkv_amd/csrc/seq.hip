@@ -5,8 +5,9 @@
 // as one serial loop of T steps on a handful of wavefronts (kernels/cuda/att_seq.cu:258-322
 // runs 64 threads per head for T steps):
 //   1. every chunk is scanned from an EMPTY state, all chunks in parallel -> local end states;
-//   2. a short serial pass over the chunks turns local end states into the true state at the
-//      start of every chunk (state_in[c+1] = decay^len(state_in[c]) + local[c]);
+//   2. the local end states are turned into the true state at the start of every chunk
+//      (state_in[c+1] = decay^len(state_in[c]) + local[c]): by doubling in LDS (RWKV-4, all in one
+//      launch) or a short serial pass over the chunks (RWKV-5);
 //   3. every chunk is scanned again from its true start state, all chunks in parallel,
 //      producing the outputs; the last chunk leaves the final state.
 // The arithmetic of pass 3 is the one-token recurrence (kernels/cuda/att.cu:30-62, :64-81);
@@ -280,28 +281,28 @@ __global__ __launch_bounds__(256) void ln_mix_wide_kernel(LnMixSeq a) {
 }
 
 // ---------------------------------------------------------------------------
-// RWKV-4 WKV scan.  k, v [T][C] fp32; r [T][C] half (already through the sigmoid),
-// overwritten with r * half(wkv).
+// RWKV-4 WKV scan, one launch.  k, v [T][C] fp32; r [T][C] half (already through the sigmoid), overwritten with
+// r * half(wkv).
+//
+// A workgroup owns CG channels and cuts time into blocks of nchunk chunks of Lc steps, a thread per (channel, chunk).
+// Per block: every chunk is scanned from an empty state (k and v stay in registers); the local end states are
+// composed into the states at the ends of the chunks by a doubling scan in LDS; every chunk is scanned again from its true
+// start state, writing the outputs; the last chunk's end state starts the next block.
+// What bounds it: about 150 vector instructions per channel and step, most of them three expf (a six-instruction
+// exponential within 2 ulp would save a tenth, but the outputs would no longer be those of the one-token kernel).  att_seq_v4
+// as a whole (products included) against a launch for pass 1, one for passes 2 and 3, which read k and v twice and
+// composed every chunk's start from all chunks before it, us: 2048 channels, T = 13: 22.2 -> 18.1, 77: 29.4 -> 25.1,
+// 1024: 81.4 -> 73.3, 4099 (a serial pass 2 of its own): 233.5 -> 221.2; 5120 channels, T = 1024: 258 both.
+// (A form with scalar bases for whole blocks and masked steps for the last one spilled registers: 1024: 75.)
 // ---------------------------------------------------------------------------
+constexpr int kWkv4MaxCg = 32;
 struct Wkv4Seq {
-  int T, C, Lc, nchunk;
+  int T, C, Lc, nchunk, nblock, cg;
   const float *k, *v, *u, *w;
   h1* r;
-  const float *aa, *bb, *pp;  // state before the sequence (read by pass 1 only; may alias aa_out / bb_out / pp_out)
-  float *la, *lb, *lp;        // [nchunk][C] local end states (pass 1)
-  float *sa, *sb, *sp;        // [nchunk][C] state at the start of each chunk (row 0: pass 1; the rest: the serial pass)
+  const float *aa, *bb, *pp;  // state before the sequence; may alias aa_out / bb_out / pp_out (a channel has one workgroup)
   float *aa_out, *bb_out, *pp_out;
 };
-
-// Steps per batch of loads in the chunk passes: a thread requests the k, v (and r) of kScanB steps
-// before the recurrence touches the first, so a chunk of 16 steps costs one memory round trip
-// instead of 16 (with two waves per SIMD little else hides them: 8.3 -> 6.9 us and 10.7 -> 9.0 us
-// per launch at T = 1024).  What remains is launch, one round trip and the library expf (~28 VALU
-// instructions; three per token and channel over the passes, one per pair: exp_pair below); a
-// six-instruction exp2-based exponential within 2 ulp was measured when the passes still took six
-// (28.4 -> 25.2 us) and was not kept: the passes then no longer compute exactly what the one-token
-// kernel does.
-constexpr int kScanB = 16;
 
 // p = max(a, b) (b on ties), ea = exp(a - p), eb = exp(b - p) with one exponential instead of two: the
 // argument of the other one is +0 and expf(+0) is exactly 1, so for finite a and b these are the bits
@@ -314,158 +315,97 @@ __device__ __forceinline__ void exp_pair(float a, float b, float& p, float& ea, 
   eb = first ? e : 1.0f;
 }
 
-__global__ __launch_bounds__(256) void wkv4_local_kernel(Wkv4Seq a) {
-  const int c = blockIdx.x * 256 + threadIdx.x, ch = blockIdx.y;
-  if (c >= a.C) return;
-  const int t0 = ch * a.Lc, t1 = min(t0 + a.Lc, a.T);
-  const float w = a.w[c];
-  float aa = 0.f, bb = 0.f, pp = -1e30f;
-  for (int tb = t0; tb < t1; tb += kScanB) {
-    float kk[kScanB], vv[kScanB];
-#pragma unroll
-    for (int i = 0; i < kScanB; i++) {
-      const int t = tb + i < t1 ? tb + i : t1 - 1;
-      kk[i] = a.k[(size_t)t * a.C + c];
-      vv[i] = a.v[(size_t)t * a.C + c];
-    }
-#pragma unroll
-    for (int i = 0; i < kScanB; i++) {
-      if (tb + i < t1) {
-        const float k = kk[i], v = vv[i];
-        float p, e1, e2;
-        exp_pair(w + pp, k, p, e1, e2);
-        aa = e1 * aa + e2 * v;
-        bb = e1 * bb + e2;
-        pp = p;
-      }
-    }
-  }
-  const size_t o = (size_t)ch * a.C + c;
-  a.la[o] = aa;
-  a.lb[o] = bb;
-  a.lp[o] = pp;
-  // The state before the sequence is copied into chunk 0's start-state slot.  The later passes read it
-  // from there, never from aa / bb / pp: the last chunk of the apply pass writes aa_out / bb_out / pp_out,
-  // which may be the same buffers, while chunks that were scheduled later have not started yet.
-  if (ch == 0) {
-    a.sa[c] = a.aa[c];
-    a.sb[c] = a.bb[c];
-    a.sp[c] = a.pp[c];
-  }
+// a: state (aa, bb, pp) followed by `steps` (times the decay w: dw) that contribute (la, lb, lp)
+__device__ __forceinline__ void wkv4_compose(float& aa, float& bb, float& pp, float dw, float la, float lb, float lp) {
+  float p, e1, e2;
+  exp_pair(pp + dw, lp, p, e1, e2);
+  aa = e1 * aa + e2 * la;
+  bb = e1 * bb + e2 * lb;
+  pp = p;
 }
 
-// The serial pass over the chunks.  A channel's step needs three values per chunk; they are read
-// eight chunks at a time ahead of the recurrence, so the pass costs one memory round trip per
-// eight chunks instead of one per chunk.
-__global__ __launch_bounds__(64) void wkv4_carry_kernel(Wkv4Seq a) {
-  const int c = blockIdx.x * 64 + threadIdx.x;
-  if (c >= a.C) return;
-  constexpr int PF = 8;
-  const float w = a.w[c];
-  float aa = a.sa[c], bb = a.sb[c], pp = a.sp[c];  // the incoming state, left there by wkv4_local_kernel
-  for (int ch0 = 0; ch0 < a.nchunk; ch0 += PF) {
-    float lp[PF], la[PF], lb[PF];
-#pragma unroll
-    for (int i = 0; i < PF; i++) {
-      const int ch = ch0 + i < a.nchunk ? ch0 + i : a.nchunk - 1;
-      const size_t o = (size_t)ch * a.C + c;
-      lp[i] = a.lp[o];
-      la[i] = a.la[o];
-      lb[i] = a.lb[o];
-    }
-#pragma unroll
-    for (int i = 0; i < PF; i++) {
-      const int ch = ch0 + i;
-      if (ch < a.nchunk) {
-        const size_t o = (size_t)ch * a.C + c;
-        a.sa[o] = aa;
-        a.sb[o] = bb;
-        a.sp[o] = pp;
-        const int len = min(a.Lc, a.T - ch * a.Lc);
-        // the incoming state decays by len steps; the chunk's own tokens contribute its local state
-        float p, e1, e2;
-        exp_pair(pp + (float)len * w, lp[i], p, e1, e2);
-        aa = e1 * aa + e2 * la[i];
-        bb = e1 * bb + e2 * lb[i];
-        pp = p;
-      }
-    }
-  }
-}
-
-// CARRY: the chunk forms its own start state by composing, in order, the incoming state with the
-// local end states of the chunks before it -- the serial pass's arithmetic, step for step, so the
-// results are the serial pass's bit for bit -- instead of reading what wkv4_carry_kernel left.  Chunk j
-// spends j compositions (two exponentials each) where the serial pass spends one launch and nchunk
-// dependent steps per channel; the local states are requested eight chunks at a time.
-template <bool CARRY>
-__global__ __launch_bounds__(256) void wkv4_apply_kernel(Wkv4Seq a) {
-  // the chunks with the longest prefix first: they decide when the launch ends
-  const int c = blockIdx.x * 256 + threadIdx.x, ch = CARRY ? (int)(gridDim.y - 1 - blockIdx.y) : (int)blockIdx.y;
-  if (c >= a.C) return;
-  const int t0 = ch * a.Lc, t1 = min(t0 + a.Lc, a.T);
+template <int LMAX>
+__global__ __launch_bounds__(1024) void wkv4_scan_kernel(Wkv4Seq a) {
+  __shared__ float ends[2][3][1024];  // end states of the chunks, by thread; two copies in turn
+  __shared__ float start[3][kWkv4MaxCg];  // state at the start of the block
+  const int CG = a.cg;
+  // neighbouring channels on one XCD: CG channels are 4 CG bytes of a row, a part of a line
+  const int n = gridDim.x, xcd = blockIdx.x & 7, grp = xcd * (n >> 3) + min(xcd, n & 7) + (blockIdx.x >> 3);
+  const int tid = threadIdx.x, cl = tid % CG, ch = tid / CG, c = grp * CG + cl;
   const float w = a.w[c], u = a.u[c];
-  const size_t o = (size_t)ch * a.C + c;
-  float aa, bb, pp;
-  if constexpr (CARRY) {
-    constexpr int PF = 8;
-    aa = a.sa[c], bb = a.sb[c], pp = a.sp[c];  // the incoming state, left there by wkv4_local_kernel
-    const float pdw = (float)a.Lc * w;  // every chunk before this one is a full chunk
-    for (int j0 = 0; j0 < ch; j0 += PF) {
-      float lp[PF], la[PF], lb[PF];
-#pragma unroll
-      for (int i = 0; i < PF; i++) {
-        const int j = j0 + i < ch ? j0 + i : ch - 1;
-        const size_t q = (size_t)j * a.C + c;
-        lp[i] = a.lp[q];
-        la[i] = a.la[q];
-        lb[i] = a.lb[q];
-      }
-#pragma unroll
-      for (int i = 0; i < PF; i++) {
-        if (j0 + i < ch) {
-          float p, e1, e2;
-          exp_pair(pp + pdw, lp[i], p, e1, e2);
-          aa = e1 * aa + e2 * la[i];
-          bb = e1 * bb + e2 * lb[i];
-          pp = p;
-        }
-      }
-    }
-  } else {
-    aa = a.sa[o], bb = a.sb[o], pp = a.sp[o];
+  if (ch == 0) {
+    start[0][cl] = a.aa[c];
+    start[1][cl] = a.bb[c];
+    start[2][cl] = a.pp[c];
   }
-  for (int tb = t0; tb < t1; tb += kScanB) {
-    float kk[kScanB], vv[kScanB];
-    h1 rr[kScanB];
+  const float dw = (float)a.Lc * w;
+  for (int blk = 0; blk < a.nblock; blk++) {
+    const int t0 = (blk * a.nchunk + ch) * a.Lc, len = min(a.Lc, a.T - t0);  // len <= 0: nothing left for this chunk
+    float kk[LMAX], vv[LMAX];
+    h1 rr[LMAX];
 #pragma unroll
-    for (int i = 0; i < kScanB; i++) {
-      const int t = tb + i < t1 ? tb + i : t1 - 1;
-      const size_t j = (size_t)t * a.C + c;
+    for (int i = 0; i < LMAX; i++) {
+      const size_t j = (size_t)min(t0 + min(i, a.Lc - 1), a.T - 1) * a.C + c;
       kk[i] = a.k[j];
       vv[i] = a.v[j];
       rr[i] = a.r[j];
     }
+    // from an empty state, without the chain of running maxima: aa = sum exp(k_i + (len - 1 - i) w - pp) v_i, bb = the same without v
+    float aa = 0.f, bb = 0.f, pp = -1e30f, q[LMAX], off = 0.f;
 #pragma unroll
-    for (int i = 0; i < kScanB; i++) {
-      if (tb + i < t1) {
+    for (int i = LMAX - 1; i >= 0; i--) {
+      q[i] = i < len ? kk[i] + off : -1e30f;
+      off = i < len ? off + w : off;
+      pp = fmaxf(pp, q[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < LMAX; i++) {
+      const float e = i < len ? expf(q[i] - pp) : 0.f;
+      aa += e * vv[i];
+      bb += e;
+    }
+    // after the step of distance s, a thread holds the contribution of its chunk and up to 2 s - 1 chunks before it
+    int cur = 0;
+    for (int s = 1; s < a.nchunk; s *= 2) {
+      ends[cur][0][tid] = aa;
+      ends[cur][1][tid] = bb;
+      ends[cur][2][tid] = pp;
+      __syncthreads();
+      if (ch >= s) {
+        float pa = ends[cur][0][tid - s * CG], pb = ends[cur][1][tid - s * CG], p = ends[cur][2][tid - s * CG];
+        wkv4_compose(pa, pb, p, (float)s * dw, aa, bb, pp);
+        aa = pa, bb = pb, pp = p;
+      }
+      cur ^= 1;
+    }
+    ends[cur][0][tid] = aa;
+    ends[cur][1][tid] = bb;
+    ends[cur][2][tid] = pp;
+    __syncthreads();
+    aa = start[0][cl], bb = start[1][cl], pp = start[2][cl];
+    if (ch > 0)
+      wkv4_compose(aa, bb, pp, (float)ch * dw, ends[cur][0][tid - CG], ends[cur][1][tid - CG], ends[cur][2][tid - CG]);
+#pragma unroll
+    for (int i = 0; i < LMAX; i++) {
+      if (i < len) {
         const float k = kk[i], v = vv[i];
         // kernels/cuda/att.cu:43-60
         float p, e1, e2;
         exp_pair(pp, u + k, p, e1, e2);
         const float wkv = (e1 * aa + e2 * v) / (e1 * bb + e2);
-        a.r[(size_t)(tb + i) * a.C + c] = rr[i] * (h1)wkv;
-        exp_pair(w + pp, k, p, e1, e2);
-        aa = e1 * aa + e2 * v;
-        bb = e1 * bb + e2;
-        pp = p;
+        a.r[(size_t)(t0 + i) * a.C + c] = rr[i] * (h1)wkv;
+        wkv4_compose(aa, bb, pp, w, v, 1.0f, k);
       }
     }
-  }
-  if (ch == a.nchunk - 1) {
-    a.aa_out[c] = aa;
-    a.bb_out[c] = bb;
-    a.pp_out[c] = pp;
+    if (len > 0 && t0 + len == a.T) {
+      a.aa_out[c] = aa;
+      a.bb_out[c] = bb;
+      a.pp_out[c] = pp;
+    }
+    if (blk + 1 < a.nblock) {
+      __syncthreads();  // everyone has read `start` and `ends`
+      if (ch == a.nchunk - 1) start[0][cl] = aa, start[1][cl] = bb, start[2][cl] = pp;  // read behind the next block's barriers
+    }
   }
 }
 
@@ -670,6 +610,31 @@ static int launch_ln_mix(int T, int C, const void* x, const void* state, const v
   return check_launch("ln_mix_seq");
 }
 
+// A workgroup's channels: about one workgroup per compute unit, at least 8 (32-byte pieces of a row), a divisor of C (a multiple
+// of 64, so 32 is one).  Chunks of at least 4 steps (2 where that still is one wave's work), of at most 16, which a thread
+// keeps in registers; up to 128 of them where 8 channels leave room, 64 otherwise (longer blocks have more doubling steps
+// than they save).  Of att_seq_v4, us: C = 5120, T = 2048: 484 with 20 channels, 501 with 16 (1.25 rounds), 492 with 8.
+static void launch_wkv4_scan(Wkv4Seq& q, hipStream_t st) {
+  constexpr int kMaxLc = 16;
+  q.cg = (q.C + compute_units() - 1) / compute_units();
+  if (q.cg < 8) q.cg = 8;
+  while (q.cg < kWkv4MaxCg && q.C % q.cg != 0) q.cg++;
+  if (q.cg > kWkv4MaxCg) q.cg = kWkv4MaxCg;
+  const int most = 1024 / q.cg, chunks = q.cg == 8 ? 128 : most < 64 ? most : 64;
+  q.nblock = (q.T + chunks * kMaxLc - 1) / (chunks * kMaxLc);
+  q.Lc = (q.T + chunks * q.nblock - 1) / (chunks * q.nblock);
+  const int least = q.T <= 32 ? 2 : 4;
+  if (q.Lc < least) q.Lc = least;
+  q.nchunk = (q.T + q.Lc * q.nblock - 1) / (q.Lc * q.nblock);
+  const dim3 grid(q.C / q.cg), block(q.nchunk * q.cg);
+  if (q.Lc <= 4)
+    hipLaunchKernelGGL(wkv4_scan_kernel<4>, grid, block, 0, st, q);
+  else if (q.Lc <= 8)
+    hipLaunchKernelGGL(wkv4_scan_kernel<8>, grid, block, 0, st, q);
+  else
+    hipLaunchKernelGGL(wkv4_scan_kernel<16>, grid, block, 0, st, q);
+}
+
 // chunk length for a scan of T steps when one chunk occupies `units` workgroup-sized units:
 // enough chunks to fill the device (~4 units per CU), chunks of at least 16 steps (the serial pass
 // over the chunks costs about 0.18 us per chunk: at T = 1024, 64 chunks of 16 beat 128 of 8)
@@ -810,31 +775,10 @@ extern "C" int frhip_att_seq_v4(int T, int C, const void* x, const void* sx, con
 
   Wkv4Seq q;
   q.T = T; q.C = C;
-  q.Lc = pick_chunk(T, (C + 255) / 256);
-  // FRHIP_WKV4_SERIAL_CARRY=1: the chunk start states from a serial pass of their own (same bits)
-  static const bool force_serial = getenv("FRHIP_WKV4_SERIAL_CARRY") != nullptr;
-  // Without the serial pass a chunk composes the local states of all chunks before it, nchunk / 2 compositions
-  // on average against Lc steps of its own: quadratic in T.  Beyond kComposeMaxChunks chunks of 32 steps
-  // (T > 4096) the serial pass takes over.
-  constexpr int kComposeMaxChunks = 128;
-  const bool serial_carry = force_serial || (T + 31) / 32 > kComposeMaxChunks;
-  // half as many, twice as long chunks (32 of 32 steps at T = 1024) cost the scans less than they save
-  // the composition
-  if (!serial_carry && q.Lc < 32 && T >= 512) q.Lc = 32;
-  q.nchunk = (T + q.Lc - 1) / q.Lc;
   q.k = w.f0; q.v = w.f1; q.u = t_first; q.w = t_decay; q.r = w.m3;
   q.aa = aa; q.bb = bb; q.pp = pp;
-  const size_t n = al256(4 * (size_t)q.nchunk * C) / 4;
-  q.la = w.scan; q.lb = q.la + n; q.lp = q.lb + n; q.sa = q.lp + n; q.sb = q.sa + n; q.sp = q.sb + n;
   q.aa_out = aa_out; q.bb_out = bb_out; q.pp_out = pp_out;
-  dim3 grid((C + 255) / 256, q.nchunk);
-  hipLaunchKernelGGL(wkv4_local_kernel, grid, dim3(256), 0, st, q);
-  if (serial_carry) {
-    hipLaunchKernelGGL(wkv4_carry_kernel, dim3((C + 63) / 64), dim3(64), 0, st, q);
-    hipLaunchKernelGGL(wkv4_apply_kernel<false>, grid, dim3(256), 0, st, q);
-  } else {
-    hipLaunchKernelGGL(wkv4_apply_kernel<true>, grid, dim3(256), 0, st, q);
-  }
+  launch_wkv4_scan(q, st);
   FR_TRY(check_launch("wkv4_seq"));
 
   GemmArgs b;

@@ -388,6 +388,15 @@ def test_att_seq_v4(T, C_, quant, fresh):
     assert np.abs(po_.numpy() - ref[4]).max() < 30  # offsets stay in a sane range
 
 
+@pytest.mark.parametrize("T,C_", [(2, 512), (3, 512), (32, 512), (33, 512),  # one wave's chunks of 2 steps; of 4
+                                  (513, 320), (1025, 192),                  # 5 of 8 and 9 of 16 registers of a chunk in use
+                                  (2049, 128), (4097, 64),                  # two and three blocks, the last one ragged
+                                  (66, 2560), (17, 5120)])                  # 10 and 20 channels a workgroup, partial waves
+def test_att_seq_v4_scan_cuts(T, C_):
+    """Every way the scan cuts time and channels.  Bounds as in test_att_seq_v4."""
+    test_att_seq_v4(T, C_, False, False)
+
+
 @pytest.mark.parametrize("T,C_,kvr,o", [(16400, 320, (256, 5, 2, 0), (256, 4, 1, 0)),  # predicated epilogues: 16 rows in the last strip
                                         (4096, 448, (256, 3, 1, 1), (64, 4, 1, 1))])   # whole tiles: the loader wave's form
 def test_att_seq_v4_on_planned_tiles(T, C_, kvr, o):
