@@ -91,7 +91,9 @@ int fr_model_run(void *m, const int *ids, int n, float *logits, int capacity) {
 long long fr_model_run_full(void *m, const int *ids, int n, float *logits, long long capacity) {
   return guarded([&]() -> long long {
     auto *model = static_cast<rwkv::Model *>(m);
-    rwkv::Tensor out = rwkv::ModelForwardSeq(model, model->_act_device, std::vector<int>(ids, ids + n), true);
+    const std::vector<int> in(ids, ids + n);
+    rwkv::Tensor out = model->_act_device == rwkv::Device::kHIP ? rwkv::hip::FullLogits(model, in)
+                                                               : rwkv::ModelForwardSeq(model, model->_act_device, in, true);
     const long long v = static_cast<long long>(out.numel());
     if (v > capacity) throw FRException("logits buffer too small");
     if (out.device() == rwkv::Device::kHIP)

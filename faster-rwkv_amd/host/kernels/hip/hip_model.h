@@ -25,8 +25,12 @@ struct ModelExtra {
 };
 
 std::shared_ptr<ModelExtra> extra_of(Model *model);
-// A device tensor into `dst` (src.nbytes() bytes of host memory), after the work queued so far; returns when it is there.
-void read_to_host(ModelExtra &ex, const Tensor &src, void *dst);
+// A device tensor of fp32 or binary16 into `dst` (src.numel() floats of host memory), after the work queued so far; returns
+// when it is there.
+void read_to_host(ModelExtra &ex, const Tensor &src, float *dst);
+// ModelForwardSeq(model, Device::kHIP, ids, full_output = true) without its last step: binary16 logits where the pass computes
+// them as such, for read_to_host to widen.
+Tensor FullLogits(Model *model, const std::vector<int> &ids);
 bool device_argmax(Model *model, const Tensor &logits, int *id);
 // `steps` greedy tokens from `first_id` with the token choice left on the device (model_forward.cpp).
 bool GreedyDecode(Model *model, int first_id, int steps, int *out_ids, Tensor *last_logits = nullptr);

@@ -502,9 +502,10 @@ bool device_argmax(Model *model, const Tensor &logits, int *id) {
 // gathered on the device, every layer runs its seq operator over all T rows (MFMA products,
 // chunked WKV scans), and only the last row goes through ln_out and the head (all rows with
 // full_output).  RWKV-4, which
-// upstream cannot run in seq mode (:111-112), goes through the `att_seq` operator.
+// upstream cannot run in seq mode (:111-112), goes through the `att_seq` operator.  `widened`: full output as fp32, as
+// the reference has it, not as the binary16 values that the head product gives.
 // FR_HIP_SEQ_FALLBACK=1 selects the loop of one-token steps (:34-46) instead.
-Tensor ModelForwardSeq(Model *model, Device device, const std::vector<int> &ids, bool full_output) {
+static Tensor forward_seq(Model *model, Device device, const std::vector<int> &ids, bool full_output, bool widened) {
   const std::string &ver = model->version();
   if (std::getenv("FR_HIP_SEQ_FALLBACK") || !(ver == "4" || ver == "5" || ver == "5.2"))
     return def::ModelForwardSeqFallback(model, device, ids, full_output);
@@ -569,7 +570,7 @@ Tensor ModelForwardSeq(Model *model, Device device, const std::vector<int> &ids,
     Tensor y = layernorm(x, p[pi], p[pi + 1]);
     Tensor lg = Tensor::Empty({T, static_cast<LengthType>(hw->N)}, DType::kFloat16, Device::kHIP);
     FRHIP_CHECK(frhip_gemm(y.data_ptr(), hw, lg.data_ptr(), T, FRHIP_F16, s));
-    return cast_dtype(lg, DType::kFloat32);
+    return widened ? cast_dtype(lg, DType::kFloat32) : lg;
   }
   // last row -> ln_out -> head -> fp32 (model_forward_seq.cpp:170-178)
   Tensor logits = Tensor::Empty({static_cast<LengthType>(hw->N)}, DType::kFloat32, Device::kHIP);
@@ -577,6 +578,12 @@ Tensor ModelForwardSeq(Model *model, Device device, const std::vector<int> &ids,
   FRHIP_CHECK(frhip_head(C, last, p[pi].data_ptr(), p[pi + 1].data_ptr(), hw, logits.data_ptr<float>(), s));
   return logits;
 }
+
+Tensor ModelForwardSeq(Model *model, Device device, const std::vector<int> &ids, bool full_output) {
+  return forward_seq(model, device, ids, full_output, true);
+}
+
+Tensor FullLogits(Model *model, const std::vector<int> &ids) { return forward_seq(model, Device::kHIP, ids, true, false); }
 
 KernelRegister model_forward_reg("model_forward", Device::kHIP, ModelForward);
 KernelRegister model_forward_seq_reg("model_forward_seq", Device::kHIP, ModelForwardSeq);

@@ -380,6 +380,29 @@ def test_the_logits_of_a_long_text_arrive_whole(rows, vocab):
     m.close()
 
 
+@pytest.mark.parametrize("rows,vocab,shift", [(4, 50000, 1), (13, 65536, 3), (61, 50277, 5), (203, 50277, 0), (203, 50277, 1)])
+def test_the_logits_of_a_long_text_are_the_same_at_any_address(rows, vocab, shift):
+    """Binary16 values widened exactly, from one copy (4 rows) and through the ring (203 rows: 20 MB, every slot of it used
+    again), into buffers that are only aligned to a float, with the words around them left alone.  The reference is the
+    operator-by-operator pass, whose logits the device widens; its layernorm and product are the same launches."""
+    m = fr.Model("synthetic:v=4,L=1,C=128,F=256,V=%d,seed=9" % vocab, "hip fp16")
+    ids = np.random.default_rng(rows).integers(0, vocab, rows).astype(np.int32)
+    os.environ["FR_HIP_GENERIC"] = "1"
+    try:
+        m.reset()
+        want = m.run_full(ids)
+    finally:
+        del os.environ["FR_HIP_GENERIC"]
+    m.reset()
+    buf = np.full(shift + rows * vocab + 8, 7.5, np.float32)
+    assert m._h.fr_model_run_full(m._m, ids.ctypes.data, rows, buf.ctypes.data + 4 * shift, rows * vocab) == rows * vocab
+    got = buf[shift:shift + rows * vocab]
+    assert np.array_equal(got.view(np.uint32), want.reshape(-1).view(np.uint32))
+    assert np.array_equal(got, got.astype(np.float16).astype(np.float32))
+    assert (buf[:shift] == 7.5).all() and (buf[shift + rows * vocab:] == 7.5).all()
+    m.close()
+
+
 def test_sampled_generation_follows_the_oracle_sampler(model_files):
     """chat.cpp's loop with a seeded Sampler: the C++ loop on the hip model picks the tokens that the
     sampler oracle picks from the same logits."""
