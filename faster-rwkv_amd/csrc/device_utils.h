@@ -119,7 +119,9 @@ __device__ __forceinline__ h2 dequant_pair(uint32_t word, float c, float mx, h2 
   const float q1 = (float)((word >> (HI ? 24 : 8)) & 0xffu);
   const float a0 = c * (float)ry.x, a1 = c * (float)ry.y;
   const float b0 = mx + (float)my.x, b1 = mx + (float)my.y;
-  return (h2){(h1)__builtin_fmaf(q0, a0, b0), (h1)__builtin_fmaf(q1, a1, b1)};
+  float w0 = __builtin_fmaf(q0, a0, b0), w1 = __builtin_fmaf(q1, a1, b1);
+  asm("" : "+v"(w0), "+v"(w1));  // rounded to fp32 before the conversion (not v_fma_mixlo_f16, which rounds once)
+  return (h2){(h1)w0, (h1)w1};
 }
 
 __device__ __forceinline__ float dot2acc(h2 a, h2 b, float acc) {

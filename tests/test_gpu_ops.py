@@ -131,6 +131,17 @@ def test_dequant_random_matrix_bit_exact(K, N):
     assert np.array_equal(out.numpy().T.view(np.uint16), po.dequant_u8(q, mx, rx, my, ry).view(np.uint16))
 
 
+@pytest.mark.parametrize("K,N", [(16, 1), (48, 7), (2064, 5), (16, 4099), (144, 6)])  # four rows per thread: N = 1, 2, 3 mod 4
+def test_dequant_rows_left_over_bit_exact_and_nothing_behind_them(K, N):
+    from synth import quantize_u8
+    q, mx, rx, my, ry = quantize_u8(h(rng.standard_normal((K, N)) * 0.02))
+    pw = PackedWeight(q=q, mx=mx, rx=rx, my=my, ry=ry)
+    out = DevBuf.from_numpy(np.full((N + 4, K), 0x7777, np.uint16))
+    fr.check(L().frhip_dequant_u8(pw.ref, out.ptr, None))
+    got = out.numpy()
+    assert np.array_equal(got[:N].T, po.dequant_u8(q, mx, rx, my, ry).view(np.uint16)) and (got[N:] == 0x7777).all()
+
+
 # K above 9216 (binary16) / 16384 (uint8): rows consumed in slices
 @pytest.mark.parametrize("K,N", [(2048, 2048), (2048, 8192), (8192, 2048), (2560, 2560), (8960, 2560), (768, 50277), (64, 3), (16, 1),
                                  (10240, 2560), (16384, 515), (20480, 130), (32768, 9), (9232, 33)])
