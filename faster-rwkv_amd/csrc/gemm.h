@@ -59,7 +59,9 @@ int launch_gemm(GemmArgs& a, bool u8, hipStream_t st, const char* what, void* dq
 // Products of a few rows in one launch, K split over the waves of a workgroup (gemm_few.hip).  plan_few: the tile that is
 // expected to be the quickest and its us; mt = 0: not a launch of this form.  It depends on the sizes alone, not on the
 // weight type, so that a uint8 weight and its binary16 image take the same sums.  few_takes: the addresses allow it.
-constexpr int kFewKernelRows = 512;
+// Up to kFewRowsMax rows: beyond, a product is at best as quick as on tiles of 64 rows (512 x 2560 x 2560: 20.5 us against
+// 20.9), and the prompts of 512 tokens that RWKV-5.2's parity is measured on keep the order of their sums.
+constexpr int kFewKernelRows = kFewRowsMax;
 struct FewPlan {
   int mt = 0, nt = 0;  // blocks of 16 rows and 16 columns of a workgroup
   double us = 0;
