@@ -109,6 +109,7 @@ _SIGS = {
     "frhip_mfma_probe": (_i, [_i, _i, _vp, _vp, _vp, _vp]),
     "frhip_seq_workspace_bytes": (_sz, [_i, _i, _i]),
     "frhip_ffn_seq": (_i, [_i, _i, _i] + [_vp] * 6 + [_WP] * 3 + [_vp, _vp, _i, _vp, _vp]),
+    "frhip_ffn_seq_v4": (_i, [_i, _i, _i] + [_vp] * 6 + [_WP] * 3 + [_vp, _vp, _i, _vp, _vp]),
     "frhip_att_seq_v4": (_i, [_i, _i] + [_vp] * 12 + [_WP] * 4 + [_vp] * 7),
     "frhip_att_seq_v5_2": (_i, [_i, _i, _i] + [_vp] * 13 + [_WP] * 5 + [_vp] * 5),
     "frhip_att_seq_v5": (_i, [_i, _i, _i] + [_vp] * 12 + [_WP] * 4 + [_vp] * 5),

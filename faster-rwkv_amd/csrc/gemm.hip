@@ -1257,8 +1257,9 @@ int launch_gemm(GemmArgs& a, bool u8, hipStream_t st, const char* what, void* dq
   // split over K in memory (64 x 20480 x 5120: 45 us against 64; 77 x 8192 x 2048: 17.3 both), many rows of wide products on
   // planned tiles (256 x 5120 x (5120 + 20480): 91 against 143).  Decided by the sizes alone: uint8 codes and their binary16
   // image, expanded here or kept by the caller, give the same bits.
-  const FewPlan fp = ldw && splitk && few && !force_bm ? few_plan(a, partial ? partial_stride : 0, partial ? max_split : 0, few_ok ? few_rows_floats : 0, compute_units())
-                                                       : FewPlan();
+  const FewPlan fp = ldw && splitk && few && !force_bm && !a.tiled_sums
+                         ? few_plan(a, partial ? partial_stride : 0, partial ? max_split : 0, few_ok ? few_rows_floats : 0, compute_units())
+                         : FewPlan();
   if (fp.mt && few_takes(a, u8)) return launch_gemm_few(a, fp, u8, st, what);
   bool direct = u8 && dq && a.M >= kDequantRows && a.M <= kU8DirectRows;
   for (int s = 0; s < a.nseg; s++)  // the uint8 kernel reads codes and row scales 16 bytes at a time; the expansion takes any address

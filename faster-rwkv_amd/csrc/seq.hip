@@ -709,10 +709,9 @@ SeqWs carve_seq(void* ws, int T, int C, int F) {
 }  // namespace
 
 // ffn_seq (kernels/cuda/ffn_seq.cu:65-109).  x [T][C]; sx [C] shift state; xx_out [C] = LN(x)[T-1].
-extern "C" int frhip_ffn_seq(int T, int C, int F, const void* x, const void* sx, const void* ln_w, const void* ln_b,
-                             const void* k_mix, const void* r_mix, const frhip_weight* kw, const frhip_weight* vw,
-                             const frhip_weight* rw, void* x_out, void* xx_out, int post_div2, void* workspace,
-                             frhip_stream s) {
+static int ffn_seq_impl(bool tiled_sums, int T, int C, int F, const void* x, const void* sx, const void* ln_w, const void* ln_b,
+                        const void* k_mix, const void* r_mix, const frhip_weight* kw, const frhip_weight* vw,
+                        const frhip_weight* rw, void* x_out, void* xx_out, int post_div2, void* workspace, frhip_stream s) {
   if (T <= 0) return set_error(FRHIP_ESHAPE, "ffn_seq: T must be positive");
   if (!x || !sx || !ln_w || !ln_b || !k_mix || !r_mix || !x_out || !xx_out || !workspace)
     return set_error(FRHIP_EINVAL, "ffn_seq: null pointer");
@@ -727,18 +726,32 @@ extern "C" int frhip_ffn_seq(int T, int C, int F, const void* x, const void* sx,
   FR_TRY(launch_ln_mix(T, C, x, sx, ln_w, ln_b, mixes, outs, 2, xx_out, st));
   GemmArgs a;
   memset(&a, 0, sizeof(a));
-  a.M = T; a.K = C;
+  a.M = T; a.K = C; a.tiled_sums = tiled_sums;
   gemm_add_seg(a, w.m1, rw, w.m2, G_SIGMOID);  // r
   gemm_add_seg(a, w.m0, kw, w.vx, G_RELU2);    // vx
   if (kw->dtype != rw->dtype) return set_error(FRHIP_EINVAL, "ffn_seq: key/receptance dtypes differ");
   FR_TRY(launch_gemm(a, kw->dtype == FRHIP_U8, st, "ffn_seq r,k", w.dq, nullptr, 0, 0, w.few, w.few_floats));
   GemmArgs b;
   memset(&b, 0, sizeof(b));
-  b.M = T; b.K = F;
+  b.M = T; b.K = F; b.tiled_sums = tiled_sums;
   b.res_x = (const h1*)x; b.res_r = w.m2; b.div2 = post_div2 ? 1 : 0;
   gemm_add_seg(b, w.vx, vw, x_out, G_FFN_OUT);
   // the four fp32 [T][C] buffers of the workspace (unused by ffn) take the partial sums of a K-split launch
   return launch_gemm(b, vw->dtype == FRHIP_U8, st, "ffn_seq v", w.dq, w.f0, (size_t)(w.f1 - w.f0), 4, w.few, w.few_floats);
+}
+
+extern "C" int frhip_ffn_seq(int T, int C, int F, const void* x, const void* sx, const void* ln_w, const void* ln_b,
+                             const void* k_mix, const void* r_mix, const frhip_weight* kw, const frhip_weight* vw,
+                             const frhip_weight* rw, void* x_out, void* xx_out, int post_div2, void* workspace,
+                             frhip_stream s) {
+  return ffn_seq_impl(true, T, C, F, x, sx, ln_w, ln_b, k_mix, r_mix, kw, vw, rw, x_out, xx_out, post_div2, workspace, s);
+}
+
+extern "C" int frhip_ffn_seq_v4(int T, int C, int F, const void* x, const void* sx, const void* ln_w, const void* ln_b,
+                                const void* k_mix, const void* r_mix, const frhip_weight* kw, const frhip_weight* vw,
+                                const frhip_weight* rw, void* x_out, void* xx_out, int post_div2, void* workspace,
+                                frhip_stream s) {
+  return ffn_seq_impl(false, T, C, F, x, sx, ln_w, ln_b, k_mix, r_mix, kw, vw, rw, x_out, xx_out, post_div2, workspace, s);
 }
 
 // RWKV-4 sequence attention.  The reference has no such operator
@@ -816,7 +829,7 @@ static int att_seq_v5_impl(bool v50, int T, int C, int H, const void* x, const v
   FR_TRY(launch_ln_mix(T, C, x, sx, ln_w, ln_b, mixes, outs, v50 ? 3 : 4, xx_out, st));
   GemmArgs a;
   memset(&a, 0, sizeof(a));
-  a.M = T; a.K = C;
+  a.M = T; a.K = C; a.tiled_sums = true;
   gemm_add_seg(a, w.m0, kw, w.f0, G_STORE_F32);  // k
   gemm_add_seg(a, w.m1, vw, w.f1, G_STORE_F32);  // v
   gemm_add_seg(a, w.m2, rw, w.f2, G_STORE_F32);  // r
@@ -841,7 +854,7 @@ static int att_seq_v5_impl(bool v50, int T, int C, int H, const void* x, const v
 
   GemmArgs b;
   memset(&b, 0, sizeof(b));
-  b.M = T; b.K = C;
+  b.M = T; b.K = C; b.tiled_sums = true;
   b.res_x = (const h1*)x;
   gemm_add_seg(b, w.gated, ow, x_out, G_RESIDUAL);
   return launch_gemm(b, ow->dtype == FRHIP_U8, st, "att_seq_v5 out", w.dq, nullptr, 0, 0, w.few, w.few_floats);

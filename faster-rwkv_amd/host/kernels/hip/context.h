@@ -43,10 +43,10 @@ const frhip_weight *find_weight(const Tensor &t);
 const frhip_weight *find_seq_weight(const Tensor &t, int rows);
 
 // ffn_seq with the halving that follows every sixth layer folded into its last epilogue (ops.cpp); same bits as
-// ffn_seq followed by scalar_div_(x, 2).
+// ffn_seq followed by scalar_div_(x, 2).  `v4`: an RWKV-4 model's (frhip_ffn_seq_v4).
 std::tuple<Tensor, Tensor> ffn_seq_div2(const Tensor &x, const Tensor &sx, const Tensor &ln_w, const Tensor &ln_b,
                                         const Tensor &k_mix, const Tensor &r_mix, const Tensor &kw, const Tensor &vw,
-                                        const Tensor &rw, bool div2);
+                                        const Tensor &rw, bool div2, bool v4);
 
 // Upload a host matrix in the reference's [K, N] layout and pack it for the kernels.
 // `dtype` kFloat16: src is binary16.  kInt8: src is binary16 and is quantised on the host
