@@ -104,6 +104,8 @@ _SIGS = {
     "frhip_gemm": (_i, [_vp, _WP, _vp, _i, _i, _vp]),
     "frhip_gemm_act": (_i, [_vp, _WP, _vp, _i, _i, _vp]),
     "frhip_gemm_route": (_i, [_i, _i, _i, _vp, _i, _vp]),
+    "frhip_gemm_few_tile": (_i, [_i, _i, _i, _vp, _i, _vp]),
+    "frhip_seq_gemm_form": (_i, [_i, _i, _i, _vp, _i, _i, _vp]),
     "frhip_copy_probe": (_i, [_vp, _vp, _sz, _vp]),
     "frhip_read_probe": (_i, [_vp, _sz, _vp, _vp]),
     "frhip_mfma_probe": (_i, [_i, _i, _vp, _vp, _vp, _vp]),

@@ -59,6 +59,7 @@ struct GemmArgs {
 // at least half of the compute units idle is split over K across the idle units, whole or product by product.
 constexpr size_t kFewRowsFloats = (size_t)512 * 64 * 128;  // two 64 x 128 tiles per compute unit of a 256-unit part
 constexpr int kFewRowsMax = 360;                          // rows up to which the seq operators carry that scratch
+constexpr int kSeqMaxSplit = 4;                           // slices of the [T][C] buffers that ffn value is given as `partial`
 int launch_gemm(GemmArgs& a, bool u8, hipStream_t st, const char* what, void* dq = nullptr, float* partial = nullptr,
                 size_t partial_stride = 0, int max_split = 0, float* few_rows = nullptr, size_t few_rows_floats = 0);
 // Products of a few rows in one launch, K split over the waves of a workgroup (gemm_few.hip).  plan_few: the tile that is

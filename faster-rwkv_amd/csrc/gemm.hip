@@ -1143,17 +1143,19 @@ static int few_rows_slices(const GemmArgs& a, size_t few_rows_floats, int cus) {
   return S < 2 ? 0 : (int)S;
 }
 
-// ... or, a group that does not fill the part, product by product, so that its narrow members are
+// ... or, a group that does not fill the part, product by product, so that its narrow members are.  A group that fits as a
+// whole and still gets no two slices has a K of four to seven steps: nor would its members get any, it stays one launch.
 static bool few_rows_one_by_one(const GemmArgs& a, int cus) {
   const int m64 = (a.M + 63) / 64;
   long tiles = 0;
-  bool any = false;
+  bool any = false, all = true;
   for (int s = 0; s < a.nseg; s++) {
     const long t = (a.seg[s].N + BN - 1) / BN;
     tiles += t;
     any = any || (t * m64 * 2 <= cus && a.seg[s].N % 16 == 0);
+    all = all && a.seg[s].N % 16 == 0;
   }
-  return a.nseg > 1 && tiles * m64 < cus && any;
+  return a.nseg > 1 && tiles * m64 < cus && any && !(all && tiles * m64 * 2 <= cus);
 }
 
 static int launch_few_rows(GemmArgs& a, bool u8, hipStream_t st, const char* what, void* dq, float* few_rows,
@@ -1447,6 +1449,39 @@ extern "C" int frhip_gemm_few_tile(int T, int K, int nproducts, const int* N, in
   out[0] = p.mt;
   out[1] = p.nt;
   return 0;
+}
+
+extern "C" int frhip_seq_gemm_form(int T, int K, int nproducts, const int* N, int which, int compute_units, int* out) {
+  if (!N || !out) return set_error(FRHIP_EINVAL, "seq_gemm_form: null pointer");
+  if (T <= 0 || K <= 0 || K % 64 != 0 || nproducts < 1 || nproducts > kGemmMaxSeg || compute_units < 1)
+    return set_error(FRHIP_ESHAPE, "seq_gemm_form: no such launch");
+  GemmArgs a;
+  memset(&a, 0, sizeof(a));
+  a.M = T;
+  a.K = K;
+  a.nseg = nproducts;
+  for (int s = 0; s < nproducts; s++) {
+    if (N[s] <= 0) return set_error(FRHIP_ESHAPE, "seq_gemm_form: no such launch");
+    a.seg[s].N = N[s];
+  }
+  const bool value = (which & FRHIP_SEQ_FFN_VALUE) != 0;
+  if (value) a.seg[0].epi = G_FFN_OUT;
+  const size_t stride = value ? (size_t)T * N[0] : 0, floats = T <= kFewRowsMax ? kFewRowsFloats : 0;
+  const int max_split = value ? kSeqMaxSplit : 0;
+  out[0] = out[1] = 0;
+  if (which & FRHIP_SEQ_V4) {
+    const FewPlan p = few_plan(a, stride, max_split, floats, compute_units);
+    out[0] = p.mt;
+    out[1] = p.nt;
+    if (p.mt) return FRHIP_FORM_FEW;
+  }
+  if (floats && K / kLdwBK >= 4) {
+    out[0] = few_rows_slices(a, floats, compute_units);
+    if (out[0]) return FRHIP_FORM_SPLIT;
+    if (few_rows_one_by_one(a, compute_units)) return FRHIP_FORM_ONE_BY_ONE;
+  }
+  out[0] = long_k_slices(a, stride, max_split, compute_units);
+  return out[0] ? FRHIP_FORM_SPLIT : FRHIP_FORM_TILES;
 }
 
 static_assert(FRHIP_ACT_SIGMOID == G_SIGMOID && FRHIP_ACT_RELU2 == G_RELU2 && FRHIP_ACT_SILU == G_SILU, "activation codes");

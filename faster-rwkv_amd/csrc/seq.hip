@@ -737,7 +737,8 @@ static int ffn_seq_impl(bool tiled_sums, int T, int C, int F, const void* x, con
   b.res_x = (const h1*)x; b.res_r = w.m2; b.div2 = post_div2 ? 1 : 0;
   gemm_add_seg(b, w.vx, vw, x_out, G_FFN_OUT);
   // the four fp32 [T][C] buffers of the workspace (unused by ffn) take the partial sums of a K-split launch
-  return launch_gemm(b, vw->dtype == FRHIP_U8, st, "ffn_seq v", w.dq, w.f0, (size_t)(w.f1 - w.f0), 4, w.few, w.few_floats);
+  return launch_gemm(b, vw->dtype == FRHIP_U8, st, "ffn_seq v", w.dq, w.f0, (size_t)(w.f1 - w.f0), kSeqMaxSplit, w.few,
+                     w.few_floats);
 }
 
 extern "C" int frhip_ffn_seq(int T, int C, int F, const void* x, const void* sx, const void* ln_w, const void* ln_b,

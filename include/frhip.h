@@ -307,10 +307,22 @@ int frhip_att_seq_v5(int T, int C, int H, const void *x, const void *sx, const f
  * out[4 i + 1]: its widest tile in blocks of 32 columns, out[4 i + 2]: its rounds over the compute units,
  * out[4 i + 3]: 1 if a wave of its own loads the tiles. */
 int frhip_gemm_route(int T, int K, int nproducts, const int *N, int compute_units, int *out);
-/* Whether such a launch goes, instead, to the kernel for a few rows (K split over the waves of a workgroup), and with which
- * tile: out[0], out[1] = blocks of 16 rows and of 16 columns of a workgroup, 0, 0 if it is cut as above.  A pure function
- * of the sizes too. */
+/* Whether such a launch (frhip_gemm's and frhip_gemm_act's are of this kind; the seq operators have scratch, see below) goes,
+ * instead, to the kernel for a few rows (K split over the waves of a workgroup), and with which tile: out[0], out[1] = blocks
+ * of 16 rows and of 16 columns of a workgroup, 0, 0 if it is cut as above.  A pure function of the sizes too. */
 int frhip_gemm_few_tile(int T, int K, int nproducts, const int *N, int compute_units, int *out);
+/* The form that a launch of the seq operators (uint8: of 4 rows and more) takes, with their scratch, for addresses that suit
+ * every form (allocations do).  `which`: 0, or FRHIP_SEQ_V4 for frhip_att_seq_v4's and frhip_ffn_seq_v4's, plus
+ * FRHIP_SEQ_FFN_VALUE for the value product of ffn_seq.  Returns the form or a negative FRHIP_E*.  out[0], out[1]:
+ * FRHIP_FORM_FEW: the tile as above; FRHIP_FORM_SPLIT (over K, with a reduction launch): slices, 0; FRHIP_FORM_TILES (as
+ * frhip_gemm_route says) and FRHIP_FORM_ONE_BY_ONE (a launch per product, each with a form of its own): 0, 0. */
+#define FRHIP_SEQ_V4 1
+#define FRHIP_SEQ_FFN_VALUE 2
+#define FRHIP_FORM_TILES 0
+#define FRHIP_FORM_FEW 1
+#define FRHIP_FORM_SPLIT 2
+#define FRHIP_FORM_ONE_BY_ONE 3
+int frhip_seq_gemm_form(int T, int K, int nproducts, const int *N, int which, int compute_units, int *out);
 
 /* ---- bandwidth probes: DIAGNOSTICS, not operators (measurement aids of bench.py and of the
  *      hardware-counter calibration; no counterpart in the reference, nothing on the model path calls them) */
