@@ -638,11 +638,12 @@ static void launch_wkv4_scan(Wkv4Seq& q, hipStream_t st) {
 // chunk length for a scan of T steps when one chunk occupies `units` workgroup-sized units:
 // enough chunks to fill the device (~4 units per CU), chunks of at least 16 steps (the serial pass
 // over the chunks costs about 0.18 us per chunk: at T = 1024, 64 chunks of 16 beat 128 of 8)
+constexpr int kMinChunk = 16;
 static int pick_chunk(int T, int units) {
   int want = (4 * compute_units() + units - 1) / units;
   if (want < 1) want = 1;
   int Lc = (T + want - 1) / want;
-  if (Lc < 16) Lc = 16;
+  if (Lc < kMinChunk) Lc = kMinChunk;
   if (Lc > 64) Lc = 64;
   return Lc;
 }
@@ -657,6 +658,9 @@ static size_t seq_dequant_bytes(int C, int F) {
   return 2 * (att > ffn ? att : ffn);
 }
 
+// RWKV-5: the chunks' end states and start states, [nchunk][C * 64] fp32 each, chunks of at least kMinChunk steps (pick_chunk)
+static size_t scan_bytes(int T, int C) { return al256(4 * (((size_t)T + kMinChunk - 1) / kMinChunk) * C * 64); }
+
 extern "C" size_t frhip_seq_workspace_bytes(int T, int C, int F) {
   if (T <= 0 || C <= 0 || F <= 0) return 0;
   const size_t tc = (size_t)T * C;
@@ -664,9 +668,7 @@ extern "C" size_t frhip_seq_workspace_bytes(int T, int C, int F) {
   size_t n = 6 * al256(2 * tc) + 4 * al256(4 * tc) + al256(2 * (size_t)T * F);
   // short prompts: partial sums of the products split over K (launch_gemm's few_rows scratch)
   if (T <= kFewRowsMax) n += al256(4 * kFewRowsFloats);
-  // scan scratch: RWKV-4 6 x [nchunk][C] fp32 with nchunk <= T/8+1; RWKV-5 2 x [nchunk][C*64] fp32
-  const size_t nchunk = (size_t)T / 8 + 1;
-  n += 6 * al256(4 * nchunk * C) + 2 * al256(4 * nchunk * (size_t)C * 64);
+  n += 2 * scan_bytes(T, C);
   // binary16 expansion of the uint8 weights of one launch: the largest group is k,v,r,g or ffn r,k
   n += al256(seq_dequant_bytes(C, F));
   return n;
@@ -701,8 +703,7 @@ SeqWs carve_seq(void* ws, int T, int C, int F) {
   w.vx = reinterpret_cast<h1*>(p);
   p += al256(2 * (size_t)T * F);
   w.scan = reinterpret_cast<float*>(p);
-  const size_t nchunk = (size_t)T / 8 + 1;
-  p += 6 * al256(4 * nchunk * C) + 2 * al256(4 * nchunk * (size_t)C * 64);
+  p += 2 * scan_bytes(T, C);
   w.dq = reinterpret_cast<h1*>(p);
   return w;
 }

@@ -30,6 +30,16 @@ def test_workspace_query_and_argument_checks_do_not_need_a_gpu():
     assert b"null" in lib.frhip_error_string()
 
 
+def test_seq_workspace_holds_what_the_operators_use():
+    """Activations (binary16: four mixed inputs, gate, gated; fp32: k, v, r, y; the ffn key), partial sums of up to 360 rows,
+    RWKV-5's chunk states (two of [64][C] per 16 steps), one launch's expanded uint8 weights; each rounded up to 256 bytes."""
+    for T, C_, F_ in ((1, 64, 64), (16, 2048, 8192), (360, 512, 1792), (361, 512, 1792), (4099, 2048, 8192), (1000, 5120, 20480)):
+        need = 6 * 2 * T * C_ + 4 * 4 * T * C_ + 2 * T * F_ + (4 * 512 * 64 * 128 if T <= 360 else 0)
+        need += 2 * 4 * -(-T // 16) * C_ * 64 + 2 * max(4 * C_ * C_, C_ * C_ + C_ * F_)
+        assert need <= fr.lib().frhip_seq_workspace_bytes(T, C_, F_) <= need + 15 * 256
+    assert fr.lib().frhip_seq_workspace_bytes(0, 64, 64) == 0
+
+
 def test_fill_many_and_copy_many_look_at_buffers_of_some_bytes_only():
     """An empty buffer is skipped whatever its address (nothing is launched); an element that would straddle its
     alignment is refused."""
