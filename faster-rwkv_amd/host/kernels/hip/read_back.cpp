@@ -8,7 +8,9 @@
 // 0.48 ms instead of 0.96 as fp32; a chunk is 2 MB because each costs the thread that issues copies about 35 us (the copy,
 // its event, the wait), as long as 2 MB take on the bus.  The whole call, 12 layers of 768 included: 2.6 -> 1.75 ms, against
 // chunks of 1 MB of fp32.
+#if defined(__x86_64__)
 #include <immintrin.h>
+#endif
 
 #include <algorithm>
 #include <condition_variable>
@@ -29,6 +31,7 @@ void widen_plain(const float16 *src, float *dst, size_t n) {
   for (size_t i = 0; i < n; i++) dst[i] = static_cast<float>(src[i]);
 }
 
+#if defined(__x86_64__)
 // The destination is not read again soon: stores past the caches, no line of it is read in first.
 __attribute__((target("avx,f16c"))) void widen_f16c(const float16 *src, float *dst, size_t n) {
   size_t i = 0;
@@ -46,6 +49,9 @@ void widen(const float16 *src, float *dst, size_t n) {
   static const bool fast = __builtin_cpu_supports("avx") && __builtin_cpu_supports("f16c");
   fast ? widen_f16c(src, dst, n) : widen_plain(src, dst, n);
 }
+#else
+void widen(const float16 *src, float *dst, size_t n) { widen_plain(src, dst, n); }
+#endif
 
 }  // namespace
 

@@ -18,3 +18,25 @@ def test_bare_barriers_stand_between_compiler_fences():
                 found += 1
                 assert (lines[i - 1], lines[i + 1]) == (fence, fence), "%s:%d" % (os.path.basename(path), i + 1)
     assert found
+
+
+def test_x86_instructions_of_the_host_layer_are_guarded():
+    """A host of another architecture compiles the plain forms: intrinsics, their header, target attributes and CPU queries
+    stand under `#if defined(__x86_64__)`."""
+    found = 0
+    for path in sorted(glob.glob(os.path.join(os.path.dirname(CSRC), "host", "**", "*.[ch]*"), recursive=True)):
+        if not path.endswith((".cpp", ".h")):
+            continue
+        under = []
+        for i, line in enumerate(open(path)):
+            word = line.split() or [""]
+            if word[0] in ("#if", "#ifdef", "#ifndef"):
+                under.append(line.strip() == "#if defined(__x86_64__)")
+            elif word[0] in ("#else", "#elif"):
+                under[-1] = False
+            elif word[0] == "#endif":
+                under.pop()
+            elif re.search(r"intrin\.h|\b_mm\d*_|__builtin_cpu_supports|\btarget\(", line):
+                found += 1
+                assert any(under), "%s:%d" % (os.path.basename(path), i + 1)
+    assert found
