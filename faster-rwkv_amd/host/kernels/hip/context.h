@@ -28,10 +28,14 @@ struct PackedWeight {
   Tensor image;
   frhip_weight image_desc{};
   bool no_image = false;  // the image could not be allocated once: not tried again
+  bool v4 = false;        // an RWKV-4 model's: its ffn_seq is frhip_ffn_seq_v4, whichever way the model runs
 };
 
 void register_weight(const void *data_ptr, std::shared_ptr<PackedWeight> w);
 void unregister_weight(const void *data_ptr);
+// Marks a registered weight as an RWKV-4 model's / whether a tensor is one.
+void mark_v4(const void *data_ptr);
+bool is_v4(const Tensor &t);
 // nullptr when `t` is not a packed weight.
 const frhip_weight *find_weight(const Tensor &t);
 // The description to hand to a product over `rows` rows of activations.  The same as
@@ -43,10 +47,10 @@ const frhip_weight *find_weight(const Tensor &t);
 const frhip_weight *find_seq_weight(const Tensor &t, int rows);
 
 // ffn_seq with the halving that follows every sixth layer folded into its last epilogue (ops.cpp); same bits as
-// ffn_seq followed by scalar_div_(x, 2).  `v4`: an RWKV-4 model's (frhip_ffn_seq_v4).
+// ffn_seq followed by scalar_div_(x, 2).
 std::tuple<Tensor, Tensor> ffn_seq_div2(const Tensor &x, const Tensor &sx, const Tensor &ln_w, const Tensor &ln_b,
                                         const Tensor &k_mix, const Tensor &r_mix, const Tensor &kw, const Tensor &vw,
-                                        const Tensor &rw, bool div2, bool v4);
+                                        const Tensor &rw, bool div2);
 
 // Upload a host matrix in the reference's [K, N] layout and pack it for the kernels.
 // `dtype` kFloat16: src is binary16.  kInt8: src is binary16 and is quantised on the host

@@ -341,6 +341,8 @@ void init_model(Model *model, Device device, const std::string &path, const std:
     build_synthetic(model, parse_spec(path.substr(tag.size())), wdtype, *ex);
   else
     build_from_fr(model, path, wdtype, *ex);
+  if (model->_version == "4")
+    for (const void *p : ex->packed) mark_v4(p);
   model->_act_dtype = DType::kFloat16;  // model.cpp:46-49 names fp32 for "int8"; this backend computes in fp16
   model->_weight_dtype = wdtype;
   // embedding rows: views into the slab (the reference allocates one tensor per row,

@@ -44,6 +44,18 @@ void unregister_weight(const void *p) {
   table().erase(p);
 }
 
+void mark_v4(const void *p) {
+  std::lock_guard<std::mutex> lock(g_mu);
+  auto it = table().find(p);
+  if (it != table().end()) it->second->v4 = true;
+}
+
+bool is_v4(const Tensor &t) {
+  std::lock_guard<std::mutex> lock(g_mu);
+  auto it = table().find(t.data_ptr());
+  return it != table().end() && it->second->v4;
+}
+
 const frhip_weight *find_weight(const Tensor &t) {
   if (!t.defined() || t.device() != Device::kHIP) return nullptr;
   std::lock_guard<std::mutex> lock(g_mu);

@@ -90,11 +90,11 @@ def test_att_seq_v5_adds_in_slices(T, gate):
     assert np.array_equal(x_out.numpy(), _h(want))
 
 
-@pytest.mark.parametrize("version,H", [("5.2", 8), ("5", 8)])
+@pytest.mark.parametrize("version,H", [("5.2", 8), ("5", 8), ("4", 0)])
 def test_model_pass_takes_the_operators_of_its_version(tmp_path, version, H, monkeypatch):
     """A short prompt through the fused pass and through the operators one by one leaves the same bits behind."""
     from synth import make_model
-    params, emb = make_model({"5": 50}.get(version, 52), 3, 512, 1792, 2048, H, seed=9)
+    params, emb = make_model({"4": 4, "5": 50}.get(version, 52), 3, 512, 1792, 2048, H, seed=9)
     path = str(tmp_path / "m.fr")
     fr.write_fr(path, version, 3, 512, 1792, H, params, emb)
     ids = [int(t) for t in np.random.default_rng(1).integers(0, 2048, 16)]
