@@ -14,6 +14,7 @@
 // only the representation of the carried state differs from a serial scan, at fp32 rounding level.
 #include <climits>
 #include <cstring>
+#include <type_traits>
 
 #include "gemm.h"
 
@@ -287,12 +288,17 @@ __global__ __launch_bounds__(256) void ln_mix_wide_kernel(LnMixSeq a) {
 // A workgroup owns CG channels and cuts time into blocks of nchunk chunks of Lc steps, a thread per (channel, chunk).
 // Per block: every chunk is scanned from an empty state (k and v stay in registers); the local end states are
 // composed into the states at the ends of the chunks by a doubling scan in LDS; every chunk is scanned again from its true
-// start state, writing the outputs; the last chunk's end state starts the next block.
+// start state, writing the outputs; the last chunk's end state starts the next block, whose k, v and r were requested step
+// by step as the registers of this one became free.
 // What bounds it: about 150 vector instructions per channel and step, most of them three expf (a six-instruction
 // exponential within 2 ulp would save a tenth, but the outputs would no longer be those of the one-token kernel).  att_seq_v4
 // as a whole (products included) against a launch for pass 1, one for passes 2 and 3, which read k and v twice and
 // composed every chunk's start from all chunks before it, us: 2048 channels, T = 13: 22.2 -> 18.1, 77: 29.4 -> 25.1,
-// 1024: 81.4 -> 73.3, 4099 (a serial pass 2 of its own): 233.5 -> 221.2; 5120 channels, T = 1024: 258 both.
+// 1024: 81.4 -> 73.3, 4099 (a serial pass 2 of its own): 240.9 -> 223.4; 5120 channels, T = 1024: 277 -> 273, 4099: 1010 -> 1019.
+// Requests ahead: the scan alone, 5120 channels, T = 4099: 117 -> 109.  Registers for every second chunk length from 8 on, not
+// for 16 only: 2048 channels, T = 4099 (11 steps): 230.5 -> 223.4.  What it still loses to: pieces of 8 to 14 channels are a
+// part of a line, fetched once for each, so 2112 to 3072 channels and more than 4096 steps were 2 to 6 % quicker in the three
+// launches (8192 x 2304: 522 against 555), whose states were two to six times further from float64.
 // (A form with scalar bases for whole blocks and masked steps for the last one spilled registers: 1024: 75.)
 // ---------------------------------------------------------------------------
 constexpr int kWkv4MaxCg = 32;
@@ -331,7 +337,8 @@ __global__ __launch_bounds__(1024) void wkv4_scan_kernel(Wkv4Seq a) {
   const int CG = a.cg;
   // neighbouring channels on one XCD: CG channels are 4 CG bytes of a row, a part of a line
   const int n = gridDim.x, xcd = blockIdx.x & 7, grp = xcd * (n >> 3) + min(xcd, n & 7) + (blockIdx.x >> 3);
-  const int tid = threadIdx.x, cl = tid % CG, ch = tid / CG, c = grp * CG + cl;
+  const int tid = threadIdx.x, cl = tid % CG, ch = tid / CG, c = min(grp * CG + cl, a.C - 1);
+  const bool live = grp * CG + cl < a.C;  // the last workgroup's channels past the end follow the last one and store nothing
   const float w = a.w[c], u = a.u[c];
   if (ch == 0) {
     start[0][cl] = a.aa[c];
@@ -339,17 +346,18 @@ __global__ __launch_bounds__(1024) void wkv4_scan_kernel(Wkv4Seq a) {
     start[2][cl] = a.pp[c];
   }
   const float dw = (float)a.Lc * w;
-  for (int blk = 0; blk < a.nblock; blk++) {
-    const int t0 = (blk * a.nchunk + ch) * a.Lc, len = min(a.Lc, a.T - t0);  // len <= 0: nothing left for this chunk
-    float kk[LMAX], vv[LMAX];
-    h1 rr[LMAX];
+  float kk[LMAX], vv[LMAX];
+  h1 rr[LMAX];
+  auto load = [&](int blk, int i) {
+    const size_t j = (size_t)min((blk * a.nchunk + ch) * a.Lc + min(i, a.Lc - 1), a.T - 1) * a.C + c;
+    kk[i] = a.k[j];
+    vv[i] = a.v[j];
+    rr[i] = a.r[j];
+  };
 #pragma unroll
-    for (int i = 0; i < LMAX; i++) {
-      const size_t j = (size_t)min(t0 + min(i, a.Lc - 1), a.T - 1) * a.C + c;
-      kk[i] = a.k[j];
-      vv[i] = a.v[j];
-      rr[i] = a.r[j];
-    }
+  for (int i = 0; i < LMAX; i++) load(0, i);
+  for (int blk = 0; blk < a.nblock; blk++) {
+    const int t0 = (blk * a.nchunk + ch) * a.Lc, len = live ? min(a.Lc, a.T - t0) : 0;  // len <= 0: nothing left for this chunk
     // from an empty state, without the chain of running maxima: aa = sum exp(k_i + (len - 1 - i) w - pp) v_i, bb = the same without v
     float aa = 0.f, bb = 0.f, pp = -1e30f, q[LMAX], off = 0.f;
 #pragma unroll
@@ -385,18 +393,23 @@ __global__ __launch_bounds__(1024) void wkv4_scan_kernel(Wkv4Seq a) {
     aa = start[0][cl], bb = start[1][cl], pp = start[2][cl];
     if (ch > 0)
       wkv4_compose(aa, bb, pp, (float)ch * dw, ends[cur][0][tid - CG], ends[cur][1][tid - CG], ends[cur][2][tid - CG]);
+    // the registers of a step take the next block's step once they have been used
+    auto apply = [&](auto more) {
 #pragma unroll
-    for (int i = 0; i < LMAX; i++) {
-      if (i < len) {
-        const float k = kk[i], v = vv[i];
-        // kernels/cuda/att.cu:43-60
-        float p, e1, e2;
-        exp_pair(pp, u + k, p, e1, e2);
-        const float wkv = (e1 * aa + e2 * v) / (e1 * bb + e2);
-        a.r[(size_t)(t0 + i) * a.C + c] = rr[i] * (h1)wkv;
-        wkv4_compose(aa, bb, pp, w, v, 1.0f, k);
+      for (int i = 0; i < LMAX; i++) {
+        if (i < len) {
+          const float k = kk[i], v = vv[i];
+          // kernels/cuda/att.cu:43-60
+          float p, e1, e2;
+          exp_pair(pp, u + k, p, e1, e2);
+          const float wkv = (e1 * aa + e2 * v) / (e1 * bb + e2);
+          a.r[(size_t)(t0 + i) * a.C + c] = rr[i] * (h1)wkv;
+          wkv4_compose(aa, bb, pp, w, v, 1.0f, k);
+        }
+        if constexpr (decltype(more)::value) load(blk + 1, i);
       }
-    }
+    };
+    if (blk + 1 < a.nblock) apply(std::true_type{}); else apply(std::false_type{});
     if (len > 0 && t0 + len == a.T) {
       a.aa_out[c] = aa;
       a.bb_out[c] = bb;
@@ -610,27 +623,39 @@ static int launch_ln_mix(int T, int C, const void* x, const void* state, const v
   return check_launch("ln_mix_seq");
 }
 
-// A workgroup's channels: about one workgroup per compute unit, at least 8 (32-byte pieces of a row), a divisor of C (a multiple
-// of 64, so 32 is one).  Chunks of at least 4 steps (2 where that still is one wave's work), of at most 16, which a thread
-// keeps in registers; up to 128 of them where 8 channels leave room, 64 otherwise (longer blocks have more doubling steps
-// than they save).  Of att_seq_v4, us: C = 5120, T = 2048: 484 with 20 channels, 501 with 16 (1.25 rounds), 492 with 8.
-static void launch_wkv4_scan(Wkv4Seq& q, hipStream_t st) {
+// A workgroup's channels: one workgroup per compute unit (or as few rounds of them as 32 channels allow), at least 8 (32-byte
+// pieces of a row); the last workgroup may have fewer (4736 channels: 250 workgroups of 19; as 148 of 32, which divides, T = 4099
+// took 945 us of att_seq_v4 against 927).  Chunks of at least 4 steps (2 where that still is one wave's work), of at most 16, which
+// a thread keeps in registers.  Up to 128 of them where 8 channels leave room; otherwise 64, of a prompt that they hold in one
+// block, and as many as there are threads of a longer one (2112 channels, 113 chunks against 64: T = 1100 107 against 115,
+// 2048 132.5 against 134; but T = 1024, ten steps a chunk against sixteen: 83 against 80.5).
+// C = 5120, T = 2048: 484 with 20 channels, 501 with 16 (1.25 rounds), 492 with 8.
+static void cut_wkv4_scan(Wkv4Seq& q, int cus) {
   constexpr int kMaxLc = 16;
-  q.cg = (q.C + compute_units() - 1) / compute_units();
+  const int rounds = (q.C + cus * kWkv4MaxCg - 1) / (cus * kWkv4MaxCg);
+  q.cg = (q.C + cus * rounds - 1) / (cus * rounds);
   if (q.cg < 8) q.cg = 8;
-  while (q.cg < kWkv4MaxCg && q.C % q.cg != 0) q.cg++;
-  if (q.cg > kWkv4MaxCg) q.cg = kWkv4MaxCg;
-  const int most = 1024 / q.cg, chunks = q.cg == 8 ? 128 : most < 64 ? most : 64;
+  const int most = 1024 / q.cg, chunks = q.cg == 8 ? 128 : most < 64 || q.T > 64 * kMaxLc ? most : 64;
   q.nblock = (q.T + chunks * kMaxLc - 1) / (chunks * kMaxLc);
   q.Lc = (q.T + chunks * q.nblock - 1) / (chunks * q.nblock);
   const int least = q.T <= 32 ? 2 : 4;
   if (q.Lc < least) q.Lc = least;
   q.nchunk = (q.T + q.Lc * q.nblock - 1) / (q.Lc * q.nblock);
-  const dim3 grid(q.C / q.cg), block(q.nchunk * q.cg);
+}
+
+static void launch_wkv4_scan(Wkv4Seq& q, hipStream_t st) {
+  cut_wkv4_scan(q, compute_units());
+  const dim3 grid((q.C + q.cg - 1) / q.cg), block(q.nchunk * q.cg);
   if (q.Lc <= 4)
     hipLaunchKernelGGL(wkv4_scan_kernel<4>, grid, block, 0, st, q);
   else if (q.Lc <= 8)
     hipLaunchKernelGGL(wkv4_scan_kernel<8>, grid, block, 0, st, q);
+  else if (q.Lc <= 10)
+    hipLaunchKernelGGL(wkv4_scan_kernel<10>, grid, block, 0, st, q);
+  else if (q.Lc <= 12)
+    hipLaunchKernelGGL(wkv4_scan_kernel<12>, grid, block, 0, st, q);
+  else if (q.Lc <= 14)
+    hipLaunchKernelGGL(wkv4_scan_kernel<14>, grid, block, 0, st, q);
   else
     hipLaunchKernelGGL(wkv4_scan_kernel<16>, grid, block, 0, st, q);
 }
@@ -802,6 +827,16 @@ extern "C" int frhip_att_seq_v4(int T, int C, const void* x, const void* sx, con
   b.res_x = (const h1*)x;
   gemm_add_seg(b, w.m3, ow, x_out, G_RESIDUAL);
   return launch_gemm(b, ow->dtype == FRHIP_U8, st, "att_seq_v4 out", w.dq, nullptr, 0, 0, w.few, w.few_floats);
+}
+
+extern "C" int frhip_wkv4_cut(int T, int C, int compute_units, int* out) {
+  if (!out) return set_error(FRHIP_EINVAL, "wkv4_cut: null pointer");
+  if (T <= 0 || C <= 0 || C % 64 != 0 || compute_units < 1) return set_error(FRHIP_ESHAPE, "wkv4_cut: no such scan");
+  Wkv4Seq q = {};
+  q.T = T; q.C = C;
+  cut_wkv4_scan(q, compute_units);
+  out[0] = q.cg; out[1] = (C + q.cg - 1) / q.cg; out[2] = q.nblock; out[3] = q.nchunk; out[4] = q.Lc;
+  return 0;
 }
 
 // Shared by RWKV-5.0 (no gate, u and w per head) and RWKV-5.2.

@@ -324,6 +324,10 @@ int frhip_gemm_few_tile(int T, int K, int nproducts, const int *N, int compute_u
 #define FRHIP_FORM_ONE_BY_ONE 3
 int frhip_seq_gemm_form(int T, int K, int nproducts, const int *N, int which, int compute_units, int *out);
 
+/* How frhip_att_seq_v4's scan of T steps of C channels is cut on a part with that many compute units.  out[0]: channels of a
+ * workgroup, out[1]: workgroups, out[2]: blocks of time one after another, out[3]: chunks of a block, out[4]: steps of a chunk. */
+int frhip_wkv4_cut(int T, int C, int compute_units, int *out);
+
 /* ---- bandwidth probes: DIAGNOSTICS, not operators (measurement aids of bench.py and of the
  *      hardware-counter calibration; no counterpart in the reference, nothing on the model path calls them) */
 /* Plain device copy, 16 bytes per lane: the kernel of known traffic (bytes read + bytes

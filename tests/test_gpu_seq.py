@@ -356,7 +356,7 @@ def _state_v4(C_, fresh):
             rng.standard_normal(C_).astype(np.float32))
 
 
-@pytest.mark.parametrize("T,C_", [(64, 512), (1024, 2048), (1, 512), (37, 768), (3000, 512), (24, 2048), (150, 2048)])  # 3000: a long, ragged prompt (94 chunks); 24, 150: short prompts at full width (split products)
+@pytest.mark.parametrize("T,C_", [(64, 512), (1024, 2048), (1, 512), (37, 768), (3000, 512), (24, 2048), (150, 2048)])  # 3000: a long, ragged prompt (two blocks); 24, 150: short prompts at full width
 @pytest.mark.parametrize("quant", [False, True])
 @pytest.mark.parametrize("fresh", [True, False])
 def test_att_seq_v4(T, C_, quant, fresh):
@@ -393,8 +393,54 @@ def test_att_seq_v4(T, C_, quant, fresh):
                                   (2049, 128), (4097, 64),                  # two and three blocks, the last one ragged
                                   (66, 2560), (17, 5120)])                  # 10 and 20 channels a workgroup, partial waves
 def test_att_seq_v4_scan_cuts(T, C_):
-    """Every way the scan cuts time and channels.  Bounds as in test_att_seq_v4."""
+    """The scan's cuts of time with 8 channels a workgroup, one to three blocks, and of one block with 10 and 20; blocks of
+    wider models: the test below.  Bounds as in test_att_seq_v4."""
     test_att_seq_v4(T, C_, False, False)
+
+
+@pytest.mark.parametrize("T,C_,cut", [(1900, 2112, (9, 235, 2, 106, 9)),    # two blocks; three channels past the end in the last workgroup
+                                      (1100, 2304, (9, 256, 1, 110, 10)),   # ten registers of a chunk in use
+                                      (1700, 2560, (10, 256, 2, 95, 9)),
+                                      (1250, 3584, (14, 256, 2, 70, 9)),    # a partial wave
+                                      (900, 5120, (20, 256, 2, 50, 9)),
+                                      (1280, 4736, (19, 250, 2, 50, 13)),   # 13 of 14 registers; 14 channels past the end
+                                      (560, 8256, (17, 486, 1, 56, 10))])   # two workgroups a compute unit
+def test_att_seq_v4_in_one_pass_and_in_parts(T, C_, cut):
+    """Blocks of time one after another with more than 8 channels a workgroup, and channels past the end: a prompt in one
+    pass against the same prompt in parts of at most 256 rows (one block each, held against the oracle above), the state
+    carried between them.  The fp32 sums are in another order, the products' as well, so that a binary16 rounding may go
+    the other way: of the output product o, by one spacing of o, and of x + o, by one of x + o; a third for an o at the edge
+    of its binade.  The inputs of o may have gone the other way too: 1 % of up to 8256 elements by 2^-12 or so, times weights
+    of 0.02, is 4e-5 rms, which the spacing at a quarter of the outputs' rms (2.4e-4 to 4.9e-4) covers six times over.
+    States as in test_att_seq_v4.  What lies past the last channel's state stays as it was."""
+    out = (C.c_int * 5)()
+    fr.check(L().frhip_wkv4_cut(T, C_, 256, out))
+    assert tuple(out) == cut
+    x, sx = h(rng.standard_normal((T, C_)) * 2), h(rng.standard_normal(C_))
+    state = _state_v4(C_, False)
+    consts = [keep(a).ptr for a in (*_common(C_), *[h(rng.uniform(0, 1, C_)) for _ in range(3)],
+                                    (-np.exp(rng.uniform(-5, 1, C_))).astype(np.float32), rng.uniform(-1, 1, C_).astype(np.float32))]
+    w = h(rng.standard_normal((C_, C_)) * 0.02)
+    ws_ = [make_weight(np.ascontiguousarray(np.roll(w, 17 * i)), False)[0] for i in range(4)]
+    ws, x_dev = DevBuf(L().frhip_seq_workspace_bytes(T, C_, 64)), keep(x)
+    results = []
+    for step in (T, 256):
+        x_out, xx = DevBuf.empty((T, C_), np.float16), [keep(sx), DevBuf.empty(C_, np.float16)]
+        st = [dev(np.concatenate([s, [7.5]]).astype(np.float32)) for s in state]
+        for lo in range(0, T, step):
+            fr.check(L().frhip_att_seq_v4(min(step, T - lo), C_, x_dev.ptr + 2 * C_ * lo, xx[0].ptr, *[s.ptr for s in st], *consts,
+                                          *[v.ref for v in ws_], x_out.ptr + 2 * C_ * lo, xx[1].ptr, *[s.ptr for s in st], ws.ptr, None))
+            xx = [xx[1], DevBuf.empty(C_, np.float16)]
+        results.append((x_out.numpy(), *[s.numpy() for s in st]))
+    (one, a1, b1, p1), (parts, a2, b2, p2) = results
+    assert a1[C_] == b1[C_] == p1[C_] == 7.5
+    one, parts = one.astype(np.float32), parts.astype(np.float32)
+    spacing = np.exp2(np.floor(np.log2(np.maximum(np.abs(parts - x), np.maximum(np.abs(parts), parts.std() / 4)))) - 10)
+    assert (np.abs(one - parts) <= 3 * spacing).all() and (one != parts).mean() < 0.1
+    scale = np.exp((p1 - p2)[:C_].astype(np.float64))
+    for got, want in ((a1, a2), (b1, b2)):
+        want = want[:C_].astype(np.float64)
+        assert np.allclose(got[:C_] * scale, want, rtol=2e-3, atol=2e-3 * np.abs(want).max())
 
 
 @pytest.mark.parametrize("T,C_,kvr,o", [(16400, 320, (256, 5, 2, 0), (256, 4, 1, 0)),  # predicated epilogues: 16 rows in the last strip
@@ -405,11 +451,11 @@ def test_att_seq_v4_on_planned_tiles(T, C_, kvr, o):
     test_att_seq_v4(T, C_, False, False)
 
 
-@pytest.mark.parametrize("T,C_", [(1024, 2048), (700, 512), (5000, 256)])  # 5000: beyond 128 chunks of 32 steps, the scan's serial pass
+@pytest.mark.parametrize("T,C_", [(1024, 2048), (700, 512), (5000, 256)])  # 5000: three blocks of time
 def test_att_seq_v4_state_updated_in_place_equals_separate_outputs(T, C_):
     """The header allows aa_out / bb_out / pp_out to be the buffers of aa / bb / pp (as frhip_att_one_v4 does).
-    The scan's last chunk writes them while other chunks may not have started: every pass must take the
-    incoming state from the copy the first pass makes.  Bit for bit the same as with separate outputs."""
+    A channel's workgroup reads the state before it writes it, and no other touches it.  Bit for bit the same as with
+    separate outputs."""
     x, sx = h(rng.standard_normal((T, C_)) * 2), h(rng.standard_normal(C_))
     aa, bb, pp = _state_v4(C_, False)
     ln_w, ln_b = _common(C_)
@@ -432,7 +478,7 @@ def test_att_seq_v4_state_updated_in_place_equals_separate_outputs(T, C_):
         results.append([x_out.numpy(), xx_out.numpy()] + [o.numpy() for o in outs])
     for sep, inp in zip(*results):
         assert np.array_equal(sep, inp)
-    if T == 5000:  # the long prompt against the oracle as well (the serial pass is otherwise only reached by a switch)
+    if T == 5000:  # the long prompt against the oracle as well
         ref = po.att_seq_v4_f16(x, sx, aa, bb, pp, ln_w, ln_b, *mixes, td, tf, *refs)
         assert_close_f16(results[0][0], ref[0], max_ulp=3, max_frac=0.1, what="x_out, T = 5000")
 
