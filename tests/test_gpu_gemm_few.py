@@ -5,7 +5,8 @@ import ctypes as C
 import numpy as np
 import pytest
 
-from hipref import DevBuf, L, dev, fr, make_weight
+import pyoracle as po
+from hipref import DevBuf, L, assert_close_f16, dev, fr, make_weight
 
 
 def tile(T, K, *N):
@@ -84,3 +85,48 @@ def test_activations_of_few_rows(T, K, N):
             assert d.max() <= 2 and (d != 0).mean() < 1e-3
         else:
             assert np.array_equal(got, ref)
+
+
+def form(T, K, *N, value=False):
+    """-> (form, blocks of 16 rows, blocks of 16 columns) of a launch of frhip_ffn_seq_v4"""
+    out = (C.c_int * 2)()
+    return L().frhip_seq_gemm_form(T, K, len(N), (C.c_int * len(N))(*N), 1 + 2 * value, 256, out), out[0], out[1]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("quant", [False, True])
+@pytest.mark.parametrize("T,C_,F_,rk,v", [(1, 512, 1024, (1, 1, 1), (1, 1, 1)), (13, 576, 1856, (1, 1, 1), (1, 1, 1)),
+                                          (16, 2048, 8192, (1, 1, 3), (1, 1, 1)),    # 2048 and 8192 are no multiples of 48
+                                          (65, 768, 3072, (1, 3, 2), (1, 1, 1)), (200, 768, 3072, (1, 5, 3), (1, 3, 1)),
+                                          (129, 512, 1792, (1, 3, 2), (1, 2, 1))])
+def test_ffn_of_few_rows(T, C_, F_, rk, v, quant):
+    """Groups (sigmoid and relu^2) and ffn's last epilogue, with rows past the end and tiles past a product's columns.
+    Bounds as for frhip_ffn_seq; halved outputs are the halves of the others, uint8 codes give the bits of their binary16 image."""
+    assert form(T, C_, C_, F_) == rk and form(T, F_, C_, value=True) == v
+    g = np.random.default_rng([T, C_])
+    h = lambda a: np.asarray(a, np.float32).astype(np.float16)
+    vecs = [h(g.standard_normal((T, C_)) * 2), h(g.standard_normal(C_)), h(1 + 0.1 * g.standard_normal(C_)), h(0.1 * g.standard_normal(C_)),
+            h(g.uniform(0, 1, C_)), h(g.uniform(0, 1, C_))]
+    (kw, kref), (vw, vref), (rw, rref) = (make_weight(h(g.standard_normal(s) * 0.02), quant) for s in ((C_, F_), (F_, C_), (C_, C_)))
+    want, xx = po.ffn_f16(*vecs, kref, vref, rref)
+    bufs, ws = [dev(a) for a in vecs], DevBuf(L().frhip_seq_workspace_bytes(T, C_, F_))
+
+    def run(weights, div2=0):
+        x_out, xx_out = DevBuf.empty((T + 1, C_), np.float16), DevBuf.empty(C_, np.float16)
+        x_out.upload(np.full((T + 1, C_), 7.5, np.float16))
+        fr.check(L().frhip_ffn_seq_v4(T, C_, F_, *[b.ptr for b in bufs], *weights, x_out.ptr, xx_out.ptr, div2, ws.ptr, None))
+        assert (x_out.numpy()[T] == 7.5).all()
+        assert_close_f16(xx_out.numpy(), xx, max_ulp=1, what="xx_last")
+        return x_out.numpy()[:T]
+
+    refs = [w.ref for w in (kw, vw, rw)]
+    got = run(refs)
+    assert_close_f16(got, want.reshape(got.shape), max_ulp=3, max_frac=0.2, what="x_out", floor_rms=1.0)
+    assert np.array_equal(run(refs, 1), got / np.float16(2))
+    if quant:
+        images = []
+        for w in (kw, vw, rw):
+            img = DevBuf.empty((w.N, w.K), np.float16)
+            fr.check(L().frhip_dequant_u8(w.ref, img.ptr, None))
+            images.append((img, fr.Weight(img.ptr, None, None, None, None, w.K, w.N, fr.F16)))
+        assert np.array_equal(run([C.byref(w) for _, w in images]).view(np.uint16), got.view(np.uint16))

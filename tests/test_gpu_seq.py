@@ -170,8 +170,8 @@ def _common(C_):
 # (1024, 2048, 8192): r and k as one round of 256-row tiles, the value product split over K in two slices;
 # (300, 2048, 8192): the value product in four slices over ragged row tiles; (512, 2560, 8960): three slices of 47, 47 and 46 K-steps
 # (16, 2048, 8192), (130, 2048, 8192), (200, 2560, 8960): short prompts at full width -- products split over K across the idle compute
-# units: r,k grouped in one split launch (16 rows), product by product because the group is too wide (130, 200 rows), the value
-# product in 16 and in fewer slices
+# units: r,k grouped in one split launch (16 rows), product by product because the group is too wide (130 rows) or on planned
+# tiles (200 rows), the value product in 16, five and three slices (test_seq_gemm_form.py holds these to it)
 @pytest.mark.parametrize("T,C_,F_", [(64, 512, 1792), (300, 2048, 8192), (1024, 2048, 8192), (512, 2560, 8960), (1, 512, 1024), (33, 768, 3072), (3000, 512, 1792),
                                      (16, 2048, 8192), (130, 2048, 8192), (200, 2560, 8960)])
 @pytest.mark.parametrize("quant", [False, True])

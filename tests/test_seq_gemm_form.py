@@ -32,6 +32,27 @@ def test_groups_that_are_split_as_a_whole_or_product_by_product():
     assert form(512, 8960, 2560, which=VALUE) == (SPLIT, 3, 0)
 
 
+@pytest.mark.parametrize("T,c,f,rk,v", [(16, 2048, 8192, (SPLIT, 3, 0), (SPLIT, 16, 0)), (130, 2048, 8192, (ONE_BY_ONE, 0, 0), (SPLIT, 5, 0)),
+                                        (200, 2560, 8960, (TILES, 0, 0), (SPLIT, 3, 0)), (300, 2048, 8192, (TILES, 0, 0), (SPLIT, 3, 0)),
+                                        (64, 512, 1792, (SPLIT, 2, 0), (SPLIT, 7, 0)), (33, 768, 3072, (SPLIT, 3, 0), (SPLIT, 12, 0)),
+                                        (13, 576, 1856, (SPLIT, 2, 0), (SPLIT, 7, 0)), (13, 2560, 8960, (SPLIT, 2, 0), (SPLIT, 12, 0)),
+                                        (64, 512, 2048, (SPLIT, 2, 0), (SPLIT, 8, 0)), (65, 768, 3072, (SPLIT, 3, 0), (SPLIT, 12, 0))])
+def test_what_the_operator_tests_of_ffn_seq_run(T, c, f, rk, v):
+    assert form(T, c, c, f) == rk and form(T, f, c, which=VALUE) == v
+
+
+@pytest.mark.parametrize("T,c", [(64, 512), (24, 2048), (37, 768), (150, 2048), (66, 2560)])
+def test_what_the_operator_tests_of_att_seq_v4_run(T, c):
+    assert form(T, c, c, c, c, which=V4)[0] == form(T, c, c, which=V4)[0] == FEW
+
+
+@pytest.mark.parametrize("T,c,f,rk,v", [(1, 512, 1024, FEW, FEW), (13, 2560, 8960, FEW, FEW), (16, 2048, 8192, FEW, FEW), (65, 768, 3072, FEW, FEW),
+                                        (200, 768, 3072, FEW, FEW), (130, 2048, 8192, FEW, SPLIT), (300, 2048, 8192, TILES, SPLIT),
+                                        (40, 2816, 11264, SPLIT, SPLIT), (17, 5120, 20480, ONE_BY_ONE, SPLIT)])
+def test_forms_of_rwkv4_ffn(T, c, f, rk, v):
+    assert form(T, c, c, f, which=V4)[0] == rk and form(T, f, c, which=V4 + VALUE)[0] == v
+
+
 @pytest.mark.parametrize("T", [4, 16, 64, 65, 128, 360])
 def test_rwkv5_sums_are_never_those_of_the_kernel_for_a_few_rows(T):
     for c, f in ((256, 896), (1024, 3584), (2560, 8960), (4096, 14336)):
