@@ -65,9 +65,11 @@ int launch_gemm(GemmArgs& a, bool u8, hipStream_t st, const char* what, void* dq
 // Products of a few rows in one launch, K split over the waves of a workgroup (gemm_few.hip).  plan_few: the tile that is
 // expected to be the quickest and its us; mt = 0: not a launch of this form.  It depends on the sizes alone, not on the
 // weight type, so that a uint8 weight and its binary16 image take the same sums.  few_takes: the addresses allow it.
-// Up to kFewRowsMax rows: beyond, a product is at best as quick as on tiles of 64 rows (512 x 2560 x 2560: 20.5 us against
-// 20.9), and the prompts of 512 tokens that RWKV-5.2's parity is measured on keep the order of their sums.
-constexpr int kFewKernelRows = kFewRowsMax;
+// Up to the rows that the times were fitted to; within them they decide.  Of 84 binary16 products of 384 to 512 rows (widths 768
+// to 5120) they send 26 here, all of them the quicker for it (512 x 2048 x 2048: 14.9 us on tiles of 64 rows, 10.2 here; 512 x
+// 3072 x 768: 20.6 and 9.0), and leave two behind that would have gained 5 % at most; a prompt of 512 tokens, 12 layers of 768:
+// 1050 -> 794 us, 2048: 1714 -> 1647, 5120 (2 layers): 1118 -> 1126.
+constexpr int kFewKernelRows = 512;
 struct FewPlan {
   int mt = 0, nt = 0;  // blocks of 16 rows and 16 columns of a workgroup
   double us = 0;

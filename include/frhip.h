@@ -260,7 +260,7 @@ int frhip_ffn_seq(int T, int C, int F, const void *x, const void *sx, const void
                   const void *k_mix, const void *r_mix,
                   const frhip_weight *kw, const frhip_weight *vw, const frhip_weight *rw,
                   void *x_out, void *xx_out, int post_div2, void *workspace, frhip_stream s);
-/* The same operator of an RWKV-4 model: products of up to 360 rows may add K in the order of a quicker kernel, as
+/* The same operator of an RWKV-4 model: products of up to 512 rows may add K in the order of a quicker kernel, as
  * frhip_att_seq_v4's do.  Rounding apart the results are the same; frhip_ffn_seq and frhip_att_seq_v5* keep the order that an
  * RWKV-5 model's first tokens need (its group normalisation turns the last bits of a sum near zero into a sign). */
 int frhip_ffn_seq_v4(int T, int C, int F, const void *x, const void *sx, const void *ln_w, const void *ln_b,

@@ -28,7 +28,7 @@ def test_cases_reach_every_tile():
 
 
 @pytest.mark.parametrize("T,K,N", [(256, 5120, (5120, 20480)),  # 91 us on planned tiles, 143 in one launch of this form
-                                   (361, 64, (64,)), (13, 2048, (2048, 2040))])  # too many rows; not a multiple of 16 columns
+                                   (513, 64, (64,)), (13, 2048, (2048, 2040))])  # too many rows; not a multiple of 16 columns
 def test_other_forms_keep_what_is_theirs(T, K, N):
     assert tile(T, K, *N) == (0, 0)
 
@@ -98,7 +98,8 @@ def form(T, K, *N, value=False):
 @pytest.mark.parametrize("T,C_,F_,rk,v", [(1, 512, 1024, (1, 1, 1), (1, 1, 1)), (13, 576, 1856, (1, 1, 1), (1, 1, 1)),
                                           (16, 2048, 8192, (1, 1, 3), (1, 1, 1)),    # 2048 and 8192 are no multiples of 48
                                           (65, 768, 3072, (1, 3, 2), (1, 1, 1)), (200, 768, 3072, (1, 5, 3), (1, 3, 1)),
-                                          (129, 512, 1792, (1, 3, 2), (1, 2, 1))])
+                                          (129, 512, 1792, (1, 3, 2), (1, 2, 1)),
+                                          (361, 768, 3072, (0, 0, 0), (1, 3, 2)), (512, 576, 1856, (0, 0, 0), (1, 3, 2))])  # the group on tiles
 def test_ffn_of_few_rows(T, C_, F_, rk, v, quant):
     """Groups (sigmoid and relu^2) and ffn's last epilogue, with rows past the end and tiles past a product's columns.
     Bounds as for frhip_ffn_seq; halved outputs are the halves of the others, uint8 codes give the bits of their binary16 image."""

@@ -356,7 +356,7 @@ def _state_v4(C_, fresh):
             rng.standard_normal(C_).astype(np.float32))
 
 
-@pytest.mark.parametrize("T,C_", [(64, 512), (1024, 2048), (1, 512), (37, 768), (3000, 512), (24, 2048), (150, 2048)])  # 3000: a long, ragged prompt (two blocks); 24, 150: short prompts at full width
+@pytest.mark.parametrize("T,C_", [(64, 512), (1024, 2048), (1, 512), (37, 768), (3000, 512), (24, 2048), (150, 2048), (500, 512)])  # 3000: a long, ragged prompt (two blocks); 24, 150: short prompts at full width; 500: products of many rows and few columns
 @pytest.mark.parametrize("quant", [False, True])
 @pytest.mark.parametrize("fresh", [True, False])
 def test_att_seq_v4(T, C_, quant, fresh):

@@ -41,7 +41,7 @@ def test_what_the_operator_tests_of_ffn_seq_run(T, c, f, rk, v):
     assert form(T, c, c, f) == rk and form(T, f, c, which=VALUE) == v
 
 
-@pytest.mark.parametrize("T,c", [(64, 512), (24, 2048), (37, 768), (150, 2048), (66, 2560)])
+@pytest.mark.parametrize("T,c", [(64, 512), (24, 2048), (37, 768), (150, 2048), (66, 2560), (500, 512)])
 def test_what_the_operator_tests_of_att_seq_v4_run(T, c):
     assert form(T, c, c, c, c, which=V4)[0] == form(T, c, c, which=V4)[0] == FEW
 
@@ -53,7 +53,14 @@ def test_forms_of_rwkv4_ffn(T, c, f, rk, v):
     assert form(T, c, c, f, which=V4)[0] == rk and form(T, f, c, which=V4 + VALUE)[0] == v
 
 
-@pytest.mark.parametrize("T", [4, 16, 64, 65, 128, 360])
+def test_the_expected_times_decide_up_to_512_rows():
+    for T, c, f in ((361, 768, 3072), (512, 768, 3072), (400, 1280, 5120)):
+        assert form(T, c, c, which=V4)[0] == form(T, f, c, which=V4 + VALUE)[0] == FEW
+    assert form(500, 512, *(512,) * 3, which=V4)[0] == form(512, 2048, 2048, which=V4)[0] == FEW
+    assert form(512, 4096, 4096, which=V4)[0] == form(513, 768, 768, which=V4)[0] == TILES
+
+
+@pytest.mark.parametrize("T", [4, 16, 64, 65, 128, 360, 361])
 def test_rwkv5_sums_are_never_those_of_the_kernel_for_a_few_rows(T):
     for c, f in ((256, 896), (1024, 3584), (2560, 8960), (4096, 14336)):
         for which, K, N in ((0, c, (c,) * 4), (0, c, (c,) * 3), (0, c, (c,)), (0, c, (c, f)), (VALUE, f, (c,))):
