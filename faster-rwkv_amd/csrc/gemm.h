@@ -52,8 +52,8 @@ struct GemmArgs {
 
 // dq: optional scratch, 2 bytes per weight of the launch.  With it, uint8 weights of a launch with at least
 // kDequantRows rows are expanded once to binary16 (the standalone dequantisation: the same bits as the
-// in-kernel one) and the launch takes the binary16 kernel, unless it has at most 64 rows and goes out split over K
-// (few_rows): the uint8 kernel dequantises those on the way into LDS.
+// in-kernel one) and the launch takes the binary16 kernel, unless it is one of gemm_few_kernel, or has at most 64 rows and goes out
+// split over K (few_rows): those kernels dequantise the codes themselves.
 // partial: optional fp32 scratch of max_split slices of partial_stride floats (>= M * N each) for splitting K.
 // few_rows: optional fp32 scratch of few_rows_floats floats; with it a launch of so few rows that 64 x 128 tiles leave
 // at least half of the compute units idle is split over K across the idle units, whole or product by product.

@@ -298,7 +298,8 @@ static void few_launch(int grid, hipStream_t st, const GemmArgs& a) {
   X(4, 2) X(4, 3) X(4, 4) X(5, 2) X(5, 3) X(5, 4) X(5, 5) X(6, 4)
 
 // What a launch with these tiles is expected to take, us; fitted to the binary16 ones of those products (2 to 512 rows, K 768 to
-// 20480, N 768 to 20480, weights from memory; 9 % rms).  Per round over the compute units: a fixed part that grows with
+// 20480, N 768 to 20480, weights from memory; 9 % rms, as on 476 others of 4 to 512 rows since, whose worst region, single narrow
+// products of 17 to 64 rows, takes 13 % longer than expected).  Per round over the compute units: a fixed part that grows with
 // the sums to be merged, then the K-steps beyond those that the rings hold at the start, each as long as its loads and
 // products; and no faster than the weights arrive, which several strips of rows read more than once.
 static double few_us(const GemmArgs& a, int mt, int nt, int cus) {

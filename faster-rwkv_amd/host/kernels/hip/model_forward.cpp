@@ -512,8 +512,11 @@ static Tensor forward_seq(Model *model, Device device, const std::vector<int> &i
   // the reference-shaped operator loop (vgather, seq operators, slice, layernorm, matmul, cast_dtype)
   if (std::getenv("FR_HIP_GENERIC")) return def::ModelForwardSeq(model, device, ids, full_output);
   RV_CHECK(!ids.empty());
-  // A prompt of two or three tokens is quicker as one-token steps (0.7 ms each for the 1.5B shape) than as a pass
-  // of the seq operators, which for so few rows costs its ~290 launches (1.9 ms); FR_HIP_SEQ_ALWAYS=1: never.
+  // A prompt of two or three tokens runs as one-token steps, because a pass of fewer than 4 rows dequantises uint8 weights on tiles
+  // for every product that gemm_few_kernel does not take, and RWKV-5's never do: 3B RWKV-5.2 width, 12 layers, uint8, two / three
+  // tokens: 0.95 / 1.41 ms as steps, 3.7 as a pass.  Where that kernel takes them a pass costs about two steps, whatever its
+  // length up to 8 (RWKV-4 1.5B shape, 168 launches in the layers: 1.43 / 2.11 ms as steps, 1.33 / 1.35 as a pass; uint8 1.23 /
+  // 1.83 and 1.29 / 1.30; 169M shape 0.43 / 0.63 and 0.48 / 0.47): three such tokens would gain.  FR_HIP_SEQ_ALWAYS=1: always a pass.
   if (!full_output && ids.size() < 4 && !std::getenv("FR_HIP_SEQ_ALWAYS")) {
     Tensor out;
     for (int id : ids) out = hip::ModelForward(model, device, id);
