@@ -39,8 +39,8 @@ struct GemmArgs {
   int vw_base[kGemmMaxSeg], vw_wide[kGemmMaxSeg], vw_maxw, vw_ns;
   int few_strips;  // gemm_few_kernel: strips of rows
   GemmSeg seg[kGemmMaxSeg];
-  // split K (ksplit >= 2; gemm_ldw_kernel<128> with one segment, gemm_ldw_kernel<64> and the uint8 gemm_kernel<64, 64> with
-  // up to four): slice z of ksplit accumulates its K-steps of segment s into partial + z * partial_stride + part_off[s] as
+  // split K (ksplit >= 2; gemm_ldw_kernel<128> with one segment, gemm_ldw_kernel<64> and
+  // gemm_q8_kernel with up to four): slice z of ksplit accumulates its K-steps of segment s into partial + z * partial_stride + part_off[s] as
   // fp32 [M][N]; gemm_splitk_reduce_kernel adds the slices and applies the epilogues
   int ksplit;
   float* partial;
@@ -52,8 +52,8 @@ struct GemmArgs {
 
 // dq: optional scratch, 2 bytes per weight of the launch.  With it, uint8 weights of a launch with at least
 // kDequantRows rows are expanded once to binary16 (the standalone dequantisation: the same bits as the
-// in-kernel one) and the launch takes the binary16 kernel, unless it is one of gemm_few_kernel, or has at most 64 rows and goes out
-// split over K (few_rows): those kernels dequantise the codes themselves.
+// in-kernel one) and the launch takes the binary16 kernel, unless it is one of gemm_few_kernel or is expected to be quicker as
+// one of gemm_q8_kernel: those dequantise the codes themselves.
 // partial: optional fp32 scratch of max_split slices of partial_stride floats (>= M * N each) for splitting K.
 // few_rows: optional fp32 scratch of few_rows_floats floats; with it a launch of so few rows that 64 x 128 tiles leave
 // at least half of the compute units idle is split over K across the idle units, whole or product by product.
@@ -77,6 +77,19 @@ struct FewPlan {
 FewPlan plan_few(const GemmArgs& a, int cus);
 bool few_takes(const GemmArgs& a, bool u8);
 int launch_gemm_few(const GemmArgs& a, const FewPlan& p, bool u8, hipStream_t st, const char* what);
+// Deals `tiles` workgroups of a strip of rows to the segments by their columns: tile_start, vw_base, vw_wide, vw_maxw.  False: too few.
+bool deal_tiles(GemmArgs& a, int tiles);
+// Products of uint8 weights that dequantise the codes on their way into LDS (gemm_q8.hip), with the tile that is expected to be
+// the quickest; rows = 0: not a launch of this form.  a.ksplit, partial and part_off as for gemm_ldw_kernel.
+struct Q8Plan {
+  int rows = 0, rounds = 0;
+  double us = 0;
+  dim3 grid;
+  GemmArgs a;
+};
+Q8Plan plan_q8(const GemmArgs& a, int cus);
+bool q8_takes(const GemmArgs& a);
+int launch_gemm_q8(const Q8Plan& p, hipStream_t st, const char* what);
 constexpr int kDequantRows = FRHIP_SEQ_EXPAND_ROWS;
 // uint8 [N][K] -> binary16 [N][K] with the frozen formula (ops.hip)
 int dequant_u8_async(const unsigned char* q, const h1* mx, const h1* rx, const h1* my, const h1* ry, h1* dst, int K, int N,

@@ -17,7 +17,7 @@
 //                    against bank conflicts), the loads of step k+1 issued before the MFMAs of
 //                    step k, and are dequantised to binary16 on the way into LDS with the same
 //                    formula as the standalone dequantisation, so the product sees exactly the
-//                    dequantised matrix (launches of up to 64 rows, and calls without scratch
+//                    dequantised matrix (what gemm_q8_kernel does not take, without scratch
 //                    for the expanded weights).
 // Products are exact in fp32, accumulation is fp32 in ascending k, and the result is rounded once
 // to the output type (kernels/cuda/matmul.cpp:38-42,64-68); all kernels give the same bits, except
@@ -35,101 +35,6 @@ namespace frhip {
 
 constexpr int BN = 128;
 constexpr int kGemmThreads = 256;
-// Fused epilogues, shared by the product kernels: acc[i][j] is the 32x32 block (i, j) of the wave's
-// (32 MI) x (32 NJ) tile whose first element is (row0, col0); acc[i][j][v] is
-// C[row = 8*(v/4) + 4*(lane/32) + v%4][col = lane%32] of the block.
-// FULL: the workgroup's tile lies inside the matrix, nothing is predicated.  (With a predicate per
-// element every store becomes a branch to an out-of-line block; on the 1024 x 6144 product that
-// was 11 of 59 us.)  The epilogue kind is uniform over the launch segment: one switch, and for the
-// kinds that read operands all 16 of a block are requested before the first is used.
-template <int MI, int NJ, bool FULL>
-__device__ __forceinline__ void gemm_epilogue_t(const GemmArgs& a, const GemmSeg& sg, const f16v (&acc)[MI][NJ],
-                                                int row0, int col0, int M, int N, int lane) {
-  auto for_tile = [&](int i, int j, auto&& f) {
-    const int col = col0 + j * 32 + (lane & 31);
-#pragma unroll
-    for (int v = 0; v < 16; v++) {
-      const int row = row0 + i * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
-      if constexpr (FULL)
-        f(v, true, (size_t)row * N + col);
-      else
-        f(v, row < M && col < N, (size_t)(row < M ? row : M - 1) * N + (col < N ? col : N - 1));
-    }
-  };
-  auto for_blocks = [&](auto&& g) {
-#pragma unroll
-    for (int i = 0; i < MI; i++)
-#pragma unroll
-      for (int j = 0; j < NJ; j++) g(i, j, acc[i][j]);
-  };
-  // blocks without a stored element; only for the costly epilogues: with the test in all of them the short launches of
-  // gemm_ldw_kernel<64> took 0.4-0.8 us longer (33 x 1024 x 5120: 6.5 -> 6.9)
-  auto outside = [&](int i, int j) { return !FULL && (row0 + i * 32 >= M || col0 + j * 32 >= N); };
-  auto live_of = [&](int i, int j) {  // bit v: element v of the block lies inside the matrix
-    uint32_t m = 0;
-    for_tile(i, j, [&](int v, bool ok, size_t) { m |= ok ? 1u << v : 0u; });
-    return m;
-  };
-  switch (sg.epi) {
-    case G_STORE_F16:
-      for_blocks([&](int i, int j, const f16v& c) {
-        for_tile(i, j, [&](int v, bool ok, size_t o) { if (ok) static_cast<h1*>(sg.out)[o] = (h1)c[v]; });
-      });
-      break;
-    case G_STORE_F32:
-      for_blocks([&](int i, int j, const f16v& c) {
-        for_tile(i, j, [&](int v, bool ok, size_t o) { if (ok) static_cast<float*>(sg.out)[o] = c[v]; });
-      });
-      break;
-    case G_SIGMOID:
-      for_blocks([&](int i, int j, const f16v& c) {
-        if (outside(i, j)) return;
-        h1 y[16];
-        sigmoid_batch(c, y, live_of(i, j));
-        for_tile(i, j, [&](int v, bool ok, size_t o) { if (ok) static_cast<h1*>(sg.out)[o] = y[v]; });
-      });
-      break;
-    case G_RELU2:
-      for_blocks([&](int i, int j, const f16v& c) {
-        for_tile(i, j, [&](int v, bool ok, size_t o) {
-          const h1 t = (h1)c[v];
-          if (ok) static_cast<h1*>(sg.out)[o] = (t > (h1)0.0f) ? (t * t) : (h1)0.0f;
-        });
-      });
-      break;
-    case G_SILU:
-      for_blocks([&](int i, int j, const f16v& c) {
-        if (outside(i, j)) return;
-        h1 y[16];
-        silu_batch(c, y, live_of(i, j));
-        for_tile(i, j, [&](int v, bool ok, size_t o) { if (ok) static_cast<h1*>(sg.out)[o] = y[v]; });
-      });
-      break;
-    case G_RESIDUAL:
-      for_blocks([&](int i, int j, const f16v& c) {
-        h1 rx[16];
-        for_tile(i, j, [&](int v, bool, size_t o) { rx[v] = a.res_x[o]; });
-        for_tile(i, j, [&](int v, bool ok, size_t o) { if (ok) static_cast<h1*>(sg.out)[o] = rx[v] + (h1)c[v]; });
-      });
-      break;
-    case G_FFN_OUT:
-      for_blocks([&](int i, int j, const f16v& c) {
-        h1 rx[16], rr[16];
-        for_tile(i, j, [&](int v, bool, size_t o) {
-          rx[v] = a.res_x[o];
-          rr[v] = a.res_r[o];
-        });
-        for_tile(i, j, [&](int v, bool ok, size_t o) {
-          h1 r = __builtin_fmaf16((h1)c[v], rr[v], rx[v]);
-          if (a.div2) r = r / (h1)2.0f;
-          if (ok) static_cast<h1*>(sg.out)[o] = r;
-        });
-      });
-      break;
-    default: break;
-  }
-}
-
 template <int BM>
 __device__ __forceinline__ void gemm_epilogue(const GemmArgs& a, const GemmSeg& sg, const f16v (&acc)[BM / 64][2], int m0,
                                               int n0, int M, int N, int lane, int wm, int wn) {
@@ -275,31 +180,17 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_kernel(GemmArgs a) {
     }
   };
 
-  // slice z of ksplit takes K-steps [z base + min(z, rem), ...): the first rem slices one step more
-  int kbeg = 0, kend = K;
-  if (U8 && a.ksplit > 1) {
-    const int z = blockIdx.z, steps = K / BK, per = steps / a.ksplit, rem = steps % a.ksplit;
-    kbeg = (z * per + min(z, rem)) * BK;
-    kend = kbeg + (per + (z < rem ? 1 : 0)) * BK;
-  }
   Stage s0;
-  load_tiles(s0, kbeg);
-  for (int k0 = kbeg; k0 < kend; k0 += BK) {
+  load_tiles(s0, 0);
+  for (int k0 = 0; k0 < K; k0 += BK) {
     __syncthreads();  // everyone is done reading the previous tile
     store_tiles(s0, k0);
     __syncthreads();
-    if (k0 + BK < kend) load_tiles(s0, k0 + BK);
+    if (k0 + BK < K) load_tiles(s0, k0 + BK);
     compute_tile();
   }
 
-  if (U8 && a.ksplit > 1) {
-    GemmSeg sp = sg;  // this slice's sums go out as fp32; the epilogue proper follows in gemm_splitk_reduce_kernel
-    sp.out = a.partial + (size_t)blockIdx.z * a.partial_stride + a.part_off[sidx];
-    sp.epi = G_STORE_F32;
-    gemm_epilogue<BM>(a, sp, acc, m0, n0, M, N, lane, wm, wn);
-  } else {
-    gemm_epilogue<BM>(a, sg, acc, m0, n0, M, N, lane, wm, wn);
-  }
+  gemm_epilogue<BM>(a, sg, acc, m0, n0, M, N, lane, wm, wn);
 }
 
 // ---------------------------------------------------------------------------
@@ -323,12 +214,7 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_kernel(GemmArgs a) {
 // ---------------------------------------------------------------------------
 constexpr int kLdwThreads = 320;
 constexpr int kLdwStages = 4;
-constexpr int kLdwBK = 64;
 static constexpr size_t gemm_ldw_lds_bytes(int bm) { return (size_t)kLdwStages * (bm + BN) * kLdwBK * 2; }
-__device__ __forceinline__ int ldw_at(int row, int q) {
-  return (row >> 3) * 1024 + (row & 7) * 128 + ((q ^ (row & 7) ^ ((row >> 3) & 1)) * 16);
-}
-
 template <int BM>
 __global__ __launch_bounds__(kLdwThreads) void gemm_ldw_kernel(GemmArgs a) {
   constexpr int MI = BM / 64;
@@ -502,67 +388,7 @@ __device__ __forceinline__ void splitk_reduce_body(const GemmArgs& a, const Gemm
 #pragma unroll
           for (int i = 0; i < 4; i++) acc[4 * q + i] += p[j][q][i];
   }
-  if (sg.epi == G_STORE_F32) {
-    float* out = static_cast<float*>(sg.out) + o;
-#pragma unroll
-    for (int q = 0; q < Q; q++) {
-      f4v v;
-#pragma unroll
-      for (int i = 0; i < 4; i++) v[i] = acc[4 * q + i];
-      *reinterpret_cast<f4v*>(out + 4 * q) = v;
-    }
-    return;
-  }
-  h1 y[W];
-  switch (sg.epi) {
-    case G_STORE_F16:
-#pragma unroll
-      for (int i = 0; i < W; i++) y[i] = (h1)acc[i];
-      break;
-    case G_SIGMOID:
-    case G_SILU:
-      if constexpr (W == 16) {
-        f16v c;
-#pragma unroll
-        for (int i = 0; i < 16; i++) c[i] = acc[i];
-        if (sg.epi == G_SIGMOID) sigmoid_batch(c, y, 0xffffu); else silu_batch(c, y, 0xffffu);
-      }
-      break;
-    case G_RELU2:
-#pragma unroll
-      for (int i = 0; i < W; i++) {
-        const h1 t = (h1)acc[i];
-        y[i] = (t > (h1)0.0f) ? (t * t) : (h1)0.0f;
-      }
-      break;
-    case G_RESIDUAL:
-#pragma unroll
-      for (int g = 0; g < W / 8; g++) {
-        const h8 x = *reinterpret_cast<const h8*>(a.res_x + o + 8 * g);
-#pragma unroll
-        for (int i = 0; i < 8; i++) y[8 * g + i] = x[i] + (h1)acc[8 * g + i];
-      }
-      break;
-    default:  // G_FFN_OUT
-#pragma unroll
-      for (int g = 0; g < W / 8; g++) {
-        const h8 x = *reinterpret_cast<const h8*>(a.res_x + o + 8 * g), r = *reinterpret_cast<const h8*>(a.res_r + o + 8 * g);
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-          h1 v = __builtin_fmaf16((h1)acc[8 * g + i], r[i], x[i]);
-          if (a.div2) v = v / (h1)2.0f;
-          y[8 * g + i] = v;
-        }
-      }
-      break;
-  }
-#pragma unroll
-  for (int g = 0; g < W / 8; g++) {
-    h8 v;
-#pragma unroll
-    for (int i = 0; i < 8; i++) v[i] = y[8 * g + i];
-    *reinterpret_cast<h8*>(static_cast<h1*>(sg.out) + o + 8 * g) = v;
-  }
+  store_row<W>(a, sg, acc, o);
 }
 
 template <int W>
@@ -734,20 +560,6 @@ __device__ __forceinline__ void vw_mma(const GemmArgs& a, const GemmSeg& sg, con
     gemm_epilogue_t<2, NJ, true>(a, sg, acc, m0 + wm * 64, n0 + brow0, M, N, lane);
   else
     gemm_epilogue_t<2, NJ, false>(a, sg, acc, m0 + wm * 64, n0 + brow0, M, N, lane);
-}
-
-// Workgroups are dealt to the eight XCDs in turn (linear index mod 8), each with an L2 of its own.  XCD x takes the
-// x-th eighth of the tiles, counted in blocks of four strips of rows by all N tiles, so that the 32 it runs at a time
-// share about four strips and eight N tiles.  Blocks of four N tiles by all strips, the other way round, gave the
-// tiles of a segment with a costly epilogue to one or two XCDs: the 4099-token prompt of a 1.5B model took 19.2 ms
-// so, 18.3 this way (same box, in turn; up to four strips the two are the same map).  (A matter of traffic and balance
-// only: the map is one to one, and any assignment of tiles to workgroups gives the same results.)
-__device__ __forceinline__ void xcd_tile(int& bx, int& by) {
-  const int gx = gridDim.x, gy = gridDim.y, lin = blockIdx.y * gx + blockIdx.x, n = gx * gy;
-  const int x = lin & 7, id = x * (n >> 3) + min(x, n & 7) + (lin >> 3);
-  const int blk = id / (4 * gx), rem = id - blk * 4 * gx, bw = min(4, gy - 4 * blk);
-  bx = rem / bw;
-  by = 4 * blk + rem % bw;
 }
 
 // BM / 32 MFMA waves of 64 rows x half the width, then the loader.  BM = 256: launches of whole tiles of at most
@@ -935,6 +747,46 @@ static double us_256(int rounds, double k, int w) { return 2 + rounds * (6.6 + k
 static double us_256_loader(int rounds, double k, int w) { return 2 + rounds * (5.7 + k * (5.8 + 6.8 * w)); }
 constexpr double kLaunchUs = 3;  // one more launch
 
+bool deal_tiles(GemmArgs& a, int P) {
+  if (P < a.nseg) return false;
+  int cb[kGemmMaxSeg], t[kGemmMaxSeg], total = 0, used = 0;
+  for (int s = 0; s < a.nseg; s++) {
+    cb[s] = (a.seg[s].N + 31) / 32;
+    total += cb[s];
+  }
+  for (int s = 0; s < a.nseg; s++) {
+    t[s] = (int)((long)P * cb[s] / total);
+    if (t[s] < 1) t[s] = 1;
+    used += t[s];
+  }
+  if (used > P) return false;
+  // the spare tiles go where the tiles are widest; among equals, to the segment whose epilogue
+  // costs most (a transcendental per element), so that its tiles are the narrow ones
+  auto heavy = [&](int s) { return a.seg[s].epi == G_SIGMOID || a.seg[s].epi == G_SILU ? 1 : 0; };
+  while (used < P) {
+    int best = 0;
+    for (int s = 1; s < a.nseg; s++) {
+      const long l = (long)cb[s] * t[best], q = (long)cb[best] * t[s];
+      if (l > q || (l == q && heavy(s) > heavy(best))) best = s;
+    }
+    t[best]++;
+    used++;
+  }
+  int tiles = 0;
+  a.vw_maxw = 0;
+  for (int s = 0; s < a.nseg; s++) {
+    const int w = (cb[s] + t[s] - 1) / t[s];
+    a.vw_maxw = w > a.vw_maxw ? w : a.vw_maxw;
+    a.tile_start[s] = tiles;
+    a.vw_base[s] = cb[s] / t[s];
+    a.vw_wide[s] = cb[s] % t[s];
+    tiles += t[s];
+  }
+  for (int s = a.nseg; s <= kGemmMaxSeg; s++) a.tile_start[s] = INT_MAX;
+  a.tile_start[a.nseg] = tiles;
+  return true;
+}
+
 // Cuts the launch into tiles of bm rows (128 or 256): the fewest rounds over `cus` compute units whose widest tile
 // fits.  r.rows stays 0 if it is too small for tiles of at least bm x 96, or too ragged.
 static GemmRoute plan_vw(const GemmArgs& args, int bm, int cus) {
@@ -945,53 +797,18 @@ static GemmRoute plan_vw(const GemmArgs& args, int bm, int cus) {
   if (bm == 256 && (size_t)a.K * 2 * 256 > 0xffffffffull) return r;
   const int mt = (a.M + bm - 1) / bm;
   const int abytes = bm * kLdwBK * 2;
-  int cb[kGemmMaxSeg], total = 0;
-  for (int s = 0; s < a.nseg; s++) {
-    cb[s] = (a.seg[s].N + 31) / 32;
-    total += cb[s];
-  }
+  int total = 0;
+  for (int s = 0; s < a.nseg; s++) total += (a.seg[s].N + 31) / 32;
   // From the fewest rounds that tiles of the largest width allow; it ends at tiles of one block at the latest.  (With a
   // limit of 32 rounds 8193 x 2048 x 65536 took 3.14 ms on fixed 128 x 128 tiles, 2.06 so, one row less 1.97.)
   for (long rounds = ((long)total * mt + (long)kVwMaxW * cus - 1) / ((long)kVwMaxW * cus);; rounds++) {
     const int P = (int)(rounds * cus / mt);  // tiles per strip of rows
-    if (P < a.nseg) continue;
-    int t[kGemmMaxSeg], used = 0;
-    for (int s = 0; s < a.nseg; s++) {
-      t[s] = (int)((long)P * cb[s] / total);
-      if (t[s] < 1) t[s] = 1;
-      used += t[s];
-    }
-    if (used > P) continue;
-    // the spare tiles go where the tiles are widest; among equals, to the segment whose epilogue
-    // costs most (a transcendental per element), so that its tiles are the narrow ones
-    auto heavy = [&](int s) { return a.seg[s].epi == G_SIGMOID || a.seg[s].epi == G_SILU ? 1 : 0; };
-    while (used < P) {
-      int best = 0;
-      for (int s = 1; s < a.nseg; s++) {
-        const long l = (long)cb[s] * t[best], q = (long)cb[best] * t[s];
-        if (l > q || (l == q && heavy(s) > heavy(best))) best = s;
-      }
-      t[best]++;
-      used++;
-    }
-    int maxw = 0, minw = INT_MAX;
-    for (int s = 0; s < a.nseg; s++) {
-      const int w = (cb[s] + t[s] - 1) / t[s];
-      maxw = w > maxw ? w : maxw;
-      minw = cb[s] / t[s] < minw ? cb[s] / t[s] : minw;
-    }
+    if (!deal_tiles(a, P)) continue;
+    const int maxw = a.vw_maxw, tiles = a.tile_start[a.nseg];
+    int minw = INT_MAX;
+    for (int s = 0; s < a.nseg; s++) minw = a.vw_base[s] < minw ? a.vw_base[s] : minw;
     if (maxw > kVwMaxW) continue;
     if (minw < 2 || maxw < 3) return r;
-    int tiles = 0;
-    for (int s = 0; s < a.nseg; s++) {
-      a.tile_start[s] = tiles;
-      a.vw_base[s] = cb[s] / t[s];
-      a.vw_wide[s] = cb[s] % t[s];
-      tiles += t[s];
-    }
-    for (int s = a.nseg; s <= kGemmMaxSeg; s++) a.tile_start[s] = INT_MAX;
-    a.tile_start[a.nseg] = tiles;
-    a.vw_maxw = maxw;
     const size_t stage = abytes + (size_t)maxw * 4096;
     if (bm == 256) {
       // Whole tiles of up to 160 columns: the loader wave's form, whose loads are two steps ahead.  All 256 compute
@@ -1117,13 +934,7 @@ static bool env_on(const char* name) {
 // launch is split over K into as many slices as there are idle compute units (at least four K-steps each), and the
 // reduction pass adds the slices in order and applies each product's epilogue.  A group that is too wide for that as a
 // whole goes out product by product, so that its narrow members still can.  FRHIP_GEMM_FEW_ROWS=0: off.
-// uint8 weights of at most kU8DirectRows rows (one strip of tiles) are dequantised on their way into LDS, once each:
-// 1 byte of traffic per weight, where the expansion and a binary16 product move 5 (1 in, 2 out, 2 in again).  The
-// slices are those of the binary16 launch, so the sums are the same bits whichever form of the weight is multiplied.
-// 13 rows of 2048 x 10240 (ffn r,k): 18.6 us against 17.7 + 9.5; 8192 x 2048: 13.7 against 15.0 + 8.6; 2048 x 2048:
-// 9.0 against 7.3 + 5.2.  Above 64 rows a second strip would dequantise every code again.
 // *taken stays false, and nothing is launched, if the launch is not of this form.
-constexpr int kU8DirectRows = 64;
 
 // Slices of K for a launch of few rows on 64 x 128 tiles, 0 if it is not split as a whole.
 static int few_rows_slices(const GemmArgs& a, size_t few_rows_floats, int cus) {
@@ -1158,31 +969,34 @@ static bool few_rows_one_by_one(const GemmArgs& a, int cus) {
   return a.nseg > 1 && tiles * m64 < cus && any && !(all && tiles * m64 * 2 <= cus);
 }
 
-static int launch_few_rows(GemmArgs& a, bool u8, hipStream_t st, const char* what, void* dq, float* few_rows,
-                           size_t few_rows_floats, bool* taken) {
+// S slices of K with their sums in `partial`: the segments side by side in every slice
+static void split_over(GemmArgs& a, int S, float* partial) {
+  size_t cols = 0;
+  for (int s = 0; s < a.nseg; s++) {
+    a.part_off[s] = (size_t)a.M * cols;
+    cols += (size_t)a.seg[s].N;
+  }
+  a.part_off[a.nseg] = (size_t)a.M * cols;
+  a.ksplit = S;
+  a.partial = partial;
+  a.partial_stride = (a.part_off[a.nseg] + 63) / 64 * 64;
+}
+
+static int launch_few_rows(GemmArgs& a, hipStream_t st, const char* what, float* few_rows, size_t few_rows_floats, bool* taken) {
   const int cus = compute_units();
   if (a.K / kLdwBK < 4) return 0;
   if (const int S = few_rows_slices(a, few_rows_floats, cus)) {
     int tiles = 0;
-    size_t cols = 0;
     for (int s = 0; s < a.nseg; s++) {
       a.tile_start[s] = tiles;
       tiles += (a.seg[s].N + BN - 1) / BN;
-      a.part_off[s] = (size_t)a.M * cols;
-      cols += (size_t)a.seg[s].N;
     }
     for (int s = a.nseg; s <= kGemmMaxSeg; s++) a.tile_start[s] = INT_MAX;
     a.tile_start[a.nseg] = tiles;
-    a.part_off[a.nseg] = (size_t)a.M * cols;
     *taken = true;
-    a.ksplit = S;
-    a.partial = few_rows;
-    a.partial_stride = (a.part_off[a.nseg] + 63) / 64 * 64;
+    split_over(a, S, few_rows);
     const dim3 grid(tiles, (a.M + 63) / 64, (unsigned)S);
-    if (u8)
-      gemm_launch_one<64, 64, true>(grid, st, a);
-    else
-      gemm_ldw_launch<64>(grid, st, a);
+    gemm_ldw_launch<64>(grid, st, a);
     if (int rc = check_launch(what)) return rc;
     launch_splitk_reduce(st, a);
     return check_launch(what);
@@ -1193,7 +1007,7 @@ static int launch_few_rows(GemmArgs& a, bool u8, hipStream_t st, const char* wha
     GemmArgs one = a;
     one.nseg = 1;
     one.seg[0] = a.seg[s];
-    if (int rc = launch_gemm(one, u8, st, what, dq, nullptr, 0, 0, few_rows, few_rows_floats)) return rc;
+    if (int rc = launch_gemm(one, false, st, what, nullptr, nullptr, 0, 0, few_rows, few_rows_floats)) return rc;
   }
   return 0;
 }
@@ -1247,6 +1061,69 @@ static FewPlan few_plan(const GemmArgs& a, size_t partial_stride, int max_split,
   return p.mt && p.us * 1.1 <= tiled_us(a, partial_stride, max_split, few_rows_floats, cus) ? p : FewPlan();
 }
 
+// uint8 weights through gemm_q8_kernel, in the slices of K that the binary16 launch would take, so with the same bits.  A group
+// whose members are split one by one stays one launch where they take the same slices and their sums fit the scratch.
+// With scratch for it (dq) the codes can be expanded instead, 3 bytes of traffic a weight at 5 TB/s, and multiplied as binary16;
+// many strips of rows dequantise every code once each, so from about 512 rows of a wide product on that is quicker (1000 x 4096 x
+// 16384: 173 us against 193; x 4096: 57 against 52).  *taken stays false, and nothing is launched, where it is expected to be.
+static int launch_codes(GemmArgs& a, hipStream_t st, const char* what, void* dq, float* partial, size_t partial_stride, int max_split,
+                        float* few_rows, size_t few_rows_floats, bool* taken) {
+  if (!q8_takes(a)) return 0;
+  const int cus = compute_units(), ksteps = a.K / kLdwBK;
+  GemmArgs b = a;
+  if (few_rows && ksteps >= 4) {
+    if (const int S = few_rows_slices(a, few_rows_floats, cus)) {
+      split_over(b, S, few_rows);
+    } else if (few_rows_one_by_one(a, cus)) {
+      int S = 0;
+      for (int s = 0; s < a.nseg; s++) {
+        GemmArgs one = a;
+        one.nseg = 1;
+        one.seg[0] = a.seg[s];
+        const int Si = few_rows_slices(one, few_rows_floats, cus);
+        S = s == 0 || Si == S ? Si : -1;
+        if (S < 2) break;
+      }
+      // (not where a member could be one of gemm_few_kernel: its binary16 image would be)
+      if (S >= 2 && a.tiled_sums) split_over(b, S, few_rows);
+      if (b.ksplit < 2 || b.ksplit * b.partial_stride > few_rows_floats) {
+        *taken = true;
+        for (int s = 0; s < a.nseg; s++) {
+          GemmArgs one = a;
+          one.nseg = 1;
+          one.seg[0] = a.seg[s];
+          if (int rc = launch_gemm(one, true, st, what, dq, nullptr, 0, 0, few_rows, few_rows_floats)) return rc;
+        }
+        return 0;
+      }
+    }
+  }
+  if (b.ksplit < 2 && partial)
+    if (const int S = long_k_slices(a, partial_stride, max_split, cus)) {
+      split_over(b, S, partial);
+      b.partial_stride = partial_stride;
+    }
+  if (b.ksplit < 2 && !a.tiled_sums && one_by_one(a, gemm_route(a, cus), cus))
+    for (int s = 0; s < a.nseg; s++) {  // the binary16 image's members could be gemm_few_kernel's
+      GemmArgs one = a;
+      one.nseg = 1;
+      one.seg[0] = a.seg[s];
+      if (few_plan(one, 0, 0, 0, cus).mt) return 0;
+    }
+  const Q8Plan q = plan_q8(b, cus);
+  if (!q.rows) return 0;
+  if (dq) {
+    double weights = 0;
+    for (int s = 0; s < a.nseg; s++) weights += (double)a.seg[s].N * a.K;
+    if (q.us > 2 + weights * 3 / 5e6 + tiled_us(a, partial ? partial_stride : 0, partial ? max_split : 0, few_rows_floats, cus)) return 0;
+  }
+  *taken = true;
+  if (int rc = launch_gemm_q8(q, st, what)) return rc;
+  if (b.ksplit < 2) return 0;
+  launch_splitk_reduce(st, q.a);
+  return check_launch(what);
+}
+
 int launch_gemm(GemmArgs& a, bool u8, hipStream_t st, const char* what, void* dq, float* partial, size_t partial_stride,
                 int max_split, float* few_rows, size_t few_rows_floats) {
   if (a.M <= 0) return 0;
@@ -1266,20 +1143,13 @@ int launch_gemm(GemmArgs& a, bool u8, hipStream_t st, const char* what, void* dq
                          ? few_plan(a, partial ? partial_stride : 0, partial ? max_split : 0, few_ok ? few_rows_floats : 0, compute_units())
                          : FewPlan();
   if (fp.mt && few_takes(a, u8)) return launch_gemm_few(a, fp, u8, st, what);
-  bool direct = u8 && dq && a.M >= kDequantRows && a.M <= kU8DirectRows;
-  for (int s = 0; s < a.nseg; s++)  // the uint8 kernel reads codes and row scales 16 bytes at a time; the expansion takes any address
-    direct = direct && ((reinterpret_cast<uintptr_t>(a.seg[s].B) | reinterpret_cast<uintptr_t>(a.seg[s].ry) |
-                         reinterpret_cast<uintptr_t>(a.seg[s].my)) & 15) == 0;
-  if (few_ok && direct) {
+  if (u8 && !fp.mt && a.M >= kDequantRows && ldw && splitk && !force_bm) {
     bool taken = false;
-    const int rc = launch_few_rows(a, true, st, what, dq, few_rows, few_rows_floats, &taken);
+    const int rc = launch_codes(a, st, what, dq, partial, partial_stride, max_split, few_ok ? few_rows : nullptr, few_ok ? few_rows_floats : 0, &taken);
     if (taken) return rc;
   }
   if (u8 && dq && a.M >= kDequantRows) {
-    // Expanding N x K codes costs 3 bytes of traffic per weight.  The uint8 kernel's in-flight dequantisation costs a launch
-    // of many rows about 0.4 x 2 T FLOP per weight at the binary16 kernel's rate, and a launch of few rows cannot be spread
-    // over the idle compute units as the binary16 one can (few_rows below): with scratch for it, one expansion and the
-    // binary16 kernels win from a handful of rows on.
+    // Expanding N x K codes costs 3 bytes of traffic per weight, once for all strips of rows (launch_codes).
     h1* dst = static_cast<h1*>(dq);
     const unsigned char* qs[kGemmMaxSeg];
     const h1 *mxs[kGemmMaxSeg], *rxs[kGemmMaxSeg], *mys[kGemmMaxSeg], *rys[kGemmMaxSeg];
@@ -1298,7 +1168,7 @@ int launch_gemm(GemmArgs& a, bool u8, hipStream_t st, const char* what, void* dq
   }
   if (!u8 && few_ok) {
     bool taken = false;
-    const int rc = launch_few_rows(a, false, st, what, dq, few_rows, few_rows_floats, &taken);
+    const int rc = launch_few_rows(a, st, what, few_rows, few_rows_floats, &taken);
     if (taken) return rc;
   }
   int tiles = 0;
@@ -1321,11 +1191,8 @@ int launch_gemm(GemmArgs& a, bool u8, hipStream_t st, const char* what, void* dq
   // differ from the unsplit launch in the last fp32 bit before the rounding to binary16.  FRHIP_GEMM_SPLITK=0: off.
   if (!u8 && ldw && splitk && !force_bm && partial) {
     if (const int S = long_k_slices(a, partial_stride, max_split, compute_units())) {
-      a.ksplit = S;
-      a.partial = partial;
+      split_over(a, S, partial);
       a.partial_stride = partial_stride;
-      a.part_off[0] = 0;
-      a.part_off[1] = (size_t)a.M * a.seg[0].N;
       gemm_ldw_launch<128>(dim3(tiles, m128, S), st, a);
       if (int rc = check_launch(what)) return rc;
       launch_splitk_reduce(st, a);

@@ -119,4 +119,214 @@ __device__ __forceinline__ void step_barrier() {
   asm volatile("" ::: "memory");
 }
 
+// 4 bytes per lane, each lane from its own address (see load_lds_saddr for M0 and the wait counts)
+__device__ __forceinline__ void load_lds_dword(const void* p, unsigned lds) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(p), "s"(lds) : "memory");
+}
+
+// c * ry and mx + my, each rounded once to fp32, with the binary16 operand taken from its half of a register
+template <int HI>
+__device__ __forceinline__ float mul_h(float c, h2 v) {
+  float r;
+  if constexpr (HI) asm("v_fma_mix_f32 %0, %1, %2, -%3 op_sel:[0,1,0] op_sel_hi:[0,1,0]" : "=v"(r) : "v"(c), "v"(v), "s"(0.0f));
+  else asm("v_fma_mix_f32 %0, %1, %2, -%3 op_sel_hi:[0,1,0]" : "=v"(r) : "v"(c), "v"(v), "s"(0.0f));
+  return r;
+}
+template <int HI>
+__device__ __forceinline__ float add_h(float m, h2 v) {
+  float r;
+  if constexpr (HI) asm("v_fma_mix_f32 %0, 1.0, %2, %1 op_sel:[0,1,0] op_sel_hi:[0,1,0]" : "=v"(r) : "v"(m), "v"(v));
+  else asm("v_fma_mix_f32 %0, 1.0, %2, %1 op_sel_hi:[0,1,0]" : "=v"(r) : "v"(m), "v"(v));
+  return r;
+}
+
+// dequant_pair's two values, the same bits, in 9 instead of up to 13 instructions: no conversion of ry and my
+template <int HI>
+__device__ __forceinline__ h2 few_dequant(uint32_t word, float c, float mx, h2 ry, h2 my) {
+  float w0 = __builtin_fmaf((float)((word >> (HI ? 16 : 0)) & 0xffu), mul_h<0>(c, ry), add_h<0>(mx, my));
+  float w1 = __builtin_fmaf((float)((word >> (HI ? 24 : 8)) & 0xffu), mul_h<1>(c, ry), add_h<1>(mx, my));
+  asm("" : "+v"(w0), "+v"(w1));  // rounded to fp32 before the conversion (not v_fma_mixlo_f16, which rounds once)
+  return (h2){(h1)w0, (h1)w1};
+}
+
+template <int N>
+__device__ __forceinline__ void wait_loads() {  // at most N of this wave's loads outstanding
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+// An operand's K-step of 64 in LDS: 8 rows x 128 bytes are 1 KB, k-segment q of row r in slot q ^ (r % 8) ^ (r / 8 % 2)
+// (gemm.hip, "LDS layout").
+constexpr int kLdwBK = 64;
+__device__ __forceinline__ int ldw_at(int row, int q) {
+  return (row >> 3) * 1024 + (row & 7) * 128 + ((q ^ (row & 7) ^ ((row >> 3) & 1)) * 16);
+}
+
+// Workgroups are dealt to the eight XCDs in turn (linear index mod 8), each with an L2 of its own.  XCD x takes the
+// x-th eighth of the tiles, counted in blocks of four strips of rows by all N tiles, so that the 32 it runs at a time
+// share about four strips and eight N tiles.  Blocks of four N tiles by all strips, the other way round, gave the
+// tiles of a segment with a costly epilogue to one or two XCDs: the 4099-token prompt of a 1.5B model took 19.2 ms
+// so, 18.3 this way (same box, in turn; up to four strips the two are the same map).  (A matter of traffic and balance
+// only: the map is one to one, and any assignment of tiles to workgroups gives the same results.)
+__device__ __forceinline__ void xcd_tile(int& bx, int& by) {
+  const int gx = gridDim.x, gy = gridDim.y, lin = blockIdx.y * gx + blockIdx.x, n = gx * gy;
+  const int x = lin & 7, id = x * (n >> 3) + min(x, n & 7) + (lin >> 3);
+  const int blk = id / (4 * gx), rem = id - blk * 4 * gx, bw = min(4, gy - 4 * blk);
+  bx = rem / bw;
+  by = 4 * blk + rem % bw;
+}
+
+// Fused epilogues, shared by the product kernels: acc[i][j] is the 32x32 block (i, j) of the wave's
+// (32 MI) x (32 NJ) tile whose first element is (row0, col0); acc[i][j][v] is
+// C[row = 8*(v/4) + 4*(lane/32) + v%4][col = lane%32] of the block.
+// FULL: the workgroup's tile lies inside the matrix, nothing is predicated.  (With a predicate per
+// element every store becomes a branch to an out-of-line block; on the 1024 x 6144 product that
+// was 11 of 59 us.)  The epilogue kind is uniform over the launch segment: one switch, and for the
+// kinds that read operands all 16 of a block are requested before the first is used.
+template <int MI, int NJ, bool FULL>
+__device__ __forceinline__ void gemm_epilogue_t(const GemmArgs& a, const GemmSeg& sg, const f16v (&acc)[MI][NJ],
+                                                int row0, int col0, int M, int N, int lane) {
+  auto for_tile = [&](int i, int j, auto&& f) {
+    const int col = col0 + j * 32 + (lane & 31);
+#pragma unroll
+    for (int v = 0; v < 16; v++) {
+      const int row = row0 + i * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
+      if constexpr (FULL)
+        f(v, true, (size_t)row * N + col);
+      else
+        f(v, row < M && col < N, (size_t)(row < M ? row : M - 1) * N + (col < N ? col : N - 1));
+    }
+  };
+  auto for_blocks = [&](auto&& g) {
+#pragma unroll
+    for (int i = 0; i < MI; i++)
+#pragma unroll
+      for (int j = 0; j < NJ; j++) g(i, j, acc[i][j]);
+  };
+  // blocks without a stored element; only for the costly epilogues: with the test in all of them the short launches of
+  // gemm_ldw_kernel<64> took 0.4-0.8 us longer (33 x 1024 x 5120: 6.5 -> 6.9)
+  auto outside = [&](int i, int j) { return !FULL && (row0 + i * 32 >= M || col0 + j * 32 >= N); };
+  auto live_of = [&](int i, int j) {  // bit v: element v of the block lies inside the matrix
+    uint32_t m = 0;
+    for_tile(i, j, [&](int v, bool ok, size_t) { m |= ok ? 1u << v : 0u; });
+    return m;
+  };
+  switch (sg.epi) {
+    case G_STORE_F16:
+      for_blocks([&](int i, int j, const f16v& c) {
+        for_tile(i, j, [&](int v, bool ok, size_t o) { if (ok) static_cast<h1*>(sg.out)[o] = (h1)c[v]; });
+      });
+      break;
+    case G_STORE_F32:
+      for_blocks([&](int i, int j, const f16v& c) {
+        for_tile(i, j, [&](int v, bool ok, size_t o) { if (ok) static_cast<float*>(sg.out)[o] = c[v]; });
+      });
+      break;
+    case G_SIGMOID:
+      for_blocks([&](int i, int j, const f16v& c) {
+        if (outside(i, j)) return;
+        h1 y[16];
+        sigmoid_batch(c, y, live_of(i, j));
+        for_tile(i, j, [&](int v, bool ok, size_t o) { if (ok) static_cast<h1*>(sg.out)[o] = y[v]; });
+      });
+      break;
+    case G_RELU2:
+      for_blocks([&](int i, int j, const f16v& c) {
+        for_tile(i, j, [&](int v, bool ok, size_t o) {
+          const h1 t = (h1)c[v];
+          if (ok) static_cast<h1*>(sg.out)[o] = (t > (h1)0.0f) ? (t * t) : (h1)0.0f;
+        });
+      });
+      break;
+    case G_SILU:
+      for_blocks([&](int i, int j, const f16v& c) {
+        if (outside(i, j)) return;
+        h1 y[16];
+        silu_batch(c, y, live_of(i, j));
+        for_tile(i, j, [&](int v, bool ok, size_t o) { if (ok) static_cast<h1*>(sg.out)[o] = y[v]; });
+      });
+      break;
+    case G_RESIDUAL:
+      for_blocks([&](int i, int j, const f16v& c) {
+        h1 rx[16];
+        for_tile(i, j, [&](int v, bool, size_t o) { rx[v] = a.res_x[o]; });
+        for_tile(i, j, [&](int v, bool ok, size_t o) { if (ok) static_cast<h1*>(sg.out)[o] = rx[v] + (h1)c[v]; });
+      });
+      break;
+    case G_FFN_OUT:
+      for_blocks([&](int i, int j, const f16v& c) {
+        h1 rx[16], rr[16];
+        for_tile(i, j, [&](int v, bool, size_t o) {
+          rx[v] = a.res_x[o];
+          rr[v] = a.res_r[o];
+        });
+        for_tile(i, j, [&](int v, bool ok, size_t o) {
+          h1 r = __builtin_fmaf16((h1)c[v], rr[v], rx[v]);
+          if (a.div2) r = r / (h1)2.0f;
+          if (ok) static_cast<h1*>(sg.out)[o] = r;
+        });
+      });
+      break;
+    default: break;
+  }
+}
+
+// The epilogue of W consecutive outputs of a row, a multiple of 8, whose sums are in `acc`; o: their place in [M][N]
+template <int W>
+__device__ __forceinline__ void store_row(const GemmArgs& a, const GemmSeg& sg, const float (&acc)[W], size_t o) {
+  if (sg.epi == G_STORE_F32) {
+    float* out = static_cast<float*>(sg.out) + o;
+#pragma unroll
+    for (int q = 0; q < W / 4; q++) {
+      f4v v;
+#pragma unroll
+      for (int i = 0; i < 4; i++) v[i] = acc[4 * q + i];
+      *reinterpret_cast<f4v*>(out + 4 * q) = v;
+    }
+    return;
+  }
+  h1 y[W];
+  switch (sg.epi) {
+    case G_STORE_F16:
+#pragma unroll
+      for (int i = 0; i < W; i++) y[i] = (h1)acc[i];
+      break;
+    case G_SIGMOID: sigmoid_batch(acc, y, (1u << W) - 1); break;
+    case G_SILU: silu_batch(acc, y, (1u << W) - 1); break;
+    case G_RELU2:
+#pragma unroll
+      for (int i = 0; i < W; i++) {
+        const h1 t = (h1)acc[i];
+        y[i] = (t > (h1)0.0f) ? (t * t) : (h1)0.0f;
+      }
+      break;
+    case G_RESIDUAL:
+#pragma unroll
+      for (int g = 0; g < W / 8; g++) {
+        const h8 x = *reinterpret_cast<const h8*>(a.res_x + o + 8 * g);
+#pragma unroll
+        for (int i = 0; i < 8; i++) y[8 * g + i] = x[i] + (h1)acc[8 * g + i];
+      }
+      break;
+    default:  // G_FFN_OUT
+#pragma unroll
+      for (int g = 0; g < W / 8; g++) {
+        const h8 x = *reinterpret_cast<const h8*>(a.res_x + o + 8 * g), r = *reinterpret_cast<const h8*>(a.res_r + o + 8 * g);
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+          h1 v = __builtin_fmaf16((h1)acc[8 * g + i], r[i], x[i]);
+          if (a.div2) v = v / (h1)2.0f;
+          y[8 * g + i] = v;
+        }
+      }
+      break;
+  }
+#pragma unroll
+  for (int g = 0; g < W / 8; g++) {
+    h8 v;
+#pragma unroll
+    for (int i = 0; i < 8; i++) v[i] = y[8 * g + i];
+    *reinterpret_cast<h8*>(static_cast<h1*>(sg.out) + o + 8 * g) = v;
+  }
+}
+
 }  // namespace frhip

@@ -40,41 +40,6 @@ constexpr int few_stages(int mt, int nt, bool u8) {
 }
 constexpr int few_wave_bytes(int mt, int nt, bool u8) { return few_stages(mt, nt, u8) * few_stage_bytes(mt, nt, u8) + (u8 ? kFewScaleBytes : 0); }
 
-// 4 bytes per lane, each lane from its own address (see load_lds_saddr for M0 and the wait counts)
-__device__ __forceinline__ void load_lds_dword(const void* p, unsigned lds) {
-  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(p), "s"(lds) : "memory");
-}
-
-// c * ry and mx + my, each rounded once to fp32, with the binary16 operand taken from its half of a register
-template <int HI>
-__device__ __forceinline__ float mul_h(float c, h2 v) {
-  float r;
-  if constexpr (HI) asm("v_fma_mix_f32 %0, %1, %2, -%3 op_sel:[0,1,0] op_sel_hi:[0,1,0]" : "=v"(r) : "v"(c), "v"(v), "s"(0.0f));
-  else asm("v_fma_mix_f32 %0, %1, %2, -%3 op_sel_hi:[0,1,0]" : "=v"(r) : "v"(c), "v"(v), "s"(0.0f));
-  return r;
-}
-template <int HI>
-__device__ __forceinline__ float add_h(float m, h2 v) {
-  float r;
-  if constexpr (HI) asm("v_fma_mix_f32 %0, 1.0, %2, %1 op_sel:[0,1,0] op_sel_hi:[0,1,0]" : "=v"(r) : "v"(m), "v"(v));
-  else asm("v_fma_mix_f32 %0, 1.0, %2, %1 op_sel_hi:[0,1,0]" : "=v"(r) : "v"(m), "v"(v));
-  return r;
-}
-
-// dequant_pair's two values, the same bits, in 9 instead of up to 13 instructions: no conversion of ry and my
-template <int HI>
-__device__ __forceinline__ h2 few_dequant(uint32_t word, float c, float mx, h2 ry, h2 my) {
-  float w0 = __builtin_fmaf((float)((word >> (HI ? 16 : 0)) & 0xffu), mul_h<0>(c, ry), add_h<0>(mx, my));
-  float w1 = __builtin_fmaf((float)((word >> (HI ? 24 : 8)) & 0xffu), mul_h<1>(c, ry), add_h<1>(mx, my));
-  asm("" : "+v"(w0), "+v"(w1));  // rounded to fp32 before the conversion (not v_fma_mixlo_f16, which rounds once)
-  return (h2){(h1)w0, (h1)w1};
-}
-
-template <int N>
-__device__ __forceinline__ void wait_loads() {  // at most N of this wave's loads outstanding
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-
 // A tile of 16 rows x 64 binary16: rows of 128 bytes, k-segment q (8 halves) of row r in slot q ^ (r % 8) ^ (r / 8)
 // (the layout of gemm_ldw_kernel: fragment reads of 16 rows are free of bank conflicts)
 __device__ __forceinline__ int few_at(int r, int q) { return r * 128 + ((q ^ (r & 7) ^ (r >> 3)) * 16); }

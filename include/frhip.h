@@ -311,6 +311,9 @@ int frhip_gemm_route(int T, int K, int nproducts, const int *N, int compute_unit
  * instead, to the kernel for a few rows (K split over the waves of a workgroup), and with which tile: out[0], out[1] = blocks
  * of 16 rows and of 16 columns of a workgroup, 0, 0 if it is cut as above.  A pure function of the sizes too. */
 int frhip_gemm_few_tile(int T, int K, int nproducts, const int *N, int compute_units, int *out);
+/* The tile of such a launch of uint8 products that dequantises the codes on their way into LDS, with K in `slices` slices: out[0],
+ * out[1], out[2] = its rows, its widest tile in blocks of 32 columns, its rounds; 0, 0, 0 if it cannot be one. */
+int frhip_gemm_q8_tile(int T, int K, int nproducts, const int *N, int slices, int compute_units, int *out);
 /* The form that a launch of the seq operators (uint8: of 4 rows and more) takes, with their scratch, for addresses that suit
  * every form (allocations do).  `which`: 0, or FRHIP_SEQ_V4 for frhip_att_seq_v4's and frhip_ffn_seq_v4's, plus
  * FRHIP_SEQ_FFN_VALUE for the value product of ffn_seq.  Returns the form or a negative FRHIP_E*.  out[0], out[1]:
