@@ -388,7 +388,10 @@ __device__ __forceinline__ void splitk_reduce_body(const GemmArgs& a, const Gemm
 #pragma unroll
           for (int i = 0; i < 4; i++) acc[4 * q + i] += p[j][q][i];
   }
-  store_row<W>(a, sg, acc, o);
+  size_t at[W / 8];
+#pragma unroll
+  for (int g = 0; g < W / 8; g++) at[g] = o + 8 * g;
+  store_groups<W / 8>(a, sg, acc, at);
 }
 
 template <int W>
@@ -516,9 +519,10 @@ __device__ __forceinline__ void vw_loader(const GemmSeg& sg, unsigned char* smem
 }
 
 template <int BM, int NJ>
-__device__ __forceinline__ void vw_mma(const GemmArgs& a, const GemmSeg& sg, const unsigned char* smem, int stage_bytes, int ns,
-                                       int brow0, int m0, int n0, int M, int N, bool full, int lane, int wm) {
+__device__ __forceinline__ void vw_mma(const GemmArgs& a, const GemmSeg& sg, unsigned char* smem, int stage_bytes, int ns,
+                                       int brow0, int m0, int n0, int M, int N, bool full, int lane, int wave) {
   constexpr int kVwABytes = BM * kLdwBK * 2;
+  const int wm = wave >> 1;
   f16v acc[2][NJ];
 #pragma unroll
   for (int i = 0; i < 2; i++)
@@ -556,10 +560,12 @@ __device__ __forceinline__ void vw_mma(const GemmArgs& a, const GemmSeg& sg, con
             acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[kb][i], fb[kb][j], acc[i][j], 0, 0, 0);
     }
   }
-  if (BM == 256 || full)  // 256 rows: whole tiles only
+  if (BM == 256 || full) {  // 256 rows: whole tiles only
     gemm_epilogue_t<2, NJ, true>(a, sg, acc, m0 + wm * 64, n0 + brow0, M, N, lane);
-  else
-    gemm_epilogue_t<2, NJ, false>(a, sg, acc, m0 + wm * 64, n0 + brow0, M, N, lane);
+  } else {
+    step_barrier();  // all fragments have been read
+    finish_wave(a, sg, acc, reinterpret_cast<float*>(smem + wave * wave_sums_bytes((a.vw_maxw + 1) / 2)), m0 + wm * 64, n0 + brow0, M, N, lane);
+  }
 }
 
 // BM / 32 MFMA waves of 64 rows x half the width, then the loader.  BM = 256: launches of whole tiles of at most
@@ -583,6 +589,7 @@ __global__ __launch_bounds__(BM * 2 + 64) void gemm_vw_kernel(GemmArgs a) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int stage_bytes = kVwABytes + a.vw_maxw * 4096, ns = a.vw_ns;
+  const bool full = m0 + BM <= M && n0 + width * 32 <= N;
   if (wave == kLoader) {
     switch (width) {
       case 2: vw_loader<BM, 2>(sg, gemm_smem, stage_bytes, ns, m0, n0, M, N, K, lane); break;
@@ -593,18 +600,18 @@ __global__ __launch_bounds__(BM * 2 + 64) void gemm_vw_kernel(GemmArgs a) {
       case 7: vw_loader<BM, kCap < 7 ? kCap : 7>(sg, gemm_smem, stage_bytes, ns, m0, n0, M, N, K, lane); break;
       default: vw_loader<BM, kCap>(sg, gemm_smem, stage_bytes, ns, m0, n0, M, N, K, lane); break;
     }
+    if (BM == 128 && !full) step_barrier();
     return;
   }
-  const int wm = wave >> 1, wn = wave & 1;
+  const int wn = wave & 1;
   const int nj0 = (width + 1) >> 1;
   const int nj = wn ? width - nj0 : nj0;
   const int brow0 = wn ? nj0 * 32 : 0;
-  const bool full = m0 + BM <= M && n0 + width * 32 <= N;
   switch (nj) {
-    case 1: vw_mma<BM, 1>(a, sg, gemm_smem, stage_bytes, ns, brow0, m0, n0, M, N, full, lane, wm); break;
-    case 2: vw_mma<BM, 2>(a, sg, gemm_smem, stage_bytes, ns, brow0, m0, n0, M, N, full, lane, wm); break;
-    case 3: vw_mma<BM, 3>(a, sg, gemm_smem, stage_bytes, ns, brow0, m0, n0, M, N, full, lane, wm); break;
-    default: vw_mma<BM, (kCap + 1) / 2>(a, sg, gemm_smem, stage_bytes, ns, brow0, m0, n0, M, N, full, lane, wm); break;
+    case 1: vw_mma<BM, 1>(a, sg, gemm_smem, stage_bytes, ns, brow0, m0, n0, M, N, full, lane, wave); break;
+    case 2: vw_mma<BM, 2>(a, sg, gemm_smem, stage_bytes, ns, brow0, m0, n0, M, N, full, lane, wave); break;
+    case 3: vw_mma<BM, 3>(a, sg, gemm_smem, stage_bytes, ns, brow0, m0, n0, M, N, full, lane, wave); break;
+    default: vw_mma<BM, (kCap + 1) / 2>(a, sg, gemm_smem, stage_bytes, ns, brow0, m0, n0, M, N, full, lane, wave); break;
   }
 }
 
@@ -684,10 +691,12 @@ __device__ __forceinline__ void vw256_body(const GemmArgs& a, const GemmSeg& sg,
         for (int j = 0; j < NJ; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[i], fb[j], acc[i][j], 0, 0, 0);
     }
   }
-  if (m0 + 256 <= M && n0 + width * 32 <= N)
+  if (m0 + 256 <= M && n0 + width * 32 <= N) {
     gemm_epilogue_t<2, NJ, true>(a, sg, acc, m0 + wm * 64, n0 + brow0, M, N, lane);
-  else
-    gemm_epilogue_t<2, NJ, false>(a, sg, acc, m0 + wm * 64, n0 + brow0, M, N, lane);
+  } else {
+    step_barrier();  // all fragments have been read
+    finish_wave(a, sg, acc, reinterpret_cast<float*>(smem + wave * wave_sums_bytes((a.vw_maxw + 1) / 2)), m0 + wm * 64, n0 + brow0, M, N, lane);
+  }
 }
 
 __global__ __launch_bounds__(kVw256Threads) void gemm_vw256_kernel(GemmArgs a) {
@@ -821,6 +830,8 @@ static GemmRoute plan_vw(const GemmArgs& args, int bm, int cus) {
     a.vw_ns = !r.loader ? 2 : stage * 4 <= 160 * 1024 ? 4 : 3;
     if (stage * a.vw_ns > 160 * 1024) return r;
     r.lds = stage * a.vw_ns;
+    const size_t sums = (size_t)(bm / 32) * wave_sums_bytes((maxw + 1) / 2);  // the epilogue's place (finish_wave)
+    if (r.lds < sums) r.lds = sums;
     r.grid = dim3(tiles, mt);
     r.blocks = maxw;
     r.rounds = (int)rounds;

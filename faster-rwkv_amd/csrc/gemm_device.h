@@ -270,28 +270,49 @@ __device__ __forceinline__ void gemm_epilogue_t(const GemmArgs& a, const GemmSeg
   }
 }
 
-// The epilogue of W consecutive outputs of a row, a multiple of 8, whose sums are in `acc`; o: their place in [M][N]
-template <int W>
-__device__ __forceinline__ void store_row(const GemmArgs& a, const GemmSeg& sg, const float (&acc)[W], size_t o) {
+// The epilogue of G groups of eight consecutive outputs of a row, whose sums are in `acc`; o: the groups' places in [M][N].  VEC:
+// operands and outputs go 16 bytes at a time; otherwise one at a time, the first n of every group.
+template <int G, bool VEC = true>
+__device__ __forceinline__ void store_groups(const GemmArgs& a, const GemmSeg& sg, const float (&acc)[8 * G], const size_t (&o)[G], int n = 8) {
+  constexpr int W = 8 * G;
   if (sg.epi == G_STORE_F32) {
-    float* out = static_cast<float*>(sg.out) + o;
 #pragma unroll
-    for (int q = 0; q < W / 4; q++) {
-      f4v v;
+    for (int g = 0; g < G; g++) {
+      float* out = static_cast<float*>(sg.out) + o[g];
+      if constexpr (VEC) {
 #pragma unroll
-      for (int i = 0; i < 4; i++) v[i] = acc[4 * q + i];
-      *reinterpret_cast<f4v*>(out + 4 * q) = v;
+        for (int q = 8 * g; q < 8 * g + 8; q += 4) *reinterpret_cast<f4v*>(out + q - 8 * g) = (f4v){acc[q], acc[q + 1], acc[q + 2], acc[q + 3]};
+      } else {
+#pragma unroll
+        for (int i = 0; i < 8; i++)
+          if (i < n) out[i] = acc[8 * g + i];
+      }
     }
     return;
   }
-  h1 y[W];
+  auto operand = [&](const h1* p, h1 (&v)[W]) {
+#pragma unroll
+    for (int g = 0; g < G; g++) {
+      if constexpr (VEC) {
+        const h8 t = *reinterpret_cast<const h8*>(p + o[g]);
+#pragma unroll
+        for (int i = 0; i < 8; i++) v[8 * g + i] = t[i];
+      } else {
+#pragma unroll
+        for (int i = 0; i < 8; i++) v[8 * g + i] = i < n ? p[o[g] + i] : (h1)0.0f;
+      }
+    }
+  };
+  static_assert(VEC || G == 1, "one bound for one group");
+  const uint32_t live = VEC ? (1u << W) - 1 : (1u << n) - 1;
+  h1 y[W], x[W], r[W];
   switch (sg.epi) {
     case G_STORE_F16:
 #pragma unroll
       for (int i = 0; i < W; i++) y[i] = (h1)acc[i];
       break;
-    case G_SIGMOID: sigmoid_batch(acc, y, (1u << W) - 1); break;
-    case G_SILU: silu_batch(acc, y, (1u << W) - 1); break;
+    case G_SIGMOID: sigmoid_batch(acc, y, live); break;
+    case G_SILU: silu_batch(acc, y, live); break;
     case G_RELU2:
 #pragma unroll
       for (int i = 0; i < W; i++) {
@@ -300,32 +321,119 @@ __device__ __forceinline__ void store_row(const GemmArgs& a, const GemmSeg& sg, 
       }
       break;
     case G_RESIDUAL:
+      operand(a.res_x, x);
 #pragma unroll
-      for (int g = 0; g < W / 8; g++) {
-        const h8 x = *reinterpret_cast<const h8*>(a.res_x + o + 8 * g);
-#pragma unroll
-        for (int i = 0; i < 8; i++) y[8 * g + i] = x[i] + (h1)acc[8 * g + i];
-      }
+      for (int i = 0; i < W; i++) y[i] = x[i] + (h1)acc[i];
       break;
     default:  // G_FFN_OUT
+      operand(a.res_x, x);
+      operand(a.res_r, r);
 #pragma unroll
-      for (int g = 0; g < W / 8; g++) {
-        const h8 x = *reinterpret_cast<const h8*>(a.res_x + o + 8 * g), r = *reinterpret_cast<const h8*>(a.res_r + o + 8 * g);
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-          h1 v = __builtin_fmaf16((h1)acc[8 * g + i], r[i], x[i]);
-          if (a.div2) v = v / (h1)2.0f;
-          y[8 * g + i] = v;
-        }
+      for (int i = 0; i < W; i++) {
+        y[i] = __builtin_fmaf16((h1)acc[i], r[i], x[i]);
+        if (a.div2) y[i] = y[i] / (h1)2.0f;
       }
       break;
   }
 #pragma unroll
-  for (int g = 0; g < W / 8; g++) {
-    h8 v;
+  for (int g = 0; g < G; g++) {
+    h1* out = static_cast<h1*>(sg.out) + o[g];
+    if constexpr (VEC) {
+      h8 v;
 #pragma unroll
-    for (int i = 0; i < 8; i++) v[i] = y[8 * g + i];
-    *reinterpret_cast<h8*>(static_cast<h1*>(sg.out) + o + 8 * g) = v;
+      for (int i = 0; i < 8; i++) v[i] = y[8 * g + i];
+      *reinterpret_cast<h8*>(out) = v;
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8; i++)
+        if (i < n) out[i] = y[8 * g + i];
+    }
+  }
+}
+
+// The end of a tile through LDS (where the operands were): an output row goes out 16 bytes a lane instead of one element a lane and
+// instruction, and a lane holds eight or sixteen sums at a time instead of its whole part of the tile.
+// Rows of sums are `pitch` floats apart: 32 columns a block and 4 more.
+__host__ __device__ constexpr int sums_pitch(int blocks) { return 32 * blocks + 4; }
+
+// One row of 32 x 32 blocks of a wave's sums: acc[j][v] is C[row = 8 * (v / 4) + 4 * (lane / 32) + v % 4][col = lane % 32] of block j.
+template <int NJ>
+__device__ __forceinline__ void sums_to_lds(const f16v (&acc)[NJ], float* sums, int pitch, int lane) {
+  float* const p = sums + 4 * (lane >> 5) * pitch + (lane & 31);
+#pragma unroll
+  for (int j = 0; j < NJ; j++)
+#pragma unroll
+    for (int v = 0; v < 16; v++) p[(8 * (v >> 2) + (v & 3)) * pitch + j * 32] = acc[j][v];
+}
+
+__device__ __forceinline__ bool vec_outputs(const GemmArgs& a, const GemmSeg& sg) {  // rows of outputs and operands, 16 bytes at a time
+  return (sg.N & 7) == 0 && ((reinterpret_cast<uintptr_t>(sg.out) | reinterpret_cast<uintptr_t>(a.res_x) |
+                              reinterpret_cast<uintptr_t>(a.res_r)) & 15) == 0;
+}
+
+__device__ __forceinline__ void read_sums(float (&s)[8], const float* sums) {
+#pragma unroll
+  for (int h = 0; h < 2; h++) {
+    const f4v v = *reinterpret_cast<const f4v*>(sums + 4 * h);
+#pragma unroll
+    for (int t = 0; t < 4; t++) s[4 * h + t] = v[t];
+  }
+}
+
+// Eight sums of row `row` from column `col`, which may lie outside the matrix
+__device__ __forceinline__ void finish_group(const GemmArgs& a, const GemmSeg& sg, const float* sums, bool vec, int row, int col, int M, int N) {
+  if (row >= M || col >= N) return;
+  float s[8];
+  read_sums(s, sums);
+  const size_t o[1] = {(size_t)row * N + col};
+  if (vec) store_groups<1>(a, sg, s, o);
+  else store_groups<1, false>(a, sg, s, o, min(8, N - col));
+}
+
+// A wave's part of a tile, from row row0 and column col0, through a place in LDS of its own, 32 rows at a time: no barriers, and
+// only the rows that follow stay in registers.  For tiles over the edge of the matrix, where a predicate per element makes every
+// store of gemm_epilogue_t a branch: 300 x 2560 x (2560 + 8960) 49.3 -> 43.7 us, 1000 x 2048 x (3 x 2048) 46.7 -> 42.5, 1000 x 768 x
+// (3 x 768) 20.1 -> 16.8.  Whole tiles store straight from the accumulators: 4099 x 2048 x (3 x 2048) 129 us, 136 through LDS.
+constexpr int wave_sums_bytes(int blocks) { return 32 * sums_pitch(blocks) * 4; }
+template <int MI, int NJ>
+__device__ __forceinline__ void finish_wave(const GemmArgs& a, const GemmSeg& sg, const f16v (&acc)[MI][NJ], float* sums, int row0,
+                                            int col0, int M, int N, int lane) {
+  const bool vec = vec_outputs(a, sg), full = vec && row0 + MI * 32 <= M && col0 + NJ * 32 <= N;
+#pragma unroll
+  for (int i = 0; i < MI; i++) {
+    sums_to_lds(acc[i], sums, sums_pitch(NJ), lane);
+    if (full) {
+#pragma unroll 1
+      for (int t = lane; t < 32 * NJ * 4; t += 128) {
+        float s[16];
+        size_t o[2];
+#pragma unroll
+        for (int g = 0; g < 2; g++) {
+          const int row = (t + 64 * g) / (NJ * 4), col = (t + 64 * g - row * (NJ * 4)) * 8;
+          read_sums(*reinterpret_cast<float(*)[8]>(s + 8 * g), sums + row * sums_pitch(NJ) + col);
+          o[g] = (size_t)(row0 + i * 32 + row) * N + col0 + col;
+        }
+        store_groups<2>(a, sg, s, o);
+      }
+      continue;
+    }
+#pragma unroll 1
+    for (int t = lane; t < 32 * NJ * 4; t += 64) {
+      const int row = t / (NJ * 4), col = (t - row * (NJ * 4)) * 8;
+      finish_group(a, sg, sums + row * sums_pitch(NJ) + col, vec, row0 + i * 32 + row, col0 + col, M, N);
+    }
+  }
+}
+
+// A tile of ROWS rows and `blocks` blocks of 32 columns, shared by all waves of the workgroup
+template <int ROWS, int THREADS>
+__device__ __forceinline__ void finish_tile(const GemmArgs& a, const GemmSeg& sg, const float* sums, int pitch, int blocks, int m0,
+                                            int n0, int M, int N) {
+  const int groups = blocks * 4;  // of 8 outputs
+  const bool vec = vec_outputs(a, sg);
+  for (int i = threadIdx.x; i < ROWS * groups; i += THREADS) {
+    const int row = i / groups, col = (i - row * groups) * 8;
+    finish_group(a, sg, sums + row * pitch + col, vec, m0 + row, n0 + col, M, N);
   }
 }
 

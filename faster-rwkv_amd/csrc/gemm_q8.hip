@@ -37,9 +37,8 @@ __host__ __device__ constexpr int q8_blocks_before(int p, int w) {
 }
 __host__ __device__ constexpr int q8_producer_at(int p, int w) { return kQ8Codes * (q8_blocks_before(p, w) * 1024 + p * 256) + p * 256; }
 constexpr int q8_lds_bytes(int bm, int w) { return kQ8Stages * bm * 128 + 2 * w * 4096 + q8_producer_at(kQ8Producers, w); }
-__host__ __device__ constexpr int q8_pitch(int w) { return 32 * w + 4; }  // floats of a row of sums
-static_assert(128 * q8_pitch(6) * 4 <= q8_lds_bytes(128, 6) && 128 * q8_pitch(2) * 4 <= q8_lds_bytes(128, 2) &&
-                  64 * q8_pitch(8) * 4 <= q8_lds_bytes(64, 8) && 64 * q8_pitch(2) * 4 <= q8_lds_bytes(64, 2), "the sums fit");
+static_assert(128 * sums_pitch(6) * 4 <= q8_lds_bytes(128, 6) && 128 * sums_pitch(2) * 4 <= q8_lds_bytes(128, 2) &&
+                  64 * sums_pitch(8) * 4 <= q8_lds_bytes(64, 8) && 64 * sums_pitch(2) * 4 <= q8_lds_bytes(64, 2), "the sums fit");
 static_assert(q8_lds_bytes(128, q8_max_blocks(128)) <= 160 * 1024 && q8_lds_bytes(64, q8_max_blocks(64)) <= 160 * 1024, "LDS of a compute unit");
 
 // few_dequant's two values, the same bits, in 8 instructions: a code in the low byte of a binary16 is the subnormal q 2^-24, which
@@ -224,15 +223,9 @@ __device__ __forceinline__ void q8_mma(unsigned char* smem, int maxw, int brow0,
     }
   }
   step_barrier();  // all fragments have been read
-  const int pitch = q8_pitch(maxw);
-  float* const sums = reinterpret_cast<float*>(smem);
+  const int pitch = sums_pitch(maxw);
 #pragma unroll
-  for (int i = 0; i < MI; i++)
-#pragma unroll
-    for (int j = 0; j < NJ; j++)
-#pragma unroll
-      for (int v = 0; v < 16; v++)
-        sums[(wm * (BM / 2) + i * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3)) * pitch + brow0 + j * 32 + (lane & 31)] = acc[i][j][v];
+  for (int i = 0; i < MI; i++) sums_to_lds(acc[i], reinterpret_cast<float*>(smem) + (wm * (BM / 2) + i * 32) * pitch + brow0, pitch, lane);
 }
 
 template <int BM>
@@ -270,26 +263,12 @@ __global__ __launch_bounds__(64 * (4 + kQ8Producers)) void gemm_q8_kernel(GemmAr
       default: q8_mma<BM, q8_max_blocks(BM) / 2>(q8_smem, a.vw_maxw, brow0, nk, lane, wm); break;
     }
   }
-  // The sums go through LDS, so that all waves share the epilogue and store 16 bytes a lane.
   __syncthreads();
   if (a.ksplit > 1) {  // this slice's sums go out as fp32; the epilogue proper follows in gemm_splitk_reduce_kernel
     sg.out = a.partial + (size_t)kz * a.partial_stride + a.part_off[sidx];
     sg.epi = G_STORE_F32;
   }
-  const int pitch = q8_pitch(a.vw_maxw), groups = width * 4;  // of 8 outputs
-  const float* const sums = reinterpret_cast<const float*>(q8_smem);
-  for (int i = threadIdx.x; i < BM * groups; i += 64 * (4 + kQ8Producers)) {
-    const int row = i / groups, col = (i - row * groups) * 8;
-    if (m0 + row >= a.M || n0 + col >= sg.N) continue;
-    float s[8];
-#pragma unroll
-    for (int h = 0; h < 2; h++) {
-      const f4v v = *reinterpret_cast<const f4v*>(sums + row * pitch + col + 4 * h);
-#pragma unroll
-      for (int t = 0; t < 4; t++) s[4 * h + t] = v[t];
-    }
-    store_row<8>(a, sg, s, (size_t)(m0 + row) * sg.N + n0 + col);
-  }
+  finish_tile<BM, 64 * (4 + kQ8Producers)>(a, sg, reinterpret_cast<const float*>(q8_smem), sums_pitch(a.vw_maxw), width, m0, n0, a.M, sg.N);
 }
 
 // What a launch of such tiles is expected to take, us: fitted to 1793 measured ones (13 to 1536 rows, widths 1024 to 4096, the
@@ -336,11 +315,11 @@ Q8Plan plan_q8(const GemmArgs& args, int cus) {
   return best;
 }
 
-// codes, residual operands and outputs go 16 bytes at a time, rows' and columns' scales 4
+// codes are loaded 16 bytes at a time, rows' and columns' scales 4
 bool q8_takes(const GemmArgs& a) {
-  uintptr_t v16 = reinterpret_cast<uintptr_t>(a.res_x) | reinterpret_cast<uintptr_t>(a.res_r), v4 = 0;
+  uintptr_t v16 = 0, v4 = 0;
   for (int s = 0; s < a.nseg; s++) {
-    v16 |= reinterpret_cast<uintptr_t>(a.seg[s].A) | reinterpret_cast<uintptr_t>(a.seg[s].B) | reinterpret_cast<uintptr_t>(a.seg[s].out);
+    v16 |= reinterpret_cast<uintptr_t>(a.seg[s].A) | reinterpret_cast<uintptr_t>(a.seg[s].B);
     for (const h1* p : {a.seg[s].mx, a.seg[s].rx, a.seg[s].my, a.seg[s].ry}) v4 |= reinterpret_cast<uintptr_t>(p);
   }
   return (v16 & 15) == 0 && (v4 & 3) == 0;

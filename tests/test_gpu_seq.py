@@ -95,6 +95,34 @@ def test_gemm_planned_tiles_against_oracle(T, K, N):
     assert np.abs(y.numpy() - ref).max() <= 3e-6 * np.sqrt(K) * np.abs(ref).max() + 1e-5
 
 
+@pytest.mark.parametrize("T,N,shift", [(300, 16384, 0), (257, 16376, 0), (300, 16377, 0), (385, 16384, 4), (513, 16377, 0), (769, 16348, 0),
+                                       (1000, 16384, 2)])
+def test_tiles_over_the_edge_give_the_bits_of_whole_ones(T, N, shift):
+    """Rows and columns that end inside a tile of 128 or 256 rows, outputs at any address (`shift` bytes past a multiple of 16),
+    against the same outputs of a product of whole tiles; nothing is written beside them."""
+    K, M, W = 192, 1024, 16384
+    x, w = h(rng.standard_normal((M, K))), h(rng.standard_normal((K, W)) * 0.3)
+    xd, whole, part = keep(x), make_weight(w, False)[0], make_weight(np.ascontiguousarray(w[:, :N]), False)[0]
+    tile = (C.c_int * 2)()
+    fr.check(L().frhip_gemm_few_tile(T, K, 1, (C.c_int * 1)(N), 256, tile))
+    assert _routes(T, K, N)[1][0][0] in (128, 256) and tuple(tile) == (0, 0)
+
+    def run(pw, T, N, shift, dt, act):
+        lead = shift // dt().itemsize
+        y = keep(np.full(lead + T * N + 16, 7.5, dt))
+        if act:
+            fr.check(L().frhip_gemm_act(xd.ptr, pw.ref, y.ptr + shift, T, act, None))
+        else:
+            fr.check(L().frhip_gemm(xd.ptr, pw.ref, y.ptr + shift, T, fr.F32 if dt is np.float32 else fr.F16, None))
+        got = y.numpy()
+        assert (got[:lead] == 7.5).all() and (got[lead + T * N:] == 7.5).all()
+        return got[lead:lead + T * N].reshape(T, N)
+
+    for dt, act in ((np.float32, 0), (np.float16, 0), (np.float16, 2), (np.float16, 3), (np.float16, 4)):
+        want = np.ascontiguousarray(run(whole, M, W, 0, dt, act)[:T, :N])
+        assert np.array_equal(np.ascontiguousarray(run(part, T, N, shift - shift % dt().itemsize, dt, act)).view(np.uint8), want.view(np.uint8))
+
+
 def test_gemm_sigmoid_and_silu_epilogues_every_binary16_bit_exact():
     """Every finite binary16 value goes through the product's sigmoid epilogue (identity weight, so the
     accumulator is the input exactly) and must come out as the oracle's double-evaluated sigmoid (and its silu), bit for bit;
