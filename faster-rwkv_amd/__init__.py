@@ -105,6 +105,7 @@ _SIGS = {
     "frhip_gemm_act": (_i, [_vp, _WP, _vp, _i, _i, _vp]),
     "frhip_gemm_route": (_i, [_i, _i, _i, _vp, _i, _vp]),
     "frhip_wkv4_cut": (_i, [_i, _i, _i, _vp]),
+    "frhip_gemm_ring_tile": (_i, [_i, _i, _i, _vp, _i, _i, _vp]),
     "frhip_gemm_q8_tile": (_i, [_i, _i, _i, _vp, _i, _i, _vp]),
     "frhip_gemm_few_tile": (_i, [_i, _i, _i, _vp, _i, _vp]),
     "frhip_seq_gemm_form": (_i, [_i, _i, _i, _vp, _i, _i, _vp]),

@@ -79,17 +79,21 @@ bool few_takes(const GemmArgs& a, bool u8);
 int launch_gemm_few(const GemmArgs& a, const FewPlan& p, bool u8, hipStream_t st, const char* what);
 // Deals `tiles` workgroups of a strip of rows to the segments by their columns: tile_start, vw_base, vw_wide, vw_maxw.  False: too few.
 bool deal_tiles(GemmArgs& a, int tiles);
-// Products of uint8 weights that dequantise the codes on their way into LDS (gemm_q8.hip), with the tile that is expected to be
-// the quickest; rows = 0: not a launch of this form.  a.ksplit, partial and part_off as for gemm_ldw_kernel.
-struct Q8Plan {
+// A launch of tiles of `rows` rows and widths of its own per segment: with the cut that is expected to be the quickest; rows = 0: not
+// a launch of the form.  a.ksplit, partial and part_off: slices of K, whose sums go there as fp32.
+struct TilePlan {
   int rows = 0, rounds = 0;
   double us = 0;
   dim3 grid;
   GemmArgs a;
 };
-Q8Plan plan_q8(const GemmArgs& a, int cus);
+// binary16 weights, four loading waves (gemm_ring.hip)
+TilePlan plan_ring(const GemmArgs& a, int cus);
+int launch_gemm_ring(const TilePlan& p, hipStream_t st, const char* what);
+// uint8 weights whose codes are dequantised on their way into LDS (gemm_q8.hip)
+TilePlan plan_q8(const GemmArgs& a, int cus);
 bool q8_takes(const GemmArgs& a);
-int launch_gemm_q8(const Q8Plan& p, hipStream_t st, const char* what);
+int launch_gemm_q8(const TilePlan& p, hipStream_t st, const char* what);
 constexpr int kDequantRows = FRHIP_SEQ_EXPAND_ROWS;
 // uint8 [N][K] -> binary16 [N][K] with the frozen formula (ops.hip)
 int dequant_u8_async(const unsigned char* q, const h1* mx, const h1* rx, const h1* my, const h1* ry, h1* dst, int K, int N,

@@ -4,23 +4,18 @@
 //
 // Both operands are K-contiguous, which is the layout v_mfma_f32_32x32x16_f16 wants:
 // a lane's A (or B) fragment is 8 consecutive k of one row, i.e. one 16-byte load.
-// Workgroup tile 128x128 (64x128 for launches that would otherwise leave CUs idle), 2x2 compute
-// waves of 64x64 (2x2 MFMA tiles, 64 fp32 accumulators per lane).  Four kernels:
-//   gemm_vw_kernel   binary16 weights, launches large enough for tiles of 128 x 96 and more:
-//                    tile widths are chosen per launch so that the workgroups fill the compute
-//                    units in whole rounds; loader wave and LDS ring as in gemm_ldw_kernel;
-//                    (128 rows; 256 rows where all tiles are whole and narrow)
-//   gemm_vw256_kernel  tiles of 256 rows and eight waves that load and multiply;
-//   gemm_ldw_kernel  binary16 weights: a fifth wave streams the tiles global -> LDS directly
-//                    through a ring of four 64-deep K steps; the compute waves never load;
-//   gemm_kernel      uint8 weights: tiles go global -> registers -> LDS (rows padded by 16 bytes
-//                    against bank conflicts), the loads of step k+1 issued before the MFMAs of
-//                    step k, and are dequantised to binary16 on the way into LDS with the same
-//                    formula as the standalone dequantisation, so the product sees exactly the
-//                    dequantised matrix (what gemm_q8_kernel does not take, without scratch
-//                    for the expanded weights).
+// The kernels:
+//   gemm_ring_kernel   (gemm_ring.hip) binary16 weights: four waves multiply a tile of 64 or 128 rows, four load;
+//   gemm_vw_kernel, gemm_vw256_kernel  binary16 weights, many rows of wide products: tiles of 256 rows, eight MFMA waves,
+//                      with a loader wave, or loading themselves;
+//   gemm_q8_kernel     (gemm_q8.hip) uint8 weights, dequantised on their way into LDS by waves of their own;
+//   gemm_few_kernel    (gemm_few.hip) a few rows: K split over the waves of a workgroup;
+//   gemm_kernel        tiles go global -> registers -> LDS (rows padded by 16 bytes against bank conflicts), the loads of step
+//                      k+1 issued before the MFMAs of step k, uint8 ones dequantised on the way: what none of the others takes
+//                      (uint8 products of fewer than four rows or of columns that are no multiple of 16, without scratch to
+//                      expand them; rows of more than 8 million elements).
 // Products are exact in fp32, accumulation is fp32 in ascending k, and the result is rounded once
-// to the output type (kernels/cuda/matmul.cpp:38-42,64-68); all kernels give the same bits, except
+// to the output type (kernels/cuda/matmul.cpp:38-42,64-68); all kernels but gemm_few_kernel give the same bits, except
 // that a launch split over K (launch_gemm) adds its slices' fp32 sums at the end.
 // Independent products over the same T and K share one launch ("segments"), each with
 // its own X, W and fused epilogue.
@@ -194,14 +189,13 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_kernel(GemmArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// binary16 weights: four MFMA waves and a fifth that only moves data.
+// binary16 weights: waves that multiply and waves that only move data.
 //
 // A compute unit keeps about 64 KB of loads in flight, and a wave that asks for more stands at its
 // load instruction with everything behind it, MFMAs included.  In gemm_kernel the waves that
-// compute also load, so requests are outstanding only between "issue" and "store to LDS".  Here
-// wave 4 streams tiles global -> LDS directly (global_load_lds_dwordx4, no registers) into a ring
-// of kLdwStages K-steps of 64 and is the only wave that ever waits for memory: two steps (64 KB
-// for a 128 x 128 tile) are in flight all the time, and the MFMA waves meet it at one barrier
+// compute also load, so requests are outstanding only between "issue" and "store to LDS".  In gemm_ring_kernel (gemm_ring.hip)
+// and gemm_vw_kernel waves of their own stream tiles global -> LDS directly (global_load_lds_dwordx4, no registers)
+// into a ring of K-steps of 64, two or three of which are in flight all the time, and the MFMA waves meet them at one barrier
 // per step.  Same products in the same order as gemm_kernel: the results are bit-identical.
 //
 // LDS layout.  One load instruction brings 8 rows x 64 k = 8 x 128 contiguous bytes (fully
@@ -212,138 +206,6 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_kernel(GemmArgs a) {
 // term moves them one slot apart: SQ_LDS_BANK_CONFLICT is 0 and a read takes 4 cycles (without
 // that term every read was a two-way conflict: 8 cycles).
 // ---------------------------------------------------------------------------
-constexpr int kLdwThreads = 320;
-constexpr int kLdwStages = 4;
-static constexpr size_t gemm_ldw_lds_bytes(int bm) { return (size_t)kLdwStages * (bm + BN) * kLdwBK * 2; }
-template <int BM>
-__global__ __launch_bounds__(kLdwThreads) void gemm_ldw_kernel(GemmArgs a) {
-  constexpr int MI = BM / 64;
-  constexpr int kABytes = BM * kLdwBK * 2, kBBytes = BN * kLdwBK * 2, kStageBytes = kABytes + kBBytes;
-  constexpr int kAInstr = kABytes / 1024, kBInstr = kBBytes / 1024, kPer = kAInstr + kBInstr;
-  static_assert(kPer == 32 || kPer == 24, "wait counts below are written for these");
-  extern __shared__ __attribute__((aligned(16))) unsigned char gemm_smem[];
-
-  int sidx = 0;
-#pragma unroll
-  for (int i = 1; i < kGemmMaxSeg; i++) sidx += (i < a.nseg && (int)blockIdx.x >= a.tile_start[i]) ? 1 : 0;
-  const GemmSeg& sg = a.seg[sidx];
-  const int n0 = ((int)blockIdx.x - a.tile_start[sidx]) * BN;
-  const int m0 = blockIdx.y * BM;
-  const int M = a.M, K = a.K, N = sg.N;
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  // slice z of ksplit takes K-steps [z base + min(z, rem), ...): the first rem slices one step more
-  const int ksplit = a.ksplit > 1 ? a.ksplit : 1;
-  const int kz = blockIdx.z, ksteps = K / kLdwBK, kper = ksteps / ksplit, krem = ksteps % ksplit;
-  const int nk = kper + (kz < krem ? 1 : 0);            // K-steps of this slice
-  const int kbase = (kz * kper + (kz < krem ? kz : krem)) * kLdwBK;
-
-  if (wave == 4) {
-    // ---- the loader ----
-    const int lr = lane >> 3, ls = (lane & 7) ^ lr;
-    // per-instruction row pointers; rows past M (N) repeat the last row and are never stored
-    const h1* pa[kAInstr];
-    const h1* pb[kBInstr];
-#pragma unroll
-    for (int b = 0; b < kAInstr; b++) {
-      int row = m0 + b * 8 + lr;
-      row = row < M ? row : M - 1;
-      pa[b] = sg.A + (size_t)row * K + kbase + (ls ^ (b & 1)) * 8;
-    }
-#pragma unroll
-    for (int b = 0; b < kBInstr; b++) {
-      int row = n0 + b * 8 + lr;
-      row = row < N ? row : N - 1;
-      pb[b] = reinterpret_cast<const h1*>(sg.B) + (size_t)row * K + kbase + (ls ^ (b & 1)) * 8;
-    }
-    // a tile wholly inside the matrices: scalar base per load plus one of two lane offsets (load_lds_saddr)
-    const bool full = m0 + BM <= M && n0 + BN <= N && (size_t)K * 16 + 128 < 0xffffffffull;
-    const unsigned voff[2] = {(unsigned)(lr * K * 2 + ls * 16), (unsigned)(lr * K * 2 + (ls ^ 1) * 16)};
-    const unsigned char* abase = uniform_ptr(reinterpret_cast<const unsigned char*>(sg.A) + ((size_t)m0 * K + kbase) * 2);
-    const unsigned char* bbase = uniform_ptr(reinterpret_cast<const unsigned char*>(sg.B) + ((size_t)n0 * K + kbase) * 2);
-    const unsigned lds0 = (unsigned)(size_t)((__attribute__((address_space(3))) unsigned char*)gemm_smem);
-    const size_t group = (size_t)__builtin_amdgcn_readfirstlane(K) * 16;
-    auto issue = [&](int step) {
-      const int k0 = step * kLdwBK;
-      if (full) {
-        const unsigned stl = lds0 + (step % kLdwStages) * kStageBytes;
-        const unsigned char* ak = abase + (size_t)k0 * 2;
-        const unsigned char* bk = bbase + (size_t)k0 * 2;
-#pragma unroll
-        for (int b = 0; b < kAInstr; b++) load_lds_saddr(voff[b & 1], ak + b * group, stl + b * 1024);
-#pragma unroll
-        for (int b = 0; b < kBInstr; b++) load_lds_saddr(voff[b & 1], bk + b * group, stl + kABytes + b * 1024);
-        return;
-      }
-      unsigned char* st = gemm_smem + (step % kLdwStages) * kStageBytes;
-#pragma unroll
-      for (int b = 0; b < kAInstr; b++)
-        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(pa[b] + k0),
-                                         (__attribute__((address_space(3))) void*)(st + b * 1024), 16, 0, 0);
-#pragma unroll
-      for (int b = 0; b < kBInstr; b++)
-        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(pb[b] + k0),
-                                         (__attribute__((address_space(3))) void*)(st + kABytes + b * 1024), 16, 0, 0);
-    };
-    issue(0);
-    if (nk > 1) issue(1);
-    for (int k = 0; k < nk; k++) {
-      // step k has landed when at most the loads of step k+1 are outstanding (loads complete in order)
-      if (k + 1 < nk) {
-        if constexpr (kPer == 32)
-          __builtin_amdgcn_s_waitcnt(0x8F70);  // vmcnt(32)
-        else
-          __builtin_amdgcn_s_waitcnt(0x4F78);  // vmcnt(24)
-      } else {
-        __builtin_amdgcn_s_waitcnt(0x0F70);    // vmcnt(0)
-      }
-      step_barrier();            // barrier k: step k may be read, step k-1 has been read by all
-      if (k + 2 < nk) issue(k + 2);            // into the slot of step k-2
-    }
-    return;
-  }
-
-  // ---- the four MFMA waves: one barrier per step, matching the loader's ----
-  const int wm = wave >> 1, wn = wave & 1;
-  f16v acc[MI][2];
-#pragma unroll
-  for (int i = 0; i < MI; i++)
-#pragma unroll
-    for (int j = 0; j < 2; j++)
-#pragma unroll
-      for (int v = 0; v < 16; v++) acc[i][j][v] = 0.f;
-  for (int k = 0; k < nk; k++) {
-    step_barrier();
-    const unsigned char* st = gemm_smem + (k % kLdwStages) * kStageBytes;
-    h8 fa[4][MI], fb[4][2];
-#pragma unroll
-    for (int kb = 0; kb < 4; kb++) {
-      const int q = kb * 2 + (lane >> 5);
-#pragma unroll
-      for (int i = 0; i < MI; i++)
-        fa[kb][i] = *reinterpret_cast<const h8*>(st + ldw_at(wm * (BM / 2) + i * 32 + (lane & 31), q));
-#pragma unroll
-      for (int j = 0; j < 2; j++)
-        fb[kb][j] = *reinterpret_cast<const h8*>(st + kABytes + ldw_at(wn * 64 + j * 32 + (lane & 31), q));
-    }
-#pragma unroll
-    for (int kb = 0; kb < 4; kb++)
-#pragma unroll
-      for (int i = 0; i < MI; i++)
-#pragma unroll
-        for (int j = 0; j < 2; j++)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[kb][i], fb[kb][j], acc[i][j], 0, 0, 0);
-  }
-  if (a.ksplit > 1) {
-    GemmSeg sp = sg;  // this slice's sums go out as fp32; the epilogue proper follows in gemm_splitk_reduce_kernel
-    sp.out = a.partial + (size_t)blockIdx.z * a.partial_stride + a.part_off[sidx];
-    sp.epi = G_STORE_F32;
-    gemm_epilogue<BM>(a, sp, acc, m0, n0, M, N, lane, wm, wn);
-  } else {
-    gemm_epilogue<BM>(a, sg, acc, m0, n0, M, N, lane, wm, wn);
-  }
-}
-
 // Adds the K slices of a split launch in slice order and applies each product's epilogue; a thread
 // takes W consecutive outputs of a row: 16, the unit the batched sigmoid / silu work on, when one of
 // the epilogues is one of those, else 8 (N % 16 == 0 either way).
@@ -421,39 +283,24 @@ static void launch_splitk_reduce(hipStream_t st, const GemmArgs& a) {
     hipLaunchKernelGGL(gemm_splitk_reduce_kernel<8>, grid, dim3(block), 0, st, a);
 }
 
-template <int BM>
-static void gemm_ldw_launch(dim3 grid, hipStream_t st, const GemmArgs& a) {
-  constexpr size_t lds = gemm_ldw_lds_bytes(BM);
-  static bool raised = false;
-  if (!raised) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_ldw_kernel<BM>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    raised = true;
-  }
-  hipLaunchKernelGGL((gemm_ldw_kernel<BM>), grid, dim3(kLdwThreads), lds, st, a);
-}
-
 // ---------------------------------------------------------------------------
-// binary16 weights, tiles of 128 (or 256) rows and a width chosen per launch.
+// binary16 weights, tiles of 256 rows and a width chosen per launch.
 //
-// A launch of 128 x 128 tiles over T = 1024 rows rarely comes out as a whole number of rounds over
-// the compute units (k,v,r of a 2048-wide model: 384 tiles on 256 CUs take as long as 512), and a
-// wider tile moves fewer bytes per product.  Here the host cuts every segment of a launch into
-// tiles of 128 rows x (32 w) columns, w = base or base + 1 per segment, so that the launch fills
-// a whole number of rounds over the compute units, and no tile straddles two segments.  The two wave columns of a workgroup take ceil(w/2) and floor(w/2)
-// 32-column blocks; the loops are instantiated per block count, so the products are the same
-// MFMAs in the same k order as in the other kernels and the results are bit-identical.  Loader
-// wave, LDS ring (three or four K-steps of 64, whatever fits 160 KB at the launch's widest tile)
-// and swizzle are those of gemm_ldw_kernel.  gemm_vw_kernel<256> has eight MFMA waves (4 x 2 of
-// 64 rows each) and takes whole tiles of at most 160 columns; gemm_vw256_kernel below takes the others.
+// A launch of fixed tiles rarely comes out as a whole number of rounds over the compute units, and a
+// wider tile moves fewer bytes per product.  Here, and for gemm_ring_kernel's tiles of 64 and 128 rows, the host cuts every segment
+// of a launch into tiles of 32 w columns, w = base or base + 1 per segment, so that the launch fills
+// a whole number of rounds over the compute units, and no tile straddles two segments.  The two wave columns of a workgroup take
+// ceil(w/2) and floor(w/2) 32-column blocks; the loops are instantiated per block count, so the products are the same
+// MFMAs in the same k order as in the other kernels and the results are bit-identical.  gemm_vw_kernel has eight MFMA waves
+// (4 x 2 of 64 rows each) and a loader wave with a ring of three K-steps, and takes whole tiles of at most 160 columns;
+// gemm_vw256_kernel below takes the others.
 // ---------------------------------------------------------------------------
-constexpr int kVwMaxW = 8;
+constexpr int kVwMaxW = 8, kVwABytes = 256 * kLdwBK * 2;
 constexpr int kVw256LoaderMaxW = 5;  // three stages of (256 + 160) x 64 halves are 156 KB of the 160 KB
 
-template <int BM, int W>
+template <int W>
 __device__ __forceinline__ void vw_loader(const GemmSeg& sg, unsigned char* smem, int stage_bytes, int ns, int m0, int n0,
                                           int M, int N, int K, int lane) {
-  constexpr int kVwABytes = BM * kLdwBK * 2;
   constexpr int kAInstr = kVwABytes / 1024, kBInstr = 4 * W, kPer = kAInstr + kBInstr;
   static_assert(kPer <= 63, "the wait counter's range");
   const int lr = lane >> 3, ls = (lane & 7) ^ lr;
@@ -474,7 +321,7 @@ __device__ __forceinline__ void vw_loader(const GemmSeg& sg, unsigned char* smem
   const int nk = K / kLdwBK;
   // a tile that lies wholly inside the matrices: rows are 8 K halves apart for every lane, so the address of
   // load b is a uniform base (row group b, this step's k) plus one of two lane offsets
-  const bool full = m0 + BM <= M && n0 + W * 32 <= N && (size_t)K * 16 + 128 < 0xffffffffull;
+  const bool full = m0 + 256 <= M && n0 + W * 32 <= N && (size_t)K * 16 + 128 < 0xffffffffull;
   const unsigned voff[2] = {(unsigned)(lr * K * 2 + ls * 16), (unsigned)(lr * K * 2 + (ls ^ 1) * 16)};
   const unsigned char* abase = uniform_ptr(reinterpret_cast<const unsigned char*>(sg.A) + (size_t)m0 * K * 2);
   const unsigned char* bbase = uniform_ptr(reinterpret_cast<const unsigned char*>(sg.B) + (size_t)n0 * K * 2);
@@ -518,10 +365,9 @@ __device__ __forceinline__ void vw_loader(const GemmSeg& sg, unsigned char* smem
   }
 }
 
-template <int BM, int NJ>
-__device__ __forceinline__ void vw_mma(const GemmArgs& a, const GemmSeg& sg, unsigned char* smem, int stage_bytes, int ns,
-                                       int brow0, int m0, int n0, int M, int N, bool full, int lane, int wave) {
-  constexpr int kVwABytes = BM * kLdwBK * 2;
+template <int NJ>
+__device__ __forceinline__ void vw_mma(const GemmArgs& a, const GemmSeg& sg, const unsigned char* smem, int stage_bytes, int ns,
+                                       int brow0, int m0, int n0, int M, int N, int lane, int wave) {
   const int wm = wave >> 1;
   f16v acc[2][NJ];
 #pragma unroll
@@ -538,7 +384,7 @@ __device__ __forceinline__ void vw_mma(const GemmArgs& a, const GemmSeg& sg, uns
     slot = slot + 1 == ns ? 0 : slot + 1;
     // fragments of KG x 16 k are requested together; with eight MFMA waves and the loader a lane has 168
     // registers and holds two of the four k-blocks of a step at a time
-    constexpr int KG = BM == 128 ? 4 : 2;
+    constexpr int KG = 2;
 #pragma unroll
     for (int kh = 0; kh < 4; kh += KG) {
       h8 fa[KG][2], fb[KG][NJ];
@@ -560,19 +406,11 @@ __device__ __forceinline__ void vw_mma(const GemmArgs& a, const GemmSeg& sg, uns
             acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[kb][i], fb[kb][j], acc[i][j], 0, 0, 0);
     }
   }
-  if (BM == 256 || full) {  // 256 rows: whole tiles only
-    gemm_epilogue_t<2, NJ, true>(a, sg, acc, m0 + wm * 64, n0 + brow0, M, N, lane);
-  } else {
-    step_barrier();  // all fragments have been read
-    finish_wave(a, sg, acc, reinterpret_cast<float*>(smem + wave * wave_sums_bytes((a.vw_maxw + 1) / 2)), m0 + wm * 64, n0 + brow0, M, N, lane);
-  }
+  gemm_epilogue_t<2, NJ, true>(a, sg, acc, m0 + wm * 64, n0 + brow0, M, N, lane);
 }
 
-// BM / 32 MFMA waves of 64 rows x half the width, then the loader.  BM = 256: launches of whole tiles of at most
-// kVw256LoaderMaxW blocks.
-template <int BM>
-__global__ __launch_bounds__(BM * 2 + 64) void gemm_vw_kernel(GemmArgs a) {
-  constexpr int kVwABytes = BM * kLdwBK * 2, kLoader = BM / 32, kCap = BM == 128 ? kVwMaxW : kVw256LoaderMaxW;
+// Eight MFMA waves of 64 rows x half the width, then the loader: launches of whole tiles of at most kVw256LoaderMaxW blocks.
+__global__ __launch_bounds__(576) void gemm_vw_kernel(GemmArgs a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char gemm_smem[];
   int bx, by;
   xcd_tile(bx, by);
@@ -584,23 +422,18 @@ __global__ __launch_bounds__(BM * 2 + 64) void gemm_vw_kernel(GemmArgs a) {
   const int base = a.vw_base[sidx], wide = a.vw_wide[sidx];
   const int width = base + (ti < wide ? 1 : 0);                  // 32-column blocks of this tile
   const int n0 = (ti * base + (ti < wide ? ti : wide)) * 32;
-  const int m0 = by * BM;
+  const int m0 = by * 256;
   const int M = a.M, K = a.K, N = sg.N;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int stage_bytes = kVwABytes + a.vw_maxw * 4096, ns = a.vw_ns;
-  const bool full = m0 + BM <= M && n0 + width * 32 <= N;
-  if (wave == kLoader) {
+  if (wave == 8) {
     switch (width) {
-      case 2: vw_loader<BM, 2>(sg, gemm_smem, stage_bytes, ns, m0, n0, M, N, K, lane); break;
-      case 3: vw_loader<BM, 3>(sg, gemm_smem, stage_bytes, ns, m0, n0, M, N, K, lane); break;
-      case 4: vw_loader<BM, 4>(sg, gemm_smem, stage_bytes, ns, m0, n0, M, N, K, lane); break;
-      case 5: vw_loader<BM, 5>(sg, gemm_smem, stage_bytes, ns, m0, n0, M, N, K, lane); break;
-      case 6: vw_loader<BM, kCap < 6 ? kCap : 6>(sg, gemm_smem, stage_bytes, ns, m0, n0, M, N, K, lane); break;
-      case 7: vw_loader<BM, kCap < 7 ? kCap : 7>(sg, gemm_smem, stage_bytes, ns, m0, n0, M, N, K, lane); break;
-      default: vw_loader<BM, kCap>(sg, gemm_smem, stage_bytes, ns, m0, n0, M, N, K, lane); break;
+      case 2: vw_loader<2>(sg, gemm_smem, stage_bytes, ns, m0, n0, M, N, K, lane); break;
+      case 3: vw_loader<3>(sg, gemm_smem, stage_bytes, ns, m0, n0, M, N, K, lane); break;
+      case 4: vw_loader<4>(sg, gemm_smem, stage_bytes, ns, m0, n0, M, N, K, lane); break;
+      default: vw_loader<kVw256LoaderMaxW>(sg, gemm_smem, stage_bytes, ns, m0, n0, M, N, K, lane); break;
     }
-    if (BM == 128 && !full) step_barrier();
     return;
   }
   const int wn = wave & 1;
@@ -608,17 +441,16 @@ __global__ __launch_bounds__(BM * 2 + 64) void gemm_vw_kernel(GemmArgs a) {
   const int nj = wn ? width - nj0 : nj0;
   const int brow0 = wn ? nj0 * 32 : 0;
   switch (nj) {
-    case 1: vw_mma<BM, 1>(a, sg, gemm_smem, stage_bytes, ns, brow0, m0, n0, M, N, full, lane, wave); break;
-    case 2: vw_mma<BM, 2>(a, sg, gemm_smem, stage_bytes, ns, brow0, m0, n0, M, N, full, lane, wave); break;
-    case 3: vw_mma<BM, 3>(a, sg, gemm_smem, stage_bytes, ns, brow0, m0, n0, M, N, full, lane, wave); break;
-    default: vw_mma<BM, (kCap + 1) / 2>(a, sg, gemm_smem, stage_bytes, ns, brow0, m0, n0, M, N, full, lane, wave); break;
+    case 1: vw_mma<1>(a, sg, gemm_smem, stage_bytes, ns, brow0, m0, n0, M, N, lane, wave); break;
+    case 2: vw_mma<2>(a, sg, gemm_smem, stage_bytes, ns, brow0, m0, n0, M, N, lane, wave); break;
+    default: vw_mma<3>(a, sg, gemm_smem, stage_bytes, ns, brow0, m0, n0, M, N, lane, wave); break;
   }
 }
 
 // ---------------------------------------------------------------------------
 // The same tiles, 256 rows high: eight waves, 4 x 2, each 64 rows x half the width.
 //
-// With one MFMA wave per SIMD (gemm_vw_kernel) nothing runs while the first fragments of a step come
+// With one MFMA wave per SIMD (gemm_ring_kernel) nothing runs while the first fragments of a step come
 // out of LDS after the barrier.  Here every SIMD has two, and a step is twice the
 // products for 1.33 times the bytes (256 x 256 against 128 x 256).  There is no loader wave: a ninth
 // wave would leave each wave 168 registers (three on one SIMD), too few for 128 accumulators; the waves
@@ -630,13 +462,13 @@ __global__ __launch_bounds__(BM * 2 + 64) void gemm_vw_kernel(GemmArgs a) {
 // 128 bytes per cycle, as many as its MFMAs take on each SIMD.  3000 x 5120 x 20480: 811 -> 580 us (1.08 PFLOP/s),
 // 4099 x 2048 x 10240: 229 -> 172 us, against the fixed 128 x 128 tiles both launches had before (in turn on one part).
 // ---------------------------------------------------------------------------
-constexpr int kVw256Threads = 512, kVw256ABytes = 256 * kLdwBK * 2;
+constexpr int kVw256Threads = 512;
 
 template <int NJ>
 __device__ __forceinline__ void vw256_body(const GemmArgs& a, const GemmSeg& sg, unsigned char* smem, int width, int brow0,
                                            int m0, int n0, int lane, int wave) {
   const int M = a.M, K = a.K, N = sg.N, nk = K / kLdwBK, wm = wave >> 1;
-  const unsigned stage_bytes = kVw256ABytes + a.vw_maxw * 4096;
+  const unsigned stage_bytes = kVwABytes + a.vw_maxw * 4096;
   // this wave's loads: row groups 4 wave .. + 3 of A, row groups wave, wave + 8, ... of B (there are 4 width)
   unsigned va[4], vb[4];
   const int lr = lane >> 3, ls = (lane & 7) ^ lr;
@@ -659,7 +491,7 @@ __device__ __forceinline__ void vw256_body(const GemmArgs& a, const GemmSeg& sg,
     for (int i = 0; i < 4; i++) load_lds_saddr(va[i], ak, st + (wave * 4 + i) * 1024);
 #pragma unroll
     for (int i = 0; i < 4; i++)
-      if (wave + 8 * i < nb) load_lds_saddr(vb[i], bk, st + kVw256ABytes + (wave + 8 * i) * 1024);
+      if (wave + 8 * i < nb) load_lds_saddr(vb[i], bk, st + kVwABytes + (wave + 8 * i) * 1024);
   };
   f16v acc[2][NJ];
 #pragma unroll
@@ -684,7 +516,7 @@ __device__ __forceinline__ void vw256_body(const GemmArgs& a, const GemmSeg& sg,
       for (int i = 0; i < 2; i++) fa[i] = *reinterpret_cast<const h8*>(st + ldw_at(wm * 64 + i * 32 + (lane & 31), q));
 #pragma unroll
       for (int j = 0; j < NJ; j++)
-        fb[j] = *reinterpret_cast<const h8*>(st + kVw256ABytes + ldw_at(brow0 + j * 32 + (lane & 31), q));
+        fb[j] = *reinterpret_cast<const h8*>(st + kVwABytes + ldw_at(brow0 + j * 32 + (lane & 31), q));
 #pragma unroll
       for (int i = 0; i < 2; i++)
 #pragma unroll
@@ -727,8 +559,8 @@ __global__ __launch_bounds__(kVw256Threads) void gemm_vw256_kernel(GemmArgs a) {
 
 // How one launch of binary16 weights, not split over K, is cut into tiles.
 struct GemmRoute {
-  int rows = 0;        // of a tile: 64 (gemm_ldw_kernel<64>), 128 (gemm_vw_kernel<128>), 256 (the other two); 0: none of these
-  bool loader = true;  // 256 rows: gemm_vw_kernel<256>, not gemm_vw256_kernel
+  int rows = 0;        // of a tile: 64 or 128 (with a loader wave; gemm_ring_kernel has taken their place), 256; 0: none of these
+  bool loader = true;  // 256 rows: gemm_vw_kernel, not gemm_vw256_kernel
   int blocks = 0;      // widest tile, in blocks of 32 columns
   int rounds = 0;      // over the compute units
   double us = 0;       // what the launch is expected to take
@@ -846,15 +678,12 @@ static GemmRoute plan_vw(const GemmArgs& args, int bm, int cus) {
 
 // The cheapest cut.  rows stays 0 where the planned tiles do not fit and fixed 64-row tiles take more than a round.
 static GemmRoute gemm_route(const GemmArgs& a, int cus) {
-  static const int force_bm = getenv("FRHIP_GEMM_VW_BM") ? atoi(getenv("FRHIP_GEMM_VW_BM")) : 0;  // measurement aid
   GemmRoute r = plan_vw(a, 128, cus);
-  if (force_bm != 128) {
-    GemmRoute r2 = plan_vw(a, 256, cus);
-    if (r2.rows && (!r.rows || r2.us < r.us || force_bm == 256)) r = r2;
-  }
+  const GemmRoute r2 = plan_vw(a, 256, cus);
+  if (r2.rows && (!r.rows || r2.us < r.us)) r = r2;
   const int rounds = (int)((tiles64(a) + cus - 1) / cus);
   const double us = us_64(rounds, a.K / 2048.0);
-  if (r.rows ? us < r.us && !force_bm : rounds == 1) {
+  if (r.rows ? us < r.us : rounds == 1) {
     r.rows = 64;
     r.blocks = BN / 32;
     r.rounds = rounds;
@@ -874,35 +703,57 @@ static GemmRoute gemm_route(const GemmArgs& a, int cus) {
 
 // A grouped launch whose products are cheaper one by one (2048 columns in one round of 64 x 128 tiles, 8192 in two of
 // 128 x 192, together three) goes out as separate launches.  FRHIP_GEMM_SEPARATE=0: never.
-static bool one_by_one(const GemmArgs& a, const GemmRoute& whole, int cus) {
+// -> what that is expected to take, us; 0: it stays one launch
+static double one_by_one(const GemmArgs& a, const GemmRoute& whole, int cus) {
   static const bool separate = !(getenv("FRHIP_GEMM_SEPARATE") && atoi(getenv("FRHIP_GEMM_SEPARATE")) == 0);
-  if (!separate || a.nseg < 2) return false;
+  if (!separate || a.nseg < 2) return 0;
   double us = kLaunchUs * (a.nseg - 1);
   for (int s = 0; s < a.nseg; s++) {
     GemmArgs one = a;
     one.nseg = 1;
     one.seg[0] = a.seg[s];
     const GemmRoute r = gemm_route(one, cus);
-    if (!r.rows) return false;
+    if (!r.rows) return 0;
     us += r.us;
   }
-  return whole.rows ? us < whole.us : true;
+  return !whole.rows || us < whole.us ? us : 0;
 }
 
 static void gemm_vw_launch(const GemmRoute& r, hipStream_t st) {
   static const bool raised = [] {
-    for (const void* f : {reinterpret_cast<const void*>(&gemm_vw_kernel<128>), reinterpret_cast<const void*>(&gemm_vw_kernel<256>),
-                          reinterpret_cast<const void*>(&gemm_vw256_kernel)})
+    for (const void* f : {reinterpret_cast<const void*>(&gemm_vw_kernel), reinterpret_cast<const void*>(&gemm_vw256_kernel)})
       (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     return true;
   }();
   (void)raised;
-  if (r.rows == 128)
-    hipLaunchKernelGGL(gemm_vw_kernel<128>, r.grid, dim3(320), r.lds, st, r.a);
-  else if (r.loader)
-    hipLaunchKernelGGL(gemm_vw_kernel<256>, r.grid, dim3(576), r.lds, st, r.a);
+  if (r.loader)
+    hipLaunchKernelGGL(gemm_vw_kernel, r.grid, dim3(576), r.lds, st, r.a);
   else
     hipLaunchKernelGGL(gemm_vw256_kernel, r.grid, dim3(kVw256Threads), r.lds, st, r.a);
+}
+
+// How a launch of binary16 weights that is not split over K goes out: gemm_ring_kernel's tiles in place of every cut of 64 or 128
+// rows (1.20 and 1.11 times as fast over 75 products of 200 to 2048 rows, none slower: 512 x 2048 x 2048 15.8 -> 11.5 us, 300 x 4096 x
+// (4 x 4096) 71.1 -> 60.5), and of 256 rows or product by product where they are expected to be quicker by a twentieth (29
+// products: five, all of them the quicker ones; 1536 x 2048 x (3 x 2048) 58.2 -> 51.7; 1024 x 2560 x (2560 + 8960) stays, 70 against 79).
+struct WholePlan {
+  bool separate = false;
+  TilePlan ring;  // rows = 0: the route
+  GemmRoute route;
+  double us = 0;
+};
+static WholePlan plan_whole(const GemmArgs& a, int cus) {
+  WholePlan w;
+  w.route = gemm_route(a, cus);
+  w.ring = plan_ring(a, cus);
+  const double apart = one_by_one(a, w.route, cus), other = apart ? apart : w.route.rows == 256 ? w.route.us : 0;
+  w.us = w.ring.us;
+  if (other && (!w.ring.rows || other <= w.ring.us * 1.05)) {
+    w.separate = apart != 0;
+    w.ring.rows = 0;
+    w.us = other;
+  }
+  return w;
 }
 
 static constexpr size_t gemm_lds_bytes(int bm, int bk) { return (size_t)(bm + BN) * (bk + 8) * 2; }
@@ -993,24 +844,22 @@ static void split_over(GemmArgs& a, int S, float* partial) {
   a.partial_stride = (a.part_off[a.nseg] + 63) / 64 * 64;
 }
 
+// A launch in slices of K, and the launch that adds them
+static int launch_split(const GemmArgs& a, int cus, hipStream_t st, const char* what) {
+  const TilePlan p = plan_ring(a, cus);
+  if (!p.rows) return set_error(FRHIP_ESHAPE, "gemm: rows too long");
+  if (int rc = launch_gemm_ring(p, st, what)) return rc;
+  launch_splitk_reduce(st, a);
+  return check_launch(what);
+}
+
 static int launch_few_rows(GemmArgs& a, hipStream_t st, const char* what, float* few_rows, size_t few_rows_floats, bool* taken) {
   const int cus = compute_units();
   if (a.K / kLdwBK < 4) return 0;
   if (const int S = few_rows_slices(a, few_rows_floats, cus)) {
-    int tiles = 0;
-    for (int s = 0; s < a.nseg; s++) {
-      a.tile_start[s] = tiles;
-      tiles += (a.seg[s].N + BN - 1) / BN;
-    }
-    for (int s = a.nseg; s <= kGemmMaxSeg; s++) a.tile_start[s] = INT_MAX;
-    a.tile_start[a.nseg] = tiles;
-    *taken = true;
     split_over(a, S, few_rows);
-    const dim3 grid(tiles, (a.M + 63) / 64, (unsigned)S);
-    gemm_ldw_launch<64>(grid, st, a);
-    if (int rc = check_launch(what)) return rc;
-    launch_splitk_reduce(st, a);
-    return check_launch(what);
+    *taken = true;
+    return launch_split(a, cus, st, what);
   }
   if (!few_rows_one_by_one(a, cus)) return 0;
   *taken = true;
@@ -1114,19 +963,21 @@ static int launch_codes(GemmArgs& a, hipStream_t st, const char* what, void* dq,
       split_over(b, S, partial);
       b.partial_stride = partial_stride;
     }
-  if (b.ksplit < 2 && !a.tiled_sums && one_by_one(a, gemm_route(a, cus), cus))
+  WholePlan w;
+  if (b.ksplit < 2) w = plan_whole(a, cus);
+  if (w.separate && !a.tiled_sums)
     for (int s = 0; s < a.nseg; s++) {  // the binary16 image's members could be gemm_few_kernel's
       GemmArgs one = a;
       one.nseg = 1;
       one.seg[0] = a.seg[s];
       if (few_plan(one, 0, 0, 0, cus).mt) return 0;
     }
-  const Q8Plan q = plan_q8(b, cus);
+  const TilePlan q = plan_q8(b, cus);
   if (!q.rows) return 0;
   if (dq) {
     double weights = 0;
     for (int s = 0; s < a.nseg; s++) weights += (double)a.seg[s].N * a.K;
-    if (q.us > 2 + weights * 3 / 5e6 + tiled_us(a, partial ? partial_stride : 0, partial ? max_split : 0, few_rows_floats, cus)) return 0;
+    if (q.us > 2 + weights * 3 / 5e6 + (b.ksplit < 2 ? w.us : plan_ring(b, cus).us)) return 0;
   }
   *taken = true;
   if (int rc = launch_gemm_q8(q, st, what)) return rc;
@@ -1140,21 +991,20 @@ int launch_gemm(GemmArgs& a, bool u8, hipStream_t st, const char* what, void* dq
   if (a.M <= 0) return 0;
   if (a.K <= 0 || a.K % 64 != 0) return set_error(FRHIP_ESHAPE, "gemm: K must be a positive multiple of 64");
   static const bool splitk = env_on("FRHIP_GEMM_SPLITK");
-  static const int force_bm = getenv("FRHIP_GEMM_BM") ? atoi(getenv("FRHIP_GEMM_BM")) : 0;  // measurement aid
-  // binary16 weights go to the kernel with the loader wave (FRHIP_GEMM_LDW=0 selects the other one:
-  // measurement aid); uint8 weights need the registers in between for the dequantisation
-  static const bool ldw = env_on("FRHIP_GEMM_LDW"), few = env_on("FRHIP_GEMM_FEW_ROWS");
-  const bool few_ok = ldw && splitk && few && !force_bm && few_rows;
+  // FRHIP_GEMM_LDW=0 selects gemm_kernel (measurement aid), which also takes rows too long for 32-bit byte offsets within a tile
+  static const bool ldw_on = env_on("FRHIP_GEMM_LDW"), few = env_on("FRHIP_GEMM_FEW_ROWS");
+  const bool ldw = ldw_on && (size_t)a.K * 2 * 256 <= 0xffffffffull;
+  const bool few_ok = ldw && splitk && few && few_rows;
   // Few rows: one launch with K split over the waves of a workgroup where that is expected to be the quicker form by a
   // tenth (both estimates are good to that).  Every workgroup of it reads all rows of X: a long K over few columns is quicker
   // split over K in memory (64 x 20480 x 5120: 45 us against 64; 77 x 8192 x 2048: 17.3 both), many rows of wide products on
   // planned tiles (256 x 5120 x (5120 + 20480): 91 against 143).  Decided by the sizes alone: uint8 codes and their binary16
   // image, expanded here or kept by the caller, give the same bits.
-  const FewPlan fp = ldw && splitk && few && !force_bm && !a.tiled_sums
+  const FewPlan fp = ldw && splitk && few && !a.tiled_sums
                          ? few_plan(a, partial ? partial_stride : 0, partial ? max_split : 0, few_ok ? few_rows_floats : 0, compute_units())
                          : FewPlan();
   if (fp.mt && few_takes(a, u8)) return launch_gemm_few(a, fp, u8, st, what);
-  if (u8 && !fp.mt && a.M >= kDequantRows && ldw && splitk && !force_bm) {
+  if (u8 && !fp.mt && a.M >= kDequantRows && ldw && splitk) {
     bool taken = false;
     const int rc = launch_codes(a, st, what, dq, partial, partial_stride, max_split, few_ok ? few_rows : nullptr, few_ok ? few_rows_floats : 0, &taken);
     if (taken) return rc;
@@ -1182,6 +1032,34 @@ int launch_gemm(GemmArgs& a, bool u8, hipStream_t st, const char* what, void* dq
     const int rc = launch_few_rows(a, st, what, few_rows, few_rows_floats, &taken);
     if (taken) return rc;
   }
+  const int cus = compute_units();
+  // Split K: a single product with few outputs and a long K (ffn value: 1024 x 8192 x 2048) fills the compute units only
+  // with 64 x 128 tiles, which ask L2 for 1.5 times the bytes of 128 x 128 tiles per product and are bound by just that
+  // (786 MB in 57 us).  With scratch for the partial sums the launch runs ksplit slices of K, and a
+  // second kernel adds the slices in order and applies the epilogue.  The sums are grouped by slice, so the result can
+  // differ from the unsplit launch in the last fp32 bit before the rounding to binary16.  FRHIP_GEMM_SPLITK=0: off.
+  if (!u8 && ldw && splitk && partial) {
+    if (const int S = long_k_slices(a, partial_stride, max_split, cus)) {
+      split_over(a, S, partial);
+      a.partial_stride = partial_stride;
+      return launch_split(a, cus, st, what);
+    }
+  }
+  if (!u8 && ldw) {
+    const WholePlan w = plan_whole(a, cus);
+    if (w.separate) {
+      for (int sgi = 0; sgi < a.nseg; sgi++) {
+        GemmArgs one = a;
+        one.nseg = 1;
+        one.seg[0] = a.seg[sgi];
+        if (int rc = launch_gemm(one, false, st, what, nullptr, nullptr, 0, 0, nullptr, 0)) return rc;
+      }
+      return 0;
+    }
+    if (w.ring.rows) return launch_gemm_ring(w.ring, st, what);
+    gemm_vw_launch(w.route, st);
+    return check_launch(what);
+  }
   int tiles = 0;
   for (int s = 0; s < a.nseg; s++) {
     a.tile_start[s] = tiles;
@@ -1191,54 +1069,9 @@ int launch_gemm(GemmArgs& a, bool u8, hipStream_t st, const char* what, void* dq
   a.tile_start[a.nseg] = tiles;
   // 128-row tiles unless that leaves fewer than ~1.5 workgroups per CU; then 64-row tiles
   const int m128 = (a.M + 127) / 128;
-  const bool small = force_bm ? force_bm == 64 : (long)tiles * m128 < (long)compute_units() * 3 / 2;
   static const int force_bk = env_bk();
-  const bool deep = force_bk ? force_bk == 128 : true;
-  const bool deep_ok = deep && a.K % 128 == 0;
-  // Split K: a single product with few outputs and a long K (ffn value: 1024 x 8192 x 2048) fills the compute units only
-  // with 64 x 128 tiles, which ask L2 for 1.5 times the bytes of 128 x 128 tiles per product and are bound by just that
-  // (786 MB in 57 us).  With scratch for the partial sums the launch runs ksplit slices of K over 128 x 128 tiles, and a
-  // second kernel adds the slices in order and applies the epilogue.  The sums are grouped by slice, so the result can
-  // differ from the unsplit launch in the last fp32 bit before the rounding to binary16.  FRHIP_GEMM_SPLITK=0: off.
-  if (!u8 && ldw && splitk && !force_bm && partial) {
-    if (const int S = long_k_slices(a, partial_stride, max_split, compute_units())) {
-      split_over(a, S, partial);
-      a.partial_stride = partial_stride;
-      gemm_ldw_launch<128>(dim3(tiles, m128, S), st, a);
-      if (int rc = check_launch(what)) return rc;
-      launch_splitk_reduce(st, a);
-      return check_launch(what);
-    }
-  }
-  // FRHIP_GEMM_VW=0 keeps binary16 launches on the fixed 128 / 64 x 128 tiles (measurement aid)
-  static const bool vw = !(getenv("FRHIP_GEMM_VW") && atoi(getenv("FRHIP_GEMM_VW")) == 0);
-  if (!u8 && ldw && vw && !force_bm) {
-    const GemmRoute r = gemm_route(a, compute_units());
-    if (one_by_one(a, r, compute_units())) {
-      for (int sgi = 0; sgi < a.nseg; sgi++) {
-        GemmArgs one = a;
-        one.nseg = 1;
-        one.seg[0] = a.seg[sgi];
-        if (int rc = launch_gemm(one, false, st, what, nullptr, nullptr, 0, 0, nullptr, 0)) return rc;
-      }
-      return 0;
-    }
-    if (r.rows) {
-      if (r.rows == 64)
-        gemm_ldw_launch<64>(r.grid, st, r.a);
-      else
-        gemm_vw_launch(r, st);
-      return check_launch(what);
-    }
-  }
-  if (!u8 && ldw) {
-    if (small)
-      gemm_ldw_launch<64>(dim3(tiles, (a.M + 63) / 64), st, a);
-    else
-      gemm_ldw_launch<128>(dim3(tiles, m128), st, a);
-    return check_launch(what);
-  }
-  if (small) {
+  const bool deep_ok = (force_bk ? force_bk == 128 : true) && a.K % 128 == 0;
+  if ((long)tiles * m128 < (long)cus * 3 / 2) {
     dim3 grid(tiles, (a.M + 63) / 64);
     if (deep_ok) FR_GEMM_LAUNCH(64, 128); else FR_GEMM_LAUNCH(64, 64);
   } else {
@@ -1311,6 +1144,43 @@ extern "C" int frhip_gemm_route(int T, int K, int nproducts, const int* N, int c
     out[4 * s + 3] = r.rows != 0 && r.loader;
   }
   return split ? nproducts : 1;
+}
+
+static int tile_args(GemmArgs& a, int T, int K, int nproducts, const int* N, int slices, int compute_units, const int* out, const char* what) {
+  if (!N || !out) return set_error(FRHIP_EINVAL, what);
+  if (T <= 0 || K <= 0 || K % 64 != 0 || nproducts < 1 || nproducts > kGemmMaxSeg || compute_units < 1 || slices < 1 || slices > K / 64)
+    return set_error(FRHIP_ESHAPE, what);
+  memset(&a, 0, sizeof(a));
+  a.M = T;
+  a.K = K;
+  a.nseg = nproducts;
+  a.ksplit = slices;
+  for (int s = 0; s < nproducts; s++) {
+    if (N[s] <= 0) return set_error(FRHIP_ESHAPE, what);
+    a.seg[s].N = N[s];
+  }
+  return 0;
+}
+
+static void tell(const TilePlan& p, int* out) {
+  out[0] = p.rows;
+  out[1] = p.rows ? p.a.vw_maxw : 0;
+  out[2] = p.rounds;
+}
+
+extern "C" int frhip_gemm_ring_tile(int T, int K, int nproducts, const int* N, int slices, int compute_units, int* out) {
+  GemmArgs a;
+  if (int rc = tile_args(a, T, K, nproducts, N, slices, compute_units, out, "gemm_ring_tile: no such launch")) return rc;
+  tell(plan_ring(a, compute_units), out);
+  out[3] = plan_whole(a, compute_units).ring.rows != 0;
+  return 0;
+}
+
+extern "C" int frhip_gemm_q8_tile(int T, int K, int nproducts, const int* N, int slices, int compute_units, int* out) {
+  GemmArgs a;
+  if (int rc = tile_args(a, T, K, nproducts, N, slices, compute_units, out, "gemm_q8_tile: no such launch")) return rc;
+  tell(plan_q8(a, compute_units), out);
+  return 0;
 }
 
 extern "C" int frhip_gemm_few_tile(int T, int K, int nproducts, const int* N, int compute_units, int* out) {

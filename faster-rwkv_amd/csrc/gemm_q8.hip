@@ -283,8 +283,8 @@ static double q8_us(const GemmArgs& a, int bm, int rounds, int w) {
   return 4.2 + sqrt(sqrt(x * x * x * x + y * y * y * y)) + (S > 1 ? 1.6 + S * a.M * cols * 8 / 4.2e6 : 0);
 }
 
-Q8Plan plan_q8(const GemmArgs& args, int cus) {
-  Q8Plan best;
+TilePlan plan_q8(const GemmArgs& args, int cus) {
+  TilePlan best;
   const int S = args.ksplit > 1 ? args.ksplit : 1;
   if ((size_t)args.K * 2 * 128 > 0xffffffffull) return best;  // 32-bit byte offsets within a tile
   for (int s = 0; s < args.nseg; s++)
@@ -296,7 +296,7 @@ Q8Plan plan_q8(const GemmArgs& args, int cus) {
       long need = 0;
       for (int s = 0; s < args.nseg; s++) need += ((args.seg[s].N + 31) / 32 + w - 1) / w;
       const int rounds = (int)((need * strips * S + cus - 1) / cus);
-      Q8Plan p;
+      TilePlan p;
       p.a = args;
       auto dealt = [&](long tiles) {  // the MFMA waves take two blocks or more of a tile
         if (!deal_tiles(p.a, (int)tiles) || p.a.vw_maxw > w) return false;
@@ -325,7 +325,7 @@ bool q8_takes(const GemmArgs& a) {
   return (v16 & 15) == 0 && (v4 & 3) == 0;
 }
 
-int launch_gemm_q8(const Q8Plan& p, hipStream_t st, const char* what) {
+int launch_gemm_q8(const TilePlan& p, hipStream_t st, const char* what) {
   static const bool raised = [] {
     for (const void* f : {reinterpret_cast<const void*>(&gemm_q8_kernel<128>), reinterpret_cast<const void*>(&gemm_q8_kernel<64>)})
       (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
@@ -341,26 +341,3 @@ int launch_gemm_q8(const Q8Plan& p, hipStream_t st, const char* what) {
 }
 
 }  // namespace frhip
-
-using namespace frhip;
-
-extern "C" int frhip_gemm_q8_tile(int T, int K, int nproducts, const int* N, int slices, int compute_units, int* out) {
-  if (!N || !out) return set_error(FRHIP_EINVAL, "gemm_q8_tile: null pointer");
-  if (T <= 0 || K <= 0 || K % 64 != 0 || nproducts < 1 || nproducts > kGemmMaxSeg || compute_units < 1 || slices < 1 || slices > K / 64)
-    return set_error(FRHIP_ESHAPE, "gemm_q8_tile: no such launch");
-  GemmArgs a;
-  memset(&a, 0, sizeof(a));
-  a.M = T;
-  a.K = K;
-  a.nseg = nproducts;
-  a.ksplit = slices;
-  for (int s = 0; s < nproducts; s++) {
-    if (N[s] <= 0) return set_error(FRHIP_ESHAPE, "gemm_q8_tile: no such launch");
-    a.seg[s].N = N[s];
-  }
-  const Q8Plan p = plan_q8(a, compute_units);
-  out[0] = p.rows;
-  out[1] = p.rows ? p.a.vw_maxw : 0;
-  out[2] = p.rounds;
-  return 0;
-}

@@ -305,12 +305,16 @@ int frhip_att_seq_v5(int T, int C, int H, const void *x, const void *sx, const f
  * Returns the number of launches (1: all products together; nproducts: one by one) or a negative FRHIP_E*.
  * out[4 i]: rows of a tile of product i's launch (64, 128, 256; 0: fixed 128 x 128 or 64 x 128 tiles, several rounds),
  * out[4 i + 1]: its widest tile in blocks of 32 columns, out[4 i + 2]: its rounds over the compute units,
- * out[4 i + 3]: 1 if a wave of its own loads the tiles. */
+ * out[4 i + 3]: 1 if a wave of its own loads the tiles.  (Cuts of 64 and 128 rows are what the choice of the kernel for a few
+ * rows is measured by; such launches go out with tiles of frhip_gemm_ring_tile.) */
 int frhip_gemm_route(int T, int K, int nproducts, const int *N, int compute_units, int *out);
 /* Whether such a launch (frhip_gemm's and frhip_gemm_act's are of this kind; the seq operators have scratch, see below) goes,
  * instead, to the kernel for a few rows (K split over the waves of a workgroup), and with which tile: out[0], out[1] = blocks
  * of 16 rows and of 16 columns of a workgroup, 0, 0 if it is cut as above.  A pure function of the sizes too. */
 int frhip_gemm_few_tile(int T, int K, int nproducts, const int *N, int compute_units, int *out);
+/* The tile of such a launch with four loading waves, with K in `slices` slices: out[0], out[1], out[2] = its rows (64, 128), its widest
+ * tile in blocks of 32 columns, its rounds; and out[3] = 1 if the launch, unsplit, takes it (0: tiles of 256 rows, or product by product). */
+int frhip_gemm_ring_tile(int T, int K, int nproducts, const int *N, int slices, int compute_units, int *out);
 /* The tile of such a launch of uint8 products that dequantises the codes on their way into LDS, with K in `slices` slices: out[0],
  * out[1], out[2] = its rows, its widest tile in blocks of 32 columns, its rounds; 0, 0, 0 if it cannot be one. */
 int frhip_gemm_q8_tile(int T, int K, int nproducts, const int *N, int slices, int compute_units, int *out);
