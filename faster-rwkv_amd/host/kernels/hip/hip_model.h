@@ -12,6 +12,7 @@ class Model;
 namespace hip {
 
 struct ReadBack;    // pinned ring for large results (read_back.cpp)
+struct SeqHost;     // pinned token ids and logits of a prompt (model_forward.cpp)
 struct DecodePlan;  // fused one-token forward: buffers + captured graphs (model_forward.cpp)
 
 struct ModelExtra {
@@ -19,6 +20,7 @@ struct ModelExtra {
   std::vector<const void *> packed; // keys registered in the weight table, released with the model
   std::shared_ptr<DecodePlan> plan;
   std::shared_ptr<ReadBack> read_back;
+  std::shared_ptr<SeqHost> seq_host;
   int32_t last_argmax = -1;               // index of the largest logit of the last fused one-token pass ...
   const void *last_argmax_of = nullptr;   // ... and the logits buffer it belongs to
   ~ModelExtra();

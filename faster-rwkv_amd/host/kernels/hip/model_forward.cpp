@@ -498,14 +498,48 @@ bool device_argmax(Model *model, const Tensor &logits, int *id) {
   return true;
 }
 
+// A prompt's token ids on their way to the device and its logits on their way back, in pinned memory that lives with the model: the
+// gather reads the ids where they are, the head kernel stores the logits there besides (as a decoded token's).  As blocking
+// copies of pageable memory they left the device idle for about 60 us ahead of a prompt's first kernel and 100 us behind its last.
+struct SeqHost {
+  int32_t *ids = nullptr;
+  float *logits = nullptr;
+  size_t ids_cap = 0, logits_cap = 0;
+  bool reading = false;  // a gather that has been queued since the last wait may still read the ids
+  ~SeqHost() {
+    frhip_stream_sync(stream());
+    if (ids) frhip_host_free(ids);
+    if (logits) frhip_host_free(logits);
+  }
+  void wait() {
+    FRHIP_CHECK(frhip_stream_sync(stream()));
+    reading = false;
+  }
+  // Room for n values, after whatever the device still does with the old one.
+  template <class T>
+  void room(T *&p, size_t &cap, size_t n) {
+    if (n <= cap) return;
+    wait();
+    if (p) frhip_host_free(p);
+    p = nullptr;
+    cap = 0;
+    void *h = nullptr;
+    FRHIP_CHECK(frhip_host_malloc(&h, n * sizeof(T)));
+    p = static_cast<T *>(h);
+    cap = n;
+  }
+};
+
 // Seq mode (reference: kernels/default/model_forward_seq.cpp:48-184): embedding rows are
 // gathered on the device, every layer runs its seq operator over all T rows (MFMA products,
 // chunked WKV scans), and only the last row goes through ln_out and the head (all rows with
 // full_output).  RWKV-4, which
 // upstream cannot run in seq mode (:111-112), goes through the `att_seq` operator.  `widened`: full output as fp32, as
 // the reference has it, not as the binary16 values that the head product gives.
-// FR_HIP_SEQ_FALLBACK=1 selects the loop of one-token steps (:34-46) instead.
-static Tensor forward_seq(Model *model, Device device, const std::vector<int> &ids, bool full_output, bool widened) {
+// FR_HIP_SEQ_FALLBACK=1 selects the loop of one-token steps (:34-46) instead.  `mirrored`: the last row's logits are wanted in
+// SeqHost::logits, too; it tells whether they will be there once the stream has been waited for.
+static Tensor forward_seq(Model *model, Device device, const std::vector<int> &ids, bool full_output, bool widened,
+                          bool *mirrored = nullptr) {
   const std::string &ver = model->version();
   if (std::getenv("FR_HIP_SEQ_FALLBACK") || !(ver == "4" || ver == "5" || ver == "5.2"))
     return def::ModelForwardSeqFallback(model, device, ids, full_output);
@@ -531,12 +565,16 @@ static Tensor forward_seq(Model *model, Device device, const std::vector<int> &i
   const int V = static_cast<int>(ex->emb_table.size(0));
   for (int id : ids) RV_CHECK(id >= 0 && id < V) << "token id " << id << " out of range";
   frhip_stream s = stream();
-  // ids -> device -> gather (reference: vgather, T separate device copies)
-  Tensor ids_cpu = Tensor::Empty({T}, DType::kInt32, Device::kCPU);
-  std::memcpy(ids_cpu.data_ptr(), ids.data(), sizeof(int32_t) * ids.size());
-  Tensor ids_dev = Copy(ids_cpu, Device::kHIP, true);
+  // the gather reads the ids from pinned memory (reference: vgather, T separate device copies)
+  if (!ex->seq_host) ex->seq_host = std::make_shared<SeqHost>();
+  SeqHost &host = *ex->seq_host;
+  host.room(host.ids, host.ids_cap, ids.size());
+  if (mirrored) host.room(host.logits, host.logits_cap, static_cast<size_t>(model->_params.back().size(1)));
+  if (host.reading) host.wait();
+  std::memcpy(host.ids, ids.data(), sizeof(int32_t) * ids.size());
   Tensor x = Tensor::Empty({T, C}, DType::kFloat16, Device::kHIP);
-  FRHIP_CHECK(frhip_gather_rows(ex->emb_table.data_ptr(), ids_dev.data_ptr<int32_t>(), x.data_ptr(), T, 2 * C, s));
+  host.reading = true;
+  FRHIP_CHECK(frhip_gather_rows(ex->emb_table.data_ptr(), host.ids, x.data_ptr(), T, 2 * C, s));
 
   auto &states = model->states();
   const auto &p = model->_params;
@@ -578,8 +616,23 @@ static Tensor forward_seq(Model *model, Device device, const std::vector<int> &i
   // last row -> ln_out -> head -> fp32 (model_forward_seq.cpp:170-178)
   Tensor logits = Tensor::Empty({static_cast<LengthType>(hw->N)}, DType::kFloat32, Device::kHIP);
   const char *last = static_cast<const char *>(x.data_ptr()) + static_cast<size_t>(T - 1) * C * 2;
-  FRHIP_CHECK(frhip_head(C, last, p[pi].data_ptr(), p[pi + 1].data_ptr(), hw, logits.data_ptr<float>(), s));
+  if (mirrored) *mirrored = true;
+  RV_CHECK(!mirrored || static_cast<size_t>(hw->N) <= host.logits_cap);
+  FRHIP_CHECK(frhip_head_mirror(C, last, p[pi].data_ptr(), p[pi + 1].data_ptr(), hw, logits.data_ptr<float>(),
+                                mirrored ? host.logits : nullptr, s));
   return logits;
+}
+
+// Model::Run on a prompt: a CPU tensor of the caller's own.
+static Tensor run_seq(Model *model, Device device, const std::vector<int> &ids) {
+  bool mirrored = false;
+  Tensor out = forward_seq(model, device, ids, false, true, &mirrored);
+  if (!mirrored) return Copy(out, Device::kCPU);
+  SeqHost &host = *extra_of(model)->seq_host;
+  host.wait();
+  Tensor owned = Tensor::Empty(out.shape(), out.dtype(), Device::kCPU);
+  std::memcpy(owned.data_ptr(), host.logits, out.nbytes());
+  return owned;
 }
 
 Tensor ModelForwardSeq(Model *model, Device device, const std::vector<int> &ids, bool full_output) {
@@ -590,6 +643,7 @@ Tensor FullLogits(Model *model, const std::vector<int> &ids) { return forward_se
 
 KernelRegister model_forward_reg("model_forward", Device::kHIP, ModelForward);
 KernelRegister model_forward_seq_reg("model_forward_seq", Device::kHIP, ModelForwardSeq);
+KernelRegister model_run_seq_reg("model_run_seq", Device::kHIP, run_seq);
 
 }  // namespace hip
 }  // namespace rwkv

@@ -134,6 +134,11 @@ inline Tensor ModelForward(Model *model, Device device, int id) {
   return KernelRegistry::Instance().Get<Fn>("model_forward", device)(model, device, id);
 }
 
+// Model::Run on several ids where a device has its own way of bringing the logits to the host ("model_run_seq"): a CPU tensor.
+inline Tensor ModelRunSeq(Model *model, Device device, const std::vector<int> &id) {
+  using Fn = Tensor (*)(Model *, Device, const std::vector<int> &);
+  return KernelRegistry::Instance().Get<Fn>("model_run_seq", device)(model, device, id);
+}
 inline Tensor ModelForwardSeq(Model *model, Device device, const std::vector<int> &id, bool full_output) {
   using Fn = Tensor (*)(Model *, Device, const std::vector<int> &, bool);
   return KernelRegistry::Instance().Get<Fn>("model_forward_seq", device)(model, device, id, full_output);

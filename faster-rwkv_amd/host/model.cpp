@@ -115,6 +115,7 @@ static Tensor CopyToCPUIfAvailable(const Tensor &x) {
 Tensor Model::Run(const std::vector<int> &ids) {
   RV_CHECK(!ids.empty());
   if (ids.size() == 1) return CopyToCPUIfAvailable(ModelForward(this, _act_device, ids[0]));
+  if (KernelRegistry::Instance().Has("model_run_seq", _act_device)) return ModelRunSeq(this, _act_device, ids);
   return CopyToCPUIfAvailable(ModelForwardSeq(this, _act_device, ids, false));
 }
 

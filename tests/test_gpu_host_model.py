@@ -254,6 +254,32 @@ def test_greedy_loop_kept_on_the_device_equals_the_loop_of_runs(spec, strategy):
     assert len(set(chained[2].tolist())) > 1  # not a constant sequence
 
 
+@pytest.mark.parametrize("spec", ["v=4,L=2,C=256,F=1024,V=1111,seed=7", "v=5.2,L=2,C=256,F=896,V=1111,H=4,seed=7"])
+def test_prompts_of_changing_length_and_texts_in_turn(spec):
+    """Ids and logits of prompts share pinned buffers that grow with the prompts: every result is that of a model of its own, also right
+    after a text whose ids a gather may still be reading, and of two models in turn."""
+    m, n = (fr.Model("synthetic:" + spec, "hip fp16") for _ in range(2))
+    g = np.random.default_rng(3)
+    prompts = [g.integers(0, 1111, k).astype(np.int32) for k in (5, 300, 7, 1300, 4, 64)]
+    want = []
+    for p in prompts:
+        f = fr.Model("synthetic:" + spec, "hip fp16")
+        want.append((f.run(p), f.run(9)))
+        f.close()
+    for p, (logits, after) in zip(prompts, want):
+        for model in (m, n):
+            model.reset()
+            model.run_full(p[:4])
+            model.reset()
+            assert np.array_equal(model.run(p), logits) and np.array_equal(model.run(9), after)
+    with pytest.raises(Exception):
+        m.run([1, 2, 1111, 4])
+    m.reset()
+    assert np.array_equal(m.run(prompts[1]), want[1][0])
+    m.close()
+    n.close()
+
+
 def test_synthetic_model_and_cpp_greedy_loop():
     m = fr.Model("synthetic:v=4,L=2,C=256,F=1024,V=1024,seed=7", "hip int8")
     toks, secs = m.greedy(1, 16)
