@@ -231,9 +231,6 @@ TilePlan plan_ring(const GemmArgs& args, int cus) {
         return true;
       };
       if (!dealt(rounds * cus / slots) && !dealt(need)) continue;
-#ifdef RING_PROBE
-      if ((getenv("R_BM") && bm != atoi(getenv("R_BM"))) || (getenv("R_W") && w != atoi(getenv("R_W")))) continue;
-#endif
       p.us = ring_us(args, bm, rounds, p.a.vw_maxw);
       p.rows = bm;
       p.rounds = (int)rounds;

@@ -76,73 +76,79 @@ __global__ __launch_bounds__(256) void ln_mix_seq_kernel(LnMixSeq a) {
 }
 
 // The same for C % 8 == 0, C <= 8 * 256 * NG: a workgroup takes kLnRows consecutive rows plus the
-// row before them (the token shift of its first row), every thread owns NG groups of 8 elements
+// row before them (the token shift of its first row), every thread owns a group of 8 elements
 // of every row in registers, all rows are loaded up front and their statistics reduced together
 // (two barriers per workgroup), and the mixed rows leave as 16-byte stores.  The launch is a chain
 // of one load, two reductions and one store per workgroup, so what counts is how many workgroups
 // a compute unit has to overlap: at T = 1024, C = 2048 four rows per workgroup (one workgroup per
 // CU, every row read 1.25 times) take 8.7 us, two 7.4 us, one (every row read twice) 7.0 us.
+// For the same reason everything is requested at the start, the mixes too (one by one in the loop over the outputs each was a round
+// trip of its own), and rows of more than 2048 elements have a thread per group: the first four waves take the sums of all of them,
+// in the order of a thread with two groups, and each thread writes its own.  A launch is 0.7 us shorter for it (48 launches of a
+// 77-token prompt of the 1.5B shape 2599 -> 2564 us, 13 tokens on a state 2626 -> 2546, 512 tokens of the 3B shape 3284 -> 3244).
 constexpr int kLnRows = 1;
 
-template <int NG>
-__global__ __launch_bounds__(256) void ln_mix_rows_kernel(LnMixSeq a) {
+template <int NG, int NMIX>
+__global__ __launch_bounds__(256 * NG) void ln_mix_rows_kernel(LnMixSeq a) {
   constexpr int NR = kLnRows + 1;  // row 0 is the row before the workgroup's first
   __shared__ float red[2][4][NR];
   const int C = a.C, ngrp = C >> 3;
   const int t0 = blockIdx.x * kLnRows;
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  h8 xr[NR][NG], gam[NG], bet[NG];
-  bool own[NG];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, g = threadIdx.x;
+  const bool own = g < ngrp, sums = NG == 1 || wv < 4, more = NG == 2 && sums && g + 256 < ngrp;
+  const int gc = own ? g : 0, gm = more ? g + 256 : 0;
+  h8 xr[NR], xm[NR], mx[NMIX];
 #pragma unroll
-  for (int n = 0; n < NG; n++) {
-    const int g = threadIdx.x + n * 256;
-    own[n] = g < ngrp;
-    const int gc = own[n] ? g : 0;
-#pragma unroll
-    for (int r = 0; r < NR; r++) {
-      int t = t0 - 1 + r;
-      t = t < 0 ? 0 : (t < a.T ? t : a.T - 1);
-      xr[r][n] = reinterpret_cast<const h8*>(a.x + (size_t)t * C)[gc];
-    }
-    gam[n] = reinterpret_cast<const h8*>(a.ln_w)[gc];
-    bet[n] = reinterpret_cast<const h8*>(a.ln_b)[gc];
+  for (int r = 0; r < NR; r++) {
+    int t = t0 - 1 + r;
+    t = t < 0 ? 0 : (t < a.T ? t : a.T - 1);
+    const h8* row = reinterpret_cast<const h8*>(a.x + (size_t)t * C);
+    xr[r] = row[gc];
+    if (NG == 2 && sums) xm[r] = row[gm];
   }
-  h8 shift0[NG];  // the shift state, used instead of LN(row -1) by the first workgroup
-  if (t0 == 0) {
+  const h8 gam = reinterpret_cast<const h8*>(a.ln_w)[gc], bet = reinterpret_cast<const h8*>(a.ln_b)[gc];
 #pragma unroll
-    for (int n = 0; n < NG; n++) shift0[n] = reinterpret_cast<const h8*>(a.state)[own[n] ? threadIdx.x + n * 256 : 0];
-  }
+  for (int m = 0; m < NMIX; m++) mx[m] = reinterpret_cast<const h8*>(a.mix[m])[gc];
+  h8 shift0;  // the shift state, used instead of LN(row -1) by the first workgroup
+  if (t0 == 0) shift0 = reinterpret_cast<const h8*>(a.state)[gc];
   float mean[NR], inv[NR];
   {
-    float s[NR];
+    if (sums) {
 #pragma unroll
-    for (int r = 0; r < NR; r++) {
-      s[r] = 0.f;
+      for (int r = 0; r < NR; r++) {
+        float s = 0.f;
+        if (own)
 #pragma unroll
-      for (int n = 0; n < NG; n++)
-        if (own[n])
+          for (int i = 0; i < 8; i++) s += (float)xr[r][i];
+        if (NG == 2 && more)
 #pragma unroll
-          for (int i = 0; i < 8; i++) s[r] += (float)xr[r][n][i];
-      s[r] = wave_sum(s[r]);
-      if (lane == 0) red[0][wv][r] = s[r];
+          for (int i = 0; i < 8; i++) s += (float)xm[r][i];
+        s = wave_sum(s);
+        if (lane == 0) red[0][wv][r] = s;
+      }
     }
     __syncthreads();
 #pragma unroll
     for (int r = 0; r < NR; r++) mean[r] = (((red[0][0][r] + red[0][1][r]) + red[0][2][r]) + red[0][3][r]) / (float)C;
-    float q[NR];
+    if (sums) {
 #pragma unroll
-    for (int r = 0; r < NR; r++) {
-      q[r] = 0.f;
-#pragma unroll
-      for (int n = 0; n < NG; n++)
-        if (own[n])
+      for (int r = 0; r < NR; r++) {
+        float q = 0.f;
+        if (own)
 #pragma unroll
           for (int i = 0; i < 8; i++) {
-            const float d = (float)xr[r][n][i] - mean[r];
-            q[r] += d * d;
+            const float d = (float)xr[r][i] - mean[r];
+            q += d * d;
           }
-      q[r] = wave_sum(q[r]);
-      if (lane == 0) red[1][wv][r] = q[r];
+        if (NG == 2 && more)
+#pragma unroll
+          for (int i = 0; i < 8; i++) {
+            const float d = (float)xm[r][i] - mean[r];
+            q += d * d;
+          }
+        q = wave_sum(q);
+        if (lane == 0) red[1][wv][r] = q;
+      }
     }
     __syncthreads();
 #pragma unroll
@@ -152,37 +158,42 @@ __global__ __launch_bounds__(256) void ln_mix_rows_kernel(LnMixSeq a) {
       inv[r] = 1.0f / sqrtf(var + 1e-5f);
     }
   }
+  if (!own) return;
+  h8 prev;
 #pragma unroll
-  for (int n = 0; n < NG; n++) {
-    if (!own[n]) continue;
-    const int g = threadIdx.x + n * 256;
-    h8 prev;
+  for (int r = 0; r < NR; r++) {
+    h8 xx;
 #pragma unroll
-    for (int r = 0; r < NR; r++) {
-      h8 xx;
-#pragma unroll
-      for (int i = 0; i < 8; i++) {  // kernels/cuda/layer_norm.cu:60-69: half, * gamma in half, + beta in half
-        const h1 nrm = (h1)(((float)xr[r][n][i] - mean[r]) * inv[r]);
-        xx[i] = (nrm * gam[n][i]) + bet[n][i];
-      }
-      if (r == 0) {
-        prev = t0 == 0 ? shift0[n] : xx;
-        continue;
-      }
-      const int t = t0 + r - 1;
-      if (t < a.T) {
-        for (int m = 0; m < a.nmix; m++) {
-          const h8 mx = reinterpret_cast<const h8*>(a.mix[m])[g];
-          h8 o;
-#pragma unroll
-          for (int i = 0; i < 8; i++) o[i] = mix1(xx[i], prev[i], mx[i]);
-          reinterpret_cast<h8*>(a.out[m] + (size_t)t * C)[g] = o;
-        }
-        if (t == a.T - 1) reinterpret_cast<h8*>(a.xx_last)[g] = xx;
-      }
-      prev = xx;
+    for (int i = 0; i < 8; i++) {  // kernels/cuda/layer_norm.cu:60-69: half, * gamma in half, + beta in half
+      const h1 nrm = (h1)(((float)xr[r][i] - mean[r]) * inv[r]);
+      xx[i] = (nrm * gam[i]) + bet[i];
     }
+    if (r == 0) {
+      prev = t0 == 0 ? shift0 : xx;
+      continue;
+    }
+    const int t = t0 + r - 1;
+    if (t < a.T) {
+#pragma unroll
+      for (int m = 0; m < NMIX; m++) {
+        h8 o;
+#pragma unroll
+        for (int i = 0; i < 8; i++) o[i] = mix1(xx[i], prev[i], mx[m][i]);
+        reinterpret_cast<h8*>(a.out[m] + (size_t)t * C)[g] = o;
+      }
+      if (t == a.T - 1) reinterpret_cast<h8*>(a.xx_last)[g] = xx;
+    }
+    prev = xx;
   }
+}
+
+template <int NMIX>
+static void launch_ln_mix_rows(const LnMixSeq& a, int nwg, hipStream_t st) {
+  const int ngrp = a.C >> 3;
+  if (ngrp <= 256)
+    hipLaunchKernelGGL((ln_mix_rows_kernel<1, NMIX>), dim3(nwg), dim3(256), 0, st, a);
+  else
+    hipLaunchKernelGGL((ln_mix_rows_kernel<2, NMIX>), dim3(nwg), dim3((ngrp + 63) / 64 * 64), 0, st, a);
 }
 
 // Rows beyond 4096 elements, up to 256 * NE: the row and the one before it stay in registers too, but
@@ -612,10 +623,8 @@ static int launch_ln_mix(int T, int C, const void* x, const void* state, const v
   }
   a.xx_last = (h1*)xx_last;
   const int nwg = (T + kLnRows - 1) / kLnRows;
-  if (C % 8 == 0 && C <= 2048)
-    hipLaunchKernelGGL(ln_mix_rows_kernel<1>, dim3(nwg), dim3(256), 0, st, a);
-  else if (C % 8 == 0 && C <= 4096)
-    hipLaunchKernelGGL(ln_mix_rows_kernel<2>, dim3(nwg), dim3(256), 0, st, a);
+  if (C % 8 == 0 && C <= 4096)
+    nmix == 2 ? launch_ln_mix_rows<2>(a, nwg, st) : nmix == 3 ? launch_ln_mix_rows<3>(a, nwg, st) : launch_ln_mix_rows<4>(a, nwg, st);
   else if (C > 4096 && C <= 6144)
     hipLaunchKernelGGL(ln_mix_wide_kernel<24>, dim3(T), dim3(256), 0, st, a);
   else

@@ -285,6 +285,13 @@ def test_ffn_seq_uint8_scales_at_any_address(T):
     assert np.array_equal(outs[0].view(np.uint16), outs[1].view(np.uint16))
 
 
+@pytest.mark.parametrize("T,C_", [(3, 2048), (1, 2112), (5, 2304), (2, 2560), (7, 4032)])  # a thread per group, one to five waves beside the first four
+def test_layernorm_of_rows_with_more_groups_than_sums(T, C_):
+    test_ffn_seq(T, C_, 128, False)
+    test_att_seq_v4(T, C_, False, True)
+    test_att_seq_v5_2(T, C_, C_ // 64, False)
+
+
 @pytest.mark.parametrize("T,C_", [(9, 4096), (5, 4160), (9, 5120), (1, 6144), (3, 6208)])  # 16-byte groups; one element at a time (three times); general form
 def test_ffn_seq_wide_rows(T, C_):
     """The layernorm and mix of wide rows, at the edges of the register forms.  Bounds as in test_ffn_seq."""
