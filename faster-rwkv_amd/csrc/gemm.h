@@ -35,13 +35,12 @@ struct GemmArgs {
   bool tiled_sums;
   int tile_start[kGemmMaxSeg + 1];  // first N-tile of each segment
   size_t part_off[kGemmMaxSeg + 1]; // split launches: where each segment's [M][N] block starts within a slice of `partial` (floats); [nseg] = all
-  // gemm_vw_kernel: a segment's tiles are vw_base (the first vw_wide of them vw_base + 1) blocks of 32 columns wide
+  // tiles of a width chosen per launch: a segment's are vw_base (the first vw_wide of them vw_base + 1) blocks of 32 columns wide
   int vw_base[kGemmMaxSeg], vw_wide[kGemmMaxSeg], vw_maxw, vw_ns;
   int few_strips;  // gemm_few_kernel: strips of rows
   GemmSeg seg[kGemmMaxSeg];
-  // split K (ksplit >= 2; gemm_ldw_kernel<128> with one segment, gemm_ldw_kernel<64> and
-  // gemm_q8_kernel with up to four): slice z of ksplit accumulates its K-steps of segment s into partial + z * partial_stride + part_off[s] as
-  // fp32 [M][N]; gemm_splitk_reduce_kernel adds the slices and applies the epilogues
+  // split K (ksplit >= 2; gemm_ring_kernel and gemm_q8_kernel): slice z of ksplit accumulates its K-steps of segment s into
+  // partial + z * partial_stride + part_off[s] as fp32 [M][N]; gemm_splitk_reduce_kernel adds the slices and applies the epilogues
   int ksplit;
   float* partial;
   size_t partial_stride;

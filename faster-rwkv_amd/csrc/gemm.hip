@@ -791,8 +791,8 @@ static bool env_on(const char* name) {
 }
 
 // Few rows (a short prompt): 64 x 128 tiles leave most compute units without a workgroup, and a workgroup pulls its
-// weights through a ring of two K-steps (48 KB in flight), so a launch takes K / 64 round trips to memory however few
-// rows there are (T = 64, 2048 x 2048: 16 workgroups, 17-25 us for 8 MB).  With scratch for the partial sums such a
+// weights through a ring of a few K-steps, so a launch takes about K / 64 round trips to memory however few
+// rows there are (64 x 2048 x 2048, two steps in flight: 16 workgroups, 17-25 us for 8 MB).  With scratch for the partial sums such a
 // launch is split over K into as many slices as there are idle compute units (at least four K-steps each), and the
 // reduction pass adds the slices in order and applies each product's epilogue.  A group that is too wide for that as a
 // whole goes out product by product, so that its narrow members still can.  FRHIP_GEMM_FEW_ROWS=0: off.
@@ -886,7 +886,10 @@ static int long_k_slices(const GemmArgs& a, size_t partial_stride, int max_split
 }
 
 // What launch_gemm's other binary16 forms are expected to take, us, in its order: split over K on 64-row tiles, product by
-// product, split over K on 128-row tiles, planned tiles.  The split forms are fitted to 600 measured products (5 to 7 % rms),
+// product, split over K on 128-row tiles, planned tiles; all with a single loader wave, which gemm_ring_kernel has replaced
+// since.  It is up to 1.4 times as quick, and still only 14 of 299 launches of 8 to 512 rows that go to gemm_few_kernel by this
+// estimate would be the quicker on its tiles (widths 768 to 5120; 77 x 5120 x 5120 20.8 us against 26.6, the others by a seventh
+// at most), of uint8 codes two: the line stays, and with it every launch's order of sums.  The split forms are fitted to 600 measured products (5 to 7 % rms),
 // their reduction launch included.  Over 476 others of 4 to 512 rows all forms together came out 5 % quicker than expected (11 %
 // rms), and what is chosen by it and few_us 0.9 % slower than the quicker form (gemm_few_kernel 295 times, 10 of them wrongly, by 14 %
 // at most).  An expansion of uint8 codes is left out, so that codes and their image take the same form: uint8 products are 10 %

@@ -203,7 +203,7 @@ __device__ __forceinline__ void gemm_epilogue_t(const GemmArgs& a, const GemmSeg
       for (int j = 0; j < NJ; j++) g(i, j, acc[i][j]);
   };
   // blocks without a stored element; only for the costly epilogues: with the test in all of them the short launches of
-  // gemm_ldw_kernel<64> took 0.4-0.8 us longer (33 x 1024 x 5120: 6.5 -> 6.9)
+  // 64-row tiles took 0.4-0.8 us longer (33 x 1024 x 5120: 6.5 -> 6.9)
   auto outside = [&](int i, int j) { return !FULL && (row0 + i * 32 >= M || col0 + j * 32 >= N); };
   auto live_of = [&](int i, int j) {  // bit v: element v of the block lies inside the matrix
     uint32_t m = 0;

@@ -41,7 +41,7 @@ constexpr int few_stages(int mt, int nt, bool u8) {
 constexpr int few_wave_bytes(int mt, int nt, bool u8) { return few_stages(mt, nt, u8) * few_stage_bytes(mt, nt, u8) + (u8 ? kFewScaleBytes : 0); }
 
 // A tile of 16 rows x 64 binary16: rows of 128 bytes, k-segment q (8 halves) of row r in slot q ^ (r % 8) ^ (r / 8)
-// (the layout of gemm_ldw_kernel: fragment reads of 16 rows are free of bank conflicts)
+// (the layout of the tiled kernels: fragment reads of 16 rows are free of bank conflicts)
 __device__ __forceinline__ int few_at(int r, int q) { return r * 128 + ((q ^ (r & 7) ^ (r >> 3)) * 16); }
 
 template <int MT, int NT, bool U8>

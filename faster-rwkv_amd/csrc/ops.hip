@@ -231,8 +231,9 @@ __global__ void dequant_u8_kernel(const uint32_t* __restrict__ q, const h1* __re
 }
 
 // The same, eight consecutive codes of four rows per thread (K a multiple of 16): ry and my are read once for four
-// rows, a wave reads 512 and writes 1024 consecutive bytes of a row per instruction.  The seq-mode products expand a
-// launch's uint8 weights with this before the binary16 GEMM, so it runs at copy rate or the expansion eats what it saves.
+// rows, a wave reads 512 and writes 1024 consecutive bytes of a row per instruction.  Where a seq-mode
+// launch does not dequantise its uint8 weights by itself (from about 512 rows on), it expands them with this before the
+// binary16 GEMM, so it runs at copy rate or the expansion eats what it saves.
 // Bound: memory, 3 bytes per code.  With 16 codes of one row per thread every thread read 64 bytes of ry and my for them
 // and stored 16 bytes at a stride of 32: four 2560 x 2560 20.0 us, 2560 x (8960 + 2560) 21.8, 8960 x 2560 18.9; now
 // 15.4 (5.1 TB/s), 17.0 and 14.3.
