@@ -926,9 +926,13 @@ static FewPlan few_plan(const GemmArgs& a, size_t partial_stride, int max_split,
 
 // uint8 weights through gemm_q8_kernel, in the slices of K that the binary16 launch would take, so with the same bits.  A group
 // whose members are split one by one stays one launch where they take the same slices and their sums fit the scratch.
-// With scratch for it (dq) the codes can be expanded instead, 3 bytes of traffic a weight at 5 TB/s, and multiplied as binary16;
-// many strips of rows dequantise every code once each, so from about 512 rows of a wide product on that is quicker (1000 x 4096 x
-// 16384: 173 us against 193; x 4096: 57 against 52).  *taken stays false, and nothing is launched, where it is expected to be.
+// With scratch for it (dq) the codes can be expanded instead, a launch of 5.5 us and 3 bytes of traffic a weight at 6.3 TB/s, and
+// multiplied as binary16; many strips of rows dequantise every code once each, so from about 512 rows of a wide product on that is
+// quicker.  Both ways measured over 488 launches of 65 to 4099 rows, widths 768 to 5120, us (expanded / on the codes): 777 x 14336
+// x 4096 142 / 162, 1024 x 5120 x (5120 + 20480) 331 / 365; 384 x 768 x (768 + 3072) 18.1 / 13.3, 1024 x 768 x 768 10.0 / 9.2.  What is
+// chosen with these figures, the 1.12 among them, is 0.7 % slower than the quicker way on average; with 2 us, 5 TB/s and 1 it was 2.5 %.
+// (Prompts of 1024 tokens of the 1.5B shape 6479 -> 6112 us, of 700 of the 7B RWKV-5.2 width 1593 -> 1508, two layers of it.)
+// *taken stays false, and nothing is launched, where expanding is expected to be quicker.
 static int launch_codes(GemmArgs& a, hipStream_t st, const char* what, void* dq, float* partial, size_t partial_stride, int max_split,
                         float* few_rows, size_t few_rows_floats, bool* taken) {
   if (!q8_takes(a)) return 0;
@@ -980,7 +984,7 @@ static int launch_codes(GemmArgs& a, hipStream_t st, const char* what, void* dq,
   if (dq) {
     double weights = 0;
     for (int s = 0; s < a.nseg; s++) weights += (double)a.seg[s].N * a.K;
-    if (q.us > 2 + weights * 3 / 5e6 + (b.ksplit < 2 ? w.us : plan_ring(b, cus).us)) return 0;
+    if (q.us * 1.12 > 5.5 + weights * 3 / 6.3e6 + (b.ksplit < 2 ? w.us : plan_ring(b, cus).us)) return 0;
   }
   *taken = true;
   if (int rc = launch_gemm_q8(q, st, what)) return rc;
