@@ -9,6 +9,9 @@ namespace frhip {
 
 typedef float f16v __attribute__((ext_vector_type(16)));
 typedef float f4v __attribute__((ext_vector_type(4)));
+// 16 bytes at any address of an element: the same one instruction (device memory is accessed in unaligned mode)
+typedef h1 h8_any __attribute__((ext_vector_type(8), aligned(2)));
+typedef float f4v_any __attribute__((ext_vector_type(4), aligned(4)));
 
 // sigmoid_h of the W accumulators a lane holds of one MFMA block (16 of 32 x 32, 4 of 16 x 16), the same bits at a
 // fraction of the cost.  Called element by element, sigmoid_h makes a wave take its double branch whenever
@@ -271,7 +274,7 @@ __device__ __forceinline__ void gemm_epilogue_t(const GemmArgs& a, const GemmSeg
 }
 
 // The epilogue of G groups of eight consecutive outputs of a row, whose sums are in `acc`; o: the groups' places in [M][N].  VEC:
-// operands and outputs go 16 bytes at a time; otherwise one at a time, the first n of every group.
+// operands and outputs go 16 bytes at a time, at any address; otherwise one at a time, the first n of every group.
 template <int G, bool VEC = true>
 __device__ __forceinline__ void store_groups(const GemmArgs& a, const GemmSeg& sg, const float (&acc)[8 * G], const size_t (&o)[G], int n = 8) {
   constexpr int W = 8 * G;
@@ -281,7 +284,7 @@ __device__ __forceinline__ void store_groups(const GemmArgs& a, const GemmSeg& s
       float* out = static_cast<float*>(sg.out) + o[g];
       if constexpr (VEC) {
 #pragma unroll
-        for (int q = 8 * g; q < 8 * g + 8; q += 4) *reinterpret_cast<f4v*>(out + q - 8 * g) = (f4v){acc[q], acc[q + 1], acc[q + 2], acc[q + 3]};
+        for (int q = 8 * g; q < 8 * g + 8; q += 4) *reinterpret_cast<f4v_any*>(out + q - 8 * g) = (f4v){acc[q], acc[q + 1], acc[q + 2], acc[q + 3]};
       } else {
 #pragma unroll
         for (int i = 0; i < 8; i++)
@@ -294,7 +297,7 @@ __device__ __forceinline__ void store_groups(const GemmArgs& a, const GemmSeg& s
 #pragma unroll
     for (int g = 0; g < G; g++) {
       if constexpr (VEC) {
-        const h8 t = *reinterpret_cast<const h8*>(p + o[g]);
+        const h8_any t = *reinterpret_cast<const h8_any*>(p + o[g]);
 #pragma unroll
         for (int i = 0; i < 8; i++) v[8 * g + i] = t[i];
       } else {
@@ -339,10 +342,10 @@ __device__ __forceinline__ void store_groups(const GemmArgs& a, const GemmSeg& s
   for (int g = 0; g < G; g++) {
     h1* out = static_cast<h1*>(sg.out) + o[g];
     if constexpr (VEC) {
-      h8 v;
+      h8_any v;
 #pragma unroll
       for (int i = 0; i < 8; i++) v[i] = y[8 * g + i];
-      *reinterpret_cast<h8*>(out) = v;
+      *reinterpret_cast<h8_any*>(out) = v;
     } else {
 #pragma unroll
       for (int i = 0; i < 8; i++)
@@ -366,11 +369,6 @@ __device__ __forceinline__ void sums_to_lds(const f16v (&acc)[NJ], float* sums, 
     for (int v = 0; v < 16; v++) p[(8 * (v >> 2) + (v & 3)) * pitch + j * 32] = acc[j][v];
 }
 
-__device__ __forceinline__ bool vec_outputs(const GemmArgs& a, const GemmSeg& sg) {  // rows of outputs and operands, 16 bytes at a time
-  return (sg.N & 7) == 0 && ((reinterpret_cast<uintptr_t>(sg.out) | reinterpret_cast<uintptr_t>(a.res_x) |
-                              reinterpret_cast<uintptr_t>(a.res_r)) & 15) == 0;
-}
-
 __device__ __forceinline__ void read_sums(float (&s)[8], const float* sums) {
 #pragma unroll
   for (int h = 0; h < 2; h++) {
@@ -380,14 +378,26 @@ __device__ __forceinline__ void read_sums(float (&s)[8], const float* sums) {
   }
 }
 
-// Eight sums of row `row` from column `col`, which may lie outside the matrix
-__device__ __forceinline__ void finish_group(const GemmArgs& a, const GemmSeg& sg, const float* sums, bool vec, int row, int col, int M, int N) {
-  if (row >= M || col >= N) return;
+// Eight sums of row `row` from column `col`; nothing if they are not all inside the matrix (finish_ends)
+__device__ __forceinline__ void finish_group(const GemmArgs& a, const GemmSeg& sg, const float* sums, int row, int col, int M, int N) {
+  if (row >= M || col + 8 > N) return;
   float s[8];
   read_sums(s, sums);
   const size_t o[1] = {(size_t)row * N + col};
-  if (vec) store_groups<1>(a, sg, s, o);
-  else store_groups<1, false>(a, sg, s, o, min(8, N - col));
+  store_groups<1>(a, sg, s, o);
+}
+
+// The last outputs of rows that are no whole groups of eight, a row a thread, after those: as a branch of finish_group every pass over the
+// rows went through it.  Whole groups go out 16 bytes a lane at whatever address such rows begin; with one output a lane and instruction,
+// 16 bytes apart from lane to lane, 384 x 768 x 50277 took 74.5 us, so 52.3, 200 rows 44.3 and 31.1, 1024 x 2048 x 16377 81.2 and 71.7.
+__device__ __forceinline__ void finish_ends(const GemmArgs& a, const GemmSeg& sg, const float* sums, int pitch, int rows, int cols,
+                                            int row0, int col0, int M, int N, int t) {
+  const int col = (N - col0) & ~7;
+  if (col0 >= N || col0 + cols <= N || col0 + col == N || t >= rows || row0 + t >= M) return;
+  float s[8];
+  read_sums(s, sums + t * pitch + col);
+  const size_t o[1] = {(size_t)(row0 + t) * N + col0 + col};
+  store_groups<1, false>(a, sg, s, o, N - col0 - col);
 }
 
 // A wave's part of a tile, from row row0 and column col0, through a place in LDS of its own, 32 rows at a time: no barriers, and
@@ -398,7 +408,7 @@ constexpr int wave_sums_bytes(int blocks) { return 32 * sums_pitch(blocks) * 4; 
 template <int MI, int NJ>
 __device__ __forceinline__ void finish_wave(const GemmArgs& a, const GemmSeg& sg, const f16v (&acc)[MI][NJ], float* sums, int row0,
                                             int col0, int M, int N, int lane) {
-  const bool vec = vec_outputs(a, sg), full = vec && row0 + MI * 32 <= M && col0 + NJ * 32 <= N;
+  const bool full = row0 + MI * 32 <= M && col0 + NJ * 32 <= N;
 #pragma unroll
   for (int i = 0; i < MI; i++) {
     sums_to_lds(acc[i], sums, sums_pitch(NJ), lane);
@@ -420,8 +430,9 @@ __device__ __forceinline__ void finish_wave(const GemmArgs& a, const GemmSeg& sg
 #pragma unroll 1
     for (int t = lane; t < 32 * NJ * 4; t += 64) {
       const int row = t / (NJ * 4), col = (t - row * (NJ * 4)) * 8;
-      finish_group(a, sg, sums + row * sums_pitch(NJ) + col, vec, row0 + i * 32 + row, col0 + col, M, N);
+      finish_group(a, sg, sums + row * sums_pitch(NJ) + col, row0 + i * 32 + row, col0 + col, M, N);
     }
+    finish_ends(a, sg, sums, sums_pitch(NJ), 32, NJ * 32, row0 + i * 32, col0, M, N, lane);
   }
 }
 
@@ -430,11 +441,12 @@ template <int ROWS, int THREADS>
 __device__ __forceinline__ void finish_tile(const GemmArgs& a, const GemmSeg& sg, const float* sums, int pitch, int blocks, int m0,
                                             int n0, int M, int N) {
   const int groups = blocks * 4;  // of 8 outputs
-  const bool vec = vec_outputs(a, sg);
   for (int i = threadIdx.x; i < ROWS * groups; i += THREADS) {
     const int row = i / groups, col = (i - row * groups) * 8;
-    finish_group(a, sg, sums + row * pitch + col, vec, m0 + row, n0 + col, M, N);
+    finish_group(a, sg, sums + row * pitch + col, m0 + row, n0 + col, M, N);
   }
+  static_assert(ROWS <= THREADS, "finish_ends");
+  finish_ends(a, sg, sums, pitch, ROWS, blocks * 32, m0, n0, M, N, threadIdx.x);
 }
 
 }  // namespace frhip
