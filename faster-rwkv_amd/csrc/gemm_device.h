@@ -122,6 +122,13 @@ __device__ __forceinline__ void step_barrier() {
   asm volatile("" ::: "memory");
 }
 
+// Between lanes of one wave that pass values through LDS: LDS serves a wave's accesses in their order, this keeps the compiler to it.
+__device__ __forceinline__ void lanes_in_order() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_wave_barrier();
+  asm volatile("" ::: "memory");
+}
+
 // 4 bytes per lane, each lane from its own address (see load_lds_saddr for M0 and the wait counts)
 __device__ __forceinline__ void load_lds_dword(const void* p, unsigned lds) {
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(p), "s"(lds) : "memory");
@@ -411,7 +418,9 @@ __device__ __forceinline__ void finish_wave(const GemmArgs& a, const GemmSeg& sg
   const bool full = row0 + MI * 32 <= M && col0 + NJ * 32 <= N;
 #pragma unroll
   for (int i = 0; i < MI; i++) {
+    if (i > 0) lanes_in_order();  // the rows before have been read
     sums_to_lds(acc[i], sums, sums_pitch(NJ), lane);
+    lanes_in_order();
     if (full) {
 #pragma unroll 1
       for (int t = lane; t < 32 * NJ * 4; t += 128) {

@@ -20,6 +20,26 @@ def test_bare_barriers_stand_between_compiler_fences():
     assert found
 
 
+def _block(text, start):
+    """text[start:] up to the brace that closes the first one"""
+    depth, i = 0, text.index("{", start)
+    while True:
+        depth += {"{": 1, "}": -1}.get(text[i], 0)
+        i += 1
+        if depth == 0:
+            return text[start:i]
+
+
+def test_sums_that_change_lanes_without_a_barrier_stay_in_order():
+    """finish_wave hands sums from lane to lane of one wave: the compiler may move neither the reads ahead of the stores nor the next rows' stores
+    ahead of the reads."""
+    text = re.sub(r"//.*", "", open(os.path.join(CSRC, "gemm_device.h")).read())
+    body = _block(text, text.index("void finish_wave"))
+    lines = [t.strip() for t in body.splitlines() if t.strip()]
+    at = [i for i, t in enumerate(lines) if t.startswith("sums_to_lds(")]
+    assert len(at) == 1 and lines[at[0] - 1].endswith("lanes_in_order();") and lines[at[0] + 1] == "lanes_in_order();"
+
+
 def test_x86_instructions_of_the_host_layer_are_guarded():
     """A host of another architecture compiles the plain forms: intrinsics, their header, target attributes and CPU queries
     stand under `#if defined(__x86_64__)`."""
