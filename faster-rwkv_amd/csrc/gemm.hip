@@ -1135,22 +1135,26 @@ extern "C" int frhip_gemm_route(int T, int K, int nproducts, const int* N, int c
     a.seg[s].N = N[s];
   }
   a.nseg = nproducts;
-  const GemmRoute whole = gemm_route(a, compute_units);
-  const bool split = one_by_one(a, whole, compute_units);
+  if ((size_t)K * 2 * 256 > 0xffffffffull) {  // launch_gemm: gemm_kernel
+    memset(out, 0, sizeof(int) * 4 * nproducts);
+    return 1;
+  }
+  const WholePlan whole = plan_whole(a, compute_units);
   for (int s = 0; s < nproducts; s++) {
-    GemmRoute r = whole;
-    if (split) {
+    WholePlan w = whole;
+    if (whole.separate) {
       GemmArgs one = a;
       one.nseg = 1;
       one.seg[0] = a.seg[s];
-      r = gemm_route(one, compute_units);
+      w = plan_whole(one, compute_units);
     }
-    out[4 * s] = r.rows;
-    out[4 * s + 1] = r.blocks;
-    out[4 * s + 2] = r.rounds;
-    out[4 * s + 3] = r.rows != 0 && r.loader;
+    const bool ring = w.ring.rows != 0;
+    out[4 * s] = ring ? w.ring.rows : w.route.rows;
+    out[4 * s + 1] = ring ? w.ring.a.vw_maxw : w.route.blocks;
+    out[4 * s + 2] = ring ? w.ring.rounds : w.route.rounds;
+    out[4 * s + 3] = ring || w.route.loader;
   }
-  return split ? nproducts : 1;
+  return whole.separate ? nproducts : 1;
 }
 
 static int tile_args(GemmArgs& a, int T, int K, int nproducts, const int* N, int slices, int compute_units, const int* out, const char* what) {

@@ -300,13 +300,12 @@ int frhip_att_seq_v5(int T, int C, int H, const void *x, const void *sx, const f
                      const frhip_weight *ow,
                      void *x_out, void *xx_out, float *s_out, void *workspace, frhip_stream s_);
 
-/* How a launch of `nproducts` (1..4) binary16 products [T][K] x [K][N[i]] would be cut into tiles on a part with that
+/* How a launch of `nproducts` (1..4) binary16 products [T][K] x [K][N[i]] goes out in tiles on a part with that
  * many compute units, without scratch to split it over K: a pure function of the sizes, for tests and measurements.
  * Returns the number of launches (1: all products together; nproducts: one by one) or a negative FRHIP_E*.
- * out[4 i]: rows of a tile of product i's launch (64, 128, 256; 0: fixed 128 x 128 or 64 x 128 tiles, several rounds),
+ * out[4 i]: rows of a tile of product i's launch (64, 128, 256; 0: rows too long for such tiles, fixed ones of 128 x 128 or 64 x 128),
  * out[4 i + 1]: its widest tile in blocks of 32 columns, out[4 i + 2]: its rounds over the compute units,
- * out[4 i + 3]: 1 if a wave of its own loads the tiles.  (Cuts of 64 and 128 rows are what the choice of the kernel for a few
- * rows is measured by; such launches go out with tiles of frhip_gemm_ring_tile.) */
+ * out[4 i + 3]: 1 if waves of their own load the tiles (of 64 and 128 rows always). */
 int frhip_gemm_route(int T, int K, int nproducts, const int *N, int compute_units, int *out);
 /* Whether such a launch (frhip_gemm's and frhip_gemm_act's are of this kind; the seq operators have scratch, see below) goes,
  * instead, to the kernel for a few rows (K split over the waves of a workgroup), and with which tile: out[0], out[1] = blocks

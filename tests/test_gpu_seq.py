@@ -34,7 +34,7 @@ def _rng_per_test(request):
 
 
 def _routes(T, K, *N):
-    """frhip_gemm_route on 256 compute units -> launches, [(rows of a tile, widest tile in blocks of 32 columns, rounds, loader wave)]"""
+    """frhip_gemm_route on 256 compute units -> launches, [(rows of a tile, widest tile in blocks of 32 columns, rounds, loading waves)]"""
     out = (C.c_int * (4 * len(N)))()
     launches = L().frhip_gemm_route(T, K, len(N), (C.c_int * len(N))(*N), 256, out)
     return launches, [tuple(out[4 * i:4 * i + 4]) for i in range(len(N))]
@@ -252,8 +252,8 @@ def test_ffn_seq(T, C_, F_, quant):
     # every product on 256-row tiles whose last strip has 16 rows: sigmoid, relu^2 and the output's epilogue, predicated
     (16400, 320, 256, (1, [(256, 8, 1, 0)] * 2), (256, 4, 1, 0)),
     (2049, 1024, 4096, (1, [(256, 6, 1, 0)] * 2), None),  # ... one row in the last strip, 16 K-steps
-    (3074, 320, 4736, (2, [(64, 4, 1, 1), (256, 8, 1, 0)]), None),  # r and k one by one, on tiles of different heights
-    (12288, 448, 896, (1, [(256, 5, 2, 1)] * 2), (256, 3, 1, 1))])  # whole tiles: the loader wave's form, grouped and alone
+    (1472, 768, 10752, (2, [(64, 3, 1, 1), (256, 8, 1, 0)]), None),  # r and k one by one, on tiles of different heights
+    (8448, 640, 1280, (1, [(256, 4, 2, 1)] * 2), (256, 3, 1, 1))])  # whole tiles: the loader wave's form, grouped and alone
 def test_ffn_seq_on_planned_tiles(T, C_, F_, rk, v):
     """The fused epilogues on 256-row tiles, with rows past the end and without, in groups and one by one.  Bounds as in
     test_ffn_seq."""
@@ -507,7 +507,7 @@ def test_att_seq_v4_in_one_pass_and_in_parts(T, C_, cut):
 
 
 @pytest.mark.parametrize("T,C_,kvr,o", [(16400, 320, (256, 5, 2, 0), (256, 4, 1, 0)),  # predicated epilogues: 16 rows in the last strip
-                                        (4096, 448, (256, 3, 1, 1), (64, 4, 1, 1))])   # whole tiles: the loader wave's form
+                                        (5632, 320, (256, 4, 1, 1), (128, 2, 1, 1))])  # whole tiles: the loader wave's form
 def test_att_seq_v4_on_planned_tiles(T, C_, kvr, o):
     """k, v, r grouped and the residual's epilogue on 256-row tiles.  Bounds as in test_att_seq_v4."""
     assert _routes(T, C_, C_, C_, C_) == (1, [kvr] * 3) and _routes(T, C_, C_) == (1, [o])
