@@ -36,7 +36,7 @@ struct GemmArgs {
   int tile_start[kGemmMaxSeg + 1];  // first N-tile of each segment
   size_t part_off[kGemmMaxSeg + 1]; // split launches: where each segment's [M][N] block starts within a slice of `partial` (floats); [nseg] = all
   // tiles of a width chosen per launch: a segment's are vw_base (the first vw_wide of them vw_base + 1) blocks of 32 columns wide
-  int vw_base[kGemmMaxSeg], vw_wide[kGemmMaxSeg], vw_maxw, vw_ns;
+  int vw_base[kGemmMaxSeg], vw_wide[kGemmMaxSeg], vw_maxw;
   int few_strips;  // gemm_few_kernel: strips of rows
   GemmSeg seg[kGemmMaxSeg];
   // split K (ksplit >= 2; gemm_ring_kernel and gemm_q8_kernel): slice z of ksplit accumulates its K-steps of segment s into

@@ -296,62 +296,33 @@ static void launch_splitk_reduce(hipStream_t st, const GemmArgs& a) {
 // gemm_vw256_kernel below takes the others.
 // ---------------------------------------------------------------------------
 constexpr int kVwMaxW = 8, kVwABytes = 256 * kLdwBK * 2;
-constexpr int kVw256LoaderMaxW = 5;  // three stages of (256 + 160) x 64 halves are 156 KB of the 160 KB
+constexpr int kVwStages = 3, kVw256LoaderMaxW = 5;  // three stages of (256 + 160) x 64 halves are 156 KB of the 160 KB
 
 template <int W>
-__device__ __forceinline__ void vw_loader(const GemmSeg& sg, unsigned char* smem, int stage_bytes, int ns, int m0, int n0,
-                                          int M, int N, int K, int lane) {
+__device__ __forceinline__ void vw_loader(const GemmSeg& sg, unsigned char* smem, int stage_bytes, int m0, int n0, int K, int lane) {
   constexpr int kAInstr = kVwABytes / 1024, kBInstr = 4 * W, kPer = kAInstr + kBInstr;
   static_assert(kPer <= 63, "the wait counter's range");
   const int lr = lane >> 3, ls = (lane & 7) ^ lr;
-  const h1* pa[kAInstr];
-  const h1* pb[kBInstr];
-#pragma unroll
-  for (int b = 0; b < kAInstr; b++) {
-    int row = m0 + b * 8 + lr;
-    row = row < M ? row : M - 1;
-    pa[b] = sg.A + (size_t)row * K + (ls ^ (b & 1)) * 8;
-  }
-#pragma unroll
-  for (int b = 0; b < kBInstr; b++) {
-    int row = n0 + b * 8 + lr;
-    row = row < N ? row : N - 1;
-    pb[b] = reinterpret_cast<const h1*>(sg.B) + (size_t)row * K + (ls ^ (b & 1)) * 8;
-  }
   const int nk = K / kLdwBK;
-  // a tile that lies wholly inside the matrices: rows are 8 K halves apart for every lane, so the address of
+  // the tile lies wholly inside the matrices: rows are 8 K halves apart for every lane, so the address of
   // load b is a uniform base (row group b, this step's k) plus one of two lane offsets
-  const bool full = m0 + 256 <= M && n0 + W * 32 <= N && (size_t)K * 16 + 128 < 0xffffffffull;
   const unsigned voff[2] = {(unsigned)(lr * K * 2 + ls * 16), (unsigned)(lr * K * 2 + (ls ^ 1) * 16)};
   const unsigned char* abase = uniform_ptr(reinterpret_cast<const unsigned char*>(sg.A) + (size_t)m0 * K * 2);
   const unsigned char* bbase = uniform_ptr(reinterpret_cast<const unsigned char*>(sg.B) + (size_t)n0 * K * 2);
   const unsigned lds0 = (unsigned)(size_t)((__attribute__((address_space(3))) unsigned char*)smem);
   const size_t group = (size_t)__builtin_amdgcn_readfirstlane(K) * 16;  // bytes between row groups of 8
   auto issue = [&](int step, int slot) {
-    const int k0 = step * kLdwBK;
-    if (full) {
-      const unsigned st = lds0 + slot * stage_bytes;
-      const unsigned char* ak = abase + (size_t)k0 * 2;
-      const unsigned char* bk = bbase + (size_t)k0 * 2;
+    const unsigned st = lds0 + slot * stage_bytes;
+    const unsigned char* ak = abase + (size_t)step * (kLdwBK * 2);
+    const unsigned char* bk = bbase + (size_t)step * (kLdwBK * 2);
 #pragma unroll
-      for (int b = 0; b < kAInstr; b++) load_lds_saddr(voff[b & 1], ak + b * group, st + b * 1024);
+    for (int b = 0; b < kAInstr; b++) load_lds_saddr(voff[b & 1], ak + b * group, st + b * 1024);
 #pragma unroll
-      for (int b = 0; b < kBInstr; b++) load_lds_saddr(voff[b & 1], bk + b * group, st + kVwABytes + b * 1024);
-      return;
-    }
-    unsigned char* st = smem + slot * stage_bytes;
-#pragma unroll
-    for (int b = 0; b < kAInstr; b++)
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(pa[b] + k0),
-                                       (__attribute__((address_space(3))) void*)(st + b * 1024), 16, 0, 0);
-#pragma unroll
-    for (int b = 0; b < kBInstr; b++)
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(pb[b] + k0),
-                                       (__attribute__((address_space(3))) void*)(st + kVwABytes + b * 1024), 16, 0, 0);
+    for (int b = 0; b < kBInstr; b++) load_lds_saddr(voff[b & 1], bk + b * group, st + kVwABytes + b * 1024);
   };
   issue(0, 0);
   if (nk > 1) issue(1, 1);
-  int slot = 2 % ns;
+  int slot = 2;
   for (int k = 0; k < nk; k++) {
     if (k + 1 < nk)
       __builtin_amdgcn_s_waitcnt(((kPer >> 4) << 14) | 0x0F70 | (kPer & 15));  // vmcnt(kPer): step k has landed
@@ -359,15 +330,15 @@ __device__ __forceinline__ void vw_loader(const GemmSeg& sg, unsigned char* smem
       __builtin_amdgcn_s_waitcnt(0x0F70);
     step_barrier();  // step k may be read; step k-1 has been read by all
     if (k + 2 < nk) {
-      issue(k + 2, slot);          // ns >= 3: not the slot of step k or k+1
-      slot = slot + 1 == ns ? 0 : slot + 1;
+      issue(k + 2, slot);  // not the slot of step k or k+1
+      slot = slot + 1 == kVwStages ? 0 : slot + 1;
     }
   }
 }
 
 template <int NJ>
-__device__ __forceinline__ void vw_mma(const GemmArgs& a, const GemmSeg& sg, const unsigned char* smem, int stage_bytes, int ns,
-                                       int brow0, int m0, int n0, int M, int N, int lane, int wave) {
+__device__ __forceinline__ void vw_mma(const GemmArgs& a, const GemmSeg& sg, const unsigned char* smem, int stage_bytes, int brow0,
+                                       int m0, int n0, int M, int N, int lane, int wave) {
   const int wm = wave >> 1;
   f16v acc[2][NJ];
 #pragma unroll
@@ -381,7 +352,7 @@ __device__ __forceinline__ void vw_mma(const GemmArgs& a, const GemmSeg& sg, con
   for (int k = 0; k < nk; k++) {
     step_barrier();
     const unsigned char* st = smem + slot * stage_bytes;
-    slot = slot + 1 == ns ? 0 : slot + 1;
+    slot = slot + 1 == kVwStages ? 0 : slot + 1;
     // fragments of KG x 16 k are requested together; with eight MFMA waves and the loader a lane has 168
     // registers and holds two of the four k-blocks of a step at a time
     constexpr int KG = 2;
@@ -409,7 +380,8 @@ __device__ __forceinline__ void vw_mma(const GemmArgs& a, const GemmSeg& sg, con
   gemm_epilogue_t<2, NJ, true>(a, sg, acc, m0 + wm * 64, n0 + brow0, M, N, lane);
 }
 
-// Eight MFMA waves of 64 rows x half the width, then the loader: launches of whole tiles of at most kVw256LoaderMaxW blocks.
+// Eight MFMA waves of 64 rows x half the width, then the loader: launches of whole tiles of at most kVw256LoaderMaxW blocks,
+// of rows of at most 8 million elements (plan_vw).
 __global__ __launch_bounds__(576) void gemm_vw_kernel(GemmArgs a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char gemm_smem[];
   int bx, by;
@@ -426,13 +398,13 @@ __global__ __launch_bounds__(576) void gemm_vw_kernel(GemmArgs a) {
   const int M = a.M, K = a.K, N = sg.N;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int stage_bytes = kVwABytes + a.vw_maxw * 4096, ns = a.vw_ns;
+  const int stage_bytes = kVwABytes + a.vw_maxw * 4096;
   if (wave == 8) {
     switch (width) {
-      case 2: vw_loader<2>(sg, gemm_smem, stage_bytes, ns, m0, n0, M, N, K, lane); break;
-      case 3: vw_loader<3>(sg, gemm_smem, stage_bytes, ns, m0, n0, M, N, K, lane); break;
-      case 4: vw_loader<4>(sg, gemm_smem, stage_bytes, ns, m0, n0, M, N, K, lane); break;
-      default: vw_loader<kVw256LoaderMaxW>(sg, gemm_smem, stage_bytes, ns, m0, n0, M, N, K, lane); break;
+      case 2: vw_loader<2>(sg, gemm_smem, stage_bytes, m0, n0, K, lane); break;
+      case 3: vw_loader<3>(sg, gemm_smem, stage_bytes, m0, n0, K, lane); break;
+      case 4: vw_loader<4>(sg, gemm_smem, stage_bytes, m0, n0, K, lane); break;
+      default: vw_loader<kVw256LoaderMaxW>(sg, gemm_smem, stage_bytes, m0, n0, K, lane); break;
     }
     return;
   }
@@ -441,9 +413,9 @@ __global__ __launch_bounds__(576) void gemm_vw_kernel(GemmArgs a) {
   const int nj = wn ? width - nj0 : nj0;
   const int brow0 = wn ? nj0 * 32 : 0;
   switch (nj) {
-    case 1: vw_mma<1>(a, sg, gemm_smem, stage_bytes, ns, brow0, m0, n0, M, N, lane, wave); break;
-    case 2: vw_mma<2>(a, sg, gemm_smem, stage_bytes, ns, brow0, m0, n0, M, N, lane, wave); break;
-    default: vw_mma<3>(a, sg, gemm_smem, stage_bytes, ns, brow0, m0, n0, M, N, lane, wave); break;
+    case 1: vw_mma<1>(a, sg, gemm_smem, stage_bytes, brow0, m0, n0, M, N, lane, wave); break;
+    case 2: vw_mma<2>(a, sg, gemm_smem, stage_bytes, brow0, m0, n0, M, N, lane, wave); break;
+    default: vw_mma<3>(a, sg, gemm_smem, stage_bytes, brow0, m0, n0, M, N, lane, wave); break;
   }
 }
 
@@ -463,6 +435,8 @@ __global__ __launch_bounds__(576) void gemm_vw_kernel(GemmArgs a) {
 // 4099 x 2048 x 10240: 229 -> 172 us, against the fixed 128 x 128 tiles both launches had before (in turn on one part).
 // ---------------------------------------------------------------------------
 constexpr int kVw256Threads = 512;
+static_assert(kVwStages * (kVwABytes + kVw256LoaderMaxW * 4096) <= 160 * 1024 && 2 * (kVwABytes + kVwMaxW * 4096) <= 160 * 1024 &&
+                  8 * wave_sums_bytes((kVwMaxW + 1) / 2) <= 160 * 1024, "LDS of a compute unit");
 
 template <int NJ>
 __device__ __forceinline__ void vw256_body(const GemmArgs& a, const GemmSeg& sg, unsigned char* smem, int width, int brow0,
@@ -628,7 +602,7 @@ bool deal_tiles(GemmArgs& a, int P) {
   return true;
 }
 
-// Cuts the launch into tiles of bm rows (128 or 256): the fewest rounds over `cus` compute units whose widest tile
+// Cuts the launch into tiles of bm rows (256, or 128 for the price alone): the fewest rounds over `cus` compute units whose widest tile
 // fits.  r.rows stays 0 if it is too small for tiles of at least bm x 96, or too ragged.
 static GemmRoute plan_vw(const GemmArgs& args, int bm, int cus) {
   GemmRoute r;
@@ -637,7 +611,6 @@ static GemmRoute plan_vw(const GemmArgs& args, int bm, int cus) {
   // gemm_vw256_kernel addresses the 256 rows of a tile with 32-bit byte offsets
   if (bm == 256 && (size_t)a.K * 2 * 256 > 0xffffffffull) return r;
   const int mt = (a.M + bm - 1) / bm;
-  const int abytes = bm * kLdwBK * 2;
   int total = 0;
   for (int s = 0; s < a.nseg; s++) total += (a.seg[s].N + 31) / 32;
   // From the fewest rounds that tiles of the largest width allow; it ends at tiles of one block at the latest.  (With a
@@ -650,7 +623,6 @@ static GemmRoute plan_vw(const GemmArgs& args, int bm, int cus) {
     for (int s = 0; s < a.nseg; s++) minw = a.vw_base[s] < minw ? a.vw_base[s] : minw;
     if (maxw > kVwMaxW) continue;
     if (minw < 2 || maxw < 3) return r;
-    const size_t stage = abytes + (size_t)maxw * 4096;
     if (bm == 256) {
       // Whole tiles of up to 160 columns: the loader wave's form, whose loads are two steps ahead.  All 256 compute
       // units multiply real data then and the clock is the lowest, which costs it less: 512 x 5120 x 20480 101 us
@@ -658,13 +630,11 @@ static GemmRoute plan_vw(const GemmArgs& args, int bm, int cus) {
       // empty the other form is the faster one (1793 x 5120 x 5120: 101 against 119): its edge tiles load like whole ones.
       r.loader = a.M % 256 == 0 && maxw <= kVw256LoaderMaxW;
       for (int s = 0; s < a.nseg; s++) r.loader = r.loader && a.seg[s].N % 32 == 0;
+      r.lds = (r.loader ? kVwStages : 2) * (size_t)(kVwABytes + maxw * 4096);
+      const size_t sums = 8 * (size_t)wave_sums_bytes((maxw + 1) / 2);  // the epilogue's place (finish_wave)
+      if (r.lds < sums) r.lds = sums;
+      r.grid = dim3(tiles, mt);
     }
-    a.vw_ns = !r.loader ? 2 : stage * 4 <= 160 * 1024 ? 4 : 3;
-    if (stage * a.vw_ns > 160 * 1024) return r;
-    r.lds = stage * a.vw_ns;
-    const size_t sums = (size_t)(bm / 32) * wave_sums_bytes((maxw + 1) / 2);  // the epilogue's place (finish_wave)
-    if (r.lds < sums) r.lds = sums;
-    r.grid = dim3(tiles, mt);
     r.blocks = maxw;
     r.rounds = (int)rounds;
     r.us = bm == 128 ? us_128(r.rounds, a.K / 2048.0, maxw)

@@ -100,8 +100,7 @@ __device__ __forceinline__ void silu_batch(const V& c, h1 (&y)[W], uint32_t live
 // needs scalar instructions only.  `lds` is the destination's LDS byte address (lane l writes 16 bytes
 // at lds + 16 l); the wait counts are the caller's business, as with the builtin.
 // M0 is written here without the compiler knowing (it refuses m0 in a clobber list: a reserved register).  That is safe
-// as used: a workgroup issues either these loads or the builtin's (a tile lies wholly inside the matrices or it does not),
-// never both, so no value the compiler keeps in M0 for the builtin is ever live across this statement.
+// as used: no kernel issues the builtin's loads besides, so the compiler keeps no value in M0 across this statement.
 __device__ __forceinline__ void load_lds_saddr(unsigned voff, const void* sbase, unsigned lds) {
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "s"(lds) : "memory");
 }

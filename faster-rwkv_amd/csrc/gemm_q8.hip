@@ -246,13 +246,11 @@ __global__ __launch_bounds__(64 * (4 + kQ8Producers)) void gemm_q8_kernel(GemmAr
   const int nk = kper + (kz < krem ? 1 : 0), kbase = (kz * kper + (kz < krem ? kz : krem)) * kLdwBK;
   if (wave >= 4) {
     const int p = wave - 4;
-    constexpr int kMost = (2 * q8_max_blocks(BM) + kQ8Producers - 1) / kQ8Producers;
+    static_assert(2 * q8_max_blocks(BM) <= 2 * kQ8Producers, "a producer has at most two blocks of 16 columns");
     switch (p < 2 * width ? (2 * width - p + kQ8Producers - 1) / kQ8Producers : 0) {
       case 0: q8_producer<BM, 0>(sg, q8_smem, a.vw_maxw, p, m0, n0, a.M, a.K, kbase, nk, lane); break;
       case 1: q8_producer<BM, 1>(sg, q8_smem, a.vw_maxw, p, m0, n0, a.M, a.K, kbase, nk, lane); break;
-      case 2: q8_producer<BM, 2>(sg, q8_smem, a.vw_maxw, p, m0, n0, a.M, a.K, kbase, nk, lane); break;
-      case 3: q8_producer<BM, kMost < 3 ? kMost : 3>(sg, q8_smem, a.vw_maxw, p, m0, n0, a.M, a.K, kbase, nk, lane); break;
-      default: q8_producer<BM, kMost>(sg, q8_smem, a.vw_maxw, p, m0, n0, a.M, a.K, kbase, nk, lane); break;
+      default: q8_producer<BM, 2>(sg, q8_smem, a.vw_maxw, p, m0, n0, a.M, a.K, kbase, nk, lane); break;
     }
   } else {
     const int wm = wave >> 1, nj0 = (width + 1) >> 1, nj = (wave & 1) ? width - nj0 : nj0, brow0 = (wave & 1) ? nj0 * 32 : 0;
