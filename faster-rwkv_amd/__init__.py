@@ -109,6 +109,7 @@ _SIGS = {
     "frhip_gemm_q8_tile": (_i, [_i, _i, _i, _vp, _i, _i, _vp]),
     "frhip_gemm_few_tile": (_i, [_i, _i, _i, _vp, _i, _vp]),
     "frhip_seq_gemm_form": (_i, [_i, _i, _i, _vp, _i, _i, _vp]),
+    "frhip_seq_codes_way": (_i, [_i, _i, _i, _vp, _i, _i, _vp]),
     "frhip_copy_probe": (_i, [_vp, _vp, _sz, _vp]),
     "frhip_read_probe": (_i, [_vp, _sz, _vp, _vp]),
     "frhip_mfma_probe": (_i, [_i, _i, _vp, _vp, _vp, _vp]),

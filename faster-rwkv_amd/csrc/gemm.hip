@@ -902,13 +902,17 @@ static FewPlan few_plan(const GemmArgs& a, size_t partial_stride, int max_split,
 // x 4096 142 / 162, 1024 x 5120 x (5120 + 20480) 331 / 365; 384 x 768 x (768 + 3072) 18.1 / 13.3, 1024 x 768 x 768 10.0 / 9.2.  What is
 // chosen with these figures, the 1.12 among them, is 0.7 % slower than the quicker way on average; with 2 us, 5 TB/s and 1 it was 2.5 %.
 // (Prompts of 1024 tokens of the 1.5B shape 6479 -> 6112 us, of 700 of the 7B RWKV-5.2 width 1593 -> 1508, two layers of it.)
-// *taken stays false, and nothing is launched, where expanding is expected to be quicker.
-static int launch_codes(GemmArgs& a, hipStream_t st, const char* what, void* dq, float* partial, size_t partial_stride, int max_split,
-                        float* few_rows, size_t few_rows_floats, bool* taken) {
-  if (!q8_takes(a)) return 0;
-  const int cus = compute_units(), ksteps = a.K / kLdwBK;
+struct CodesPlan {
+  int way = FRHIP_CODES_EXPANDED;  // or FRHIP_CODES_TILES: q, FRHIP_CODES_ONE_BY_ONE: a launch per product, each with a plan of its own
+  TilePlan q;
+};
+// dq: with scratch for the expanded codes.  max_split, few_rows_floats: 0 without scratch for slices of that kind.
+static CodesPlan plan_codes(const GemmArgs& a, bool dq, float* partial, size_t partial_stride, int max_split, float* few_rows,
+                            size_t few_rows_floats, int cus) {
+  CodesPlan c;
+  const int ksteps = a.K / kLdwBK;
   GemmArgs b = a;
-  if (few_rows && ksteps >= 4) {
+  if (few_rows_floats && ksteps >= 4) {
     if (const int S = few_rows_slices(a, few_rows_floats, cus)) {
       split_over(b, S, few_rows);
     } else if (few_rows_one_by_one(a, cus)) {
@@ -924,18 +928,12 @@ static int launch_codes(GemmArgs& a, hipStream_t st, const char* what, void* dq,
       // (not where a member could be one of gemm_few_kernel: its binary16 image would be)
       if (S >= 2 && a.tiled_sums) split_over(b, S, few_rows);
       if (b.ksplit < 2 || b.ksplit * b.partial_stride > few_rows_floats) {
-        *taken = true;
-        for (int s = 0; s < a.nseg; s++) {
-          GemmArgs one = a;
-          one.nseg = 1;
-          one.seg[0] = a.seg[s];
-          if (int rc = launch_gemm(one, true, st, what, dq, nullptr, 0, 0, few_rows, few_rows_floats)) return rc;
-        }
-        return 0;
+        c.way = FRHIP_CODES_ONE_BY_ONE;
+        return c;
       }
     }
   }
-  if (b.ksplit < 2 && partial)
+  if (b.ksplit < 2 && max_split)
     if (const int S = long_k_slices(a, partial_stride, max_split, cus)) {
       split_over(b, S, partial);
       b.partial_stride = partial_stride;
@@ -947,19 +945,38 @@ static int launch_codes(GemmArgs& a, hipStream_t st, const char* what, void* dq,
       GemmArgs one = a;
       one.nseg = 1;
       one.seg[0] = a.seg[s];
-      if (few_plan(one, 0, 0, 0, cus).mt) return 0;
+      if (few_plan(one, 0, 0, 0, cus).mt) return c;
     }
-  const TilePlan q = plan_q8(b, cus);
-  if (!q.rows) return 0;
+  c.q = plan_q8(b, cus);
+  if (!c.q.rows) return c;
   if (dq) {
     double weights = 0;
     for (int s = 0; s < a.nseg; s++) weights += (double)a.seg[s].N * a.K;
-    if (q.us * 1.12 > 5.5 + weights * 3 / 6.3e6 + (b.ksplit < 2 ? w.us : plan_ring(b, cus).us)) return 0;
+    if (c.q.us * 1.12 > 5.5 + weights * 3 / 6.3e6 + (b.ksplit < 2 ? w.us : plan_ring(b, cus).us)) return c;
   }
+  c.way = FRHIP_CODES_TILES;
+  return c;
+}
+
+// *taken stays false, and nothing is launched, where the codes are to be expanded.
+static int launch_codes(GemmArgs& a, hipStream_t st, const char* what, void* dq, float* partial, size_t partial_stride, int max_split,
+                        float* few_rows, size_t few_rows_floats, bool* taken) {
+  if (!q8_takes(a)) return 0;
+  const CodesPlan c = plan_codes(a, dq != nullptr, partial, partial_stride, partial ? max_split : 0, few_rows, few_rows_floats, compute_units());
+  if (c.way == FRHIP_CODES_EXPANDED) return 0;
   *taken = true;
-  if (int rc = launch_gemm_q8(q, st, what)) return rc;
-  if (b.ksplit < 2) return 0;
-  launch_splitk_reduce(st, q.a);
+  if (c.way == FRHIP_CODES_ONE_BY_ONE) {
+    for (int s = 0; s < a.nseg; s++) {
+      GemmArgs one = a;
+      one.nseg = 1;
+      one.seg[0] = a.seg[s];
+      if (int rc = launch_gemm(one, true, st, what, dq, nullptr, 0, 0, few_rows, few_rows_floats)) return rc;
+    }
+    return 0;
+  }
+  if (int rc = launch_gemm_q8(c.q, st, what)) return rc;
+  if (c.q.a.ksplit < 2) return 0;
+  launch_splitk_reduce(st, c.q.a);
   return check_launch(what);
 }
 
@@ -1183,37 +1200,57 @@ extern "C" int frhip_gemm_few_tile(int T, int K, int nproducts, const int* N, in
   return 0;
 }
 
-extern "C" int frhip_seq_gemm_form(int T, int K, int nproducts, const int* N, int which, int compute_units, int* out) {
-  if (!N || !out) return set_error(FRHIP_EINVAL, "seq_gemm_form: null pointer");
-  if (T <= 0 || K <= 0 || K % 64 != 0 || nproducts < 1 || nproducts > kGemmMaxSeg || compute_units < 1)
-    return set_error(FRHIP_ESHAPE, "seq_gemm_form: no such launch");
+// A launch of the seq operators as frhip_seq_gemm_form and frhip_seq_codes_way are asked about, with the scratch it has
+struct AskedLaunch {
   GemmArgs a;
-  memset(&a, 0, sizeof(a));
-  a.M = T;
-  a.K = K;
-  a.nseg = nproducts;
-  for (int s = 0; s < nproducts; s++) {
-    if (N[s] <= 0) return set_error(FRHIP_ESHAPE, "seq_gemm_form: no such launch");
-    a.seg[s].N = N[s];
+  size_t stride = 0, floats = 0;
+  int max_split = 0;
+  bool v4 = false;
+};
+static int asked_launch(AskedLaunch& q, int T, int K, int nproducts, const int* N, int which, int compute_units, const int* out, const char* what) {
+  if (int rc = tile_args(q.a, T, K, nproducts, N, 1, compute_units, out, what)) return rc;
+  q.v4 = (which & FRHIP_SEQ_V4) != 0;
+  q.floats = T <= kFewRowsMax ? kFewRowsFloats : 0;
+  if (which & FRHIP_SEQ_FFN_VALUE) {
+    q.a.seg[0].epi = G_FFN_OUT;
+    q.stride = (size_t)T * N[0];
+    q.max_split = kSeqMaxSplit;
   }
-  const bool value = (which & FRHIP_SEQ_FFN_VALUE) != 0;
-  if (value) a.seg[0].epi = G_FFN_OUT;
-  const size_t stride = value ? (size_t)T * N[0] : 0, floats = T <= kFewRowsMax ? kFewRowsFloats : 0;
-  const int max_split = value ? kSeqMaxSplit : 0;
+  return 0;
+}
+
+extern "C" int frhip_seq_gemm_form(int T, int K, int nproducts, const int* N, int which, int compute_units, int* out) {
+  AskedLaunch q;
+  if (int rc = asked_launch(q, T, K, nproducts, N, which, compute_units, out, "seq_gemm_form: no such launch")) return rc;
   out[0] = out[1] = 0;
-  if (which & FRHIP_SEQ_V4) {
-    const FewPlan p = few_plan(a, stride, max_split, floats, compute_units);
+  if (q.v4) {
+    const FewPlan p = few_plan(q.a, q.stride, q.max_split, q.floats, compute_units);
     out[0] = p.mt;
     out[1] = p.nt;
     if (p.mt) return FRHIP_FORM_FEW;
   }
-  if (floats && K / kLdwBK >= 4) {
-    out[0] = few_rows_slices(a, floats, compute_units);
+  if (q.floats && K / kLdwBK >= 4) {
+    out[0] = few_rows_slices(q.a, q.floats, compute_units);
     if (out[0]) return FRHIP_FORM_SPLIT;
-    if (few_rows_one_by_one(a, compute_units)) return FRHIP_FORM_ONE_BY_ONE;
+    if (few_rows_one_by_one(q.a, compute_units)) return FRHIP_FORM_ONE_BY_ONE;
   }
-  out[0] = long_k_slices(a, stride, max_split, compute_units);
+  out[0] = long_k_slices(q.a, q.stride, q.max_split, compute_units);
   return out[0] ? FRHIP_FORM_SPLIT : FRHIP_FORM_TILES;
+}
+
+extern "C" int frhip_seq_codes_way(int T, int K, int nproducts, const int* N, int which, int compute_units, int* out) {
+  AskedLaunch q;
+  if (int rc = asked_launch(q, T, K, nproducts, N, which, compute_units, out, "seq_codes_way: no such launch")) return rc;
+  out[0] = out[1] = out[2] = 0;
+  q.a.tiled_sums = !q.v4;
+  if (q.v4 && few_plan(q.a, q.stride, q.max_split, q.floats, compute_units).mt) return FRHIP_CODES_FEW;
+  if (T < kDequantRows || (size_t)K * 2 * 256 > 0xffffffffull) return FRHIP_CODES_EXPANDED;
+  const CodesPlan c = plan_codes(q.a, true, nullptr, q.stride, q.max_split, nullptr, q.floats, compute_units);
+  if (c.way == FRHIP_CODES_TILES) {
+    tell(c.q, out);
+    out[2] = c.q.a.ksplit > 1 ? c.q.a.ksplit : 1;
+  }
+  return c.way;
 }
 
 static_assert(FRHIP_ACT_SIGMOID == G_SIGMOID && FRHIP_ACT_RELU2 == G_RELU2 && FRHIP_ACT_SILU == G_SILU, "activation codes");

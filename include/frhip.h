@@ -329,6 +329,14 @@ int frhip_gemm_q8_tile(int T, int K, int nproducts, const int *N, int slices, in
 #define FRHIP_FORM_SPLIT 2
 #define FRHIP_FORM_ONE_BY_ONE 3
 int frhip_seq_gemm_form(int T, int K, int nproducts, const int *N, int which, int compute_units, int *out);
+/* What such a launch of uint8 weights, of FRHIP_SEQ_EXPAND_ROWS rows and more, does with the codes: returns one of the below or a negative
+ * FRHIP_E*.  FRHIP_CODES_TILES: they are dequantised on their way into LDS, out[0], out[1], out[2] = rows of a tile, its widest in
+ * blocks of 32 columns, slices of K; otherwise 0, 0, 0. */
+#define FRHIP_CODES_EXPANDED 0   /* to binary16, ahead of the product */
+#define FRHIP_CODES_TILES 1
+#define FRHIP_CODES_ONE_BY_ONE 2 /* a launch per product, each with an answer of its own */
+#define FRHIP_CODES_FEW 3        /* FRHIP_FORM_FEW, which dequantises in registers */
+int frhip_seq_codes_way(int T, int K, int nproducts, const int *N, int which, int compute_units, int *out);
 
 /* How frhip_att_seq_v4's scan of T steps of C channels is cut on a part with that many compute units.  out[0]: channels of a
  * workgroup, out[1]: workgroups, out[2]: blocks of time one after another, out[3]: chunks of a block, out[4]: steps of a chunk. */

@@ -8,21 +8,69 @@ import pytest
 from hipref import DevBuf, L, dev, fr
 
 
+EXPANDED, TILES, ONE_BY_ONE, FEW = range(4)
+V4, VALUE = 1, 2
+
+
 def tile(T, K, *N, slices=1):
     out = (C.c_int * 3)()
     fr.check(L().frhip_gemm_q8_tile(T, K, len(N), (C.c_int * len(N))(*N), slices, 256, out))
     return tuple(out)
 
 
-# more rows than the kernel for a few rows takes; one to seven K-steps (the producers hold four)
+def few(T, K, N):
+    out = (C.c_int * 2)()
+    fr.check(L().frhip_gemm_few_tile(T, K, 1, (C.c_int * 1)(N), 256, out))
+    return out[0] != 0
+
+
+def way(T, K, *N, which=0):
+    """frhip_seq_codes_way -> way, (rows of a tile, its widest in blocks of 32 columns, slices of K)"""
+    out = (C.c_int * 3)()
+    w = L().frhip_seq_codes_way(T, K, len(N), (C.c_int * len(N))(*N), which, 256, out)
+    assert w >= 0, fr.lib().frhip_error_string()
+    return w, tuple(out)
+
+
+# one to sixteen K-steps (the producers hold four), and not the kernel for a few rows
 CASES = [((64, 2, 1), 513, 64, 64), ((64, 3, 1), 520, 128, 80), ((64, 2, 1), 577, 192, 1600), ((64, 3, 1), 513, 256, 2672),
          ((128, 2, 1), 641, 320, 2608), ((128, 3, 1), 700, 384, 3600), ((128, 4, 1), 641, 448, 5232), ((128, 5, 1), 700, 128, 6416),
-         ((128, 6, 1), 769, 320, 6384), ((128, 6, 2), 1025, 192, 10016)]
+         ((128, 6, 1), 769, 320, 6384), ((128, 6, 2), 1025, 192, 10016), ((64, 4, 1), 385, 64, 3536), ((64, 5, 1), 129, 192, 12400),
+         ((64, 8, 1), 129, 1024, 20560)]
+# RWKV-5's ffn (rows, width, ffn width): what its r,k and its value product do with the codes
+FFN = [((TILES, (64, 4, 1)), (TILES, (64, 2, 33)), 129, 64, 8512), ((TILES, (64, 5, 1)), (TILES, (64, 3, 42)), 129, 192, 12352),
+       ((TILES, (64, 7, 1)), (EXPANDED, (0, 0, 0)), 257, 2240, 8960), ((TILES, (64, 8, 1)), (TILES, (64, 4, 10)), 129, 1024, 19648),
+       ((TILES, (128, 4, 1)), (EXPANDED, (0, 0, 0)), 1024, 768, 3072), ((EXPANDED, (0, 0, 0)), (EXPANDED, (0, 0, 0)), 1030, 2048, 7168)]
 
 
-def test_cases_reach_tiles_of_every_width():
+def test_cases_reach_their_tiles():
     assert [tile(T, K, N) for _, T, K, N in CASES] == [t for t, *_ in CASES]
+    assert not any(few(T, K, N) for _, T, K, N in CASES)
     assert tile(13, 2560, 2560, slices=10)[0] == 64 and tile(300, 2560, 2560, 8960) == (128, 5, 1)
+    assert [(way(T, c, c, f), way(T, f, c, which=VALUE)) for _, _, T, c, f in FFN] == [v[:2] for v in FFN]
+
+
+def test_every_tile_that_launches_of_the_operators_take_is_among_the_cases():
+    """Rows of tiles and widths over models of 256 to 5120 channels; a wave's part of a tile follows from the two."""
+    taken = set()
+
+    def go(T, K, *N, which):
+        w, out = way(T, K, *N, which=which)
+        if w == ONE_BY_ONE:
+            for n in N:
+                go(T, K, n, which=which & V4)
+        elif w == TILES:
+            taken.add(out[:2])
+
+    for T in [4, 13, 40, 64, 65, 100, 129, 150, 193, 257, 300, 361, 513, 641, 777, 1024, 1536, 4099]:
+        for c in range(256, 5184, 64):
+            for f in (4 * c, 7 * c // 128 * 64):
+                for v4 in (V4, 0):
+                    go(T, c, c, f, which=v4)
+                    go(T, f, c, which=v4 + VALUE)
+                    go(T, c, *(c,) * (3 if v4 else 4), which=v4)
+                    go(T, c, c, which=v4)
+    assert taken == {t[:2] for t, *_ in CASES} | {rk[1][:2] for rk, *_ in FFN if rk[0] == TILES}
 
 
 @pytest.mark.parametrize("T,K,N", [(64, 64, (16,)), (64, 64, (32,)), (100, 128, (2048, 24))])  # one block of columns; not a multiple of 16
@@ -81,6 +129,17 @@ def test_activations(act):
 @pytest.mark.parametrize("C_,F_", [(320, 1088), (576, 2000 // 64 * 64), (1024, 3584)])
 def test_ffn_in_slices_and_whole(T, C_, F_):
     """RWKV-5's operator, whose products keep the slices of the binary16 launches: a group, its members one by one, split or whole."""
+    _ffn_gives_the_bits_of_the_images(T, C_, F_)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,C_,F_", [v[2:] for v in FFN])
+def test_groups_on_wide_tiles_and_expanded_codes(T, C_, F_):
+    """Two products on one launch of the wide tiles of 64 rows; codes expanded ahead of one product or of all."""
+    _ffn_gives_the_bits_of_the_images(T, C_, F_)
+
+
+def _ffn_gives_the_bits_of_the_images(T, C_, F_):
     g = np.random.default_rng([T, C_])
     h = lambda a: np.asarray(a, np.float32).astype(np.float16)
     vecs = [dev(a) for a in (h(g.standard_normal((T, C_)) * 2), h(g.standard_normal(C_)), h(1 + 0.1 * g.standard_normal(C_)),

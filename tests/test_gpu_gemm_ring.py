@@ -13,15 +13,48 @@ def tile(T, K, *N, slices=1):
     return tuple(out)
 
 
-# more rows than the kernel for a few rows takes; one to seven K-steps (the ring holds three or four)
+def few(T, K, N):
+    out = (C.c_int * 2)()
+    fr.check(L().frhip_gemm_few_tile(T, K, 1, (C.c_int * 1)(N), 256, out))
+    return out[0] != 0
+
+
+# one to seven K-steps (the ring holds three or four), and not the kernel for a few rows
 CASES = [((64, 1), 513, 64, 20), ((64, 2), 577, 128, 1085), ((64, 3), 513, 256, 2672), ((64, 4), 1000, 192, 2048), ((64, 5), 513, 320, 3792),
          ((64, 6), 529, 384, 5040), ((128, 3), 513, 128, 4624), ((128, 4), 520, 192, 5450), ((128, 5), 700, 384, 6416), ((128, 6), 641, 448, 8000),
-         ((128, 7), 600, 192, 10600), ((128, 8), 513, 448, 12000), ((128, 8), 1537, 128, 9408)]
+         ((128, 7), 600, 192, 10600), ((128, 8), 513, 448, 12000), ((128, 8), 1537, 128, 9408), ((64, 7), 129, 64, 16421), ((64, 8), 129, 192, 20565),
+         ((128, 2), 321, 192, 5429)]
 
 
 def test_cases_reach_their_tiles():
     assert [tile(T, K, N)[:2] for _, T, K, N in CASES] == [t for t, *_ in CASES]
-    assert all(tile(T, K, N)[3] for _, T, K, N in CASES)
+    assert all(tile(T, K, N)[3] for _, T, K, N in CASES) and not any(few(T, K, N) for _, T, K, N in CASES)
+
+
+def test_every_tile_that_launches_of_the_operators_take_is_among_the_cases():
+    """Rows of tiles and widths over models of 256 to 5120 channels; a wave's part of a tile follows from the two."""
+    taken = set()
+
+    def go(T, K, *N, which):
+        out = (C.c_int * 2)()
+        form = L().frhip_seq_gemm_form(T, K, len(N), (C.c_int * len(N))(*N), which, 256, out)
+        if form == 3:  # one by one
+            for n in N:
+                go(T, K, n, which=which & 1)
+        elif form != 1:  # not the kernel for a few rows
+            t = tile(T, K, *N, slices=out[0] if form == 2 else 1)
+            if form == 2 or t[3]:
+                taken.add(t[:2])
+
+    for T in [4, 13, 40, 64, 65, 100, 129, 150, 193, 257, 300, 361, 513, 641, 777, 1024, 1536, 4099]:
+        for c in range(256, 5184, 64):
+            for f in (4 * c, 7 * c // 128 * 64):
+                for v4 in (1, 0):
+                    go(T, c, c, f, which=v4)
+                    go(T, f, c, which=v4 + 2)
+                    go(T, c, *(c,) * (3 if v4 else 4), which=v4)
+                    go(T, c, c, which=v4)
+    assert taken == {t for t, *_ in CASES}
 
 
 @pytest.mark.gpu
