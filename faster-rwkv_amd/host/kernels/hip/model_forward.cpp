@@ -515,10 +515,12 @@ struct SeqHost {
     FRHIP_CHECK(frhip_stream_sync(stream()));
     reading = false;
   }
-  // Room for n values, after whatever the device still does with the old one.
+  // Room for n values, after whatever the device still does with the old one.  It grows by a factor: a new buffer is a pinned allocation,
+  // which prompts that are each a little longer than the one before would otherwise pay every time.
   template <class T>
   void room(T *&p, size_t &cap, size_t n) {
     if (n <= cap) return;
+    n = std::max({n, 2 * cap, static_cast<size_t>(4096)});
     wait();
     if (p) frhip_host_free(p);
     p = nullptr;
