@@ -184,9 +184,10 @@ def test_rows_past_the_end_do_not_slow_an_epilogue(act):
     assert best[777] <= 1.2 * best[1024], best
 
 
-@pytest.mark.parametrize("T,K,N", [(384, 768, 50277), (777, 768, 50277), (1024, 192, 16377)])  # tiles of 128 rows; of 256, the last ones over the edge
-def test_rows_at_any_address_do_not_slow_an_epilogue(T, K, N):
-    """50277 outputs a row (the vocabulary of the 169M model) begin at any even address; 50280 at multiples of 16 bytes.  The bound is between
+@pytest.mark.parametrize("T,K,N,most", [(384, 768, 50277, 1.25), (777, 768, 50277, 1.25),  # tiles of 128 rows; of 256, the last ones over the edge
+                                        (1024, 192, 16377, 1.6)])
+def test_rows_at_any_address_do_not_slow_an_epilogue(T, K, N, most):
+    """50277 outputs a row (the vocabulary of the 169M model) begin at any even address; 50280 at multiples of 16 bytes.  The bounds are between
     what was measured: 1.0 times as long, 1.2 to 1.27 the small one; 1.40, 1.46 and 1.95 where such rows went out one element a lane and instruction."""
     more = -(-N // 8) * 8
     x, w = keep(h(rng.standard_normal((T, K)))), h(rng.standard_normal((K, more)) * 0.02)
@@ -209,7 +210,7 @@ def test_rows_at_any_address_do_not_slow_an_epilogue(T, K, N):
     for e in events:
         fr.check(L().frhip_event_destroy(e))
     print(best)
-    assert best[N] <= 1.3 * best[more], best
+    assert best[N] <= most * best[more], best
 
 
 def test_gemm_rejects_bad_shapes():
@@ -264,8 +265,8 @@ def test_ffn_seq_on_planned_tiles(T, C_, F_, rk, v):
 
 @pytest.mark.parametrize("T,C_,F_", [(4, 512, 1792), (64, 512, 2048), (65, 768, 3072), (128, 2048, 8192), (129, 512, 1792)])
 def test_ffn_seq_uint8_dequantised_in_the_product(T, C_, F_):
-    """Up to 64 rows the split product dequantises by itself; from 65 rows on the codes are expanded first.  Bounds as in
-    test_ffn_seq."""
+    """uint8 weights of RWKV-5's operator, up to 129 rows: in slices of K and whole, a group on one launch and its members one by one.
+    Bounds as in test_ffn_seq."""
     test_ffn_seq(T, C_, F_, True)
 
 
@@ -273,8 +274,8 @@ def test_ffn_seq_uint8_dequantised_in_the_product(T, C_, F_):
 @pytest.mark.parametrize("T", [4, 13, 63, 64, 65, 129])
 @pytest.mark.parametrize("C_,F_", [(576, 1856), (2560, 8960)])
 def test_ffn_seq_uint8_gives_the_bits_of_its_binary16_image(T, C_, F_):
-    """A uint8 weight and its dequantised image as a binary16 weight: the same slices of K, so the same bits, whether the
-    product dequantises (up to 64 rows) or the codes are expanded first."""
+    """A uint8 weight, whose codes these products dequantise on their way into LDS, and its dequantised image as a binary16 weight: the
+    same slices of K, so the same bits.  (Codes expanded ahead of the product: test_gpu_gemm_q8.py.)"""
     x, sx = h(rng.standard_normal((T, C_)) * 2), h(rng.standard_normal(C_))
     vecs = [keep(a) for a in (x, sx, *_common(C_), h(rng.uniform(0, 1, C_)), h(rng.uniform(0, 1, C_)))]
     coded = [make_weight(h(rng.standard_normal(s) * 0.02), True)[0] for s in ((C_, F_), (F_, C_), (C_, C_))]
@@ -290,6 +291,31 @@ def test_ffn_seq_uint8_gives_the_bits_of_its_binary16_image(T, C_, F_):
         fr.check(L().frhip_ffn_seq(T, C_, F_, *[a.ptr for a in vecs], kw, vw, rw, x_out.ptr, xx_out.ptr, 0, ws.ptr, None))
         outs.append(x_out.numpy())
     assert np.array_equal(outs[0].view(np.uint16), outs[1].view(np.uint16))
+
+
+# Of the value product: slices of K, the tile of the whole binary16 product, and that of the codes (0: expanded ahead of it)
+@pytest.mark.parametrize("T,C_,F_,slices,tile,coded", [
+    (13, 512, 1792, 7, None, 64), (129, 576, 1856, 7, None, 64),     # the reduction launch
+    (700, 1024, 256, 0, (64, 2), 64), (777, 3072, 128, 0, (128, 3), 128),  # the last strip over the edge
+    (16400, 320, 256, 0, (256, 4), 0), (8448, 640, 1280, 0, (256, 3), 0)])  # tiles of 256 rows, over the edge and whole
+@pytest.mark.parametrize("quant", [False, True])
+def test_ffn_seq_rows_at_any_address(T, C_, F_, slices, tile, coded, quant):
+    """The residual epilogue reads x and writes x_out wherever they begin (2 and 6 bytes past a multiple of 16): the bits of aligned ones."""
+    out = (C.c_int * 3)()
+    assert L().frhip_seq_gemm_form(T, F_, 1, (C.c_int * 1)(C_), 2, 256, out) == (2 if slices else 0) and out[0] == slices
+    assert slices or _routes(T, F_, C_)[1][0][:2] == tile
+    assert L().frhip_seq_codes_way(T, F_, 1, (C.c_int * 1)(C_), 2, 256, out) == (1 if coded else 0) and out[0] == coded
+    g = np.random.default_rng([T, C_])
+    x = h(g.standard_normal((T, C_)) * 2)
+    vecs = [keep(v) for v in (h(g.standard_normal(C_)), h(1 + 0.1 * g.standard_normal(C_)), h(0.1 * g.standard_normal(C_)), h(g.uniform(0, 1, C_)), h(g.uniform(0, 1, C_)))]
+    kw, vw, rw = [make_weight(h(g.standard_normal(s) * 0.02), quant)[0] for s in ((C_, F_), (F_, C_), (C_, C_))]
+    outs = []
+    for at_x, at_out in ((0, 0), (1, 3)):  # elements
+        xs = keep(np.concatenate([np.zeros(at_x, np.float16), x.reshape(-1)]))
+        out, xx, ws = DevBuf.empty(T * C_ + 8, np.float16), DevBuf.empty(C_, np.float16), DevBuf(L().frhip_seq_workspace_bytes(T, C_, F_))
+        fr.check(L().frhip_ffn_seq(T, C_, F_, xs.ptr + 2 * at_x, *[v.ptr for v in vecs], kw.ref, vw.ref, rw.ref, out.ptr + 2 * at_out, xx.ptr, 0, ws.ptr, None))
+        outs.append((out.numpy()[at_out:at_out + T * C_].view(np.uint16), xx.numpy().view(np.uint16)))
+    assert all(np.array_equal(a, b) for a, b in zip(*outs))
 
 
 @pytest.mark.parametrize("T", [4, 13, 64, 65])
