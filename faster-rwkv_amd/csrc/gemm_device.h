@@ -1,4 +1,4 @@
-// Device helpers shared by the MFMA product kernels (gemm.hip, gemm_few.hip).
+// Device helpers shared by the MFMA product kernels (gemm.hip, gemm_few.hip, gemm_ring.hip, gemm_q8.hip).
 #pragma once
 
 #include "gemm.h"

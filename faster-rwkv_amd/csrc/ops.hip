@@ -687,12 +687,12 @@ int frhip_scalar_div_f16(void* x, float divisor, size_t n, frhip_stream s) {
   return check_launch("scalar_div");
 }
 
-int frhip_gather_rows(const void* table, const int32_t* ids_dev, void* out, int n_ids, int row_bytes, frhip_stream s) {
-  if (!table || !ids_dev || !out) return set_error(FRHIP_EINVAL, "gather: null pointer");
+int frhip_gather_rows(const void* table, const int32_t* ids, void* out, int n_ids, int row_bytes, frhip_stream s) {
+  if (!table || !ids || !out) return set_error(FRHIP_EINVAL, "gather: null pointer");
   if (n_ids < 0 || row_bytes <= 0 || row_bytes % 16 != 0) return set_error(FRHIP_ESHAPE, "gather: row_bytes must be a multiple of 16");
   if (n_ids == 0) return 0;
   hipLaunchKernelGGL(gather_rows_kernel, dim3(n_ids), dim3(256), 0, static_cast<hipStream_t>(s),
-                     (const unsigned char*)table, ids_dev, (unsigned char*)out, row_bytes);
+                     (const unsigned char*)table, ids, (unsigned char*)out, row_bytes);
   return check_launch("gather_rows");
 }
 

@@ -129,8 +129,9 @@ int frhip_fill_many(int n, void *const *dst, const int *dtype, const float *valu
 int frhip_copy_many(int n, void *const *dst, const void *const *src, const size_t *bytes, frhip_stream s);
 /* scalar_div_: kernels/cuda/element_wise.cu:8-19 (binary16, divisor rounded to half first). */
 int frhip_scalar_div_f16(void *x, float divisor, size_t n, frhip_stream s);
-/* vgather of embedding rows: kernels/default/gather_ops.cpp:46-89.  table [V][C]; ids on the device. */
-int frhip_gather_rows(const void *table, const int32_t *ids_dev, void *out, int n_ids, int row_bytes, frhip_stream s);
+/* vgather of embedding rows: kernels/default/gather_ops.cpp:46-89.  table [V][C]; ids on the device,
+ * or in pinned host memory (frhip_host_malloc) that stays as it is until the gather has run. */
+int frhip_gather_rows(const void *table, const int32_t *ids, void *out, int n_ids, int row_bytes, frhip_stream s);
 
 /* slice: kernels/cuda/slice.cu:38-136.  dst[i] = src[start + i * interval] per dimension, ndim 1..4;
  * the caller has resolved negative / whole-dimension ranges (slice.cu:54-66) into start, interval and
