@@ -1,6 +1,8 @@
 // Argument structures of the MFMA GEMM shared by gemm.hip and seq.hip.
 #pragma once
 
+#include <cstddef>
+
 #include "device_utils.h"
 #include "frhip_internal.h"
 
@@ -38,7 +40,10 @@ struct GemmArgs {
   // tiles of a width chosen per launch: a segment's are vw_base (the first vw_wide of them vw_base + 1) blocks of 32 columns wide
   int vw_base[kGemmMaxSeg], vw_wide[kGemmMaxSeg], vw_maxw;
   int few_strips;  // gemm_few_kernel: strips of rows
-  GemmSeg seg[kGemmMaxSeg];
+  // A segment, and ksplit with all behind it, are one 64-byte line each of the kernel's arguments, counted from their beginning.  Over two,
+  // 8 bytes earlier, a launch of gemm_ring_kernel took 0.2 us longer (1024 x 8192 x 2048 in two slices 37.84 -> 38.05, 77 rows in
+  // slices 11.95 -> 12.2), the reduction launch of 1024 rows 0.25 (6.04 -> 6.28).
+  alignas(16) GemmSeg seg[kGemmMaxSeg];
   // split K (ksplit >= 2; gemm_ring_kernel and gemm_q8_kernel): slice z of ksplit accumulates its K-steps of segment s into
   // partial + z * partial_stride + part_off[s] as fp32 [M][N]; gemm_splitk_reduce_kernel adds the slices and applies the epilogues
   int ksplit;
@@ -48,6 +53,7 @@ struct GemmArgs {
   const h1* res_r;  // [M][N] G_FFN_OUT
   int div2;
 };
+static_assert(sizeof(GemmSeg) == 64 && offsetof(GemmArgs, seg) % 64 == 0 && offsetof(GemmArgs, ksplit) / 64 == offsetof(GemmArgs, div2) / 64, "one line each");
 
 // dq: optional scratch, 2 bytes per weight of the launch.  With it, uint8 weights of a launch with at least
 // kDequantRows rows are expanded once to binary16 (the standalone dequantisation: the same bits as the
